@@ -1,0 +1,47 @@
+"""Kernels at the sizes where their tiling can go wrong (edges of blocks,
+strips and tiles, remainders, the smallest and largest of a range), against
+the oracle."""
+import numpy as np
+import pytest
+
+from fake_spectra_amd import spectra_priv as SP, synth
+from fake_spectra_amd.lines import HI_1215
+from gpu_util import assert_colden_close, assert_tau_close
+
+pytestmark = pytest.mark.gpu
+
+
+def small_gas(n, box, nlos, nbins, kernel, hfrac, seed=3, line=HI_1215, compute_tau=True):
+    """_Particle_Interpolate arguments for n particles of support about
+    hfrac * box, two of them at one position, mixed axes."""
+    rng = np.random.default_rng(seed)
+    pos = (rng.random((n, 3)) * box).astype(np.float32)
+    np.minimum(pos, np.nextafter(np.float32(box), np.float32(0)), out=pos)
+    if n > 3:
+        pos[n // 2] = pos[1]
+    h = (hfrac * box * np.exp(0.2 * rng.standard_normal(n))).astype(np.float32)
+    temp = (1e4 * np.exp(rng.standard_normal(n))).astype(np.float32)
+    vel = (30.0 * rng.standard_normal((n, 3))).astype(np.float32)
+    dens = np.exp(25.0 + rng.standard_normal(n)).astype(np.float32)
+    axis = (1 + np.arange(nlos) % 3).astype(np.int32)
+    cofm = rng.random((nlos, 3)) * box
+    c = synth.Cosmology()
+    none = np.zeros(1, dtype=np.float32)
+    return (int(compute_tau), nbins, kernel, float(box), c.velfac(), c.atime, line.lambda_cm, line.gamma, line.fosc,
+            line.amumass, 1e-7, pos, vel if compute_tau else none, dens, temp if compute_tau else none, h, axis, cofm)
+
+
+# boxes of 2049, 2048, 2047 and 64 grid points 0.1 apart, one point, and rows
+# of more particles than the candidates a block holds (every particle of the
+# 850 of a row lies nearer than a block's stretch of points is long)
+@pytest.mark.parametrize("box,n,nlos,hfrac", [(204.95, 400, 7, 0.3), (204.85, 400, 7, 0.3), (204.75, 300, 5, 0.3),
+                                              (6.45, 60, 6, 0.4), (0.15, 5, 3, 0.4), (50.0, 3000, 4, 0.3),
+                                              (1000.0, 3, 9, 0.4), (2000.0, 1500, 3, 0.15)])
+def test_mesh_cells(oracle, box, n, nlos, hfrac):
+    """The column density of kernel 2 is the overlap of a pixel with the
+    particle's segment, so it pins the cells' ends."""
+    for ct in (False, True):
+        args = small_gas(n, box, nlos, 40, 2, hfrac, compute_tau=ct)
+        ref = oracle.interpolate(*args)
+        got = SP._Particle_Interpolate(*args)
+        (assert_tau_close if ct else assert_colden_close)(got, ref, "mesh %g %d" % (box, n))
