@@ -45,3 +45,17 @@ def test_mesh_cells(oracle, box, n, nlos, hfrac):
         ref = oracle.interpolate(*args)
         got = SP._Particle_Interpolate(*args)
         (assert_tau_close if ct else assert_colden_close)(got, ref, "mesh %g %d" % (box, n))
+
+
+# mask words of 64 particles with every remainder kind, no, few and nearly all
+# particles near a sightline, particles outside the box
+@pytest.mark.parametrize("n,nlos,hfrac", [(1, 1, 0.4), (63, 2, 0.05), (64, 3, 0.3), (65, 1, 1e-4), (257, 700, 0.03),
+                                          (4097, 50, 0.004), (1000, 1, 0.01)])
+def test_near_lines(oracle, n, nlos, hfrac):
+    args = small_gas(n, 1000.0, nlos, 8, 1, hfrac)
+    box, pos, h, axis, cofm = args[3], args[11], args[15], args[16], args[17]
+    if n > 64:
+        pos[5] = [-3.0, 1001.0, 500.0]
+    _, parts, _ = oracle.near_particles(box, pos, h, axis, cofm)
+    got = SP._near_lines(box, pos, h, axis, cofm)
+    assert got.dtype == np.int32 and np.array_equal(got, np.unique(parts))
