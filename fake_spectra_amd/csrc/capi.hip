@@ -71,7 +71,7 @@ static long long tune_key(int nbins, int nlines, int kernel)
     return ((long long)nbins << 20) ^ ((long long)nlines << 4) ^ kernel;
 }
 
-// Work items for K lines in the plan's heaviest-first order; a sightline
+// Work items for K lines (or parts of the fields) in the plan's heaviest-first order; a sightline
 // with more than `chunk` pairs is split into non-direct items.  Cached.
 static int item_set(fsamd_plan *P, int K, long long chunk, fsamd_plan::ItemSet **out)
 {
@@ -294,10 +294,13 @@ static int run_deposit(bool tau, fsamd_plan *P, int nbins, int kernel, double ve
         A.stats = g_stats_on ? P->stats.as<long long>() : nullptr;
         A.npairs = P->npairs;
         A.win = rec ? P->win.as<int>() + (size_t)k0 * 2 * P->npairs : nullptr;
+        // column density: one item takes several fields of its sightline
+        A.fields = tau ? 1 : lds ? colden_fields(K, nbins) : K;
+        const int parts = tau ? K : (K + A.fields - 1) / A.fields;
         fsamd_plan::ItemSet *set = nullptr;
-        if (capturing && !find_item_set(P, K, chunk_key))
+        if (capturing && !find_item_set(P, parts, chunk_key))
             return fail(FSAMD_ERR_ARG, "run one uncaptured fsamd_tau call before capturing");
-        if ((rc = item_set(P, K, chunk_key, &set))) return rc;
+        if ((rc = item_set(P, parts, chunk_key, &set))) return rc;
         const std::vector<WorkItem> &items = set->host;
         for (int attempt = 0;; ++attempt) {
             A.fix = P->fix.as<Fixup>();
@@ -314,7 +317,8 @@ static int run_deposit(bool tau, fsamd_plan *P, int nbins, int kernel, double ve
             if (!plain) {
                 A.nitems = (int)items.size();
                 if ((rc = launch_fill_i32(A.queue, 0, 1, s))) return rc;
-                const int per_cu = deposit_blocks_per_cu(tau, lds, gsize, effective_waves(lds, g_stats_on, waves), nbins);
+                const int per_cu = deposit_blocks_per_cu(tau, lds, gsize, effective_waves(lds, g_stats_on, waves), nbins,
+                                                         A.fields);
                 const int nblocks = (int)std::min<long long>((long long)per_cu * dev.ncu, A.nitems);
                 if (g_timing_on) FSAMD_HIP(hipEventRecord(P->ev[2], s));
                 if ((rc = launch_deposit(tau, lds, gsize, waves, A, set->buf.as<WorkItem>(), 0, nblocks, 1, s)))

@@ -24,7 +24,10 @@ size_t deposit_static_lds(bool tau, int gsize, int waves);
 size_t adjoint_static_lds(int gsize);
 int launch_deposit(bool tau, bool lds, int gsize, int waves, const DepositArgs &A, const WorkItem *items, int item_base,
                    int nblocks, int use_queue, hipStream_t s);
-int deposit_blocks_per_cu(bool tau, bool lds, int gsize, int waves, int nbins);
+// fields: rows a column-density block holds (1 for tau)
+int deposit_blocks_per_cu(bool tau, bool lds, int gsize, int waves, int nbins, int fields);
+// rows a column-density work item takes of nlines
+int colden_fields(int nlines, int nbins);
 int effective_waves(bool lds, bool stats, int waves);
 int launch_tau_adjoint(int gsize, const DepositArgs &A, const WorkItem *items, int nblocks, hipStream_t s);
 // the FP64 pairs tau_adjoint_kernel listed in A.fix (after it, on the same stream)

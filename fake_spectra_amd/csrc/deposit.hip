@@ -25,7 +25,8 @@
 //    re-evaluated in FP64 so the tail-cut decision matches the reference;
 //    pairs with a damping parameter above kA32Max are evaluated in FP64.
 // Column density (compute_colden, part_int.cpp:53-84 with
-// add_colden_particle, absorption.cpp:167-210) is all FP64, one lane per pair.
+// add_colden_particle, absorption.cpp:167-210) is all FP64, one lane per
+// (pair, pixel).
 #include "fsamd_internal.h"
 #include "plan.h"
 #include "voigt.h"
@@ -41,6 +42,7 @@ __constant__ __attribute__((aligned(16))) float c_gtab[kGTableSize] = FSAMD_G_CO
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
+constexpr int kColThreads = 512;   // column density
 constexpr double kGuard = 2e-5;
 constexpr int kWingTerms = 10;
 
@@ -1592,37 +1594,126 @@ int adjoint_blocks_per_cu(int gsize, int nbins)
 // ---------------------------------------------------------------------------
 // Column density
 
-// absorption.cpp:53-74 (cubic), 76-97 (quintic) / 109-115 (tophat, also the
-// reference's default for any other id, absorption.cpp:136-148)
-__device__ inline double kern_frac(int kernel, double zlow, double zhigh, double smooth, double dr2,
-                                   double zrange)
+// sqrt(x) for 1e-300 < x < 1e300 to about an ulp: the hardware's reciprocal
+// square root, one step of Goldschmidt's iteration and a Newton correction.
+__device__ inline double sqrt_nr(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+
+// Sums over kernel samples of the truncated powers the splines consist of
+// (singleabs.h:17-42): the cubic is 2 ((1-q)+^3 - 4 (1/2-q)+^3) over its norm,
+// the quintic (3-3q)+^5 - 6 (2-3q)+^5 + 15 (1-3q)+^5.  No branch on q.
+template <int kKernel>
+struct ShapeSum {
+    double s1 = 0, s2 = 0, s3 = 0;
+    __device__ inline void add(double q2)
+    {
+        const double q = sqrt_nr(q2);
+        if (kKernel == kCubicSpline) {
+            const double t = fmax(1.0 - q, 0.0), h = fmax(0.5 - q, 0.0);
+            s1 = __builtin_fma(t * t, t, s1);
+            s2 = __builtin_fma(h * h, h, s2);
+        } else {
+            const double t3 = fmax(__builtin_fma(-3.0, q, 3.0), 0.0), t2 = fmax(__builtin_fma(-3.0, q, 2.0), 0.0),
+                         t1 = fmax(__builtin_fma(-3.0, q, 1.0), 0.0);
+            const double p3 = t3 * t3, p2 = t2 * t2, p1 = t1 * t1;
+            s1 = __builtin_fma(p3 * p3, t3, s1);
+            s2 = __builtin_fma(p2 * p2, t2, s2);
+            s3 = __builtin_fma(p1 * p1, t1, s3);
+        }
+    }
+    __device__ inline void halve()
+    {
+        s1 *= 0.5;
+        s2 *= 0.5;
+        if (kKernel != kCubicSpline) s3 *= 0.5;
+    }
+    __device__ inline double kernel_sum() const
+    {
+        if (kKernel == kCubicSpline) return 32. / 4 / kPi * 2.0 * (s1 - 4.0 * s2);
+        return 9. / 40 / kPi * (s1 - 6.0 * s2 + 15.0 * s3);
+    }
+};
+
+// absorption.cpp:53-74 (cubic), 76-97 (quintic): the trapezoid of 8 intervals
+template <int kKernel>
+__device__ inline double kern_trapezoid(double zlow, double zhigh, double inv_s2, double dr2)
+{
+    const double dz = (zhigh - zlow) / kNGrid;
+    const double d2 = dr2 * inv_s2 + 1e-290;   // keeps q^2 above zero for sqrt_nr
+    ShapeSum<kKernel> sum;
+    sum.add(__builtin_fma(zlow * zlow, inv_s2, d2));
+    sum.add(__builtin_fma(zhigh * zhigh, inv_s2, d2));
+    sum.halve();
+#pragma unroll
+    for (int i = 1; i < kNGrid; ++i) {
+        const double zz = __builtin_fma((double)i, dz, zlow);
+        sum.add(__builtin_fma(zz * zz, inv_s2, d2));
+    }
+    return dz * sum.kernel_sum();
+}
+
+// kern_frac of one pixel [zlow, zhigh]: absorption.cpp:129-134 (mesh), 53-97
+// and 109-115 (tophat, also the reference's default for any other id,
+// absorption.cpp:136-148)
+__device__ inline double kern_frac(int kernel, double zlow, double zhigh, double inv_s2, double dr2, double zrange)
 {
     zlow = fmax(zlow, -zrange);
     zhigh = fmin(zhigh, zrange);
-    if (kernel == kVoronoiMesh) return fmax(0., zhigh - zlow);     // absorption.cpp:129-134
-    if (kernel != kCubicSpline && kernel != kSphQuintic) return 3. / 4. / kPi * fmax(0., zhigh - zlow);
-    if (zlow > zhigh) return 0;
-    double total = kernel_weight(kernel, sqrt(dr2 + zlow * zlow) / smooth) / 2.;
-    const double dz = (zhigh - zlow) / kNGrid;
-    for (int i = 1; i < kNGrid; ++i) {
-        const double zz = i * dz + zlow;
-        total += kernel_weight(kernel, sqrt(dr2 + zz * zz) / smooth);
-    }
-    total += kernel_weight(kernel, sqrt(dr2 + zhigh * zhigh) / smooth) / 2.;
-    return dz * total;
+    if (kernel == kCubicSpline) return zlow > zhigh ? 0.0 : kern_trapezoid<kCubicSpline>(zlow, zhigh, inv_s2, dr2);
+    if (kernel == kSphQuintic) return zlow > zhigh ? 0.0 : kern_trapezoid<kSphQuintic>(zlow, zhigh, inv_s2, dr2);
+    const double len = fmax(0., zhigh - zlow);
+    return kernel == kVoronoiMesh ? len : 3. / 4. / kPi * len;
 }
 
+// One pair as its pixels need it.
+struct ColPair {
+    double pos1, zrange, dr2, inv_s2;
+    long long start;          // first of the pair's slots in the batch
+    int zlow, pad;
+};
+
+// Dynamic LDS of a column-density block per field: its row and its density
+// of each pair the wavefronts hold.
+static size_t colden_lds_bytes(int nbins) { return deposit_lds_bytes(nbins) + sizeof(float) * kColThreads; }
+
+// Work item: one sightline (or a range of its pairs) and up to A.fields
+// fields, part w.line of them; their rows lie side by side in LDS.
+//
+// Bound: FP64 VALU (9 kernel values a pixel and pair).  A wavefront takes 64
+// pairs, one per lane, and then runs over all their (pair, pixel) slots 64 at
+// a time, so that supports of a few pixels and of hundreds fill the lanes
+// alike, and a pixel's kernel fraction serves every field.  12.5M pairs of
+// ~45 pixels, 5 fields of 1024 pixels: 168 ms with one lane a pair and one
+// field an item, 5.6 ms so (81% of the VALU issue slots busy, 98% of lanes;
+// the samples rolled instead of unrolled: 6.1 ms).
 template <bool kLds>
-__global__ __launch_bounds__(kThreads) void colden_kernel(DepositArgs A, const WorkItem *items, int item_base,
-                                                          int use_queue)
+__global__ __launch_bounds__(kColThreads) void colden_kernel(DepositArgs A, const WorkItem *items, int item_base,
+                                                             int use_queue)
 {
     extern __shared__ double smem[];
     __shared__ int s_item;
+    __shared__ unsigned long long s_next;
+    __shared__ ColPair pairs[kColThreads];
+    __shared__ int marks[kColThreads];
+    const int lane = threadIdx.x & 63, wbase = threadIdx.x & ~63;
+    ColPair *mine = pairs + wbase;
+    int *mark = marks + wbase;
+    // [field][pair of the block], after the rows
+    float *dens = (float *)(smem + (kLds ? (size_t)A.fields * A.nbins : 0)) + wbase;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const double boxtokpc = A.vbox / A.nbins / A.velfac;   // absorption.cpp:188
     int it = use_queue ? 0 : blockIdx.x;
     for (;;) {
         int item;
+        __syncthreads();
         if (use_queue) {
-            __syncthreads();
             if (threadIdx.x == 0) s_item = atomicAdd(A.queue, 1);
             __syncthreads();
             item = s_item;
@@ -1632,53 +1723,108 @@ __global__ __launch_bounds__(kThreads) void colden_kernel(DepositArgs A, const W
         }
         if (item >= A.nitems) break;
         const WorkItem w = items[item_base + item];
-        const LineDesc L = line_of(A, w.line);
-        double *out_row = L.out + (size_t)w.los * A.nbins;
-        double *row = kLds ? smem : out_row;
-        if (kLds) {
-            for (int j = threadIdx.x; j < A.nbins; j += kThreads) row[j] = 0.0;
-            __syncthreads();
-        }
+        const int f0 = w.line * A.fields, nf = min(A.fields, A.nlines - f0);
+        if (kLds)
+            for (int j = threadIdx.x; j < nf * A.nbins; j += kColThreads) smem[j] = 0.0;
+        if (threadIdx.x == 0) s_next = (unsigned long long)w.p0;
+        __syncthreads();
         const LosInfo los = los_info(A, w.los);
-        const double boxtokpc = A.vbox / A.nbins / A.velfac;   // absorption.cpp:188
-        for (long long k = w.p0 + threadIdx.x; k < w.p1; k += kThreads) {
-            const int p = A.pair_part[k];
-            const float *pp = &A.pos[3 * (size_t)p];
-            const float dens = L.dens[p];
-            double pos1 = pp[los.ax - 1], zrange, dr2;
-            float smooth;
-            if (A.seg) {
-                // Voronoi mesh: the segment ends replace dr2 and h
-                // (absorption.cpp:170-187): centre and half length
-                const float2 sg = A.seg[k];
-                dr2 = (double)sg.x;
-                smooth = sg.y;
-                if (dr2 > 2 * A.vbox / A.velfac || (double)smooth > 2 * A.vbox / A.velfac) continue;
-                pos1 = (dr2 + (double)smooth) / 2.;
-                zrange = ((double)smooth - dr2) / 2.;
-            } else {
-                dr2 = pair_dr2(los, pp, A.box);
-                smooth = A.h[p];
-                const float sm2 = smooth * smooth;
-                if ((double)sm2 - dr2 <= 0) continue;              // absorption.cpp:182
-                zrange = sqrt((double)sm2 - dr2);
+        for (;;) {
+            unsigned long long base = 0;
+            if (lane == 0) base = atomicAdd(&s_next, 64ull);
+            base = (unsigned long long)__shfl((long long)base, 0, 64);
+            if ((long long)base >= w.p1) break;
+            const long long k = (long long)base + lane;
+            // the pair of this lane
+            bool have = k < w.p1;
+            ColPair P;
+            int p = 0;
+            long long npix = 0;
+            if (have) {
+                p = A.pair_part[k];
+                const float *pp = &A.pos[3 * (size_t)p];
+                float smooth;
+                P.pos1 = pp[los.ax - 1];
+                if (A.seg) {
+                    // Voronoi mesh: the segment ends replace dr2 and h
+                    // (absorption.cpp:170-187): centre and half length
+                    const float2 sg = A.seg[k];
+                    P.dr2 = (double)sg.x;
+                    smooth = sg.y;
+                    have = !(P.dr2 > 2 * A.vbox / A.velfac || (double)smooth > 2 * A.vbox / A.velfac);
+                    P.pos1 = (P.dr2 + (double)smooth) / 2.;
+                    P.zrange = ((double)smooth - P.dr2) / 2.;
+                } else {
+                    P.dr2 = pair_dr2(los, pp, A.box);
+                    smooth = A.h[p];
+                    const float sm2 = smooth * smooth;
+                    have = !((double)sm2 - P.dr2 <= 0);              // absorption.cpp:182
+                    P.zrange = have ? sqrt((double)sm2 - P.dr2) : 0.0;
+                }
+                P.inv_s2 = 1.0 / ((double)smooth * (double)smooth);
+                if (have) {
+                    P.zlow = (int)floor((P.pos1 - P.zrange) / boxtokpc);
+                    npix = max(0ll, (long long)(int)ceil((P.pos1 + P.zrange) / boxtokpc) - P.zlow + 1);
+                }
             }
-            const int zlow = floor((pos1 - zrange) / boxtokpc);
-            const int zhigh = ceil((pos1 + zrange) / boxtokpc);
-            for (int z = zlow; z <= zhigh; ++z) {
-                const double plow = (boxtokpc * z - pos1);
-                const double v = (double)dens * kern_frac(A.kernel, plow, plow + boxtokpc, smooth, dr2, zrange);
-                row_add<kLds>(&row[wrap_pixel(z, A.nbins)], v);
+            have = npix > 0;
+            // its slots: exclusive scan of the pixel counts
+            long long incl = npix;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const long long t = __shfl_up(incl, d, 64);
+                if (lane >= d) incl += t;
+            }
+            const long long total = __shfl(incl, 63, 64);
+            P.start = incl - npix;
+            const unsigned long long live = __ballot(have);
+            wave_sync();   // the previous batch's pairs have been read
+            if (have) {
+                const int at = __popcll(live & below);
+                ColPair &d = mine[at];
+                for (int f = 0; f < nf; ++f) dens[f * kColThreads + at] = A.lines[f0 + f].dens[p];
+                d.pos1 = P.pos1;
+                d.zrange = P.zrange;
+                d.dr2 = P.dr2;
+                d.inv_s2 = P.inv_s2;
+                d.start = P.start;
+                d.zlow = P.zlow;
+            }
+            for (long long s0 = 0; s0 < total; s0 += 64) {
+                // pair of slot s0 + lane: the pairs that start at or before it,
+                // by marking the slots at which one starts
+                mark[lane] = 0;
+                wave_sync();
+                const long long rel = P.start - s0;
+                if (have && rel >= 0 && rel < 64) mark[(int)rel] = 1;
+                wave_sync();
+                const unsigned long long starts = __ballot(mark[lane] != 0);
+                const int before = __popcll(__ballot(have && rel < 0));
+                if (s0 + lane < total) {
+                    const int at = before + __popcll(starts & (below << 1 | 1ull)) - 1;
+                    const ColPair &c = mine[at];
+                    const int z = c.zlow + (int)(s0 + lane - c.start);
+                    const double plow = boxtokpc * z - c.pos1;
+                    const double frac = kern_frac(A.kernel, plow, plow + boxtokpc, c.inv_s2, c.dr2, c.zrange);
+                    const int j = wrap_pixel(z, A.nbins);
+                    for (int f = 0; f < nf; ++f) {
+                        double *row = kLds ? smem + (size_t)f * A.nbins : A.lines[f0 + f].out + (size_t)w.los * A.nbins;
+                        row_add<kLds>(&row[j], (double)dens[f * kColThreads + at] * frac);
+                    }
+                }
+                wave_sync();   // the marks have been read
             }
         }
         if (kLds) {
             __syncthreads();
-            if (w.direct) {
-                for (int j = threadIdx.x; j < A.nbins; j += kThreads) out_row[j] = row[j];
-            } else {
-                for (int j = threadIdx.x; j < A.nbins; j += kThreads) {
-                    const double v = row[j];
-                    if (v != 0.0) unsafeAtomicAdd(&out_row[j], v);
+            for (int f = 0; f < nf; ++f) {
+                double *out_row = A.lines[f0 + f].out + (size_t)w.los * A.nbins;
+                const double *row = smem + (size_t)f * A.nbins;
+                for (int j = threadIdx.x; j < A.nbins; j += kColThreads) {
+                    if (w.direct)
+                        out_row[j] = row[j];
+                    else if (row[j] != 0.0)
+                        unsafeAtomicAdd(&out_row[j], row[j]);
                 }
             }
         }
@@ -1738,6 +1884,11 @@ int launch_voigt_eval(const double *u, long long n, double a, float *out, hipStr
 
 size_t deposit_lds_bytes(int nbins) { return sizeof(double) * (size_t)nbins; }
 
+static size_t colden_shm(bool lds, int nbins, int fields)
+{
+    return (size_t)fields * (lds ? colden_lds_bytes(nbins) : colden_lds_bytes(0));
+}
+
 // A kernel's static LDS, or a conservative 64 KiB if the runtime cannot say.
 static size_t static_lds(const void *fn)
 {
@@ -1761,7 +1912,8 @@ static size_t tau_static_lds(int waves)
 
 size_t deposit_static_lds(bool tau, int gsize, int waves)
 {
-    if (!tau) return static_lds((const void *)colden_kernel<true>);
+    // (column density: with the densities of one field)
+    if (!tau) return static_lds((const void *)colden_kernel<true>) + colden_lds_bytes(0);
     return gsize == 16 ? tau_static_lds<16>(waves) : gsize == 32 ? tau_static_lds<32>(waves) : tau_static_lds<64>(waves);
 }
 
@@ -1822,7 +1974,7 @@ static int launch_tau(const DepositArgs &A, const WorkItem *items, int item_base
 int launch_deposit(bool tau, bool lds, int gsize, int waves, const DepositArgs &A, const WorkItem *items,
                    int item_base, int nblocks, int use_queue, hipStream_t s)
 {
-    const size_t shm = lds ? deposit_lds_bytes(A.nbins) : 0;
+    const size_t shm = tau ? (lds ? deposit_lds_bytes(A.nbins) : 0) : colden_shm(lds, A.nbins, A.fields);
     int rc = FSAMD_OK;
     if (tau) {
         if (gsize == 16)
@@ -1838,9 +1990,9 @@ int launch_deposit(bool tau, bool lds, int gsize, int waves, const DepositArgs &
     } else {
         if (lds) {
             if (int rc2 = raise_lds_limit((const void *)colden_kernel<true>, shm)) return rc2;
-            colden_kernel<true><<<nblocks, kThreads, shm, s>>>(A, items, item_base, use_queue);
+            colden_kernel<true><<<nblocks, kColThreads, shm, s>>>(A, items, item_base, use_queue);
         } else {
-            colden_kernel<false><<<nblocks, kThreads, 0, s>>>(A, items, item_base, use_queue);
+            colden_kernel<false><<<nblocks, kColThreads, shm, s>>>(A, items, item_base, use_queue);
         }
     }
     FSAMD_HIP(hipGetLastError());
@@ -1890,16 +2042,28 @@ static int occ_tau(bool lds, size_t shm, int waves)
     }
 }
 
-int deposit_blocks_per_cu(bool tau, bool lds, int gsize, int waves, int nbins)
+// Fields a column-density item takes: all of them, or as many (in parts of
+// nearly equal size) as leave room for a second block on the CU, and one
+// where a single row is larger than that.
+int colden_fields(int nlines, int nbins)
+{
+    constexpr size_t kCuLds = 160 * 1024;
+    const size_t room = kCuLds / 2 - std::min(kCuLds / 2, static_lds((const void *)colden_kernel<true>) + 1024);
+    const int most = (int)std::max<size_t>(1, room / colden_lds_bytes(nbins));
+    const int parts = (nlines + most - 1) / most;
+    return (nlines + parts - 1) / parts;
+}
+
+int deposit_blocks_per_cu(bool tau, bool lds, int gsize, int waves, int nbins, int fields)
 {
     int nb = 0;
-    const size_t shm = lds ? deposit_lds_bytes(nbins) : 0;
+    const size_t shm = tau ? (lds ? deposit_lds_bytes(nbins) : 0) : colden_shm(lds, nbins, fields);
     if (tau) {
         nb = gsize == 16 ? occ_tau<16>(lds, shm, waves)
              : gsize == 32 ? occ_tau<32>(lds, shm, waves) : occ_tau<64>(lds, shm, waves);
     } else {
-        hipError_t e = lds ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, colden_kernel<true>, kThreads, shm)
-                           : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, colden_kernel<false>, kThreads, 0);
+        hipError_t e = lds ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, colden_kernel<true>, kColThreads, shm)
+                           : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, colden_kernel<false>, kColThreads, shm);
         if (e != hipSuccess) {
             (void)hipGetLastError();
             nb = 1;

@@ -113,6 +113,7 @@ struct DepositArgs {
     const float2 *seg;          // [M] Voronoi segment ends (kernel 2), else nullptr
     const LineDesc *lines;      // device [nlines], lines of this launch
     int nlines;
+    int fields;                 // column density: fields of a work item (part i takes fields i * fields ..)
     int nitems;
     int claim;                  // most pairs a wavefront of the tau kernel claims at once (1..kWaveClaim)
     int *queue;                 // work-queue counter (zeroed before launch)

@@ -6,7 +6,7 @@ import pytest
 
 from fake_spectra_amd import spectra_priv as SP, synth
 from fake_spectra_amd.lines import HI_1215
-from gpu_util import assert_colden_close, assert_tau_close
+from gpu_util import assert_colden_close, assert_tau_close, dev
 
 pytestmark = pytest.mark.gpu
 
@@ -59,3 +59,30 @@ def test_near_lines(oracle, n, nlos, hfrac):
     _, parts, _ = oracle.near_particles(box, pos, h, axis, cofm)
     got = SP._near_lines(box, pos, h, axis, cofm)
     assert got.dtype == np.int32 and np.array_equal(got, np.unique(parts))
+
+
+# rows of fewer than 64, of 64, 65 and many pairs; supports of one or two pixels
+# and of most of the row; every kernel; fields in one part, in several, and
+# more than a launch takes; rows too long for two blocks and for LDS
+@pytest.mark.parametrize("n,nlos,nbins,kernel,hfrac,fields", [
+    (3, 4, 7, 1, 0.3, 1), (200, 3, 64, 3, 0.3, 5), (230, 5, 257, 0, 0.01, 2), (3000, 4, 1024, 1, 0.2, 5),
+    (700, 3, 2048, 1, 0.02, 5), (700, 3, 4099, 3, 0.2, 4), (500, 2, 9001, 1, 0.1, 3), (300, 2, 20011, 1, 0.1, 2),
+    (400, 3, 100, 9, 0.2, 11), (1, 1, 1, 1, 0.4, 1), (300, 4, 513, 2, 0.3, 3)])
+def test_colden_fields(oracle, n, nlos, nbins, kernel, hfrac, fields):
+    """Several fields of one plan, each against a call of its own; FP64
+    throughout, so to rounding (a sum of up to ~1e4 positive terms)."""
+    args = small_gas(n, 400.0, nlos, nbins, kernel, hfrac, compute_tau=False)
+    pos, dens, h, axis, cofm = (args[i] for i in (11, 13, 15, 16, 17))
+    rng = np.random.default_rng(9)
+    all_dens = [dens] + [(dens * rng.random(n)).astype(np.float32) for _ in range(fields - 1)]
+    plan = SP.Plan(args[3], dev(pos), dev(h), dev(axis), dev(cofm))
+    if kernel == 2:
+        plan.assign_cells()
+    outs = SP.colden(plan, nbins, kernel, args[4], [dev(d) for d in all_dens])
+    assert len(outs) == fields
+    for d, o in zip(all_dens, outs):
+        a = list(args)
+        a[13] = d
+        ref, got = oracle.interpolate(*a), o.cpu().numpy()
+        assert np.array_equal(got == 0, ref == 0)
+        assert np.max(np.abs(got - ref)) <= 1e-12 * max(ref.max(), 1e-300)
