@@ -39,6 +39,8 @@
 namespace fsamd {
 
 __constant__ __attribute__((aligned(16))) float c_gtab[kGTableSize] = FSAMD_G_COEF_INIT;
+constexpr int kG64Size = FSAMD_G64_NPIECE * FSAMD_G64_NCOEF;
+__device__ const double d_gtab64[kG64Size] = FSAMD_G64_COEF_INIT;
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
@@ -264,30 +266,29 @@ __device__ inline double inner32(const PairTau &P, double vouter, const float *g
     return (double)acc;
 }
 
-// Same sum with the FP64 profile and FP64 kernel weights; out of line and
-// with scalar arguments because it only runs for rare pixels.
-__device__ __noinline__ double inner64(double aa, double b, double dvk, double vhigh, double vdr2,
-                                       double vsmooth, double vouter, int kernel)
+// One sample of that sum (i = 1 .. kNGrid - 1) with the FP64 profile and FP64
+// kernel weights.
+__device__ inline double sample64(const PairTau &P, double vouter, int kernel, int i, const double *gtab64)
 {
-    double total = 0;
-    for (int i = 1; i < kNGrid; ++i) {
-        const double vv = i * dvk - vhigh;
-        const double q = sqrt(vdr2 + vv * vv) / vsmooth;
-        const double t0 = (vv - vouter) / b;
-        total += voigt64(aa, t0) * kernel_weight(kernel, q);
-    }
-    return total;
+    const double vv = i * P.dvk - P.vhigh;
+    const double q = sqrt(P.vdr2 + vv * vv) / P.vsmooth;
+    const double u = (vv - vouter) / P.b;
+    return kernel_weight(kernel, q) * (P.aa <= (double)kA32Max ? voigt64_small(P.aa, u, gtab64) : voigt64(P.aa, u));
 }
 
-__device__ inline double inner64(const PairTau &P, double vouter, int kernel)
+// The whole sum on one lane.
+__device__ __noinline__ double inner64(const PairTau &P, double vouter, int kernel, const double *gtab64)
 {
-    return inner64(P.aa, P.b, P.dvk, P.vhigh, P.vdr2, P.vsmooth, vouter, kernel);
+    double total = 0;
+#pragma unroll 1
+    for (int i = 1; i < kNGrid; ++i) total += sample64(P, vouter, kernel, i, gtab64);
+    return total;
 }
 
 // amp*dens*tau_kern_outer(vlow, vlow+bintov)/velfac  (absorption.cpp:255; singleabs.h:104-126)
 template <bool k64>
 __device__ inline double taulast_pixel(const PairTau &P, double vlow, double bintov, double velfac, int kernel,
-                                       const float *gtab)
+                                       const float *gtab, const double *gtab64)
 {
     const double vhighp = vlow + bintov;
     const double width = vhighp - vlow;
@@ -301,19 +302,45 @@ __device__ inline double taulast_pixel(const PairTau &P, double vlow, double bin
             return P.scale * (double)(S * Y);
         }
     }
-    if (width < P.b / 2.) {
-        const double mid = (vhighp + vlow) / 2.;
-        return P.scale * (k64 ? inner64(P, mid, kernel) : inner32(P, mid, gtab));
-    }
+    auto inner = [&](double v) { return k64 ? inner64(P, v, kernel, gtab64) : inner32(P, v, gtab); };
+    if (width < P.b / 2.) return P.scale * inner((vhighp + vlow) / 2.);
     const int np = 2 * ceil(width / (P.b / 2.) / 2) + 1.;
     const double dv = width / (np - 1);
-    double total = 0.5 * (k64 ? inner64(P, vlow, kernel) : inner32(P, vlow, gtab));
-    for (int i = 1; i < np - 1; ++i) {
-        const double vv = i * dv + vlow;
-        total += k64 ? inner64(P, vv, kernel) : inner32(P, vv, gtab);
-    }
-    total += 0.5 * (k64 ? inner64(P, vhighp, kernel) : inner32(P, vhighp, gtab));
+    double total = 0.5 * inner(vlow);
+    for (int i = 1; i < np - 1; ++i) total += inner(i * dv + vlow);
+    total += 0.5 * inner(vhighp);
     return P.scale * (total / (np - 1));
+}
+
+template <int kG>
+__device__ inline double group_sum(double v)
+{
+#pragma unroll
+    for (int o = kG / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kG);
+    return v;
+}
+
+// taulast_pixel<true> of one pixel by a whole lane group, its 7 x np samples
+// over the lanes: a pixel that decides a tail cut is usually the only one of
+// its group, and its samples in turn on one lane would be the walk's latency.
+template <int kG>
+__device__ inline double taulast_group64(const PairTau &P, double vlow, double bintov, int kernel, int glane,
+                                         const double *gtab64)
+{
+    const double vhighp = vlow + bintov;
+    const double width = vhighp - vlow;
+    int np = 1;
+    if (!(width < P.b / 2.)) np = 2 * ceil(width / (P.b / 2.) / 2) + 1.;
+    const double dv = width / (np - 1);
+    double total = 0;
+    for (int m = glane; m < (kNGrid - 1) * np; m += kG) {
+        const int j = m / (kNGrid - 1), i = m - j * (kNGrid - 1) + 1;
+        const double v = np == 1 ? (vhighp + vlow) / 2. : j == 0 ? vlow : j == np - 1 ? vhighp : j * dv + vlow;
+        const double h = sample64(P, v, kernel, i, gtab64);
+        total += np > 1 && (j == 0 || j == np - 1) ? 0.5 * h : h;
+    }
+    total = group_sum<kG>(total);
+    return P.scale * (np == 1 ? total : total / (np - 1));
 }
 
 // x^n for 0 <= n < 16 by squaring, with a uniform instruction stream.
@@ -799,35 +826,31 @@ __device__ inline void row_add(double *p, double v)
         unsafeAtomicAdd(p, v);    // global_atomic_add_f64
 }
 
-// Walk modes: the FP32 deposit kernel defers any decision it cannot make
-// exactly; the fix-up kernel re-evaluates guard-band pixels in FP64, or
-// evaluates whole pairs in FP64.
-enum { kWalkMain = 0, kWalkGuarded = 1, kWalkFull64 = 2 };
+// The FP32 deposit kernel defers any decision it cannot make exactly; the
+// fix-up kernel re-evaluates guard-band pixels in FP64, or evaluates whole
+// pairs in FP64.
+enum { kWalkGuarded = 1, kWalkFull64 = 2 };
 
-
-
-// One step of kG consecutive pixels of a walk (lane glane of the group), each
-// pixel evaluated on its own as tau_kern_outer does (singleabs.h:104-126,
-// sub-sample grid from the pixel's own vhigh - vlow): the fix-up kernel's
-// walk (walk_fix), in the guarded or the all-FP64 mode.  Returns true when the
-// walk is over (tail cut reached, end of the window, or in kWalkMain mode the
-// decision deferred).
-template <int kG, int kMode, bool kLds, bool kStats>
-__device__ inline bool walk_chunk(const DepositArgs &A, const PairTau &P, double *row, const float *gtab, int z0,
-                                  int dir, int count, int c, int lane, LaneStats &st, long long k, int item,
-                                  bool active, int &walked)
+// One step of kG consecutive pixels of a fix-up walk (lane glane of the group),
+// each pixel evaluated on its own as tau_kern_outer does (singleabs.h:104-126,
+// sub-sample grid from the pixel's own vhigh - vlow), in FP32 with the guard
+// band re-evaluated in FP64 (kWalkGuarded), or all in FP64.  Returns true when
+// the walk is over (tail cut reached or end of the window).
+template <int kG, int kMode, bool kStats>
+__device__ inline bool walk_chunk(const DepositArgs &A, const PairTau &P, double *row, const float *gtab,
+                                  const double *gtab64, int z0, int dir, int count, int c, int lane, LaneStats &st,
+                                  int &walked)
 {
     const int glane = lane % kG;
     const double bintov = A.vbox / A.nbins;
     const double tt = A.tautail;
     const int idx = c + glane;
-    const bool valid = active && idx < count;
+    const bool valid = idx < count;
     const int z = z0 + dir * idx;
     double t = 0, vlow = 0;
-    bool guard = false;
     if (valid) {
         vlow = z * bintov - P.vel;                                  // absorption.cpp:252
-        t = taulast_pixel<kMode == kWalkFull64>(P, vlow, bintov, A.velfac, A.kernel, gtab);
+        t = taulast_pixel<kMode == kWalkFull64>(P, vlow, bintov, A.velfac, A.kernel, gtab, gtab64);
         if (kStats) {
             st.evaluated++;
             if (kMode != kWalkFull64 && fabs((vlow + 0.5 * bintov) * P.inv_b) >= P.ufar)
@@ -835,31 +858,32 @@ __device__ inline bool walk_chunk(const DepositArgs &A, const PairTau &P, double
             else
                 st.sums += pixel_samples(P, vlow, bintov) / (kNGrid - 1);
         }
-        if (kMode != kWalkFull64 && fabs(t - tt) <= kGuard * tt) {
-            if (kMode == kWalkGuarded) {
-                t = taulast_pixel<true>(P, vlow, bintov, A.velfac, A.kernel, gtab);
+    }
+    if (kMode == kWalkGuarded) {
+        // pixels past the first certain cut are not needed
+        const unsigned long long sure =
+            group_bits<kG>(__ballot(valid && t < tt && !(fabs(t - tt) <= kGuard * tt)), lane);
+        unsigned long long band = group_bits<kG>(__ballot(valid && fabs(t - tt) <= kGuard * tt), lane);
+        if (sure) band &= (sure & (0ull - sure)) - 1ull;
+        while (band) {
+            const int g = __builtin_ctzll(band);
+            band &= band - 1ull;
+            const double t64 = taulast_group64<kG>(P, (z0 + dir * (c + g)) * bintov - P.vel, bintov, A.kernel, glane,
+                                                   gtab64);
+            if (glane == g) {
+                t = t64;
                 if (kStats) st.px64++;
-            } else {
-                guard = true;
             }
         }
     }
-    const unsigned long long mb = group_bits<kG>(__ballot(valid && !guard && t < tt), lane);
-    const unsigned long long mg = group_bits<kG>(__ballot(guard), lane);
-    const unsigned long long mall = mb | mg;
-    const int first = mall ? __builtin_ctzll(mall) : kG;
-    if (valid && (glane < first || (glane == first && ((mb >> glane) & 1ull)))) {
-        row_add<kLds>(&row[wrap_pixel(z, A.nbins)], t);
+    const unsigned long long mb = group_bits<kG>(__ballot(valid && t < tt), lane);
+    const int first = mb ? __builtin_ctzll(mb) : kG;
+    if (valid && glane <= first) {
+        row_add<false>(&row[wrap_pixel(z, A.nbins)], t);
         if (kStats) {
             st.pixels++;
             st.samples += pixel_samples(P, vlow, bintov);
         }
-    }
-    if (kMode == kWalkMain && first < kG && ((mg >> first) & 1ull)) {
-        // the FP32 value of the deciding pixel is too close to tautail
-        if (active && glane == 0) push_fixup(A, k, item, z0 + dir * (c + first), count - (c + first), dir);
-        walked = -1;
-        return true;
     }
     if (mb != 0) {
         walked = c + first + 1;
@@ -1036,8 +1060,8 @@ __device__ inline bool step_needs_wing(const PairTau &P, double bintov, int z0, 
 // Walk one direction with a kG-lane group (fix-up kernel): pixels z0,
 // z0+dir, ... for at most `count` pixels, until and including the tail cut.
 template <int kG, int kMode, bool kStats>
-__device__ inline int walk_fix(const DepositArgs &A, PairTau &P, double *row, const float *gtab, int z0, int dir,
-                               int count, int lane, LaneStats &st, long long k, int item)
+__device__ inline int walk_fix(const DepositArgs &A, PairTau &P, double *row, const float *gtab,
+                               const double *gtab64, int z0, int dir, int count, int lane, LaneStats &st)
 {
     const double bintov = A.vbox / A.nbins;
     const int glane = lane % kG;
@@ -1048,14 +1072,15 @@ __device__ inline int walk_fix(const DepositArgs &A, PairTau &P, double *row, co
             if (glane == 0) P.wing_ready = 1;
             wave_sync();
         }
-        if (walk_chunk<kG, kMode, false, kStats>(A, P, row, gtab, z0, dir, count, c, lane, st, k, item, true, walked))
+        if (walk_chunk<kG, kMode, kStats>(A, P, row, gtab, gtab64, z0, dir, count, c, lane, st, walked))
             return walked;
     }
     return walked;
 }
 
 // Lanes per fix-up entry: most deferred walks end a few pixels past the
-// deciding pixel, so a wavefront works on four entries at once.
+// deciding pixel, and its 7 (or 21) samples fill half of 16 lanes, so a
+// wavefront works on four entries at once.
 constexpr int kFixG = 16;
 
 // 4 waves per SIMD: measured 8% faster at c1 than the 3 the register count
@@ -1223,20 +1248,29 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     }
 }
 
-// Deferred walks, after the deposit kernel has written its rows: one wave per
-// fix-up entry, deposits straight into the output with FP64 atomics.
+// Deferred walks, after the deposit kernel has written its rows: one lane
+// group per fix-up entry, deposits straight into the output with FP64 atomics.
+//
+// Bound: the latency of an entry's FP64 samples where few walks are deferred,
+// FP64 VALU where millions are.  With voigt64_small in place of w64 and a
+// deciding pixel's samples over the group instead of in turn on one lane: 109M
+// pair-lines of 2048 pixels 3192 -> 224 us, 1.4M of 1501 1089 -> 28 us, 32768
+// particles and 64 sightlines 174 -> 18 us.
 template <bool kStats>
 __global__ __launch_bounds__(kThreads) void tau_fixup_kernel(DepositArgs A, const WorkItem *items)
 {
     constexpr int kGroups = kThreads / kFixG;
     __shared__ __attribute__((aligned(16))) float gtab[kGTableSize];
     __shared__ PairTau pslot[kGroups];
+    __shared__ double gtab64[kG64Size];
+    const int n = (int)min(A.fix_count[0], (unsigned long long)A.fix_cap);
+    if (blockIdx.x * kGroups >= n) return;
     for (int i = threadIdx.x; i < kGTableSize; i += kThreads) gtab[i] = c_gtab[i];
+    for (int i = threadIdx.x; i < kG64Size; i += kThreads) gtab64[i] = d_gtab64[i];
     __syncthreads();
     const int lane = threadIdx.x & 63, gid = threadIdx.x / kFixG, glane = lane % kFixG;
     PairTau &P = pslot[gid];
     LaneStats st;
-    const int n = (int)min(A.fix_count[0], (unsigned long long)A.fix_cap);
     const int half = A.nbins / 2;
     for (int e = blockIdx.x * kGroups + gid; e < n; e += gridDim.x * kGroups) {
         const Fixup f = A.fix[e];
@@ -1246,17 +1280,14 @@ __global__ __launch_bounds__(kThreads) void tau_fixup_kernel(DepositArgs A, cons
         const LosInfo los = los_info(A, w.los);
         if (!setup_pair<kFixG>(A, w.line, L, los, f.k, P, glane)) continue;
         if (f.dir == 0) {
-            const int lf = walk_fix<kFixG, kWalkFull64, kStats>(A, P, out_row, gtab, P.zmax, 1, half, lane, st, f.k,
-                                                                  f.item);
-            const int lb = walk_fix<kFixG, kWalkFull64, kStats>(A, P, out_row, gtab, P.zmax - 1, -1, half, lane, st,
-                                                                  f.k, f.item);
+            const int lf = walk_fix<kFixG, kWalkFull64, kStats>(A, P, out_row, gtab, gtab64, P.zmax, 1, half, lane, st);
+            const int lb = walk_fix<kFixG, kWalkFull64, kStats>(A, P, out_row, gtab, gtab64, P.zmax - 1, -1, half, lane, st);
             if (glane == 0) {
                 record_window(A, w.line, f.k, 1, lf);
                 record_window(A, w.line, f.k, -1, lb);
             }
         } else {
-            const int l = walk_fix<kFixG, kWalkGuarded, kStats>(A, P, out_row, gtab, f.z0, f.dir, f.count, lane, st,
-                                                                  f.k, f.item);
+            const int l = walk_fix<kFixG, kWalkGuarded, kStats>(A, P, out_row, gtab, gtab64, f.z0, f.dir, f.count, lane, st);
             if (glane == 0) record_window(A, w.line, f.k, f.dir, (half - f.count) + l);
         }
     }
@@ -1365,14 +1396,6 @@ __device__ inline void adj_far(const PairTau &P, double vlow, double bintov, dou
     S = (double)(s * Y);
     SU = 2.0 / U * (double)(d * Y);
     SF = (double)(f * Y);
-}
-
-template <int kG>
-__device__ inline double group_sum(double v)
-{
-#pragma unroll
-    for (int o = kG / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kG);
-    return v;
 }
 
 template <int kG>

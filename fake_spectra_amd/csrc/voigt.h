@@ -39,6 +39,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include "dawson_table.h"
+#include "dawson64_table.h"
 
 namespace fsamd {
 
@@ -315,6 +316,54 @@ __device__ inline void w64(double x, double y, double &wr, double &wi)
     }
     wr = r;
     wi = x < 0 ? -i : i;
+}
+
+// Re w(u + ia) for 0 <= a <= kA32Max to ~1e-13 relative, without the sums and
+// recurrences of w64: nearly every guard-band pixel has such an a.
+// |u| < 10: w's Taylor series in a about the real axis to a^9 D^(9): its even
+// terms are exp(a^2 - u^2) cos(2au), its odd ones the odd derivatives of
+// Dawson's integral, G = D' from pieces of degree 11 in u (gtab64,
+// dawson64_table.h) and the others by
+//   D''' = (4u^2 - 6) D' + 2,  D^(n+2) = (4u^2 - 4n - 2) D^(n) - 4n(n-1) D^(n-2);
+// |u| >= 10: the asymptotic series w ~ (i/sqrt(pi)) sum_n (2n-1)!!/2^n z^-(2n+1),
+// 14 terms in complex arithmetic.
+__device__ inline double voigt64_small(double a, double u, const double *gtab64)
+{
+    const double x = fabs(u), p = u * u;
+    if (x >= FSAMD_G64_UMAX) {
+        // r = 1/z^2, s = sum_n c_n r^n
+        const double q = 1.0 / (p + a * a);
+        const double ir = x * q, ii = -a * q;              // 1/z
+        const double rr = ir * ir - ii * ii, ri = 2.0 * ir * ii;
+        double sr = 1.0, si = 0.0;
+#pragma unroll 1
+        for (int n = 14; n >= 1; --n) {
+            const double c = n - 0.5;                      // c_n / c_(n-1)
+            const double tr = sr * rr - si * ri, ti = sr * ri + si * rr;
+            sr = 1.0 + c * tr;
+            si = c * ti;
+        }
+        // Re (i s / z), and the Gaussian for a = 0
+        return exp(a * a - p) - (ir * si + ii * sr) * (1.0 / kSqrtPi);
+    }
+    const int k = (int)(x * FSAMD_G64_PER_UNIT);
+    const double v = x - (k + 0.5) * (1.0 / FSAMD_G64_PER_UNIT);
+    const double *c = gtab64 + k * FSAMD_G64_NCOEF;
+    double d1 = c[FSAMD_G64_NCOEF - 1];
+#pragma unroll
+    for (int i = FSAMD_G64_NCOEF - 2; i >= 0; --i) d1 = __builtin_fma(d1, v, c[i]);
+    const double a2 = a * a, p4 = 4.0 * p;
+    const double d3 = (p4 - 6.0) * d1 + 2.0;
+    const double d5 = (p4 - 14.0) * d3 - 24.0 * d1;
+    const double d7 = (p4 - 22.0) * d5 - 80.0 * d3;
+    const double d9 = (p4 - 30.0) * d7 - 168.0 * d5;
+    const double odd = d1 - a2 * (1.0 / 6.0) * (d3 - a2 * (1.0 / 20.0) * (d5 - a2 * (1.0 / 42.0) * (d7 - a2 * (1.0 / 72.0) * d9)));
+    // cos(2au), 2au <= 0.8
+    const double m = -4.0 * a2 * p;
+    double cs = 1.0;
+#pragma unroll
+    for (int n = 9; n >= 1; --n) cs = __builtin_fma(cs, m * (1.0 / ((2 * n - 1) * (2 * n))), 1.0);
+    return exp(a2 - p) * cs - kTwoOverSqrtPi * a * odd;
 }
 
 __device__ inline double voigt64(double a, double u)

@@ -86,3 +86,25 @@ def test_colden_fields(oracle, n, nlos, nbins, kernel, hfrac, fields):
         ref, got = oracle.interpolate(*a), o.cpu().numpy()
         assert np.array_equal(got == 0, ref == 0)
         assert np.max(np.abs(got - ref)) <= 1e-12 * max(ref.max(), 1e-300)
+
+
+# damping parameters of 0, of cold and hot gas below 0.04, and above it; pixels
+# of one midpoint and of many sub-samples; windows of one group step, several,
+# and cut by half the row
+@pytest.mark.parametrize("nbins,kernel,tscale,gscale", [(7, 1, 1.0, 1.0), (64, 3, 1e-4, 1.0), (300, 0, 1.0, 0.0),
+                                                        (300, 1, 1.0, 40.0), (129, 1, 1e-3, 5.0), (1024, 1, 1.0, 1.0),
+                                                        (200, 9, 1.0, 1e3)])
+def test_fp64_walks(oracle, nbins, kernel, tscale, gscale):
+    """Every pair on the FP64 path: the profile is good to ~1e-13 relative and
+    the sums have positive terms, so tau to 1e-11."""
+    args = list(small_gas(60, 1500.0, 3, nbins, kernel, 0.1))
+    args[14] = (args[14] * tscale).astype(np.float32)
+    args[7] *= gscale
+    ref = oracle.interpolate(*args)
+    SP.set_fp64(True)
+    try:
+        got = SP._Particle_Interpolate(*args)
+    finally:
+        SP.set_fp64(False)
+    assert np.max(ref) > 0 and np.array_equal(got == 0, ref == 0)
+    assert np.max(np.abs(got - ref) / np.maximum(ref, 1e-300)) <= 1e-11
