@@ -39,6 +39,7 @@
 namespace fsamd {
 
 __constant__ __attribute__((aligned(16))) float c_gtab[kGTableSize] = FSAMD_G_COEF_INIT;
+__device__ __attribute__((aligned(16))) const float d_ptab[kPTableSize] = FSAMD_P_COEF_INIT;
 constexpr int kG64Size = FSAMD_G64_NPIECE * FSAMD_G64_NCOEF;
 __device__ const double d_gtab64[kG64Size] = FSAMD_G64_COEF_INIT;
 
@@ -162,42 +163,21 @@ __device__ inline int wrap_pixel(int z, int nbins)
 // Each wavefront keeps the constants of its current pair in an LDS slot: the
 // values are uniform across the wave, and reading them with broadcast LDS
 // loads keeps them out of the vector registers of the per-pixel loop.
-// One interior kernel sample of a pair (singleabs.h:146-157): its offset
-// vv_i / b as a two-float split (cv_hi + cv_lo, ~48 bits) and its weight
-// K(q_i), read together (one 16-byte LDS read) in the sample loop.
+// One interior kernel sample of a pair (singleabs.h:146-157): twice its offset
+// vv_i / b (the profile's table takes 2u, voigt.h) and its weight K(q_i).
 struct KernelSample {
-    float cv_hi, cv_lo;
+    double cv2;
     float w;
     float pad;
 };
 
-__device__ inline void set_sample_offset(KernelSample &k, double cv)
-{
-    k.cv_hi = (float)cv;
-    k.cv_lo = (float)(cv - (double)k.cv_hi);
-}
+__device__ inline void set_sample_offset(KernelSample &k, double cv) { k.cv2 = 2.0 * cv; }
 
-__device__ inline double sample_offset(const KernelSample &k) { return (double)k.cv_hi + (double)k.cv_lo; }
+__device__ inline double sample_offset(const KernelSample &k) { return 0.5 * k.cv2; }
 
-// The sub-sample velocity in units of b as a two-float split.
-struct Split {
-    float hi, lo;
-};
-
-__device__ inline Split split_s(double s)
-{
-    Split r;
-    r.hi = (float)s;
-    r.lo = (float)(s - (double)r.hi);
-    return r;
-}
-
-// u = (vv_i - vouter)/b in FP32 from the two splits: the high parts cancel
-// exactly where u is small (Sterbenz), so u keeps ~1 ulp relative error.
-__device__ inline float sample_u(const KernelSample &k, Split s)
-{
-    return (k.cv_hi - s.hi) + (k.cv_lo - s.lo);
-}
+// 2u = 2 (vv_i - vouter)/b from s2 = 2 vouter/b: subtracted in FP64 and rounded
+// once, so u keeps half an ulp where the two nearly cancel.
+__device__ inline float sample_u2(const KernelSample &k, double s2) { return (float)(k.cv2 - s2); }
 
 // The constants a walk of the main kernel reads, in one layout in the pair
 // set-up record and in the group's PairTau slot, so that taking a record
@@ -209,22 +189,28 @@ struct WalkHead {
     double inv_nm1;  // 1 / (np - 1)
     // Far wing: for a pixel centred at U (units of b) with |U| >= ufar the
     // 7 x np samples sum to Y (C0 + C1 Y + ... + C9 Y^9), Y = (ufar/U)^2.
-    double ufar;
+    float ufar;
     int zmax;
-    int nm1, rounds, pstep;   // near-step shape of the main kernel (step_shape)
+    int shape;       // near-step shape of the main kernel (step_shape)
+    int k;           // the pair, counted from the work item's first (main kernel)
 };
-static_assert(sizeof(WalkHead) == 56, "WalkHead is seven 8-byte words");
+static_assert(sizeof(WalkHead) == 48, "WalkHead is six 8-byte words");
 
-struct PairTau : WalkHead {
+// What a walk of the main kernel reads of its pair.
+struct PairWalk : WalkHead {
     KernelSample smp[kNGrid - 1];   // kernel sample velocities / b and weights
+    float Cw[kWingTerms];
+    VoigtP vp;
     double b;        // btherm (absorption.cpp:220)
+};
+
+struct PairTau : PairWalk {
     double dvk;      // 2 vhigh / NGRID (singleabs.h:146)
     double vhigh, vdr2, vsmooth, aa;
     float ufar2;     // ufar^2 (fix-up and adjoint kernels)
     double scale_nd; // amp * dvk / velfac (scale without the density)
     double temp;     // particle temperature
     int part;        // particle index
-    float Cw[kWingTerms];
     float CwF[kWingTerms];   // adjoint: far-wing coefficients of sum w (u dH/du + a dH/da)
     VoigtA va;
     int fp64;
@@ -250,20 +236,23 @@ __device__ inline double shfl_d(double v, int src)
 }
 
 // sum_i K(q_i) Re w((vv_i - vouter)/b + i a), FP32 profile; the sample
-// offsets from the FP64 anchor vouter/b (one split per sum).  kA3 = false:
-// without the profile's a^3 term (pairs with a <= kA3Drop).
+// offsets from the FP64 anchor vouter/b.  kA3 = false: the light form of the
+// profile (pairs with a <= kA3Drop).
 template <bool kA3 = true>
-__device__ inline double inner32(const PairTau &P, double vouter, const float *gtab)
+__device__ inline float inner32(const PairWalk &P, double vouter, const float *ptab)
 {
-    const Split s = split_s(vouter * P.inv_b);
-    const VoigtA va = P.va;
-    float acc = 0.0f;
+    const double s2 = vouter * (2.0 * P.inv_b);
+    const VoigtP vp = P.vp;
+    float sE = 0.0f, sG = 0.0f;
 #pragma unroll  // full: 5% faster than unrolling by 2 at 256^3 and 512^3 (same operation order)
     for (int i = 0; i < kNGrid - 1; ++i) {
         const KernelSample k = P.smp[i];
-        acc = __builtin_fmaf(k.w, voigt32<kA3>(va, sample_u(k, s), gtab), acc);
+        float E, G;
+        voigt_terms<kA3>(vp, sample_u2(k, s2), ptab, E, G);
+        sE = __builtin_fmaf(k.w, E, sE);
+        sG = __builtin_fmaf(k.w, G, sG);
     }
-    return (double)acc;
+    return __builtin_fmaf(-vp.two_a_sqpi, sG, sE);
 }
 
 // One sample of that sum (i = 1 .. kNGrid - 1) with the FP64 profile and FP64
@@ -288,7 +277,7 @@ __device__ __noinline__ double inner64(const PairTau &P, double vouter, int kern
 // amp*dens*tau_kern_outer(vlow, vlow+bintov)/velfac  (absorption.cpp:255; singleabs.h:104-126)
 template <bool k64>
 __device__ inline double taulast_pixel(const PairTau &P, double vlow, double bintov, double velfac, int kernel,
-                                       const float *gtab, const double *gtab64)
+                                       const float *ptab, const double *gtab64)
 {
     const double vhighp = vlow + bintov;
     const double width = vhighp - vlow;
@@ -302,7 +291,7 @@ __device__ inline double taulast_pixel(const PairTau &P, double vlow, double bin
             return P.scale * (double)(S * Y);
         }
     }
-    auto inner = [&](double v) { return k64 ? inner64(P, v, kernel, gtab64) : inner32(P, v, gtab); };
+    auto inner = [&](double v) { return k64 ? inner64(P, v, kernel, gtab64) : inner32(P, v, ptab); };
     if (width < P.b / 2.) return P.scale * inner((vhighp + vlow) / 2.);
     const int np = 2 * ceil(width / (P.b / 2.) / 2) + 1.;
     const double dv = width / (np - 1);
@@ -444,7 +433,11 @@ struct StepShape {
     int nm1;      // np - 1 (0: midpoint)
     int rounds;   // lane rounds per step
     int pstep;    // pixels per step
+    __device__ inline int packed() const { return nm1 | (rounds << 16) | (pstep << 24); }
 };
+static_assert(64 * kRoundsMax < (1 << 16) && kRoundsMax < (1 << 8), "StepShape::packed");
+
+__device__ inline StepShape unpack_shape(int s) { return StepShape{s & 0xffff, (s >> 16) & 0xff, s >> 24}; }
 
 __device__ inline StepShape step_shape(int np, int kg)
 {
@@ -556,10 +549,14 @@ __device__ inline bool pair_consts(const DepositArgs &A, int line, const LineDes
     // differ between pixels (bintov/b at a switch point to 1e-12) goes to the
     // FP64 path, which follows the reference pixel by pixel.
     const bool grid_edge = fabs(bintov - b / 2.) <= 1e-12 * bintov || (np > 1 && fabs(xs - rint(xs)) <= 1e-12 * xs);
-    // pixels wider than max_sums sub-samples do not fit one walk step
-    C.fp64 = A.force_fp64 || !(aa <= (double)kA32Max) || grid_edge || np - 1 > max_sums - 1;
     const double dmax = (vhigh - dvk) * inv_b + (np > 1 ? 0.5 * bintov * inv_b : 0.0);
     C.ufar = fmax(7.0 + dmax, 3.0 * dmax);
+    // pixels wider than max_sums sub-samples do not fit one walk step; samples
+    // of a near step (up to 4 * 64 sub-samples of half a b past ufar) must lie
+    // within the profile's table, which leaves out only supports of thousands
+    // of Doppler widths
+    C.fp64 = A.force_fp64 || !(aa <= (double)kA32Max) || grid_edge || np - 1 > max_sums - 1 ||
+             !(C.ufar + dmax + 130.0 <= kVoigtUMax);
     C.vel = vel;
     C.b = b;
     C.inv_b = inv_b;
@@ -611,20 +608,17 @@ __device__ inline bool setup_pair(const DepositArgs &A, int line, const LineDesc
         P.zmax = C.zmax;
         P.fp64 = C.fp64;
         P.va = make_voigt_a(C.fp64 ? 0.0 : C.aa);
+        P.vp = make_voigt_p(C.fp64 ? 0.0 : C.aa, C.aa <= (double)kA3Drop);
         P.scale = C.scale;
         P.scale_nd = C.scale_nd;
         P.temp = (double)C.temp;
         P.part = p;
         P.np = C.np;
-        P.ufar = C.ufar;
-        P.ufar2 = (float)(C.ufar * C.ufar);
+        P.ufar = (float)C.ufar;
+        P.ufar2 = (float)((double)P.ufar * P.ufar);
         P.wing_ready = 0;
         P.inv_nm1 = C.np > 1 ? 1.0 / (C.np - 1) : 1.0;
         P.dv = C.np > 1 ? bintov * P.inv_nm1 : 0.0;
-        const StepShape sh = step_shape(C.np, kG);
-        P.nm1 = sh.nm1;
-        P.rounds = sh.rounds;
-        P.pstep = sh.pstep;
     }
     wave_sync();
     return true;
@@ -641,13 +635,13 @@ constexpr int kWaveQueue = kWaveClaim;
 struct PairLite {
     WalkHead h;
     double vhigh;
-    long long k;      // pair index
     float W[4];       // kernel weights of the centre sample and the 3 above it
     float Cw[kWingTerms];   // far-wing coefficients (wing_coeffs)
-    VoigtA va;        // constants of the FP32 profile
+    VoigtP vp;        // constants of the FP32 profile
 };
-static_assert(sizeof(PairLite) == 168, "PairLite layout");
-static_assert(sizeof(VoigtA) == kWingTerms * sizeof(float), "the activation copies VoigtA with the Cw lanes");
+static_assert(sizeof(PairLite) == 136, "PairLite layout");
+constexpr int kVoigtWords = sizeof(VoigtP) / sizeof(float);
+static_assert(kVoigtWords <= 16, "the activation copies VoigtP one word a lane");
 
 // The far-wing coefficients of wing_setup for one pair, all ten on one lane
 // (the batched set-up of the main kernel), in FP32: every term is positive,
@@ -743,18 +737,13 @@ __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int 
         r.h.inv_b = C.inv_b;
         r.h.scale = C.scale;
         r.vhigh = C.vhigh;
-        r.va = make_voigt_a(C.aa);
         // the walk uses the light form of the profile for a <= kA3Drop, as a
         // property of the pair: its coefficients are zero, so the full form
         // gives the same values and the result does not depend on which
         // pairs share a wavefront
-        if (C.aa <= (double)kA3Drop) {
-            r.va.a3_sqpi3 = 0.0f;
-            r.va.lc2 = 0.0f;
-            r.va.lc3 = 0.0f;
-        }
+        r.vp = make_voigt_p(C.aa, C.aa <= (double)kA3Drop);
         r.h.inv_nm1 = C.np > 1 ? 1.0 / (C.np - 1) : 1.0;
-        r.k = kk;
+        r.h.k = (int)(kk - w.p0);   // a row has fewer than 2^31 pairs (one per particle)
         const double inv_vs = 1.0 / C.vsmooth;
         float W[4];
 #pragma unroll
@@ -765,12 +754,10 @@ __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int 
         }
         // the walk compares with ufar rounded to FP32, the unit of the coefficients
         const float ufar = (float)C.ufar;
-        r.h.ufar = (double)ufar;
+        r.h.ufar = ufar;
         r.h.zmax = C.zmax;
         const StepShape sh = step_shape(C.np, kG);
-        r.h.nm1 = sh.nm1;
-        r.h.rounds = sh.rounds;
-        r.h.pstep = sh.pstep;
+        r.h.shape = sh.packed();
         // far-wing coefficients, in units of that ufar
         const double iu = 1.0 / (double)ufar;
         wing_coeffs((float)(C.vhigh * C.inv_b * iu), (float)(0.5 * bintov * C.inv_b * iu), sh.nm1, W[0], W[1], W[2],
@@ -786,17 +773,16 @@ __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int 
 // per lane (setup_pair and wing_setup fill the same values for the other
 // kernels).  Only the lanes of the groups taking a record call it.
 template <bool kStats>
-__device__ inline void activate_pair(const PairLite &r, PairTau &P, int glane)
+__device__ inline void activate_pair(const PairLite &r, PairWalk &P, int glane)
 {
     if (glane < kNGrid - 1) {
         const double dvk = 2. * r.vhigh / kNGrid;
         set_sample_offset(P.smp[glane], ((glane + 1) * dvk - r.vhigh) * r.h.inv_b);
         P.smp[glane].w = r.W[glane < 3 ? 3 - glane : glane - 3];   // K(q) is even in the sample offset
     }
-    if (glane < kWingTerms) {
-        P.Cw[glane] = r.Cw[glane];
-        reinterpret_cast<float *>(&P.va)[glane] = reinterpret_cast<const float *>(&r.va)[glane];
-    }
+    if (glane < kWingTerms) P.Cw[glane] = r.Cw[glane];
+    if (glane < kVoigtWords)
+        reinterpret_cast<float *>(&P.vp)[glane] = reinterpret_cast<const float *>(&r.vp)[glane];
     constexpr int kHeadWords = sizeof(WalkHead) / sizeof(long long);
     if (glane < kHeadWords)
         reinterpret_cast<long long *>(static_cast<WalkHead *>(&P))[glane] =
@@ -808,7 +794,7 @@ __device__ inline void activate_pair(const PairLite &r, PairTau &P, int glane)
 }
 
 // Voigt samples the reference evaluates for one pixel (singleabs.h:110-125).
-__device__ inline int pixel_samples(const PairTau &P, double vlow, double bintov)
+__device__ inline int pixel_samples(const PairWalk &P, double vlow, double bintov)
 {
     const double vhighp = vlow + bintov;
     const double width = vhighp - vlow;
@@ -837,7 +823,7 @@ enum { kWalkGuarded = 1, kWalkFull64 = 2 };
 // band re-evaluated in FP64 (kWalkGuarded), or all in FP64.  Returns true when
 // the walk is over (tail cut reached or end of the window).
 template <int kG, int kMode, bool kStats>
-__device__ inline bool walk_chunk(const DepositArgs &A, const PairTau &P, double *row, const float *gtab,
+__device__ inline bool walk_chunk(const DepositArgs &A, const PairTau &P, double *row, const float *ptab,
                                   const double *gtab64, int z0, int dir, int count, int c, int lane, LaneStats &st,
                                   int &walked)
 {
@@ -850,7 +836,7 @@ __device__ inline bool walk_chunk(const DepositArgs &A, const PairTau &P, double
     double t = 0, vlow = 0;
     if (valid) {
         vlow = z * bintov - P.vel;                                  // absorption.cpp:252
-        t = taulast_pixel<kMode == kWalkFull64>(P, vlow, bintov, A.velfac, A.kernel, gtab, gtab64);
+        t = taulast_pixel<kMode == kWalkFull64>(P, vlow, bintov, A.velfac, A.kernel, ptab, gtab64);
         if (kStats) {
             st.evaluated++;
             if (kMode != kWalkFull64 && fabs((vlow + 0.5 * bintov) * P.inv_b) >= P.ufar)
@@ -907,7 +893,7 @@ constexpr int kFarRounds = 4;
 // fix-up kernel when that decision falls in the guard band.  Returns true
 // when the walk is over, with `walked` set.
 template <int kG, bool kLds, bool kStats>
-__device__ inline bool settle(const DepositArgs &A, const PairTau &P, double *row, int lane, bool valid, double t,
+__device__ inline bool settle(const DepositArgs &A, const PairWalk &P, double *row, int lane, bool valid, double t,
                               int z, double vlow, int z0, int dir, int cstep, int pcount, int count, LaneStats &st,
                               long long k, int item, int &walked)
 {
@@ -952,8 +938,8 @@ __device__ inline bool settle(const DepositArgs &A, const PairTau &P, double *ro
 // or the decision deferred to the fix-up kernel); `adv` is the number of
 // pixels the step covered.
 template <int kG, bool kLds, bool kStats>
-__device__ inline bool walk_step(const DepositArgs &A, const PairTau &P, float *sbuf, double *row,
-                                 const float *gtab, int z0, int dir, int count, int c, bool far, int lane,
+__device__ inline bool walk_step(const DepositArgs &A, const PairWalk &P, float *sbuf, double *row,
+                                 const float *ptab, int z0, int dir, int count, int c, bool far, int lane,
                                  LaneStats &st, long long k, int item, bool active, int &walked, int &adv)
 {
     adv = 0;
@@ -970,7 +956,7 @@ __device__ inline bool walk_step(const DepositArgs &A, const PairTau &P, float *
             double t = 0;
             if (valid) {
                 const double U = (vlow + 0.5 * bintov) * P.inv_b;
-                const float Y = (float)(P.ufar * P.ufar) * __builtin_amdgcn_rcpf((float)(U * U));
+                const float Y = (float)((double)P.ufar * P.ufar) * __builtin_amdgcn_rcpf((float)(U * U));
                 float S = P.Cw[kWingTerms - 1];
 #pragma unroll
                 for (int q = kWingTerms - 2; q >= 0; --q) S = __builtin_fmaf(S, Y, P.Cw[q]);
@@ -987,19 +973,20 @@ __device__ inline bool walk_step(const DepositArgs &A, const PairTau &P, float *
         adv = kFarRounds * kG;
         return false;
     }
-    const int nm1 = P.nm1;
-    const int pcount = min(P.pstep, count - c);
+    const StepShape sh = unpack_shape(P.shape);
+    const int nm1 = sh.nm1;
+    const int pcount = min(sh.pstep, count - c);
     // pairs with a <= kA3Drop carry the light form of the profile (zero a^3
     // and exponent coefficients); when every pair of this near step of the
     // wavefront does, the light code runs (a wavefront-uniform branch with
     // the same results)
-    const bool a3 = __ballot(P.va.a3_sqpi3 != 0.0f) != 0ull;
+    const bool a3 = __ballot(P.vp.a3 != 0.0f) != 0ull;
     wave_sync();   // the previous step's reads of sbuf are done
     {
         const int nsub = nm1 == 0 ? pcount : pcount * nm1 + 1;
         const int zlo = dir > 0 ? z0 + c : z0 - c - (pcount - 1);
         const double vlo = zlo * bintov - P.vel;   // vlow of the step's lowest pixel (absorption.cpp:252)
-        for (int r = 0; r < P.rounds; ++r) {
+        for (int r = 0; r < sh.rounds; ++r) {
             const int m = glane + r * kG;
             if (m < nsub) {
                 double v;
@@ -1012,7 +999,7 @@ __device__ inline bool walk_step(const DepositArgs &A, const PairTau &P, float *
                     // rounding of m dv against the pixel's own vlow
                     v = __builtin_fma((double)m, bintov * P.inv_nm1, vlo);
                 }
-                sbuf[m] = (float)(a3 ? inner32<true>(P, v, gtab) : inner32<false>(P, v, gtab));
+                sbuf[m] = a3 ? inner32<true>(P, v, ptab) : inner32<false>(P, v, ptab);
                 if (kStats) st.sums++;
             }
         }
@@ -1060,7 +1047,7 @@ __device__ inline bool step_needs_wing(const PairTau &P, double bintov, int z0, 
 // Walk one direction with a kG-lane group (fix-up kernel): pixels z0,
 // z0+dir, ... for at most `count` pixels, until and including the tail cut.
 template <int kG, int kMode, bool kStats>
-__device__ inline int walk_fix(const DepositArgs &A, PairTau &P, double *row, const float *gtab,
+__device__ inline int walk_fix(const DepositArgs &A, PairTau &P, double *row, const float *ptab,
                                const double *gtab64, int z0, int dir, int count, int lane, LaneStats &st)
 {
     const double bintov = A.vbox / A.nbins;
@@ -1072,7 +1059,7 @@ __device__ inline int walk_fix(const DepositArgs &A, PairTau &P, double *row, co
             if (glane == 0) P.wing_ready = 1;
             wave_sync();
         }
-        if (walk_chunk<kG, kMode, kStats>(A, P, row, gtab, gtab64, z0, dir, count, c, lane, st, walked))
+        if (walk_chunk<kG, kMode, kStats>(A, P, row, ptab, gtab64, z0, dir, count, c, lane, st, walked))
             return walked;
     }
     return walked;
@@ -1094,19 +1081,27 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     constexpr int kWavesPerBlock = kBlock / 64;
     constexpr int kGroupsPerWave = 64 / kG;
     extern __shared__ double smem[];
-    __shared__ __attribute__((aligned(16))) float gtab[kGTableSize];
-    __shared__ PairTau pslot[kGroups];
-    __shared__ float sub_sums[kBlock * kRoundsMax];
-    __shared__ PairLite wqueue[kWavesPerBlock * kWaveQueue];
+    // The table comes first: a row number has 5 exponent bits, so a NaN's names
+    // a place past the table's octaves, which still lies in this block's LDS.
+    struct Lds {
+        __attribute__((aligned(16))) float ptab[kPTableSize];
+        PairWalk pslot[kGroups];
+        float sub_sums[kBlock * kRoundsMax];
+        PairLite wqueue[kWavesPerBlock * kWaveQueue];
+    };
+    static_assert(sizeof(Lds) >= 32 * FSAMD_P_BINS * 16, "every row number lies in the block's LDS");
+    __shared__ Lds lds;
     __shared__ int s_item;
     __shared__ unsigned long long s_next;
-    for (int i = threadIdx.x; i < kGTableSize; i += kBlock) gtab[i] = c_gtab[i];
+    const float *ptab = lds.ptab;
+    for (int i = threadIdx.x; i < kPTableSize / 4; i += kBlock)
+        reinterpret_cast<float4 *>(lds.ptab)[i] = reinterpret_cast<const float4 *>(d_ptab)[i];
     const int lane = threadIdx.x & 63;
     const int glane = lane % kG;
     const int gid = threadIdx.x / kG;
-    PairTau &P = pslot[gid];
-    float *sbuf = sub_sums + gid * kG * kRoundsMax;
-    PairLite *q = wqueue + (threadIdx.x / 64) * kWaveQueue;
+    PairWalk &P = lds.pslot[gid];
+    float *sbuf = lds.sub_sums + gid * kG * kRoundsMax;
+    PairLite *q = lds.wqueue + (threadIdx.x / 64) * kWaveQueue;
     // the wavefront's leader lanes of its groups, below this lane's group
     const unsigned long long leaders = kG == 64 ? 1ull : (kG == 32 ? 0x0000000100000001ull :
                                                          0x0001000100010001ull);
@@ -1175,7 +1170,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                     if (rank < avail) {
                         const PairLite &r = q[(head + rank) % kWaveQueue];
                         activate_pair<kStats>(r, P, glane);
-                        k = r.k;
+                        k = w.p0 + r.h.k;
                         dir = 1;
                         c = 0;
                         fresh = true;
@@ -1197,7 +1192,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             long long tc2 = 0;
             if (kStats) tc2 = clock64();
             int walked = 0, adv = 0;
-            const bool done = walk_step<kG, kLds, kStats>(A, P, sbuf, row, gtab, z0, dir, half, c, far, lane, st, k,
+            const bool done = walk_step<kG, kLds, kStats>(A, P, sbuf, row, ptab, z0, dir, half, c, far, lane, st, k,
                                                           gitem, walking, walked, adv);
             if (kStats && lane == 0) {
                 const long long tc3 = clock64();
@@ -1260,16 +1255,22 @@ template <bool kStats>
 __global__ __launch_bounds__(kThreads) void tau_fixup_kernel(DepositArgs A, const WorkItem *items)
 {
     constexpr int kGroups = kThreads / kFixG;
-    __shared__ __attribute__((aligned(16))) float gtab[kGTableSize];
-    __shared__ PairTau pslot[kGroups];
+    struct Lds {
+        __attribute__((aligned(16))) float ptab[kPTableSize];   // first: see tau_kernel
+        PairTau pslot[kGroups];
+    };
+    static_assert(sizeof(Lds) >= 32 * FSAMD_P_BINS * 16, "every row number lies in the block's LDS");
+    __shared__ Lds lds;
     __shared__ double gtab64[kG64Size];
+    const float *ptab = lds.ptab;
     const int n = (int)min(A.fix_count[0], (unsigned long long)A.fix_cap);
     if (blockIdx.x * kGroups >= n) return;
-    for (int i = threadIdx.x; i < kGTableSize; i += kThreads) gtab[i] = c_gtab[i];
+    for (int i = threadIdx.x; i < kPTableSize / 4; i += kThreads)
+        reinterpret_cast<float4 *>(lds.ptab)[i] = reinterpret_cast<const float4 *>(d_ptab)[i];
     for (int i = threadIdx.x; i < kG64Size; i += kThreads) gtab64[i] = d_gtab64[i];
     __syncthreads();
     const int lane = threadIdx.x & 63, gid = threadIdx.x / kFixG, glane = lane % kFixG;
-    PairTau &P = pslot[gid];
+    PairTau &P = lds.pslot[gid];
     LaneStats st;
     const int half = A.nbins / 2;
     for (int e = blockIdx.x * kGroups + gid; e < n; e += gridDim.x * kGroups) {
@@ -1280,14 +1281,14 @@ __global__ __launch_bounds__(kThreads) void tau_fixup_kernel(DepositArgs A, cons
         const LosInfo los = los_info(A, w.los);
         if (!setup_pair<kFixG>(A, w.line, L, los, f.k, P, glane)) continue;
         if (f.dir == 0) {
-            const int lf = walk_fix<kFixG, kWalkFull64, kStats>(A, P, out_row, gtab, gtab64, P.zmax, 1, half, lane, st);
-            const int lb = walk_fix<kFixG, kWalkFull64, kStats>(A, P, out_row, gtab, gtab64, P.zmax - 1, -1, half, lane, st);
+            const int lf = walk_fix<kFixG, kWalkFull64, kStats>(A, P, out_row, ptab, gtab64, P.zmax, 1, half, lane, st);
+            const int lb = walk_fix<kFixG, kWalkFull64, kStats>(A, P, out_row, ptab, gtab64, P.zmax - 1, -1, half, lane, st);
             if (glane == 0) {
                 record_window(A, w.line, f.k, 1, lf);
                 record_window(A, w.line, f.k, -1, lb);
             }
         } else {
-            const int l = walk_fix<kFixG, kWalkGuarded, kStats>(A, P, out_row, gtab, gtab64, f.z0, f.dir, f.count, lane, st);
+            const int l = walk_fix<kFixG, kWalkGuarded, kStats>(A, P, out_row, ptab, gtab64, f.z0, f.dir, f.count, lane, st);
             if (glane == 0) record_window(A, w.line, f.k, f.dir, (half - f.count) + l);
         }
     }
@@ -1319,12 +1320,12 @@ __global__ __launch_bounds__(kThreads) void tau_fixup_kernel(DepositArgs A, cons
 __device__ inline void adj_inner32(const PairTau &P, double vouter, const float *gtab, float &S, float &SU,
                                    float &SF)
 {
-    const Split s = split_s(vouter * P.inv_b);
+    const double s2 = vouter * (2.0 * P.inv_b);
     const VoigtA va = P.va;
 #pragma unroll  // full: the adjoint kernel 6% faster than unrolling by 2 at 128^3
     for (int i = 0; i < kNGrid - 1; ++i) {
         const KernelSample k = P.smp[i];
-        const VoigtGrad g = voigt32_grad(va, sample_u(k, s), gtab);
+        const VoigtGrad g = voigt32_grad(va, 0.5f * sample_u2(k, s2), gtab);
         const float w = k.w;
         S = __builtin_fmaf(w, g.H, S);
         SU = __builtin_fmaf(w, g.Hu, SU);
@@ -1862,10 +1863,10 @@ __global__ __launch_bounds__(kColThreads) void colden_kernel(DepositArgs A, cons
 __global__ __launch_bounds__(kThreads) void voigt_peak_kernel(long long per_thread, double du, double umax,
                                                               float a, float *sink)
 {
-    __shared__ __attribute__((aligned(16))) float gtab[kGTableSize];
-    for (int i = threadIdx.x; i < kGTableSize; i += kThreads) gtab[i] = c_gtab[i];
+    __shared__ __attribute__((aligned(16))) float ptab[32 * FSAMD_P_BINS * 4];
+    for (int i = threadIdx.x; i < kPTableSize; i += kThreads) ptab[i] = d_ptab[i];
     __syncthreads();
-    const VoigtA va = make_voigt_a(a);
+    const VoigtP va = make_voigt_p(a, false);
     const long long tid = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     const long long nthreads = (long long)gridDim.x * blockDim.x;
     float acc = 0.0f;
@@ -1873,7 +1874,7 @@ __global__ __launch_bounds__(kThreads) void voigt_peak_kernel(long long per_thre
     double u = fmod((double)tid * du, umax);
     const double step = fmod((double)nthreads * du, umax);
     for (long long i = 0; i < per_thread; ++i) {
-        acc = __builtin_fmaf(w, voigt32(va, (float)u, gtab), acc);
+        acc = __builtin_fmaf(w, voigt32(va, (float)u, ptab), acc);
         u += step;
         if (u >= umax) u -= umax;
     }
@@ -1885,12 +1886,12 @@ __global__ __launch_bounds__(kThreads) void voigt_peak_kernel(long long per_thre
 // parameter is set up as for a pair.
 __global__ __launch_bounds__(kThreads) void voigt_eval_kernel(const double *u, long long n, double a, float *out)
 {
-    __shared__ __attribute__((aligned(16))) float gtab[kGTableSize];
-    for (int i = threadIdx.x; i < kGTableSize; i += kThreads) gtab[i] = c_gtab[i];
+    __shared__ __attribute__((aligned(16))) float ptab[32 * FSAMD_P_BINS * 4];
+    for (int i = threadIdx.x; i < kPTableSize; i += kThreads) ptab[i] = d_ptab[i];
     __syncthreads();
-    const VoigtA va = make_voigt_a(a);
+    const VoigtP va = make_voigt_p(a, false);
     for (long long i = blockIdx.x * (long long)kThreads + threadIdx.x; i < n; i += (long long)gridDim.x * kThreads)
-        out[i] = voigt32(va, (float)u[i], gtab);
+        out[i] = voigt32(va, (float)u[i], ptab);
 }
 
 int launch_voigt_eval(const double *u, long long n, double a, float *out, hipStream_t s)

@@ -1,0 +1,76 @@
+"""Generate profile_table.h: G(u) = 1 - 2u D(u) (D: Dawson's integral) as cubics
+in t = 4u^2 + 2, indexed by the bits of t.
+
+G is the real-axis factor of the damping term of the Voigt function,
+    Re w(u + ia) = exp(a^2 - u^2) cos(2au) - (2/sqrt(pi)) (a G(u) - a^3/6 D'''(u) + ...),
+and an even entire function of u.  Every octave of t is cut into BINS equal
+bins, so that a bin's number is the low exponent bits and the first mantissa
+bits of t as a float, and its left edge is t with the other mantissa bits
+cleared: neither core and wing nor small and large u need a case of their
+own.  The 2 keeps t at or above an exponent whose low five bits are zero; the
+4 puts the first bins, near u = 0, where G has structure on p = u^2 ~ 1, at a
+width of 1/64 in p.  Row r holds the four coefficients of the cubic in
+t - edge (one 128-bit LDS read), a Chebyshev fit in float64 weighted by
+1/|G|: within a bin t varies by at most 1/32 of itself, which holds the
+truncation below 2e-8 of G (4.2e-8 of 0.01 next to its zero), less than the
+float32 rounding that the evaluation adds (4.5e-8 rms).  G comes from scipy.special.dawsn, beyond u = 9 from its
+asymptotic series -sum_n (2n-1)!!/(2 u^2)^n.
+
+Run:  python fake_spectra_amd/csrc/gen_profile_table.py > fake_spectra_amd/csrc/profile_table.h
+"""
+import numpy as np
+from scipy.special import dawsn
+
+OCTAVES = 28
+BINS = 32
+
+
+def g64(p):
+    """G at u^2 = p."""
+    u = np.sqrt(p)
+    x = 1 / np.maximum(p, 1e-300)
+    s = np.zeros_like(p)
+    coef = np.cumprod([1.0] + [(2 * n - 1) / 2.0 for n in range(1, 16)])
+    for n in range(15, 0, -1):
+        s = (s + coef[n]) * x
+    return np.where(u > 9.0, -s, 1 - 2 * u * dawsn(u))
+
+
+def rows():
+    th = np.cos(np.pi * (np.arange(24) + 0.5) / 24)
+    out, worst = [], 0.0
+    for e in range(1, OCTAVES + 1):
+        w = 2.0 ** e / BINS
+        for m in range(BINS):
+            lo = 2.0 ** e + m * w
+            g = g64((lo + (th + 1) / 2 * w - 2) / 4)
+            c = np.polynomial.chebyshev.chebfit(th, g, 3, w=1 / np.maximum(np.abs(g), 0.01 if lo < 16 else 0.0))
+            # a polynomial in t - lo
+            mono = np.polynomial.Polynomial(np.polynomial.chebyshev.cheb2poly(c))(
+                np.polynomial.Polynomial([-1.0, 2.0 / w])).coef
+            v = np.linspace(0, w, 101)
+            ref = g64((lo + v - 2) / 4)
+            err = np.abs(np.polyval(mono[::-1], v) - ref) / np.maximum(np.abs(ref), 0.01 if lo < 16 else 0.0)
+            worst = max(worst, float(err.max()))
+            out.append(mono)
+    return out, worst
+
+
+def main():
+    r, worst = rows()
+    print("/* Generated by gen_profile_table.py; do not edit. */")
+    print("/* G(u) = 1 - 2u D(u): cubics in t - edge, t = 4u^2 + 2, %d bins in each of %d octaves of t from 2" % (
+        BINS, OCTAVES))
+    print("   (max float64 fit error %.2g of G, of 0.01 near its zero). */" % worst)
+    print("#pragma once")
+    print("#define FSAMD_P_OCTAVES %d" % OCTAVES)
+    print("#define FSAMD_P_BINS %d" % BINS)
+    print("/* initializer for a float[FSAMD_P_OCTAVES * FSAMD_P_BINS * 4] array */")
+    print("#define FSAMD_P_COEF_INIT { \\")
+    for c in r:
+        print("    " + ", ".join("%.9ef" % v for v in c) + ", \\")
+    print("}")
+
+
+if __name__ == "__main__":
+    main()

@@ -9,21 +9,15 @@
 //  with G = 1 - 2u D(u) = D'(u) (D: Dawson's integral).  This is the Taylor
 //  series of w about the real axis, whose even terms sum to Re exp(-z^2) and
 //  whose odd terms are those of the entire function (2i/sqrt(pi)) D(z); the
-//  a^5 term is below 1e-7 relative for a <= 0.04.
-//  |u| < 7:  G from a piecewise polynomial table, Z = -D'''/3 with
-//            D''' = (4u^2 - 6) G + 2;
-//  |u| >= 7: G = x R(x), x = 1/u^2, R a polynomial that follows the
-//            asymptotic series w ~ (i/sqrt(pi)) sum_n (2n-1)!!/2^n z^-(2n+1)
-//            (the last table row holds x R(x) as a polynomial in x); Z = x^2 Q(x), Q = sum C(2n+3,3) (2n-1)!!/2^n x^n (3 terms),
-//            the a^3 term of the same series, free of the cancellation in D'''.
-//  Each lane picks its table row (a core piece or the wing row) and its a^3
-//  form by selects, and every lane runs the same instructions, so the
-//  wavefront never diverges on |u|.
+//  a^5 term is below 1e-7 relative for a <= 0.04.  G comes from one table of
+//  cubics in t = 4u^2 + 2 (profile_table.h) whose row number and bin edge are
+//  bits of t, so core, transition and wing are one code without selects, and
+//  exp(a^2 - u^2) cos(2au) is one exp2 of a polynomial in u^2;
+//  D''' = (4u^2 - 6) G + 2, and -12 G^2 beyond u = 20.
 //
-// u arrives in FP32.  The deposit forms it as (c_hi - s_hi) + (c_lo - s_lo)
-// from two-float splits of the kernel-sample offset c and of the sub-sample
-// velocity s (s from the pixel's FP64 position), so u carries ~1 ulp relative
-// error even where c and s nearly cancel; u^2 and the exponent of
+// u arrives in FP32.  The deposit subtracts the sub-sample velocity from the
+// kernel-sample offset in FP64 and rounds the difference, so u carries half
+// an ulp even where the two nearly cancel; u^2 and the exponent of
 // exp(a^2 - u^2) are FP32, and exp amplifies their relative error by ~2u^2
 // ln2: the Gaussian term carries ~1.2e-7 u^2 relative error on top of the
 // expansions' 3.6e-7 (measured against scipy.special.wofz, a <= 0.04,
@@ -39,6 +33,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include "dawson_table.h"
+#include "profile_table.h"
 #include "dawson64_table.h"
 
 namespace fsamd {
@@ -58,17 +53,14 @@ constexpr int kGTableSize = FSAMD_G_NROW * FSAMD_G_STRIDE;
 // C(2n+3,3) (2n-1)!!/2^n, n = 0..2
 #define FSAMD_WING_Q {1.0f, 5.0f, 26.25f}
 
-// Per-pair constants of the FP32 profile.
+// Per-pair constants of the FP32 profile's derivatives (voigt32_grad).
 struct VoigtA {
     float a;            // damping parameter
     float a2;           // a^2
     float a2_6;         // a^2 / 6
     float two_a_sqpi;   // 2a/sqrt(pi)
     float a_sqpi;       // a/sqrt(pi)
-    float a3_sqpi3;     // a^3/(3 sqrt(pi))
     float a2_log2e;     // a^2 log2(e)
-    // log2 of Re exp(-(u + ia)^2) = a2_log2e + lc1 u^2 + lc2 u^4 + lc3 u^6 (voigt32)
-    float lc1, lc2, lc3;
 };
 
 __device__ inline VoigtA make_voigt_a(double a)
@@ -79,12 +71,7 @@ __device__ inline VoigtA make_voigt_a(double a)
     v.a2_6 = (float)(a * a * (1.0 / 6.0));
     v.two_a_sqpi = (float)(a * kTwoOverSqrtPi);
     v.a_sqpi = (float)(a * (1.0 / kSqrtPi));
-    v.a3_sqpi3 = (float)(a * a * a * (1.0 / (3.0 * kSqrtPi)));
     v.a2_log2e = (float)(a * a * kLog2E);
-    const double a2 = a * a;
-    v.lc1 = (float)(-(1.0 + 2.0 * a2) * kLog2E);
-    v.lc2 = (float)(-(4.0 / 3.0) * a2 * a2 * kLog2E);
-    v.lc3 = (float)(-(64.0 / 45.0) * a2 * a2 * a2 * kLog2E);
     return v;
 }
 
@@ -95,49 +82,76 @@ __device__ inline VoigtA make_voigt_a(double a)
 // scipy.special.wofz).
 constexpr float kA3Drop = 2e-3f;
 
-// H(a, u) with u the sample's offset from the line centre in units of b,
-// any u.  The table `tab` is 16-byte aligned.  kA3 = false: the light form
-// (for a <= kA3Drop), which equals the full one when a3_sqpi3, lc2 and lc3
-// are zero.
-template <bool kA3 = true>
-__device__ inline float voigt32(const VoigtA &v, float u, const float *tab)
+// Per-pair constants of the FP32 profile.
+struct VoigtP {
+    // log2 of Re exp(-(u + ia)^2) = exp(a^2 - u^2) cos(2au), with ln cos x =
+    // -x^2/2 - x^4/12 - x^6/45 - ...:  l0 + l1 t + l2 u^4 + l3 u^6, t = 4u^2 + 2,
+    // from log2(e) (a^2 - (1 + 2a^2) u^2 - (4/3) a^4 u^4 - (64/45) a^6 u^6); the
+    // dropped term, (17/2520)(2au)^8, changes H by < 5e-9 relative for a <= 0.04
+    float l0, l1, l2, l3;
+    float two_a_sqpi;   // 2a/sqrt(pi)
+    float a3;           // -a^2/6, 0 in the light form
+};
+
+// light (a <= kA3Drop): the terms of the light form are zero, so the full
+// code gives the light form's values.
+__device__ inline VoigtP make_voigt_p(double a, bool light)
 {
-    static_assert(FSAMD_G_DEG == 6 && FSAMD_G_STRIDE % 4 == 0 && FSAMD_G_STRIDE >= 8, "voigt32 evaluates 7 coefficients per row");
-    const float uh = __builtin_fabsf(u);
-    const float p = u * u;
-    // Re exp(-(u + ia)^2) = exp(a^2 - u^2) cos(2au) = 2^y, with ln cos x =
-    // -x^2/2 - x^4/12 - x^6/45 - ...:  y = log2(e) (a^2 - (1 + 2a^2) u^2 -
-    // (4/3) a^4 u^4 - (64/45) a^6 u^6).  The dropped term, (17/2520)(2au)^8,
-    // changes H by < 5e-9 relative for a <= 0.04 (against scipy's wofz); the
-    // u^4 and u^6 terms are small next to the u^2 one, so y keeps the
-    // rounding of its first fma.  2^y is 0 once y passes the FP32 range.
-    const float y = __builtin_fmaf(p, v.lc1, v.a2_log2e);
-    const float re_exp = __builtin_amdgcn_exp2f(kA3 ? __builtin_fmaf(p * p, __builtin_fmaf(p, v.lc3, v.lc2), y) : y);
-    // G: table piece (|u| < 7) or the wing row, selected per lane; both rows
-    // are polynomials in their variable, so G is the row's Horner sum
-    const float x = __builtin_amdgcn_rcpf(p);
-    const bool core = uh < kVoigtCoreMax;
-    const float q = uh * (1.0f / FSAMD_G_WIDTH);
-    // piece q (variable: the fractional part of q) or the wing row (variable x)
-    constexpr int kRowBytes = FSAMD_G_STRIDE * (int)sizeof(float);
-    const int off = core ? (int)q * kRowBytes : FSAMD_G_NPIECE * kRowBytes;
-    const float var = core ? __builtin_amdgcn_fractf(q) : x;
-    const float *row = (const float *)((const char *)tab + off);
-    const float4 lo = *(const float4 *)row;
-    const float4 hi = *(const float4 *)(row + 4);
-    float r = __builtin_fmaf(hi.z, var, hi.y);
-    r = __builtin_fmaf(r, var, hi.x);
-    r = __builtin_fmaf(r, var, lo.w);
-    r = __builtin_fmaf(r, var, lo.z);
-    r = __builtin_fmaf(r, var, lo.y);
-    const float G = __builtin_fmaf(r, var, lo.x);
-    if constexpr (!kA3) return __builtin_fmaf(-v.two_a_sqpi, G, re_exp);
-    // a^3 term, -(a^3/sqrt(pi)) Z = (a^3/(3 sqrt(pi))) D with D = D''' =
-    // (4u^2 - 6) G + 2, or D = -3 Z = -3 x^2 (1 + 5x + 26.25x^2) in the wing
-    const float Dc = __builtin_fmaf(__builtin_fmaf(4.0f, p, -6.0f), G, 2.0f);
-    const float Dw = x * x * __builtin_fmaf(__builtin_fmaf(-78.75f, x, -15.0f), x, -3.0f);
-    const float D = core ? Dc : Dw;
-    return __builtin_fmaf(v.a3_sqpi3, D, __builtin_fmaf(-v.two_a_sqpi, G, re_exp));
+    const double a2 = a * a, lc1 = -(1.0 + 2.0 * a2) * kLog2E;
+    VoigtP v;
+    v.l0 = (float)(a2 * kLog2E - 0.5 * lc1);
+    v.l1 = (float)(0.25 * lc1);
+    v.l2 = light ? 0.0f : (float)(-(4.0 / 3.0) * a2 * a2 * kLog2E);
+    v.l3 = light ? 0.0f : (float)(-(64.0 / 45.0) * a2 * a2 * a2 * kLog2E);
+    v.two_a_sqpi = (float)(a * kTwoOverSqrtPi);
+    v.a3 = light ? 0.0f : (float)(a2 * (-1.0 / 6.0));
+    return v;
+}
+
+// Largest |u| whose t lies in the table, and the LDS the table takes.
+constexpr double kVoigtUMax = 1.1e4;
+constexpr int kPTableSize = FSAMD_P_OCTAVES * FSAMD_P_BINS * 4;
+static_assert(FSAMD_P_BINS == 32 && 4.0 * kVoigtUMax * kVoigtUMax + 2.0 < (double)(2u << FSAMD_P_OCTAVES),
+              "profile_table.h");
+
+// The two terms of H(a, u) = E - (2a/sqrt(pi)) G at u = us/2, |u| <= kVoigtUMax:
+// sums over samples take them separately and combine them once.  The
+// Gaussian's exponent and the table's argument come from the same t; its
+// mantissa's first 5 bits and exponent name the row, its remaining bits are
+// the cubic's variable.  14 VALU instructions and one 16-byte LDS read a
+// sample in the light form (kA3 = false; 22 and two reads with a table in u and
+// a selected wing row), 22 in the full one (35).
+template <bool kA3 = true>
+__device__ inline void voigt_terms(const VoigtP &v, float us, const float *tab, float &E, float &G)
+{
+    const float t = __builtin_fmaf(us, us, 2.0f);
+    float y = __builtin_fmaf(t, v.l1, v.l0);
+    if (kA3) {
+        const float p = __builtin_fmaf(t, 0.25f, -0.5f);
+        y = __builtin_fmaf(p * p, __builtin_fmaf(p, v.l3, v.l2), y);
+    }
+    E = __builtin_amdgcn_exp2f(y);    // 0 once y passes the FP32 range
+    const unsigned edge = __float_as_uint(t) & 0xfffc0000u;
+    const float d = t - __uint_as_float(edge);
+    const float4 c = *(const float4 *)((const char *)tab + __builtin_amdgcn_ubfe(edge, 14, 14));
+    G = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(c.w, d, c.z), d, c.y), d, c.x);
+    if (kA3) {
+        // -(a^2/6) D''': (4u^2 - 6) G + 2 loses its digits as 1/u^4, where G -> -1/(2u^2)
+        const float D = t > 1602.0f ? G * (G * -12.0f) : __builtin_fmaf(t - 8.0f, G, 2.0f);
+        G = __builtin_fmaf(v.a3, D, G);
+    }
+}
+
+// H(a, u) at any u (diagnostics): beyond the table the asymptotic series.
+__device__ inline float voigt32(const VoigtP &v, float u, const float *tab)
+{
+    if (!(__builtin_fabsf(u) <= (float)kVoigtUMax)) {
+        const float x = 1.0f / (u * u);
+        return 0.5f * v.two_a_sqpi * __builtin_fmaf(1.5f * x, x, x);
+    }
+    float E, G;
+    voigt_terms(v, 2.0f * u, tab, E, G);
+    return __builtin_fmaf(-v.two_a_sqpi, G, E);
 }
 
 // ---------------------------------------------------------------------------
@@ -177,7 +191,7 @@ __device__ inline VoigtGrad voigt32_grad(const VoigtA &v, float u, const float *
         r.F = v.a_sqpi * x * f;
         return r;
     }
-    // exp(a^2 - u^2) as in voigt32
+    // exp(a^2 - u^2)
     const float p = uh * uh;
     const float E = __builtin_amdgcn_exp2f(__builtin_fmaf(p, -kLog2EF, v.a2_log2e));
     const float c = 2.0f * v.a * uh;
