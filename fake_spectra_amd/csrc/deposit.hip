@@ -159,6 +159,22 @@ __device__ inline int wrap_pixel(int z, int nbins)
     return j < 0 ? j + nbins : j;
 }
 
+// Box lengths by which pixel z lies outside [0, nbins): a walk from there is
+// the same walk moved back by as many.
+__device__ inline int box_shift(int z, int nbins)
+{
+    if (z >= 0 && z < nbins) return 0;
+    const int q = z / nbins;
+    return z - q * nbins < 0 ? q - 1 : q;
+}
+
+// A pixel of a walk that starts inside the box (walks go at most half a box).
+__device__ inline int wrap_near(int z, int nbins)
+{
+    if (z >= nbins) z -= nbins;
+    return z < 0 ? z + nbins : z;
+}
+
 // Per-pair constants of LineAbsorption::add_tau_particle and SingleAbsorber.
 // Each wavefront keeps the constants of its current pair in an LDS slot: the
 // values are uniform across the wave, and reading them with broadcast LDS
@@ -236,12 +252,11 @@ __device__ inline double shfl_d(double v, int src)
 }
 
 // sum_i K(q_i) Re w((vv_i - vouter)/b + i a), FP32 profile; the sample
-// offsets from the FP64 anchor vouter/b.  kA3 = false: the light form of the
-// profile (pairs with a <= kA3Drop).
+// offsets from the FP64 anchor s2 = 2 vouter/b.  kA3 = false: the light form
+// of the profile (pairs with a <= kA3Drop).
 template <bool kA3 = true>
-__device__ inline float inner32(const PairWalk &P, double vouter, const float *ptab)
+__device__ inline float inner32(const PairWalk &P, double s2, const float *ptab)
 {
-    const double s2 = vouter * (2.0 * P.inv_b);
     const VoigtP vp = P.vp;
     float sE = 0.0f, sG = 0.0f;
 #pragma unroll  // full: 5% faster than unrolling by 2 at 256^3 and 512^3 (same operation order)
@@ -291,7 +306,7 @@ __device__ inline double taulast_pixel(const PairTau &P, double vlow, double bin
             return P.scale * (double)(S * Y);
         }
     }
-    auto inner = [&](double v) { return k64 ? inner64(P, v, kernel, gtab64) : inner32(P, v, ptab); };
+    auto inner = [&](double v) { return k64 ? inner64(P, v, kernel, gtab64) : inner32(P, v * (2.0 * P.inv_b), ptab); };
     if (width < P.b / 2.) return P.scale * inner((vhighp + vlow) / 2.);
     const int np = 2 * ceil(width / (P.b / 2.) / 2) + 1.;
     const double dv = width / (np - 1);
@@ -474,6 +489,27 @@ __device__ inline unsigned long long group_bits(unsigned long long m, int lane)
 {
     if (kG == 64) return m;
     return (m >> ((lane / kG) * kG)) & ((1ull << kG) - 1ull);
+}
+
+// The first lane of this lane's group whose bit is set in m (counted from the
+// group's first lane), kG if none.
+template <int kG>
+__device__ inline int group_first(unsigned long long m, int lane)
+{
+    if (kG == 64) return m ? __builtin_ctzll(m) : 64;
+    unsigned b = lane & 32 ? (unsigned)(m >> 32) : (unsigned)m;
+    if (kG == 32) return b ? __builtin_ctz(b) : 32;
+    b = (b >> (lane & 16)) & 0xffffu;
+    return __builtin_ctz(b | 0x10000u);
+}
+
+// Bit `i` (< kG) of this lane's group in m.
+template <int kG>
+__device__ inline bool group_bit(unsigned long long m, int lane, int i)
+{
+    if (kG == 64) return (m >> i) & 1ull;
+    const unsigned b = lane & 32 ? (unsigned)(m >> 32) : (unsigned)m;
+    return (b >> ((kG == 16 ? lane & 16 : 0) + i)) & 1u;
 }
 
 struct LaneStats {
@@ -733,7 +769,9 @@ __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int 
     wave_sync();   // the records taken earlier have been read
     if (enq) {
         PairLite &r = q[(tail + __popcll(m & ((1ull << lane) - 1ull))) % kWaveQueue];
-        r.h.vel = C.vel;
+        const int shift = box_shift(C.zmax, A.nbins);
+        r.h.vel = shift ? C.vel - shift * A.vbox : C.vel;
+        r.h.zmax = C.zmax - shift * A.nbins;
         r.h.inv_b = C.inv_b;
         r.h.scale = C.scale;
         r.vhigh = C.vhigh;
@@ -755,7 +793,6 @@ __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int 
         // the walk compares with ufar rounded to FP32, the unit of the coefficients
         const float ufar = (float)C.ufar;
         r.h.ufar = ufar;
-        r.h.zmax = C.zmax;
         const StepShape sh = step_shape(C.np, kG);
         r.h.shape = sh.packed();
         // far-wing coefficients, in units of that ufar
@@ -882,97 +919,76 @@ __device__ inline bool walk_chunk(const DepositArgs &A, const PairTau &P, double
     return false;
 }
 
-// Far steps cover this many groups of kG pixels (the moment expansion is a
-// few FMAs per pixel, so a far walk advances several sub-steps while the
-// other groups of the wavefront evaluate their near pixels).
-constexpr int kFarRounds = 4;
+// The tail cut's guard band as two limits: a pixel above hi goes on, below lo
+// it ends the walk, between them FP64 decides (the fix-up kernel).
+struct CutBand {
+    double lo, hi;
+};
 
-// End of one sub-step of a walk (lanes glane < pcount hold the pixels
-// cstep + glane of the walk, value t): deposit up to and including the first
-// pixel below tautail (absorption.cpp:260-263), or hand the walk to the
-// fix-up kernel when that decision falls in the guard band.  Returns true
-// when the walk is over, with `walked` set.
-template <int kG, bool kLds, bool kStats>
-__device__ inline bool settle(const DepositArgs &A, const PairWalk &P, double *row, int lane, bool valid, double t,
-                              int z, double vlow, int z0, int dir, int cstep, int pcount, int count, LaneStats &st,
-                              long long k, int item, int &walked)
+__device__ inline CutBand cut_band(double tautail) { return CutBand{tautail - kGuard * tautail, tautail + kGuard * tautail}; }
+
+// A walk that has reached the far wing, by the whole wavefront, 64 pixels at a
+// time: |U| only grows from there, so this ends the walk.  zf: its next pixel,
+// count: the pixels left.  P and the arguments are uniform, so the tail cut
+// (deposit up to and including the first pixel below tautail,
+// absorption.cpp:260-263) is scalar work.  In steps of 4 x kG pixels by the
+// walk's own group (four rounds of ~90 instructions in which the other groups
+// idle) the kernel took 127 instead of 94 ms at 256^3 x 5000 x 2048, two lines.
+// Returns the pixels walked, or -1 where the decision went to the fix-up
+// kernel.
+template <bool kLds, bool kStats>
+__device__ inline int far_walk(const DepositArgs &A, const PairWalk &P, double *row, int zf, int dir, int count,
+                               const CutBand &cut, int lane, LaneStats &st, long long k, int item)
 {
-    const int glane = lane % kG;
-    const double tt = A.tautail;
-    const bool guard = valid && fabs(t - tt) <= kGuard * tt;
-    const unsigned long long mb = group_bits<kG>(__ballot(valid && !guard && t < tt), lane);
-    const unsigned long long mg = group_bits<kG>(__ballot(guard), lane);
-    const unsigned long long mall = mb | mg;
-    const int first = mall ? __builtin_ctzll(mall) : kG;
-    if (valid && (glane < first || (glane == first && ((mb >> glane) & 1ull)))) {
-        row_add<kLds>(&row[wrap_pixel(z, A.nbins)], t);
-        if (kStats) {
-            st.pixels++;
-            st.samples += pixel_samples(P, vlow, A.vbox / A.nbins);
+    const double bintov = A.vbox / A.nbins;
+    const float uf2 = (float)((double)P.ufar * P.ufar);
+    for (int i0 = 0; i0 < count; i0 += 64) {
+        const int i = i0 + lane;
+        const bool valid = i < count;
+        const int z = zf + dir * i;
+        const double vlow = z * bintov - P.vel;
+        const double U = (vlow + 0.5 * bintov) * P.inv_b;
+        const float Y = uf2 * __builtin_amdgcn_rcpf((float)(U * U));
+        float S = P.Cw[kWingTerms - 1];
+#pragma unroll
+        for (int q = kWingTerms - 2; q >= 0; --q) S = __builtin_fmaf(S, Y, P.Cw[q]);
+        const double t = P.scale * (double)(S * Y);
+        const unsigned long long stop = __ballot(valid && t <= cut.hi), below = __ballot(valid && t < cut.lo);
+        const int first = stop ? __builtin_ctzll(stop) : 64;
+        const bool sure = stop && ((below >> (first & 63)) & 1ull);
+        if (kStats && valid) {
+            st.evaluated++;
+            st.far++;
+        }
+        if (valid && (lane < first || (lane == first && sure))) {
+            row_add<kLds>(&row[wrap_near(z, A.nbins)], t);
+            if (kStats) {
+                st.pixels++;
+                st.samples += pixel_samples(P, vlow, bintov);
+            }
+        }
+        if (stop) {
+            if (sure) return i0 + first + 1;
+            // the FP32 value of the deciding pixel is too close to tautail
+            if (lane == 0) push_fixup(A, k, item, zf + dir * (i0 + first), count - (i0 + first), dir);
+            return -1;
         }
     }
-    if (first < kG && ((mg >> first) & 1ull)) {
-        // the FP32 value of the deciding pixel is too close to tautail
-        if (glane == 0) push_fixup(A, k, item, z0 + dir * (cstep + first), count - (cstep + first), dir);
-        walked = -1;
-        return true;
-    }
-    if (mb != 0) {
-        walked = cstep + first + 1;
-        return true;
-    }
-    if (cstep + pcount >= count) {
-        walked = count;
-        return true;
-    }
-    return false;
+    return count;
 }
 
-// One step of a walk in the main kernel (lane glane of a kG-lane group):
-// the next pixels z0 + dir*(c + p) of the walk.  Pixels whose centre lies in
-// the far wing take the moment expansion: a step is a far step when its
-// first pixel is (|U| only grows along a walk) and then covers kFarRounds
-// sub-steps of kG pixels.  A near step covers P.pstep pixels on the shared
-// sub-sample grid; `sbuf` is the group's LDS scratch of kG * kRoundsMax
-// floats.  Returns true when the walk is over (tail cut, end of the window,
-// or the decision deferred to the fix-up kernel); `adv` is the number of
-// pixels the step covered.
+// One near step of a walk (lane glane of a kG-lane group): the next sh.pstep
+// pixels z0 + dir*(c + p), on the sub-sample grid they share; `sbuf` is the
+// group's LDS scratch of kG * kRoundsMax floats.  Returns true when the walk is
+// over (tail cut, end of the window, or the decision deferred to the fix-up
+// kernel), with `walked` set; `adv` is the number of pixels the step covered.
 template <int kG, bool kLds, bool kStats>
-__device__ inline bool walk_step(const DepositArgs &A, const PairWalk &P, float *sbuf, double *row,
-                                 const float *ptab, int z0, int dir, int count, int c, bool far, int lane,
-                                 LaneStats &st, long long k, int item, bool active, int &walked, int &adv)
+__device__ inline bool near_step(const DepositArgs &A, const PairWalk &P, float *sbuf, double *row, const float *ptab,
+                                 int z0, int dir, int count, int c, const CutBand &cut, int lane, LaneStats &st,
+                                 long long p0, int item, int &walked, int &adv)
 {
-    adv = 0;
-    if (!active) return false;
     const int glane = lane % kG;
     const double bintov = A.vbox / A.nbins;
-    if (far) {
-        for (int r = 0; r < kFarRounds; ++r) {
-            const int cc = c + r * kG;
-            const int pc = min(kG, count - cc);
-            const bool valid = glane < pc;
-            const int z = z0 + dir * (cc + glane);
-            const double vlow = z * bintov - P.vel;
-            double t = 0;
-            if (valid) {
-                const double U = (vlow + 0.5 * bintov) * P.inv_b;
-                const float Y = (float)((double)P.ufar * P.ufar) * __builtin_amdgcn_rcpf((float)(U * U));
-                float S = P.Cw[kWingTerms - 1];
-#pragma unroll
-                for (int q = kWingTerms - 2; q >= 0; --q) S = __builtin_fmaf(S, Y, P.Cw[q]);
-                t = P.scale * (double)(S * Y);
-                if (kStats) {
-                    st.evaluated++;
-                    st.far++;
-                }
-            }
-            if (settle<kG, kLds, kStats>(A, P, row, lane, valid, t, z, vlow, z0, dir, cc, pc, count, st, k, item,
-                                         walked))
-                return true;
-        }
-        adv = kFarRounds * kG;
-        return false;
-    }
     const StepShape sh = unpack_shape(P.shape);
     const int nm1 = sh.nm1;
     const int pcount = min(sh.pstep, count - c);
@@ -983,49 +999,58 @@ __device__ inline bool walk_step(const DepositArgs &A, const PairWalk &P, float 
     const bool a3 = __ballot(P.vp.a3 != 0.0f) != 0ull;
     wave_sync();   // the previous step's reads of sbuf are done
     {
+        // Sub-sample m of the step, in increasing velocity: sub-sample m mod
+        // (np-1) of its pixel (singleabs.h:118-121) up to the rounding of m dv
+        // against the pixel's own vlow, or (np = 1) pixel m's centre
+        // (singleabs.h:113); positions as 2 v / b.
         const int nsub = nm1 == 0 ? pcount : pcount * nm1 + 1;
         const int zlo = dir > 0 ? z0 + c : z0 - c - (pcount - 1);
-        const double vlo = zlo * bintov - P.vel;   // vlow of the step's lowest pixel (absorption.cpp:252)
+        const double ib2 = 2.0 * P.inv_b;
+        double vlo = zlo * bintov - P.vel;   // vlow of the step's lowest pixel (absorption.cpp:252)
+        if (nm1 == 0) vlo += 0.5 * bintov;
+        const double s2 = vlo * ib2, ds2 = bintov * P.inv_nm1 * ib2;
         for (int r = 0; r < sh.rounds; ++r) {
             const int m = glane + r * kG;
             if (m < nsub) {
-                double v;
-                if (nm1 == 0) {
-                    const double vlow = (z0 + dir * (c + m)) * bintov - P.vel;   // absorption.cpp:252
-                    v = ((vlow + bintov) + vlow) / 2.;                           // singleabs.h:113
-                } else {
-                    // sub-sample m of the step, in increasing velocity: sub-sample
-                    // m mod (np-1) of its pixel (singleabs.h:118-121), up to the
-                    // rounding of m dv against the pixel's own vlow
-                    v = __builtin_fma((double)m, bintov * P.inv_nm1, vlo);
-                }
-                sbuf[m] = a3 ? inner32<true>(P, v, ptab) : inner32<false>(P, v, ptab);
+                const double at = __builtin_fma((double)m, ds2, s2);
+                sbuf[m] = a3 ? inner32<true>(P, at, ptab) : inner32<false>(P, at, ptab);
                 if (kStats) st.sums++;
             }
         }
     }
     wave_sync();
     const bool valid = glane < pcount;
-    const int z = z0 + dir * (c + glane);
-    const double vlow = z * bintov - P.vel;
     double t = 0;
     if (valid) {
-        if (nm1 == 0) {
-            t = P.scale * (double)sbuf[glane];
-        } else {
-            // trapezoid over the pixel's sub-samples (singleabs.h:116-125)
-            const int j = dir > 0 ? glane : pcount - 1 - glane;
-            const float *sp = sbuf + j * nm1;
-            double tot = 0.5 * (double)sp[0];
-            for (int kk = 1; kk < nm1; ++kk) tot += (double)sp[kk];
-            tot += 0.5 * (double)sp[nm1];
-            t = P.scale * (tot * P.inv_nm1);
-        }
+        // trapezoid over the pixel's sub-samples (singleabs.h:116-125); np = 1:
+        // both ends are the one sample
+        const int j = dir > 0 ? glane : pcount - 1 - glane;
+        const float *sp = sbuf + (nm1 == 0 ? j : j * nm1);
+        double tot = 0.5 * ((double)sp[0] + (double)sp[nm1]);
+        for (int kk = 1; kk < nm1; ++kk) tot += (double)sp[kk];
+        t = P.scale * (tot * P.inv_nm1);
         if (kStats) st.evaluated++;
     }
     adv = pcount;
-    return settle<kG, kLds, kStats>(A, P, row, lane, valid, t, z, vlow, z0, dir, c, pcount, count, st, k, item,
-                                    walked);
+    const unsigned long long stop = __ballot(valid && t <= cut.hi), below = __ballot(valid && t < cut.lo);
+    const int first = group_first<kG>(stop, lane);
+    const bool sure = first < kG && group_bit<kG>(below, lane, first & (kG - 1));
+    const int z = z0 + dir * (c + glane);
+    if (valid && (glane < first || (glane == first && sure))) {
+        row_add<kLds>(&row[wrap_near(z, A.nbins)], t);
+        if (kStats) {
+            st.pixels++;
+            st.samples += pixel_samples(P, z * bintov - P.vel, bintov);
+        }
+    }
+    if (first < kG) {
+        walked = sure ? c + first + 1 : -1;
+        // the FP32 value of the deciding pixel is too close to tautail
+        if (!sure && glane == 0) push_fixup(A, p0 + P.k, item, z0 + dir * (c + first), count - (c + first), dir);
+        return true;
+    }
+    walked = count;
+    return c + pcount >= count;
 }
 
 // Record the pixels walked in one direction of pair k (for the adjoint).
@@ -1106,8 +1131,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     const unsigned long long leaders = kG == 64 ? 1ull : (kG == 32 ? 0x0000000100000001ull :
                                                          0x0001000100010001ull);
     const unsigned long long leaders_below = leaders & ((1ull << ((lane / kG) * kG)) - 1ull);
+    const PairWalk *wslots = lds.pslot + (threadIdx.x / 64) * kGroupsPerWave;
     const double bintov = A.vbox / A.nbins;
     const int half = A.nbins / 2;
+    const CutBand cut = cut_band(A.tautail);
     LaneStats st;
     int it = use_queue ? 0 : blockIdx.x;
     for (;;) {
@@ -1133,7 +1160,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         __syncthreads();
         const LosInfo los = los_info(A, w.los);
         // group state: dir 0 = needs a pair, +1/-1 = walking, 2 = no pairs left
-        long long k = 0;
         int dir = 0, c = 0, z0 = 0;
         // the wavefront's ring of set-up pairs: records head .. tail - 1
         int head = 0, tail = 0;
@@ -1170,7 +1196,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                     if (rank < avail) {
                         const PairLite &r = q[(head + rank) % kWaveQueue];
                         activate_pair<kStats>(r, P, glane);
-                        k = w.p0 + r.h.k;
                         dir = 1;
                         c = 0;
                         fresh = true;
@@ -1186,14 +1211,23 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             if (!__ballot(dir != 2)) break;
             long long tc1 = 0;
             if (kStats) tc1 = clock64();
-            // the step's first pixel in the far wing: |U| only grows along a walk
-            // (the record brought the far-wing coefficients)
+            // a step whose first pixel lies in the far wing takes the rest of its
+            // walk there, one such walk of the wavefront after the other
             const bool far = walking && fabs(((z0 + dir * c) * bintov - P.vel + 0.5 * bintov) * P.inv_b) >= P.ufar;
+            int walked = 0, adv = 0;
+            bool done = far;
+            for (unsigned long long fm = __ballot(far) & leaders; fm; fm &= fm - 1ull) {
+                const int src = __builtin_ctzll(fm);
+                const PairWalk &Q = wslots[src / kG];
+                const int fd = __builtin_amdgcn_readlane(dir, src), fc = __builtin_amdgcn_readlane(c, src),
+                          fz = __builtin_amdgcn_readlane(z0, src);
+                const int n = far_walk<kLds, kStats>(A, Q, row, fz + fd * fc, fd, half - fc, cut, lane, st, w.p0 + Q.k, gitem);
+                if (lane / kG == src / kG) walked = n < 0 ? -1 : fc + n;
+            }
             long long tc2 = 0;
             if (kStats) tc2 = clock64();
-            int walked = 0, adv = 0;
-            const bool done = walk_step<kG, kLds, kStats>(A, P, sbuf, row, ptab, z0, dir, half, c, far, lane, st, k,
-                                                          gitem, walking, walked, adv);
+            if (walking && !far)
+                done = near_step<kG, kLds, kStats>(A, P, sbuf, row, ptab, z0, dir, half, c, cut, lane, st, w.p0, gitem, walked, adv);
             if (kStats && lane == 0) {
                 const long long tc3 = clock64();
                 st.cyc_setup += tc1 - tc0;
@@ -1201,7 +1235,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                 st.cyc_walk += tc3 - tc2;
             }
             if (walking) {
-                if (done && walked >= 0 && glane == 0) record_window(A, w.line, k, dir, walked);
+                if (done && walked >= 0 && glane == 0) record_window(A, w.line, w.p0 + P.k, dir, walked);
                 if (!done) {
                     c += adv;
                 } else if (dir == 1) {
@@ -1288,6 +1322,9 @@ __global__ __launch_bounds__(kThreads) void tau_fixup_kernel(DepositArgs A, cons
                 record_window(A, w.line, f.k, -1, lb);
             }
         } else {
+            // the walk's z0 counts from the box that holds its first pixel
+            if (glane == 0) P.vel -= box_shift(P.zmax, A.nbins) * A.vbox;
+            wave_sync();
             const int l = walk_fix<kFixG, kWalkGuarded, kStats>(A, P, out_row, ptab, gtab64, f.z0, f.dir, f.count, lane, st);
             if (glane == 0) record_window(A, w.line, f.k, f.dir, (half - f.count) + l);
         }
