@@ -59,10 +59,10 @@ static void line_consts(const fsamd_line &l, LineDesc &d)
     d.out = l.out;
 }
 
-static bool find_item_set(const fsamd_plan *P, int K, long long chunk)
+static bool find_item_set(const fsamd_plan *P, int K, long long chunk, int slots, long long unit)
 {
     for (auto &it : P->item_sets)
-        if (it->K == K && it->chunk == chunk) return true;
+        if (it->K == K && it->chunk == chunk && it->slots == slots && it->unit == unit) return true;
     return false;
 }
 
@@ -71,35 +71,55 @@ static long long tune_key(int nbins, int nlines, int kernel)
     return ((long long)nbins << 20) ^ ((long long)nlines << 4) ^ kernel;
 }
 
-// Work items for K lines (or parts of the fields) in the plan's heaviest-first order; a sightline
-// with more than `chunk` pairs is split into non-direct items.  Cached.
-static int item_set(fsamd_plan *P, int K, long long chunk, fsamd_plan::ItemSet **out)
+// Parts of a split sightline are multiples of this many pairs.  tau: below some
+// 16 pairs a wavefront the row's zeroing and flush cost more than the balance
+// gains.  Column density: a block's wavefronts take 64 pairs at a time.
+constexpr long long kTauPart = 128;
+constexpr long long kColdenPart = kColThreads;
+
+// Work items for K lines (or parts of the fields) in the plan's heaviest-first
+// order; a sightline with more than `chunk` pairs is split into non-direct
+// items.  slots > 0 (blocks the launch keeps resident): besides, sightlines are
+// split as guided scheduling does, into parts of about the pairs still to be
+// handed out over 2 x slots.  With many more items than slots that cuts up only
+// the last ones, which would otherwise leave part of the chip idle (10000
+// items on 512 slots: 102.1 -> 99.3 ms a call); with fewer, every sightline (333
+// items 2.07 -> 1.77 ms, 64 items 1.20 -> 0.83 ms, 50 items forward and backward
+// 3.4 -> 1.2 ms).  Cached.
+static int item_set(fsamd_plan *P, int K, long long chunk, int slots, long long unit, fsamd_plan::ItemSet **out)
 {
     for (auto &it : P->item_sets)
-        if (it->K == K && it->chunk == chunk) {
+        if (it->K == K && it->chunk == chunk && it->slots == slots && it->unit == unit) {
             *out = it.get();
             return FSAMD_OK;
         }
     auto set = std::make_unique<fsamd_plan::ItemSet>();
     set->K = K;
     set->chunk = chunk;
+    set->slots = slots;
+    set->unit = unit;
     set->split = false;
     std::vector<WorkItem> &items = set->host;
     const long long stride = chunk < 0 ? -chunk : 1;
     if (chunk < 0) chunk = 1ll << 62;
-    long long nsel = 0;
+    long long nsel = 0, left = 0;
+    if (slots > 0) {
+        for (int s : P->order_host)
+            if (nsel++ % stride == 0) left += K * (P->off_host[s + 1] - P->off_host[s]);
+        nsel = 0;
+    }
     for (int s : P->order_host) {
         const long long a = P->off_host[s], b = P->off_host[s + 1];
         const long long n = b - a;
         if (nsel++ % stride) continue;
         for (int k = 0; k < K; ++k) {
-            if (n <= chunk) {
-                items.push_back(WorkItem{s, k, a, b, 1, 0});
-            } else {
-                set->split = true;
-                for (long long c = a; c < b; c += chunk)
-                    items.push_back(WorkItem{s, k, c, std::min(b, c + chunk), 0, 0});
-            }
+            const long long part = slots > 0 ? unit * std::max(1ll, (left / (2 * slots) + unit / 2) / unit) : chunk;
+            left -= n;
+            // not for a part of less than half the size
+            const long long parts = n <= std::min(chunk, part + part / 2) ? 1 : (n + part - 1) / part;
+            if (parts > 1) set->split = true;
+            for (long long i = 0; i < parts; ++i)
+                items.push_back(WorkItem{s, k, a + i * n / parts, a + (i + 1) * n / parts, parts == 1, 0});
         }
     }
     if (items.size() >= (size_t)INT32_MAX) return fail(FSAMD_ERR_ARG, "too many work items");
@@ -297,10 +317,13 @@ static int run_deposit(bool tau, fsamd_plan *P, int nbins, int kernel, double ve
         // column density: one item takes several fields of its sightline
         A.fields = tau ? 1 : lds ? colden_fields(K, nbins) : K;
         const int parts = tau ? K : (K + A.fields - 1) / A.fields;
+        const int slots = plain ? 0 : dev.ncu * deposit_blocks_per_cu(tau, lds, gsize, effective_waves(lds, g_stats_on, waves),
+                                                                      nbins, A.fields);
+        const long long unit = tau ? kTauPart : kColdenPart;
         fsamd_plan::ItemSet *set = nullptr;
-        if (capturing && !find_item_set(P, parts, chunk_key))
+        if (capturing && !find_item_set(P, parts, chunk_key, slots, unit))
             return fail(FSAMD_ERR_ARG, "run one uncaptured fsamd_tau call before capturing");
-        if ((rc = item_set(P, parts, chunk_key, &set))) return rc;
+        if ((rc = item_set(P, parts, chunk_key, slots, unit, &set))) return rc;
         const std::vector<WorkItem> &items = set->host;
         for (int attempt = 0;; ++attempt) {
             A.fix = P->fix.as<Fixup>();
@@ -317,9 +340,7 @@ static int run_deposit(bool tau, fsamd_plan *P, int nbins, int kernel, double ve
             if (!plain) {
                 A.nitems = (int)items.size();
                 if ((rc = launch_fill_i32(A.queue, 0, 1, s))) return rc;
-                const int per_cu = deposit_blocks_per_cu(tau, lds, gsize, effective_waves(lds, g_stats_on, waves), nbins,
-                                                         A.fields);
-                const int nblocks = (int)std::min<long long>((long long)per_cu * dev.ncu, A.nitems);
+                const int nblocks = std::min(slots, A.nitems);
                 if (g_timing_on) FSAMD_HIP(hipEventRecord(P->ev[2], s));
                 if ((rc = launch_deposit(tau, lds, gsize, waves, A, set->buf.as<WorkItem>(), 0, nblocks, 1, s)))
                     return rc;
@@ -748,7 +769,8 @@ int fsamd_tau_adjoint(fsamd_plan *P, int nbins, int kernel, double velfac, const
         A.grad_temp = grad_temp;
         A.grad_vel = grad_vel;
         fsamd_plan::ItemSet *set = nullptr;
-        if ((rc = item_set(P, K, 1ll << 62, &set))) return rc;
+        const int slots = adjoint_blocks_per_cu(gsize, nbins) * dev.ncu;
+        if ((rc = item_set(P, K, 1ll << 62, slots, kTauPart, &set))) return rc;
         if (set->host.empty()) continue;
         A.nitems = (int)set->host.size();
         A.fix = P->fix.as<Fixup>();
@@ -756,7 +778,7 @@ int fsamd_tau_adjoint(fsamd_plan *P, int nbins, int kernel, double velfac, const
         A.fix_cap = P->fix_cap;
         if ((rc = launch_fill_i32(A.queue, 0, 1, s))) return rc;
         if ((rc = launch_fill_i32((int *)A.fix_count, 0, 4, s))) return rc;
-        const int nblocks = (int)std::min<long long>((long long)adjoint_blocks_per_cu(gsize, nbins) * dev.ncu, A.nitems);
+        const int nblocks = std::min(slots, A.nitems);
         if ((rc = launch_tau_adjoint(gsize, A, set->buf.as<WorkItem>(), nblocks, s))) return rc;
         if ((rc = launch_tau_adjoint64(A, set->buf.as<WorkItem>(), dev.ncu * 2, s))) return rc;
         unsigned long long fc[2] = {0, 0};

@@ -16,6 +16,8 @@ struct WorkItem {
     int pad;
 };
 
+constexpr int kColThreads = 512;   // threads of a column-density block
+
 size_t deposit_lds_bytes(int nbins);
 // LDS a deposit kernel declares itself (queues, per-group state, tables):
 // the tau kernel at group width gsize and `waves` wavefronts per block, or

@@ -45,7 +45,6 @@ __device__ const double d_gtab64[kG64Size] = FSAMD_G64_COEF_INIT;
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
-constexpr int kColThreads = 512;   // column density
 constexpr double kGuard = 2e-5;
 constexpr int kWingTerms = 10;
 

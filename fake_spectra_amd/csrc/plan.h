@@ -99,6 +99,8 @@ struct fsamd_plan {
     struct ItemSet {
         int K;
         long long chunk;
+        int slots;
+        long long unit;
         bool split;
         fsamd::DevBuf buf;
         std::vector<fsamd::WorkItem> host;

@@ -108,3 +108,30 @@ def test_fp64_walks(oracle, nbins, kernel, tscale, gscale):
         SP.set_fp64(False)
     assert np.max(ref) > 0 and np.array_equal(got == 0, ref == 0)
     assert np.max(np.abs(got - ref) / np.maximum(ref, 1e-300)) <= 1e-11
+
+
+# fewer sightlines than blocks (every row split, into one pair and into many),
+# a row of no pairs, rows around the size of a part, and rows too long for LDS
+@pytest.mark.parametrize("n,nlos,nbins,hfrac", [(1, 1, 8, 0.4), (127, 2, 64, 0.5), (129, 1, 64, 0.5), (5000, 1, 300, 0.3),
+                                                (400, 40, 100, 0.2), (3000, 2, 25000, 0.2), (3, 20, 50, 0.05)])
+def test_split_rows(oracle, n, nlos, nbins, hfrac):
+    """Rows cut into parts that add into the output: tau to the stated
+    tolerance, column density to rounding, and forward and backward windows."""
+    import torch
+    from fake_spectra_amd import autograd as AG
+    args = small_gas(n, 900.0, nlos, nbins, 1, hfrac)
+    assert_tau_close(SP._Particle_Interpolate(*args), oracle.interpolate(*args), "split tau")
+    cargs = small_gas(n, 900.0, nlos, nbins, 1, hfrac, compute_tau=False)
+    ref, got = oracle.interpolate(*cargs), SP._Particle_Interpolate(*cargs)
+    assert np.max(np.abs(got - ref)) <= 1e-12 * max(ref.max(), 1e-300)
+    if nbins > 5000:
+        return      # the adjoint keeps its rows in LDS
+    # the gradient of the sum with respect to the densities is linear: sum over
+    # particles of dens * grad equals the sum of tau (FP32 profile, 1e-5)
+    plan = SP.Plan(args[3], dev(args[11]), dev(args[15]), dev(args[16]), dev(args[17]))
+    d = dev(args[13]).requires_grad_(True)
+    tau = AG.tau_autograd(plan, nbins, 1, args[4], dev(args[12]), dev(args[14]), [HI_1215], [d])[0]
+    total = tau.sum()
+    if total.item() > 0:
+        total.backward()
+        assert float((d.grad.double() * d.detach().double()).sum()) == pytest.approx(total.item(), rel=1e-5)
