@@ -97,6 +97,18 @@ __device__ inline double kernel_weight(int kernel, double q)
     return 1.0;
 }
 
+// sqrt(x) for 1e-300 < x < 1e300 to about an ulp: the hardware's reciprocal
+// square root, one step of Goldschmidt's iteration and a Newton correction.
+__device__ inline double sqrt_nr(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+
 __device__ inline LineDesc line_of(const DepositArgs &A, int k) { return A.lines[k]; }
 
 // Sightline data needed to recompute dr2 exactly as the binning did.
@@ -174,55 +186,36 @@ __device__ inline int wrap_near(int z, int nbins)
     return z < 0 ? z + nbins : z;
 }
 
-// Per-pair constants of LineAbsorption::add_tau_particle and SingleAbsorber.
-// Each wavefront keeps the constants of its current pair in an LDS slot: the
-// values are uniform across the wave, and reading them with broadcast LDS
-// loads keeps them out of the vector registers of the per-pixel loop.
-// One interior kernel sample of a pair (singleabs.h:146-157): twice its offset
-// vv_i / b (the profile's table takes 2u, voigt.h) and its weight K(q_i).
-struct KernelSample {
-    double cv2;
-    float w;
-    float pad;
-};
-
-__device__ inline void set_sample_offset(KernelSample &k, double cv) { k.cv2 = 2.0 * cv; }
-
-__device__ inline double sample_offset(const KernelSample &k) { return 0.5 * k.cv2; }
-
-// 2u = 2 (vv_i - vouter)/b from s2 = 2 vouter/b: subtracted in FP64 and rounded
-// once, so u keeps half an ulp where the two nearly cancel.
-__device__ inline float sample_u2(const KernelSample &k, double s2) { return (float)(k.cv2 - s2); }
-
-// The constants a walk of the main kernel reads, in one layout in the pair
-// set-up record and in the group's PairTau slot, so that taking a record
-// copies them with one 8-byte move per lane.
-struct WalkHead {
+// Per-pair constants of LineAbsorption::add_tau_particle and SingleAbsorber as
+// the walks read them.  They lie in LDS: uniform over a lane group, they are
+// read with broadcast loads where they are used and take no vector registers
+// of the per-pixel loop.  Velocities in units of b carry the factor kUScale of
+// the profile's argument (voigt.h).
+struct PairRec {
     double vel;      // velfac*ppos + pvel (absorption.cpp:234)
-    double inv_b;
+    double ibs;      // kUScale / b
+    double dss;      // sub-sample spacing, bintov / max(np - 1, 1) * ibs
     double scale;    // amp * dens * dvk / velfac: taulast = scale * (sample sum)
-    double inv_nm1;  // 1 / (np - 1)
+    double snear;    // scale / max(np - 1, 1), for the sum over sub-samples
+    double qs;       // spacing of the kernel samples (singleabs.h:146-157), vhigh / 4 * ibs
+    float W[4];      // kernel weights of the centre sample and the 3 above it (K is even)
     // Far wing: for a pixel centred at U (units of b) with |U| >= ufar the
     // 7 x np samples sum to Y (C0 + C1 Y + ... + C9 Y^9), Y = (ufar/U)^2.
-    float ufar;
+    float Cw[kWingTerms];
+    VoigtP vp;       // constants of the FP32 profile
+    float ufs;       // kUScale ufar
     int zmax;
     int shape;       // near-step shape of the main kernel (step_shape)
     int k;           // the pair, counted from the work item's first (main kernel)
 };
-static_assert(sizeof(WalkHead) == 48, "WalkHead is six 8-byte words");
+static_assert(sizeof(PairRec) == 144, "PairRec layout: W on a 16-byte boundary");
 
-// What a walk of the main kernel reads of its pair.
-struct PairWalk : WalkHead {
-    KernelSample smp[kNGrid - 1];   // kernel sample velocities / b and weights
-    float Cw[kWingTerms];
-    VoigtP vp;
+struct PairTau : PairRec {
     double b;        // btherm (absorption.cpp:220)
-};
-
-struct PairTau : PairWalk {
+    double inv_b;
     double dvk;      // 2 vhigh / NGRID (singleabs.h:146)
     double vhigh, vdr2, vsmooth, aa;
-    float ufar2;     // ufar^2 (fix-up and adjoint kernels)
+    double ufar;
     double scale_nd; // amp * dvk / velfac (scale without the density)
     double temp;     // particle temperature
     int part;        // particle index
@@ -231,8 +224,14 @@ struct PairTau : PairWalk {
     int fp64;
     int np;          // sub-samples per pixel (1 = midpoint)
     int wing_ready;  // Cw computed
+    double inv_nm1;  // 1 / (np - 1)
     double dv;       // sub-sample spacing bintov / (np - 1)
 };
+
+// kUScale u, u = (vv_i - vouter)/b of the kernel sample i - 3 = j from the centre,
+// from s = kUScale vouter/b: in FP64 and rounded once, so u keeps half an ulp
+// where the two nearly cancel.
+__device__ inline float sample_us(double qs, int j, double s) { return (float)__builtin_fma((double)j, qs, -s); }
 
 __device__ inline void wave_sync()
 {
@@ -251,20 +250,23 @@ __device__ inline double shfl_d(double v, int src)
 }
 
 // sum_i K(q_i) Re w((vv_i - vouter)/b + i a), FP32 profile; the sample
-// offsets from the FP64 anchor s2 = 2 vouter/b.  kA3 = false: the light form
+// offsets from the FP64 anchor s = kUScale vouter/b.  kA3 = false: the light form
 // of the profile (pairs with a <= kA3Drop).
 template <bool kA3 = true>
-__device__ inline float inner32(const PairWalk &P, double s2, const float *ptab)
+__device__ inline float inner32(const PairRec &P, double s, const float *ptab)
 {
     const VoigtP vp = P.vp;
+    const double qs = P.qs;
+    const float4 w4 = *(const float4 *)P.W;
+    const float W[4] = {w4.x, w4.y, w4.z, w4.w};
     float sE = 0.0f, sG = 0.0f;
 #pragma unroll  // full: 5% faster than unrolling by 2 at 256^3 and 512^3 (same operation order)
-    for (int i = 0; i < kNGrid - 1; ++i) {
-        const KernelSample k = P.smp[i];
+    for (int j = -3; j <= 3; ++j) {
         float E, G;
-        voigt_terms<kA3>(vp, sample_u2(k, s2), ptab, E, G);
-        sE = __builtin_fmaf(k.w, E, sE);
-        sG = __builtin_fmaf(k.w, G, sG);
+        voigt_terms<kA3>(vp, sample_us(qs, j, s), ptab, E, G);
+        const float w = W[j < 0 ? -j : j];
+        sE = __builtin_fmaf(w, E, sE);
+        sG = __builtin_fmaf(w, G, sG);
     }
     return __builtin_fmaf(-vp.two_a_sqpi, sG, sE);
 }
@@ -298,14 +300,14 @@ __device__ inline double taulast_pixel(const PairTau &P, double vlow, double bin
     if (!k64) {
         const double U = (vlow + 0.5 * bintov) * P.inv_b;
         if (fabs(U) >= P.ufar) {
-            const float Y = P.ufar2 * __builtin_amdgcn_rcpf((float)(U * U));
+            const float Y = (float)(P.ufar * P.ufar) * __builtin_amdgcn_rcpf((float)(U * U));
             float S = P.Cw[kWingTerms - 1];
 #pragma unroll
             for (int t = kWingTerms - 2; t >= 0; --t) S = __builtin_fmaf(S, Y, P.Cw[t]);
             return P.scale * (double)(S * Y);
         }
     }
-    auto inner = [&](double v) { return k64 ? inner64(P, v, kernel, gtab64) : inner32(P, v * (2.0 * P.inv_b), ptab); };
+    auto inner = [&](double v) { return k64 ? inner64(P, v, kernel, gtab64) : inner32(P, v * P.ibs, ptab); };
     if (width < P.b / 2.) return P.scale * inner((vhighp + vlow) / 2.);
     const int np = 2 * ceil(width / (P.b / 2.) / 2) + 1.;
     const double dv = width / (np - 1);
@@ -395,17 +397,14 @@ __device__ inline void wing_setup(PairTau &P, double bintov, int lane)
         }
     }
     // m'_n = sum_k C(2n,2k) X_k Y_(n-k), X_k by running powers
-    const double c4 = sample_offset(P.smp[4]) * inv_u, c5 = sample_offset(P.smp[5]) * inv_u,
-                 c6 = sample_offset(P.smp[6]) * inv_u;
+    const double c4 = P.qs * (inv_u / kUScale), c5 = 2.0 * c4, c6 = 3.0 * c4;
     const double x4 = c4 * c4, x5 = c5 * c5, x6 = c6 * c6;
-    const double w4 = (double)P.smp[4].w + (double)P.smp[2].w;
-    const double w5 = (double)P.smp[5].w + (double)P.smp[1].w;
-    const double w6 = (double)P.smp[6].w + (double)P.smp[0].w;
+    const double w4 = 2.0 * P.W[1], w5 = 2.0 * P.W[2], w6 = 2.0 * P.W[3];
     double p4 = 1.0, p5 = 1.0, p6 = 1.0, mom = 0.0;
 #pragma unroll 1
     for (int k = 0; k < kWingTerms; ++k) {
         double xk = w4 * p4 + w5 * p5 + w6 * p6;
-        if (k == 0) xk += (double)P.smp[3].w;
+        if (k == 0) xk += (double)P.W[0];
         p4 *= x4;
         p5 *= x5;
         p6 *= x6;
@@ -627,10 +626,7 @@ __device__ inline bool setup_pair(const DepositArgs &A, int line, const LineDesc
     const int p = A.pair_part[kk];
     const double bintov = A.vbox / A.nbins;
     wave_sync();   // the previous pair's constants are no longer read
-    if (lane < kNGrid - 1) {
-        set_sample_offset(P.smp[lane], ((lane + 1) * C.dvk - C.vhigh) * C.inv_b);
-        P.smp[lane].w = sample_weight(A, C, lane);
-    }
+    if (lane < 4) P.W[lane] = sample_weight(A, C, lane + 3);
     if (lane == 0) {
         P.vel = C.vel;
         P.b = C.b;
@@ -649,8 +645,9 @@ __device__ inline bool setup_pair(const DepositArgs &A, int line, const LineDesc
         P.temp = (double)C.temp;
         P.part = p;
         P.np = C.np;
-        P.ufar = (float)C.ufar;
-        P.ufar2 = (float)((double)P.ufar * P.ufar);
+        P.ufar = C.ufar;
+        P.ibs = kUScale * C.inv_b;
+        P.qs = 0.25 * C.vhigh * P.ibs;
         P.wing_ready = 0;
         P.inv_nm1 = C.np > 1 ? 1.0 / (C.np - 1) : 1.0;
         P.dv = C.np > 1 ? bintov * P.inv_nm1 : 0.0;
@@ -659,24 +656,21 @@ __device__ inline bool setup_pair(const DepositArgs &A, int line, const LineDesc
     return true;
 }
 
-// The main kernel sets pairs up in batches, one pair per lane of a
-// wavefront, into a per-wavefront ring of compact records: the FP64 set-up
-// (pair constants, kernel weights and the ten far-wing coefficients) runs on
-// up to kWaveQueue lanes at once instead of on the few lanes of one lane
-// group, and a group taking the next record only expands it into its PairTau
-// slot.  The ring is shared by the wavefront's groups.
-constexpr int kWaveQueue = kWaveClaim;
-
-struct PairLite {
-    WalkHead h;
-    double vhigh;
-    float W[4];       // kernel weights of the centre sample and the 3 above it
-    float Cw[kWingTerms];   // far-wing coefficients (wing_coeffs)
-    VoigtP vp;        // constants of the FP32 profile
-};
-static_assert(sizeof(PairLite) == 136, "PairLite layout");
-constexpr int kVoigtWords = sizeof(VoigtP) / sizeof(float);
-static_assert(kVoigtWords <= 16, "the activation copies VoigtP one word a lane");
+// The main kernel sets pairs up in batches, one pair per lane of a wavefront,
+// into the wavefront's kRecs records: the FP64 set-up (pair constants, kernel
+// weights and the ten far-wing coefficients) runs on up to kRecs lanes at once
+// instead of on the few lanes of one lane group.  A group walks its pair in
+// the record where it lies.  Which records are free, and which hold pairs of
+// the light and of the full profile, are three masks of the wavefront: the
+// groups take pairs of one class as long as there are some, so that the near
+// steps of the wavefront mostly run the light code (a step runs the full code,
+// 180 instead of 85 instructions a sum, if any of its groups needs it).  Against
+// a ring in claim order whose records were copied to a slot per group: 99.3 ->
+// 89.6 ms at 256^3 x 5000 x 2048, two lines; 301 -> 269 with a metal line (half
+// of its pairs full) at 12288 x 1024.
+constexpr int kRecs = kWaveClaim;
+static_assert(kRecs == 32, "the record masks are 32-bit");
+constexpr int kRefillRoom = 12;   // fewest free records worth a set-up while others wait
 
 // The far-wing coefficients of wing_setup for one pair, all ten on one lane
 // (the batched set-up of the main kernel), in FP32: every term is positive,
@@ -739,14 +733,30 @@ __device__ __noinline__ void wing_coeffs(float c0, float h, int m1, float W0, fl
     }
 }
 
-// Claim up to `want` pairs of item w for the wavefront, set up one per lane,
-// and append those walked in FP32 to the wavefront's ring (tail advances);
-// FP64 pairs go straight to the fix-up list.  Every lane of the wavefront
-// calls it; `more` says whether the item has pairs left.
+// K(q) (singleabs.h:17-42 and kernel_weight), q^2 > 0, without branches on q.
+__device__ inline float kernel_weight_q2(int kernel, double q2)
+{
+    const double q = sqrt_nr(q2 + 1e-290);
+    if (kernel == kCubicSpline) {
+        const double t = fmax(1.0 - q, 0.0), h = fmax(0.5 - q, 0.0);
+        return (float)(32. / 4 / kPi * 2.0 * (t * t * t - 4.0 * (h * h * h)));
+    }
+    if (kernel == kSphQuintic) {
+        const double t3 = fmax(3.0 - 3.0 * q, 0.0), t2 = fmax(2.0 - 3.0 * q, 0.0), t1 = fmax(1.0 - 3.0 * q, 0.0);
+        const double p3 = t3 * t3, p2 = t2 * t2, p1 = t1 * t1;
+        return (float)(9. / 40 / kPi * (p3 * p3 * t3 - 6.0 * (p2 * p2 * t2) + 15.0 * (p1 * p1 * t1)));
+    }
+    return kernel == kTopHat ? (float)(3. / 4. / kPi) : 1.0f;
+}
+
+// Claim up to `want` (at most the free records) pairs of item w for the
+// wavefront, set them up one per lane and put those walked in FP32 into free
+// records; FP64 pairs go straight to the fix-up list.  Every lane of the
+// wavefront calls it; `more` says whether the item has pairs left.
 template <int kG, bool kStats>
 __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int gitem, const LineDesc &L,
-                                   const LosInfo &los, unsigned long long *next, PairLite *q, int lane, int want,
-                                   int &tail, bool &more, LaneStats &st)
+                                   const LosInfo &los, unsigned long long *next, PairRec *recs, int lane, int want,
+                                   unsigned &free, unsigned &light, unsigned &full, bool &more, LaneStats &st)
 {
     unsigned long long base = 0;
     if (lane == 0) base = atomicAdd(next, (unsigned long long)want);
@@ -765,77 +775,68 @@ __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int 
         }
     }
     const unsigned long long m = __ballot(enq);
-    wave_sync();   // the records taken earlier have been read
+    const int n = __popcll(m);
+    // the r-th pair goes to the r-th free record: lane l stands for record l
+    // and sends its number to the lane of its rank
+    const bool isfree = lane < kRecs && ((free >> (lane & 31)) & 1u);
+    const int frank = __popc(free & ((1u << (lane & 31)) - 1u));
+    const int nth = __builtin_amdgcn_ds_permute(4 * (isfree ? frank : 63), lane);
+    const int slot = __shfl(nth, __popcll(m & ((1ull << lane) - 1ull)), 64);
+    wave_sync();   // the records' former pairs have been read
     if (enq) {
-        PairLite &r = q[(tail + __popcll(m & ((1ull << lane) - 1ull))) % kWaveQueue];
+        PairRec &r = recs[slot];
         const int shift = box_shift(C.zmax, A.nbins);
-        r.h.vel = shift ? C.vel - shift * A.vbox : C.vel;
-        r.h.zmax = C.zmax - shift * A.nbins;
-        r.h.inv_b = C.inv_b;
-        r.h.scale = C.scale;
-        r.vhigh = C.vhigh;
+        const double ibs = kUScale * C.inv_b;
+        const double inv_m = C.np > 1 ? 1.0 / (C.np - 1) : 1.0;
+        r.vel = shift ? C.vel - shift * A.vbox : C.vel;
+        r.zmax = C.zmax - shift * A.nbins;
+        r.ibs = ibs;
+        r.dss = bintov * inv_m * ibs;
+        r.scale = C.scale;
+        r.snear = C.scale * inv_m;
+        r.qs = 0.25 * C.vhigh * ibs;
         // the walk uses the light form of the profile for a <= kA3Drop, as a
         // property of the pair: its coefficients are zero, so the full form
         // gives the same values and the result does not depend on which
         // pairs share a wavefront
         r.vp = make_voigt_p(C.aa, C.aa <= (double)kA3Drop);
-        r.h.inv_nm1 = C.np > 1 ? 1.0 / (C.np - 1) : 1.0;
-        r.h.k = (int)(kk - w.p0);   // a row has fewer than 2^31 pairs (one per particle)
-        const double inv_vs = 1.0 / C.vsmooth;
+        r.k = (int)(kk - w.p0);   // a row has fewer than 2^31 pairs (one per particle)
+        const double inv_s2 = 1.0 / (C.vsmooth * C.vsmooth);
         float W[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const double vv = (i + 4) * C.dvk - C.vhigh;
-            W[i] = (float)kernel_weight(A.kernel, sqrt(C.vdr2 + vv * vv) * inv_vs);
-            r.W[i] = W[i];
+            W[i] = kernel_weight_q2(A.kernel, (C.vdr2 + vv * vv) * inv_s2);
         }
+        *(float4 *)r.W = make_float4(W[0], W[1], W[2], W[3]);
         // the walk compares with ufar rounded to FP32, the unit of the coefficients
         const float ufar = (float)C.ufar;
-        r.h.ufar = ufar;
+        r.ufs = (float)kUScale * ufar;
         const StepShape sh = step_shape(C.np, kG);
-        r.h.shape = sh.packed();
+        r.shape = sh.packed();
         // far-wing coefficients, in units of that ufar
         const double iu = 1.0 / (double)ufar;
         wing_coeffs((float)(C.vhigh * C.inv_b * iu), (float)(0.5 * bintov * C.inv_b * iu), sh.nm1, W[0], W[1], W[2],
                     W[3], (float)C.aa, ufar, r.Cw);
     }
     wave_sync();
-    tail += __popcll(m);
+    const bool used = isfree && frank < n;
+    const unsigned mine = (unsigned)__ballot(used);
+    const unsigned a3 = (unsigned)__ballot(used && recs[lane & 31].vp.a3 != 0.0f);
+    free &= ~mine;
+    light |= mine & ~a3;
+    full |= a3;
     more = (long long)base + want < w.p1;
 }
 
-// Expand queued record r into the group's PairTau slot: the fields the main
-// kernel's walk reads, one 8-byte word, weight, coefficient or sample offset
-// per lane (setup_pair and wing_setup fill the same values for the other
-// kernels).  Only the lanes of the groups taking a record call it.
-template <bool kStats>
-__device__ inline void activate_pair(const PairLite &r, PairWalk &P, int glane)
-{
-    if (glane < kNGrid - 1) {
-        const double dvk = 2. * r.vhigh / kNGrid;
-        set_sample_offset(P.smp[glane], ((glane + 1) * dvk - r.vhigh) * r.h.inv_b);
-        P.smp[glane].w = r.W[glane < 3 ? 3 - glane : glane - 3];   // K(q) is even in the sample offset
-    }
-    if (glane < kWingTerms) P.Cw[glane] = r.Cw[glane];
-    if (glane < kVoigtWords)
-        reinterpret_cast<float *>(&P.vp)[glane] = reinterpret_cast<const float *>(&r.vp)[glane];
-    constexpr int kHeadWords = sizeof(WalkHead) / sizeof(long long);
-    if (glane < kHeadWords)
-        reinterpret_cast<long long *>(static_cast<WalkHead *>(&P))[glane] =
-            reinterpret_cast<const long long *>(&r.h)[glane];
-    if (kStats && glane == kHeadWords) {
-        // read by the counters (pixel_samples)
-        P.b = 1.0 / r.h.inv_b;
-    }
-}
-
 // Voigt samples the reference evaluates for one pixel (singleabs.h:110-125).
-__device__ inline int pixel_samples(const PairWalk &P, double vlow, double bintov)
+__device__ inline int pixel_samples(const PairRec &P, double vlow, double bintov)
 {
+    const double b = kUScale / P.ibs;
     const double vhighp = vlow + bintov;
     const double width = vhighp - vlow;
-    if (width < P.b / 2.) return kNGrid - 1;
-    const int np = 2 * ceil(width / (P.b / 2.) / 2) + 1.;
+    if (width < b / 2.) return kNGrid - 1;
+    const int np = 2 * ceil(width / (b / 2.) / 2) + 1.;
     return (kNGrid - 1) * np;
 }
 
@@ -936,18 +937,18 @@ __device__ inline CutBand cut_band(double tautail) { return CutBand{tautail - kG
 // Returns the pixels walked, or -1 where the decision went to the fix-up
 // kernel.
 template <bool kLds, bool kStats>
-__device__ inline int far_walk(const DepositArgs &A, const PairWalk &P, double *row, int zf, int dir, int count,
+__device__ inline int far_walk(const DepositArgs &A, const PairRec &P, double *row, int zf, int dir, int count,
                                const CutBand &cut, int lane, LaneStats &st, long long k, int item)
 {
     const double bintov = A.vbox / A.nbins;
-    const float uf2 = (float)((double)P.ufar * P.ufar);
+    const float ufsq = (float)((double)P.ufs * P.ufs);
     for (int i0 = 0; i0 < count; i0 += 64) {
         const int i = i0 + lane;
         const bool valid = i < count;
         const int z = zf + dir * i;
         const double vlow = z * bintov - P.vel;
-        const double U = (vlow + 0.5 * bintov) * P.inv_b;
-        const float Y = uf2 * __builtin_amdgcn_rcpf((float)(U * U));
+        const double Us = (vlow + 0.5 * bintov) * P.ibs;
+        const float Y = ufsq * __builtin_amdgcn_rcpf((float)(Us * Us));
         float S = P.Cw[kWingTerms - 1];
 #pragma unroll
         for (int q = kWingTerms - 2; q >= 0; --q) S = __builtin_fmaf(S, Y, P.Cw[q]);
@@ -977,20 +978,21 @@ __device__ inline int far_walk(const DepositArgs &A, const PairWalk &P, double *
 }
 
 // One near step of a walk (lane glane of a kG-lane group): the next sh.pstep
-// pixels z0 + dir*(c + p), on the sub-sample grid they share; `sbuf` is the
-// group's LDS scratch of kG * kRoundsMax floats.  Returns true when the walk is
-// over (tail cut, end of the window, or the decision deferred to the fix-up
-// kernel), with `walked` set; `adv` is the number of pixels the step covered.
+// pixels from zf in direction dir, on the sub-sample grid they share; vf =
+// zf's lower end relative to the pair, `left` the pixels left; `sbuf` is the
+// group's LDS scratch of kG * kRoundsMax floats.  Returns the pixels walked if
+// the walk is over (tail cut or end of the window), -1 where that decision
+// goes to the fix-up kernel, 0 if it goes on after the sh.pstep pixels.
 template <int kG, bool kLds, bool kStats>
-__device__ inline bool near_step(const DepositArgs &A, const PairWalk &P, float *sbuf, double *row, const float *ptab,
-                                 int z0, int dir, int count, int c, const CutBand &cut, int lane, LaneStats &st,
-                                 long long p0, int item, int &walked, int &adv)
+__device__ inline int near_step(const DepositArgs &A, const PairRec &P, float *sbuf, double *row, const float *ptab,
+                                int zf, double vf, int dir, int left, const CutBand &cut, int lane, LaneStats &st,
+                                long long p0, int item, int &adv)
 {
     const int glane = lane % kG;
     const double bintov = A.vbox / A.nbins;
     const StepShape sh = unpack_shape(P.shape);
     const int nm1 = sh.nm1;
-    const int pcount = min(sh.pstep, count - c);
+    const int pcount = min(sh.pstep, left);
     // pairs with a <= kA3Drop carry the light form of the profile (zero a^3
     // and exponent coefficients); when every pair of this near step of the
     // wavefront does, the light code runs (a wavefront-uniform branch with
@@ -1001,17 +1003,16 @@ __device__ inline bool near_step(const DepositArgs &A, const PairWalk &P, float 
         // Sub-sample m of the step, in increasing velocity: sub-sample m mod
         // (np-1) of its pixel (singleabs.h:118-121) up to the rounding of m dv
         // against the pixel's own vlow, or (np = 1) pixel m's centre
-        // (singleabs.h:113); positions as 2 v / b.
+        // (singleabs.h:113); positions as kUScale v / b.
         const int nsub = nm1 == 0 ? pcount : pcount * nm1 + 1;
-        const int zlo = dir > 0 ? z0 + c : z0 - c - (pcount - 1);
-        const double ib2 = 2.0 * P.inv_b;
-        double vlo = zlo * bintov - P.vel;   // vlow of the step's lowest pixel (absorption.cpp:252)
-        if (nm1 == 0) vlo += 0.5 * bintov;
-        const double s2 = vlo * ib2, ds2 = bintov * P.inv_nm1 * ib2;
+        const double dss = P.dss;
+        double sv = vf * P.ibs;
+        if (nm1 == 0) sv = __builtin_fma(0.5, dss, sv);
+        if (dir < 0) sv = __builtin_fma((double)((1 - pcount) * max(nm1, 1)), dss, sv);   // its lowest pixel
         for (int r = 0; r < sh.rounds; ++r) {
             const int m = glane + r * kG;
             if (m < nsub) {
-                const double at = __builtin_fma((double)m, ds2, s2);
+                const double at = __builtin_fma((double)m, dss, sv);
                 sbuf[m] = a3 ? inner32<true>(P, at, ptab) : inner32<false>(P, at, ptab);
                 if (kStats) st.sums++;
             }
@@ -1027,14 +1028,14 @@ __device__ inline bool near_step(const DepositArgs &A, const PairWalk &P, float 
         const float *sp = sbuf + (nm1 == 0 ? j : j * nm1);
         double tot = 0.5 * ((double)sp[0] + (double)sp[nm1]);
         for (int kk = 1; kk < nm1; ++kk) tot += (double)sp[kk];
-        t = P.scale * (tot * P.inv_nm1);
+        t = P.snear * tot;
         if (kStats) st.evaluated++;
     }
     adv = pcount;
     const unsigned long long stop = __ballot(valid && t <= cut.hi), below = __ballot(valid && t < cut.lo);
     const int first = group_first<kG>(stop, lane);
     const bool sure = first < kG && group_bit<kG>(below, lane, first & (kG - 1));
-    const int z = z0 + dir * (c + glane);
+    const int z = zf + dir * glane;
     if (valid && (glane < first || (glane == first && sure))) {
         row_add<kLds>(&row[wrap_near(z, A.nbins)], t);
         if (kStats) {
@@ -1043,13 +1044,12 @@ __device__ inline bool near_step(const DepositArgs &A, const PairWalk &P, float 
         }
     }
     if (first < kG) {
-        walked = sure ? c + first + 1 : -1;
+        if (sure) return first + 1;
         // the FP32 value of the deciding pixel is too close to tautail
-        if (!sure && glane == 0) push_fixup(A, p0 + P.k, item, z0 + dir * (c + first), count - (c + first), dir);
-        return true;
+        if (glane == 0) push_fixup(A, p0 + P.k, item, zf + dir * first, left - first, dir);
+        return -1;
     }
-    walked = count;
-    return c + pcount >= count;
+    return pcount >= left ? left : 0;
 }
 
 // Record the pixels walked in one direction of pair k (for the adjoint).
@@ -1101,7 +1101,6 @@ template <int kG, bool kLds, bool kStats, int kBlock>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void tau_kernel(DepositArgs A, const WorkItem *items, int item_base,
                                                        int use_queue)
 {
-    constexpr int kGroups = kBlock / kG;
     constexpr int kWavesPerBlock = kBlock / 64;
     constexpr int kGroupsPerWave = 64 / kG;
     extern __shared__ double smem[];
@@ -1109,9 +1108,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     // a place past the table's octaves, which still lies in this block's LDS.
     struct Lds {
         __attribute__((aligned(16))) float ptab[kPTableSize];
-        PairWalk pslot[kGroups];
+        PairRec recs[kWavesPerBlock * kRecs];
         float sub_sums[kBlock * kRoundsMax];
-        PairLite wqueue[kWavesPerBlock * kWaveQueue];
     };
     static_assert(sizeof(Lds) >= 32 * FSAMD_P_BINS * 16, "every row number lies in the block's LDS");
     __shared__ Lds lds;
@@ -1123,14 +1121,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     const int lane = threadIdx.x & 63;
     const int glane = lane % kG;
     const int gid = threadIdx.x / kG;
-    PairWalk &P = lds.pslot[gid];
     float *sbuf = lds.sub_sums + gid * kG * kRoundsMax;
-    PairLite *q = lds.wqueue + (threadIdx.x / 64) * kWaveQueue;
-    // the wavefront's leader lanes of its groups, below this lane's group
+    PairRec *recs = lds.recs + (threadIdx.x / 64) * kRecs;
+    // the leader lanes of the wavefront's groups
     const unsigned long long leaders = kG == 64 ? 1ull : (kG == 32 ? 0x0000000100000001ull :
                                                          0x0001000100010001ull);
-    const unsigned long long leaders_below = leaders & ((1ull << ((lane / kG) * kG)) - 1ull);
-    const PairWalk *wslots = lds.pslot + (threadIdx.x / 64) * kGroupsPerWave;
     const double bintov = A.vbox / A.nbins;
     const int half = A.nbins / 2;
     const CutBand cut = cut_band(A.tautail);
@@ -1158,11 +1153,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         if (threadIdx.x == 0) s_next = (unsigned long long)w.p0;
         __syncthreads();
         const LosInfo los = los_info(A, w.los);
-        // group state: dir 0 = needs a pair, +1/-1 = walking, 2 = no pairs left
-        int dir = 0, c = 0, z0 = 0;
-        // the wavefront's ring of set-up pairs: records head .. tail - 1
-        int head = 0, tail = 0;
-        bool more = true;
+        // group state: dir 0 = needs a pair, +1/-1 = walking, 2 = no pairs left;
+        // rec: its record; c: pixels walked in this direction
+        int dir = 0, c = 0, z0 = 0, rec = 0;
+        // the wavefront's records, and the class it takes pairs from
+        unsigned free = ~0u, light = 0, full = 0;
+        bool more = half > 0, take_full = false;   // a row of one pixel has no window (absorption.cpp:249-279)
         for (;;) {
             long long tc0 = 0;
             const unsigned long long needing = __ballot(dir == 0) & leaders;
@@ -1175,76 +1171,80 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             }
             if (needing) {
                 const int nneed = __popcll(needing);
-                if (tail - head < nneed && more) {
-                    // claim up to a ring's worth, fewer near the end of the item so
+                if (more && __popc(take_full ? full : light) < nneed && __popc(free) >= kRefillRoom) {
+                    // claim up to the free records, fewer near the end of the item so
                     // that the block's wavefronts finish together
                     const long long rem = (long long)w.p1 - (long long)__atomic_load_n(&s_next, __ATOMIC_RELAXED);
                     const long long share = rem / (2 * kWavesPerBlock);
-                    int want = kWaveQueue - (tail - head);
+                    int want = __popc(free);
                     if (share < want) want = (int)(share > 2 * kGroupsPerWave ? share : 2 * kGroupsPerWave);
                     if (A.claim < want) want = A.claim;
                     if (want < 1) want = 1;
                     want = __builtin_amdgcn_readfirstlane(want);
-                    refill_wave<kG, kStats>(A, w, gitem, L, los, &s_next, q, lane, want, tail, more, st);
+                    refill_wave<kG, kStats>(A, w, gitem, L, los, &s_next, recs, lane, want, free, light, full, more, st);
                 }
-                const int avail = tail - head;
-                const int rank = __popcll(needing & leaders_below);
-                bool fresh = false;
-                wave_sync();   // the previous pairs' constants are no longer read
-                if (dir == 0) {
-                    if (rank < avail) {
-                        const PairLite &r = q[(head + rank) % kWaveQueue];
-                        activate_pair<kStats>(r, P, glane);
+                if ((take_full ? full : light) == 0) take_full = !take_full;
+                for (unsigned long long nm = needing; nm && (light | full); nm &= nm - 1ull) {
+                    const bool f = light == 0 || (take_full && full != 0);
+                    const int at = __builtin_ctz(f ? full : light);
+                    if (f)
+                        full &= full - 1u;
+                    else
+                        light &= light - 1u;
+                    if (lane / kG == __builtin_ctzll(nm) / kG) {
+                        rec = at;
                         dir = 1;
                         c = 0;
-                        fresh = true;
-                    } else if (!more) {
-                        dir = 2;
+                        z0 = recs[at].zmax;
                     }
                 }
-                wave_sync();
-                if (fresh) z0 = P.zmax;
-                head += nneed < avail ? nneed : avail;
+                if (dir == 0 && !more) dir = 2;   // neither records nor pairs left
             }
             const bool walking = (dir == 1 || dir == -1);
             if (!__ballot(dir != 2)) break;
             long long tc1 = 0;
             if (kStats) tc1 = clock64();
+            const PairRec &P = recs[rec];
             // a step whose first pixel lies in the far wing takes the rest of its
             // walk there, one such walk of the wavefront after the other
-            const bool far = walking && fabs(((z0 + dir * c) * bintov - P.vel + 0.5 * bintov) * P.inv_b) >= P.ufar;
-            int walked = 0, adv = 0;
-            bool done = far;
+            const int zf = z0 + dir * c;
+            const double vf = zf * bintov - P.vel;   // absorption.cpp:252
+            const bool far = walking && fabs((vf + 0.5 * bintov) * P.ibs) >= (double)P.ufs;
+            int n = 0, adv = 0;
             for (unsigned long long fm = __ballot(far) & leaders; fm; fm &= fm - 1ull) {
                 const int src = __builtin_ctzll(fm);
-                const PairWalk &Q = wslots[src / kG];
-                const int fd = __builtin_amdgcn_readlane(dir, src), fc = __builtin_amdgcn_readlane(c, src),
-                          fz = __builtin_amdgcn_readlane(z0, src);
-                const int n = far_walk<kLds, kStats>(A, Q, row, fz + fd * fc, fd, half - fc, cut, lane, st, w.p0 + Q.k, gitem);
-                if (lane / kG == src / kG) walked = n < 0 ? -1 : fc + n;
+                const PairRec &Q = recs[__builtin_amdgcn_readlane(rec, src)];
+                const int fn = far_walk<kLds, kStats>(A, Q, row, __builtin_amdgcn_readlane(zf, src),
+                                                      __builtin_amdgcn_readlane(dir, src),
+                                                      half - __builtin_amdgcn_readlane(c, src), cut, lane, st, w.p0 + Q.k, gitem);
+                if (lane / kG == src / kG) n = fn;
             }
             long long tc2 = 0;
             if (kStats) tc2 = clock64();
             if (walking && !far)
-                done = near_step<kG, kLds, kStats>(A, P, sbuf, row, ptab, z0, dir, half, c, cut, lane, st, w.p0, gitem, walked, adv);
+                n = near_step<kG, kLds, kStats>(A, P, sbuf, row, ptab, zf, vf, dir, half - c, cut, lane, st, w.p0, gitem, adv);
             if (kStats && lane == 0) {
                 const long long tc3 = clock64();
                 st.cyc_setup += tc1 - tc0;
                 st.cyc_wing += tc2 - tc1;
                 st.cyc_walk += tc3 - tc2;
             }
+            bool ended = false;
             if (walking) {
-                if (done && walked >= 0 && glane == 0) record_window(A, w.line, w.p0 + P.k, dir, walked);
-                if (!done) {
+                if (n > 0 && glane == 0) record_window(A, w.line, w.p0 + P.k, dir, c + n);
+                if (n == 0) {
                     c += adv;
                 } else if (dir == 1) {
                     dir = -1;
-                    z0 = P.zmax - 1;
+                    z0 -= 1;
                     c = 0;
                 } else {
                     dir = 0;
+                    ended = true;
                 }
             }
+            for (unsigned long long em = __ballot(ended) & leaders; em; em &= em - 1ull)
+                free |= 1u << __builtin_amdgcn_readlane(rec, __builtin_ctzll(em));
         }
         if (kLds) {
             __syncthreads();
@@ -1356,13 +1356,12 @@ __global__ __launch_bounds__(kThreads) void tau_fixup_kernel(DepositArgs A, cons
 __device__ inline void adj_inner32(const PairTau &P, double vouter, const float *gtab, float &S, float &SU,
                                    float &SF)
 {
-    const double s2 = vouter * (2.0 * P.inv_b);
+    const double s = vouter * P.ibs;
     const VoigtA va = P.va;
 #pragma unroll  // full: the adjoint kernel 6% faster than unrolling by 2 at 128^3
-    for (int i = 0; i < kNGrid - 1; ++i) {
-        const KernelSample k = P.smp[i];
-        const VoigtGrad g = voigt32_grad(va, 0.5f * sample_u2(k, s2), gtab);
-        const float w = k.w;
+    for (int j = -3; j <= 3; ++j) {
+        const VoigtGrad g = voigt32_grad(va, (float)(1 / kUScale) * sample_us(P.qs, j, s), gtab);
+        const float w = P.W[j < 0 ? -j : j];
         S = __builtin_fmaf(w, g.H, S);
         SU = __builtin_fmaf(w, g.Hu, SU);
         SF = __builtin_fmaf(w, g.F, SF);
@@ -1422,7 +1421,7 @@ __device__ inline void adj_pixel64(const PairTau &P, double vlow, double bintov,
 __device__ inline void adj_far(const PairTau &P, double vlow, double bintov, double &S, double &SU, double &SF)
 {
     const double U = (vlow + 0.5 * bintov) * P.inv_b;
-    const float Y = P.ufar2 * __builtin_amdgcn_rcpf((float)(U * U));
+    const float Y = (float)(P.ufar * P.ufar) * __builtin_amdgcn_rcpf((float)(U * U));
     float s = P.Cw[kWingTerms - 1], d = kWingTerms * P.Cw[kWingTerms - 1], f = P.CwF[kWingTerms - 1];
 #pragma unroll
     for (int t = kWingTerms - 2; t >= 0; --t) {
@@ -1653,18 +1652,6 @@ int adjoint_blocks_per_cu(int gsize, int nbins)
 
 // ---------------------------------------------------------------------------
 // Column density
-
-// sqrt(x) for 1e-300 < x < 1e300 to about an ulp: the hardware's reciprocal
-// square root, one step of Goldschmidt's iteration and a Newton correction.
-__device__ inline double sqrt_nr(double x)
-{
-    const double y = __builtin_amdgcn_rsq(x);
-    double g = x * y, h = 0.5 * y;
-    const double r = __builtin_fma(-h, g, 0.5);
-    g = __builtin_fma(g, r, g);
-    h = __builtin_fma(h, r, h);
-    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
-}
 
 // Sums over kernel samples of the truncated powers the splines consist of
 // (singleabs.h:17-42): the cubic is 2 ((1-q)+^3 - 4 (1/2-q)+^3) over its norm,

@@ -1,5 +1,5 @@
 """Generate profile_table.h: G(u) = 1 - 2u D(u) (D: Dawson's integral) as cubics
-in t = 4u^2 + 2, indexed by the bits of t.
+in t = 16u^2 + 2, indexed by the bits of t.
 
 G is the real-axis factor of the damping term of the Voigt function,
     Re w(u + ia) = exp(a^2 - u^2) cos(2au) - (2/sqrt(pi)) (a G(u) - a^3/6 D'''(u) + ...),
@@ -8,8 +8,9 @@ bins, so that a bin's number is the low exponent bits and the first mantissa
 bits of t as a float, and its left edge is t with the other mantissa bits
 cleared: neither core and wing nor small and large u need a case of their
 own.  The 2 keeps t at or above an exponent whose low five bits are zero; the
-4 puts the first bins, near u = 0, where G has structure on p = u^2 ~ 1, at a
-width of 1/64 in p.  Row r holds the four coefficients of the cubic in
+16 makes it small against u^2 where the Gaussian, whose exponent is taken from
+the same t, still matters (with 4u^2 + 2 the rounding of t cost the Gaussian
+up to 1.6 times the error for u < 1).  Row r holds the four coefficients of the cubic in
 t - edge (one 128-bit LDS read), a Chebyshev fit in float64 weighted by
 1/|G|: within a bin t varies by at most 1/32 of itself, which holds the
 truncation below 2e-8 of G (4.2e-8 of 0.01 next to its zero), less than the
@@ -21,7 +22,7 @@ Run:  python fake_spectra_amd/csrc/gen_profile_table.py > fake_spectra_amd/csrc/
 import numpy as np
 from scipy.special import dawsn
 
-OCTAVES = 28
+OCTAVES = 30
 BINS = 32
 
 
@@ -43,14 +44,14 @@ def rows():
         w = 2.0 ** e / BINS
         for m in range(BINS):
             lo = 2.0 ** e + m * w
-            g = g64((lo + (th + 1) / 2 * w - 2) / 4)
-            c = np.polynomial.chebyshev.chebfit(th, g, 3, w=1 / np.maximum(np.abs(g), 0.01 if lo < 16 else 0.0))
+            g = g64((lo + (th + 1) / 2 * w - 2) / 16)
+            c = np.polynomial.chebyshev.chebfit(th, g, 3, w=1 / np.maximum(np.abs(g), 0.01 if lo < 64 else 0.0))
             # a polynomial in t - lo
             mono = np.polynomial.Polynomial(np.polynomial.chebyshev.cheb2poly(c))(
                 np.polynomial.Polynomial([-1.0, 2.0 / w])).coef
             v = np.linspace(0, w, 101)
-            ref = g64((lo + v - 2) / 4)
-            err = np.abs(np.polyval(mono[::-1], v) - ref) / np.maximum(np.abs(ref), 0.01 if lo < 16 else 0.0)
+            ref = g64((lo + v - 2) / 16)
+            err = np.abs(np.polyval(mono[::-1], v) - ref) / np.maximum(np.abs(ref), 0.01 if lo < 64 else 0.0)
             worst = max(worst, float(err.max()))
             out.append(mono)
     return out, worst
@@ -59,7 +60,7 @@ def rows():
 def main():
     r, worst = rows()
     print("/* Generated by gen_profile_table.py; do not edit. */")
-    print("/* G(u) = 1 - 2u D(u): cubics in t - edge, t = 4u^2 + 2, %d bins in each of %d octaves of t from 2" % (
+    print("/* G(u) = 1 - 2u D(u): cubics in t - edge, t = 16u^2 + 2, %d bins in each of %d octaves of t from 2" % (
         BINS, OCTAVES))
     print("   (max float64 fit error %.2g of G, of 0.01 near its zero). */" % worst)
     print("#pragma once")

@@ -10,7 +10,7 @@
 //  series of w about the real axis, whose even terms sum to Re exp(-z^2) and
 //  whose odd terms are those of the entire function (2i/sqrt(pi)) D(z); the
 //  a^5 term is below 1e-7 relative for a <= 0.04.  G comes from one table of
-//  cubics in t = 4u^2 + 2 (profile_table.h) whose row number and bin edge are
+//  cubics in t = 16u^2 + 2 (profile_table.h) whose row number and bin edge are
 //  bits of t, so core, transition and wing are one code without selects, and
 //  exp(a^2 - u^2) cos(2au) is one exp2 of a polynomial in u^2;
 //  D''' = (4u^2 - 6) G + 2, and -12 G^2 beyond u = 20.
@@ -85,7 +85,7 @@ constexpr float kA3Drop = 2e-3f;
 // Per-pair constants of the FP32 profile.
 struct VoigtP {
     // log2 of Re exp(-(u + ia)^2) = exp(a^2 - u^2) cos(2au), with ln cos x =
-    // -x^2/2 - x^4/12 - x^6/45 - ...:  l0 + l1 t + l2 u^4 + l3 u^6, t = 4u^2 + 2,
+    // -x^2/2 - x^4/12 - x^6/45 - ...:  l0 + l1 t + l2 u^4 + l3 u^6, t = 16u^2 + 2,
     // from log2(e) (a^2 - (1 + 2a^2) u^2 - (4/3) a^4 u^4 - (64/45) a^6 u^6); the
     // dropped term, (17/2520)(2au)^8, changes H by < 5e-9 relative for a <= 0.04
     float l0, l1, l2, l3;
@@ -99,8 +99,8 @@ __device__ inline VoigtP make_voigt_p(double a, bool light)
 {
     const double a2 = a * a, lc1 = -(1.0 + 2.0 * a2) * kLog2E;
     VoigtP v;
-    v.l0 = (float)(a2 * kLog2E - 0.5 * lc1);
-    v.l1 = (float)(0.25 * lc1);
+    v.l0 = (float)(a2 * kLog2E - 0.125 * lc1);
+    v.l1 = (float)(0.0625 * lc1);
     v.l2 = light ? 0.0f : (float)(-(4.0 / 3.0) * a2 * a2 * kLog2E);
     v.l3 = light ? 0.0f : (float)(-(64.0 / 45.0) * a2 * a2 * a2 * kLog2E);
     v.two_a_sqpi = (float)(a * kTwoOverSqrtPi);
@@ -108,13 +108,15 @@ __device__ inline VoigtP make_voigt_p(double a, bool light)
     return v;
 }
 
-// Largest |u| whose t lies in the table, and the LDS the table takes.
+// The profile takes kUScale u, so that t is one fma.
+constexpr double kUScale = 4.0;
+// Largest |u| whose t lies in the table, and the floats the table takes.
 constexpr double kVoigtUMax = 1.1e4;
 constexpr int kPTableSize = FSAMD_P_OCTAVES * FSAMD_P_BINS * 4;
-static_assert(FSAMD_P_BINS == 32 && 4.0 * kVoigtUMax * kVoigtUMax + 2.0 < (double)(2u << FSAMD_P_OCTAVES),
+static_assert(FSAMD_P_BINS == 32 && kUScale * kUScale * kVoigtUMax * kVoigtUMax + 2.0 < (double)(2ull << FSAMD_P_OCTAVES),
               "profile_table.h");
 
-// The two terms of H(a, u) = E - (2a/sqrt(pi)) G at u = us/2, |u| <= kVoigtUMax:
+// The two terms of H(a, u) = E - (2a/sqrt(pi)) G at u = us/kUScale, |u| <= kVoigtUMax:
 // sums over samples take them separately and combine them once.  The
 // Gaussian's exponent and the table's argument come from the same t; its
 // mantissa's first 5 bits and exponent name the row, its remaining bits are
@@ -127,7 +129,7 @@ __device__ inline void voigt_terms(const VoigtP &v, float us, const float *tab, 
     const float t = __builtin_fmaf(us, us, 2.0f);
     float y = __builtin_fmaf(t, v.l1, v.l0);
     if (kA3) {
-        const float p = __builtin_fmaf(t, 0.25f, -0.5f);
+        const float p = __builtin_fmaf(t, 0.0625f, -0.125f);
         y = __builtin_fmaf(p * p, __builtin_fmaf(p, v.l3, v.l2), y);
     }
     E = __builtin_amdgcn_exp2f(y);    // 0 once y passes the FP32 range
@@ -137,7 +139,7 @@ __device__ inline void voigt_terms(const VoigtP &v, float us, const float *tab, 
     G = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(c.w, d, c.z), d, c.y), d, c.x);
     if (kA3) {
         // -(a^2/6) D''': (4u^2 - 6) G + 2 loses its digits as 1/u^4, where G -> -1/(2u^2)
-        const float D = t > 1602.0f ? G * (G * -12.0f) : __builtin_fmaf(t - 8.0f, G, 2.0f);
+        const float D = t > 6402.0f ? G * (G * -12.0f) : __builtin_fmaf(__builtin_fmaf(t, 0.25f, -6.5f), G, 2.0f);
         G = __builtin_fmaf(v.a3, D, G);
     }
 }
@@ -150,7 +152,7 @@ __device__ inline float voigt32(const VoigtP &v, float u, const float *tab)
         return 0.5f * v.two_a_sqpi * __builtin_fmaf(1.5f * x, x, x);
     }
     float E, G;
-    voigt_terms(v, 2.0f * u, tab, E, G);
+    voigt_terms(v, (float)kUScale * u, tab, E, G);
     return __builtin_fmaf(-v.two_a_sqpi, G, E);
 }
 

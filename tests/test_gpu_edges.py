@@ -111,9 +111,11 @@ def test_fp64_walks(oracle, nbins, kernel, tscale, gscale):
 
 
 # fewer sightlines than blocks (every row split, into one pair and into many),
-# a row of no pairs, rows around the size of a part, and rows too long for LDS
+# a row of no pairs, rows around the size of a part, rows too long for LDS, and
+# rows of one to three pixels (windows of none and one a direction)
 @pytest.mark.parametrize("n,nlos,nbins,hfrac", [(1, 1, 8, 0.4), (127, 2, 64, 0.5), (129, 1, 64, 0.5), (5000, 1, 300, 0.3),
-                                                (400, 40, 100, 0.2), (3000, 2, 25000, 0.2), (3, 20, 50, 0.05)])
+                                                (400, 40, 100, 0.2), (3000, 2, 25000, 0.2), (3, 20, 50, 0.05),
+                                                (5, 2, 1, 0.4), (5, 2, 2, 0.4), (40, 2, 3, 0.4)])
 def test_split_rows(oracle, n, nlos, nbins, hfrac):
     """Rows cut into parts that add into the output: tau to the stated
     tolerance, column density to rounding, and forward and backward windows."""

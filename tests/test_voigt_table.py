@@ -1,4 +1,4 @@
-"""profile_table.h (the FP32 profile's cubics of G = 1 - 2u D in t = 4u^2 + 2)
+"""profile_table.h (the FP32 profile's cubics of G = 1 - 2u D in t = 16u^2 + 2)
 on the CPU: the header is its generator's output, and rows addressed by the
 bits of t as voigt_terms does follow scipy's dawsn."""
 import os
@@ -32,14 +32,14 @@ def table():
 def test_rows_follow_dawson(table, lo, hi):
     coef, octaves = table
     u = np.linspace(lo, hi, 40001)
-    t = (4.0 * u * u + 2.0).astype(np.float32)
+    t = (16.0 * u * u + 2.0).astype(np.float32)
     edge = t.view(np.uint32) & np.uint32(0xFFFC0000)
     row = ((edge >> 14) & np.uint32(0x3FFF)) // 16
     assert row.max() < octaves * 32
     d = t.astype(np.float64) - edge.view(np.float32)
     c = coef[row].astype(np.float64)
     got = c[:, 0] + d * (c[:, 1] + d * (c[:, 2] + d * c[:, 3]))
-    uu = np.sqrt(np.maximum((t.astype(np.float64) - 2.0) / 4.0, 0.0))
+    uu = np.sqrt(np.maximum((t.astype(np.float64) - 2.0) / 16.0, 0.0))
     x = 1.0 / np.maximum(uu * uu, 1e-300)
     series = -0.5 * x * (1 + 1.5 * x * (1 + 2.5 * x * (1 + 3.5 * x * (1 + 4.5 * x * (1 + 5.5 * x * (1 + 6.5 * x))))))
     ref = np.where(uu < 12.0, 1.0 - 2.0 * uu * dawsn(uu), series)
