@@ -1104,14 +1104,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     constexpr int kWavesPerBlock = kBlock / 64;
     constexpr int kGroupsPerWave = 64 / kG;
     extern __shared__ double smem[];
-    // The table comes first: a row number has 5 exponent bits, so a NaN's names
-    // a place past the table's octaves, which still lies in this block's LDS.
+    // The table has a row for every row number (5 exponent and 5 mantissa bits),
+    // a NaN's too.
     struct Lds {
         __attribute__((aligned(16))) float ptab[kPTableSize];
         PairRec recs[kWavesPerBlock * kRecs];
         float sub_sums[kBlock * kRoundsMax];
     };
-    static_assert(sizeof(Lds) >= 32 * FSAMD_P_BINS * 16, "every row number lies in the block's LDS");
     __shared__ Lds lds;
     __shared__ int s_item;
     __shared__ unsigned long long s_next;
@@ -1289,10 +1288,9 @@ __global__ __launch_bounds__(kThreads) void tau_fixup_kernel(DepositArgs A, cons
 {
     constexpr int kGroups = kThreads / kFixG;
     struct Lds {
-        __attribute__((aligned(16))) float ptab[kPTableSize];   // first: see tau_kernel
+        __attribute__((aligned(16))) float ptab[kPTableSize];
         PairTau pslot[kGroups];
     };
-    static_assert(sizeof(Lds) >= 32 * FSAMD_P_BINS * 16, "every row number lies in the block's LDS");
     __shared__ Lds lds;
     __shared__ double gtab64[kG64Size];
     const float *ptab = lds.ptab;
@@ -1886,7 +1884,7 @@ __global__ __launch_bounds__(kColThreads) void colden_kernel(DepositArgs A, cons
 __global__ __launch_bounds__(kThreads) void voigt_peak_kernel(long long per_thread, double du, double umax,
                                                               float a, float *sink)
 {
-    __shared__ __attribute__((aligned(16))) float ptab[32 * FSAMD_P_BINS * 4];
+    __shared__ __attribute__((aligned(16))) float ptab[kPTableSize];
     for (int i = threadIdx.x; i < kPTableSize; i += kThreads) ptab[i] = d_ptab[i];
     __syncthreads();
     const VoigtP va = make_voigt_p(a, false);
@@ -1909,7 +1907,7 @@ __global__ __launch_bounds__(kThreads) void voigt_peak_kernel(long long per_thre
 // parameter is set up as for a pair.
 __global__ __launch_bounds__(kThreads) void voigt_eval_kernel(const double *u, long long n, double a, float *out)
 {
-    __shared__ __attribute__((aligned(16))) float ptab[32 * FSAMD_P_BINS * 4];
+    __shared__ __attribute__((aligned(16))) float ptab[kPTableSize];
     for (int i = threadIdx.x; i < kPTableSize; i += kThreads) ptab[i] = d_ptab[i];
     __syncthreads();
     const VoigtP va = make_voigt_p(a, false);

@@ -22,7 +22,7 @@ Run:  python fake_spectra_amd/csrc/gen_profile_table.py > fake_spectra_amd/csrc/
 import numpy as np
 from scipy.special import dawsn
 
-OCTAVES = 30
+OCTAVES = 32
 BINS = 32
 
 

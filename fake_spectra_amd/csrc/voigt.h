@@ -111,10 +111,11 @@ __device__ inline VoigtP make_voigt_p(double a, bool light)
 // The profile takes kUScale u, so that t is one fma.
 constexpr double kUScale = 4.0;
 // Largest |u| whose t lies in the table, and the floats the table takes.
-constexpr double kVoigtUMax = 1.1e4;
+constexpr double kVoigtUMax = 2.3e4;
 constexpr int kPTableSize = FSAMD_P_OCTAVES * FSAMD_P_BINS * 4;
 static_assert(FSAMD_P_BINS == 32 && kUScale * kUScale * kVoigtUMax * kVoigtUMax + 2.0 < (double)(2ull << FSAMD_P_OCTAVES),
               "profile_table.h");
+static_assert(FSAMD_P_OCTAVES == 32, "a row for every value of the five exponent bits");
 
 // The two terms of H(a, u) = E - (2a/sqrt(pi)) G at u = us/kUScale, |u| <= kVoigtUMax:
 // sums over samples take them separately and combine them once.  The
