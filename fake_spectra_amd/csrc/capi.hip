@@ -73,9 +73,13 @@ static long long tune_key(int nbins, int nlines, int kernel)
 
 // Parts of a split sightline are multiples of this many pairs.  tau: below some
 // 16 pairs a wavefront the row's zeroing and flush cost more than the balance
-// gains.  Column density: a block's wavefronts take 64 pairs at a time.
+// gains (the adjoint's blocks have 16).  Column density: a block's wavefronts
+// take 64 pairs at a time.
 constexpr long long kTauPart = 128;
+constexpr long long kAdjointPart = 256;
 constexpr long long kColdenPart = kColThreads;
+// Longest row fsamd_tau_adjoint takes.
+constexpr int kAdjointMaxBins = 19536;
 
 // Work items for K lines (or parts of the fields) in the plan's heaviest-first
 // order; a sightline with more than `chunk` pairs is split into non-direct
@@ -710,9 +714,9 @@ int fsamd_tau_adjoint(fsamd_plan *P, int nbins, int kernel, double velfac, const
     static thread_local DeviceInfo dev;
     int rc;
     if (dev.ncu == 0 && (rc = device_info(dev))) return rc;
-    if (deposit_lds_bytes(nbins) + adjoint_static_lds(g_group_size.load(std::memory_order_relaxed)) >
-        (size_t)dev.max_lds)
-        return fail(FSAMD_ERR_UNSUPPORTED, "adjoint rows must fit in LDS (nbins too large)");
+    if (nbins > kAdjointMaxBins)
+        return fail(FSAMD_ERR_UNSUPPORTED, "the adjoint takes rows of at most " + std::to_string(kAdjointMaxBins) +
+                                               " pixels (nbins too large)");
     std::vector<LineDesc> ld(nlines);
     for (int i = 0; i < nlines; ++i) {
         if (!lines[i].dens || !lines[i].grad_tau || !lines[i].grad_dens)
@@ -769,8 +773,8 @@ int fsamd_tau_adjoint(fsamd_plan *P, int nbins, int kernel, double velfac, const
         A.grad_temp = grad_temp;
         A.grad_vel = grad_vel;
         fsamd_plan::ItemSet *set = nullptr;
-        const int slots = adjoint_blocks_per_cu(gsize, nbins) * dev.ncu;
-        if ((rc = item_set(P, K, 1ll << 62, slots, kTauPart, &set))) return rc;
+        const int slots = dev.ncu;
+        if ((rc = item_set(P, K, 1ll << 62, slots, kAdjointPart, &set))) return rc;
         if (set->host.empty()) continue;
         A.nitems = (int)set->host.size();
         A.fix = P->fix.as<Fixup>();

@@ -38,8 +38,8 @@
 
 namespace fsamd {
 
-__constant__ __attribute__((aligned(16))) float c_gtab[kGTableSize] = FSAMD_G_COEF_INIT;
 __device__ __attribute__((aligned(16))) const float d_ptab[kPTableSize] = FSAMD_P_COEF_INIT;
+__device__ __attribute__((aligned(16))) const float d_dtab[kPTableSize] = FSAMD_P_DCOEF_INIT;   // dG/d(u^2)
 constexpr int kG64Size = FSAMD_G64_NPIECE * FSAMD_G64_NCOEF;
 __device__ const double d_gtab64[kG64Size] = FSAMD_G64_COEF_INIT;
 
@@ -189,11 +189,11 @@ __device__ inline int wrap_near(int z, int nbins)
 // Per-pair constants of LineAbsorption::add_tau_particle and SingleAbsorber as
 // the walks read them.  They lie in LDS: uniform over a lane group, they are
 // read with broadcast loads where they are used and take no vector registers
-// of the per-pixel loop.  Velocities in units of b carry the factor kUScale of
-// the profile's argument (voigt.h).
+// of the per-pixel loop.  Velocities in units of b carry the scale of the
+// profile's argument (voigt_uscale, close to kUScale).
 struct PairRec {
     double vel;      // velfac*ppos + pvel (absorption.cpp:234)
-    double ibs;      // kUScale / b
+    double ibs;      // voigt_uscale / b
     double dss;      // sub-sample spacing, bintov / max(np - 1, 1) * ibs
     double scale;    // amp * dens * dvk / velfac: taulast = scale * (sample sum)
     double snear;    // scale / max(np - 1, 1), for the sum over sub-samples
@@ -203,7 +203,7 @@ struct PairRec {
     // 7 x np samples sum to Y (C0 + C1 Y + ... + C9 Y^9), Y = (ufar/U)^2.
     float Cw[kWingTerms];
     VoigtP vp;       // constants of the FP32 profile
-    float ufs;       // kUScale ufar
+    float ufsq;      // (voigt_uscale ufar)^2
     int zmax;
     int shape;       // near-step shape of the main kernel (step_shape)
     int k;           // the pair, counted from the work item's first (main kernel)
@@ -219,8 +219,6 @@ struct PairTau : PairRec {
     double scale_nd; // amp * dvk / velfac (scale without the density)
     double temp;     // particle temperature
     int part;        // particle index
-    float CwF[kWingTerms];   // adjoint: far-wing coefficients of sum w (u dH/du + a dH/da)
-    VoigtA va;
     int fp64;
     int np;          // sub-samples per pixel (1 = midpoint)
     int wing_ready;  // Cw computed
@@ -228,8 +226,8 @@ struct PairTau : PairRec {
     double dv;       // sub-sample spacing bintov / (np - 1)
 };
 
-// kUScale u, u = (vv_i - vouter)/b of the kernel sample i - 3 = j from the centre,
-// from s = kUScale vouter/b: in FP64 and rounded once, so u keeps half an ulp
+// u times its scale, u = (vv_i - vouter)/b of the kernel sample i - 3 = j from the
+// centre, from s = vouter/b times the scale: in FP64 and rounded once, so u keeps half an ulp
 // where the two nearly cancel.
 __device__ inline float sample_us(double qs, int j, double s) { return (float)__builtin_fma((double)j, qs, -s); }
 
@@ -250,7 +248,7 @@ __device__ inline double shfl_d(double v, int src)
 }
 
 // sum_i K(q_i) Re w((vv_i - vouter)/b + i a), FP32 profile; the sample
-// offsets from the FP64 anchor s = kUScale vouter/b.  kA3 = false: the light form
+// offsets from the FP64 anchor s, vouter/b times its scale.  kA3 = false: the light form
 // of the profile (pairs with a <= kA3Drop).
 template <bool kA3 = true>
 __device__ inline float inner32(const PairRec &P, double s, const float *ptab)
@@ -373,7 +371,7 @@ __device__ inline double ipow(double x, int n)
 // positive offsets with the summed weights of each +- pair; Y_k = h^2k T[m][k]
 // for a pixel of half-width h in np = m + 1 sub-samples, with T tabulated
 // exactly (wing_table.h) up to m = FSAMD_WING_TMAX.
-template <int kG, bool kAdj = false>
+template <int kG>
 __device__ inline void wing_setup(PairTau &P, double bintov, int lane)
 {
     const double inv_u = 1.0 / P.ufar;
@@ -397,7 +395,7 @@ __device__ inline void wing_setup(PairTau &P, double bintov, int lane)
         }
     }
     // m'_n = sum_k C(2n,2k) X_k Y_(n-k), X_k by running powers
-    const double c4 = P.qs * (inv_u / kUScale), c5 = 2.0 * c4, c6 = 3.0 * c4;
+    const double c4 = 0.25 * P.vhigh * P.inv_b * inv_u, c5 = 2.0 * c4, c6 = 3.0 * c4;
     const double x4 = c4 * c4, x5 = c5 * c5, x6 = c6 * c6;
     const double w4 = 2.0 * P.W[1], w5 = 2.0 * P.W[2], w6 = 2.0 * P.W[3];
     double p4 = 1.0, p5 = 1.0, p6 = 1.0, mom = 0.0;
@@ -414,7 +412,7 @@ __device__ inline void wing_setup(PairTau &P, double bintov, int lane)
     // C'_n = sum_(k+j=n) g_k ufar^(-2k-2) C(2n+1, 2j) m'_j
     const double a = P.aa, a2 = a * a, iu2 = inv_u * inv_u, u2 = P.ufar * P.ufar;
     // j = 0..n walks k = n..0: start from ufar^(-2n-2)
-    double C = 0.0, CF = 0.0, gs = a * (1.0 / kSqrtPi) * iu2 * ipow(iu2, n);
+    double C = 0.0, gs = a * (1.0 / kSqrtPi) * iu2 * ipow(iu2, n);
 #pragma unroll 1
     for (int j = 0; j < kWingTerms; ++j) {
         const double mj = shfl_d<kG>(mom, j);
@@ -424,14 +422,9 @@ __device__ inline void wing_setup(PairTau &P, double bintov, int lane)
             const double binom = c_binom_odd[n * kWingTerms + j];
             const double qk = k > 0 ? c_wing_q[k - 1] : 0.0;
             C += gs * (c_wing_p[k] - a2 * qk) * binom * mj;
-            // u dH/du + a dH/da of the term a p_k u^(-2k-2) - a^3 q_(k-1) u^(-2k-2)
-            if (kAdj) CF += gs * (-(2.0 * k + 1.0) * c_wing_p[k] + (2.0 * k - 1.0) * a2 * qk) * binom * mj;
         }
     }
-    if (lane < kWingTerms) {
-        P.Cw[lane] = (float)C;
-        if (kAdj) P.CwF[lane] = (float)CF;
-    }
+    if (lane < kWingTerms) P.Cw[lane] = (float)C;
 }
 
 // Sub-sample grid of one walk step in the main kernel.  A step evaluates one
@@ -638,7 +631,6 @@ __device__ inline bool setup_pair(const DepositArgs &A, int line, const LineDesc
         P.aa = C.aa;
         P.zmax = C.zmax;
         P.fp64 = C.fp64;
-        P.va = make_voigt_a(C.fp64 ? 0.0 : C.aa);
         P.vp = make_voigt_p(C.fp64 ? 0.0 : C.aa, C.aa <= (double)kA3Drop);
         P.scale = C.scale;
         P.scale_nd = C.scale_nd;
@@ -646,7 +638,7 @@ __device__ inline bool setup_pair(const DepositArgs &A, int line, const LineDesc
         P.part = p;
         P.np = C.np;
         P.ufar = C.ufar;
-        P.ibs = kUScale * C.inv_b;
+        P.ibs = voigt_uscale(P.vp, C.fp64 ? 0.0 : C.aa) * C.inv_b;
         P.qs = 0.25 * C.vhigh * P.ibs;
         P.wing_ready = 0;
         P.inv_nm1 = C.np > 1 ? 1.0 / (C.np - 1) : 1.0;
@@ -679,8 +671,12 @@ constexpr int kRefillRoom = 12;   // fewest free records worth a set-up while ot
 // kernel extents 0..30 b and a <= 0.04).  c0 = vhigh/b and h = half the
 // pixel width over b, both in units of ufar; W the kernel weights at offsets
 // 0, 1/4, 1/2, 3/4 of vhigh; m1 = sub-samples - 1 (at most FSAMD_WING_TMAX).
+// kAdj: CwT receives the coefficients of the sum of W (H + u dH/du + a dH/da),
+// from that operator on the term a p_k u^(-2k-2) - a^3 q_(k-1) u^(-2k-2); its
+// leading one is zero.
+template <bool kAdj>
 __device__ __noinline__ void wing_coeffs(float c0, float h, int m1, float W0, float W1, float W2, float W3, float a,
-                                         float ufar, float *Cw)
+                                         float ufar, float *Cw, float *CwT)
 {
     float Y[kWingTerms];
     if (m1 == 0) {
@@ -720,15 +716,18 @@ __device__ __noinline__ void wing_coeffs(float c0, float h, int m1, float W0, fl
     float lead = a * kInvSqrtPiF * iu2;   // a/sqrt(pi) ufar^(-2n-2) at n = 0
 #pragma unroll
     for (int n = 0; n < kWingTerms; ++n) {
-        float cn = 0.0f, gs = lead;
+        float cn = 0.0f, cf = 0.0f, gs = lead;
 #pragma unroll
         for (int j = 0; j <= n; ++j) {
             if (j > 0) gs *= u2;
             const int k = n - j;
             const float qk = k > 0 ? (float)c_wing_q[k - 1] : 0.0f;
-            cn += gs * ((float)c_wing_p[k] - a2 * qk) * (float)c_binom_odd[n * kWingTerms + j] * m[j];
+            const float bm = gs * (float)c_binom_odd[n * kWingTerms + j] * m[j];
+            cn += ((float)c_wing_p[k] - a2 * qk) * bm;
+            if (kAdj) cf += ((2.0f * k - 2.0f) * a2 * qk - 2.0f * k * (float)c_wing_p[k]) * bm;
         }
         Cw[n] = cn;
+        if (kAdj) CwT[n] = cf;
         lead *= iu2;
     }
 }
@@ -747,6 +746,28 @@ __device__ inline float kernel_weight_q2(int kernel, double q2)
         return (float)(9. / 40 / kPi * (p3 * p3 * t3 - 6.0 * (p2 * p2 * t2) + 15.0 * (p1 * p1 * t1)));
     }
     return kernel == kTopHat ? (float)(3. / 4. / kPi) : 1.0f;
+}
+
+// The record of this lane's pair if its bit is set in m: the r-th pair goes to
+// the r-th free record.  Lane l stands for record l and sends its number to the
+// lane of its rank; `used` says whether record l gets a pair.
+__device__ inline int free_record(unsigned free, unsigned long long m, int lane, bool &used)
+{
+    const bool isfree = lane < kRecs && ((free >> (lane & 31)) & 1u);
+    const int frank = __popc(free & ((1u << (lane & 31)) - 1u));
+    used = isfree && frank < __popcll(m);
+    const int nth = __builtin_amdgcn_ds_permute(4 * (isfree ? frank : 63), lane);
+    return __shfl(nth, __popcll(m & ((1ull << lane) - 1ull)), 64);
+}
+
+// Pairs to claim for a wavefront: its free records, fewer near the end of the
+// item so that the block's wavefronts finish together.
+__device__ inline int pairs_wanted(long long left, int waves, int groups, int nfree)
+{
+    const long long share = left / (2 * waves);
+    int want = nfree;
+    if (share < want) want = (int)(share > 2 * groups ? share : 2 * groups);
+    return min(want, nfree);
 }
 
 // Claim up to `want` (at most the free records) pairs of item w for the
@@ -775,18 +796,19 @@ __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int 
         }
     }
     const unsigned long long m = __ballot(enq);
-    const int n = __popcll(m);
-    // the r-th pair goes to the r-th free record: lane l stands for record l
-    // and sends its number to the lane of its rank
-    const bool isfree = lane < kRecs && ((free >> (lane & 31)) & 1u);
-    const int frank = __popc(free & ((1u << (lane & 31)) - 1u));
-    const int nth = __builtin_amdgcn_ds_permute(4 * (isfree ? frank : 63), lane);
-    const int slot = __shfl(nth, __popcll(m & ((1ull << lane) - 1ull)), 64);
+    bool used;
+    const int slot = free_record(free, m, lane, used);
     wave_sync();   // the records' former pairs have been read
     if (enq) {
         PairRec &r = recs[slot];
         const int shift = box_shift(C.zmax, A.nbins);
-        const double ibs = kUScale * C.inv_b;
+        // the walk uses the light form of the profile for a <= kA3Drop, as a
+        // property of the pair: its coefficients are zero, so the full form
+        // gives the same values and the result does not depend on which
+        // pairs share a wavefront
+        const VoigtP vp = make_voigt_p(C.aa, C.aa <= (double)kA3Drop);
+        r.vp = vp;
+        const double us = voigt_uscale(vp, C.aa), ibs = us * C.inv_b;
         const double inv_m = C.np > 1 ? 1.0 / (C.np - 1) : 1.0;
         r.vel = shift ? C.vel - shift * A.vbox : C.vel;
         r.zmax = C.zmax - shift * A.nbins;
@@ -795,11 +817,6 @@ __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int 
         r.scale = C.scale;
         r.snear = C.scale * inv_m;
         r.qs = 0.25 * C.vhigh * ibs;
-        // the walk uses the light form of the profile for a <= kA3Drop, as a
-        // property of the pair: its coefficients are zero, so the full form
-        // gives the same values and the result does not depend on which
-        // pairs share a wavefront
-        r.vp = make_voigt_p(C.aa, C.aa <= (double)kA3Drop);
         r.k = (int)(kk - w.p0);   // a row has fewer than 2^31 pairs (one per particle)
         const double inv_s2 = 1.0 / (C.vsmooth * C.vsmooth);
         float W[4];
@@ -811,16 +828,15 @@ __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int 
         *(float4 *)r.W = make_float4(W[0], W[1], W[2], W[3]);
         // the walk compares with ufar rounded to FP32, the unit of the coefficients
         const float ufar = (float)C.ufar;
-        r.ufs = (float)kUScale * ufar;
+        r.ufsq = (float)((us * ufar) * (us * ufar));
         const StepShape sh = step_shape(C.np, kG);
         r.shape = sh.packed();
         // far-wing coefficients, in units of that ufar
         const double iu = 1.0 / (double)ufar;
-        wing_coeffs((float)(C.vhigh * C.inv_b * iu), (float)(0.5 * bintov * C.inv_b * iu), sh.nm1, W[0], W[1], W[2],
-                    W[3], (float)C.aa, ufar, r.Cw);
+        wing_coeffs<false>((float)(C.vhigh * C.inv_b * iu), (float)(0.5 * bintov * C.inv_b * iu), sh.nm1, W[0], W[1],
+                           W[2], W[3], (float)C.aa, ufar, r.Cw, nullptr);
     }
     wave_sync();
-    const bool used = isfree && frank < n;
     const unsigned mine = (unsigned)__ballot(used);
     const unsigned a3 = (unsigned)__ballot(used && recs[lane & 31].vp.a3 != 0.0f);
     free &= ~mine;
@@ -941,14 +957,13 @@ __device__ inline int far_walk(const DepositArgs &A, const PairRec &P, double *r
                                const CutBand &cut, int lane, LaneStats &st, long long k, int item)
 {
     const double bintov = A.vbox / A.nbins;
-    const float ufsq = (float)((double)P.ufs * P.ufs);
     for (int i0 = 0; i0 < count; i0 += 64) {
         const int i = i0 + lane;
         const bool valid = i < count;
         const int z = zf + dir * i;
         const double vlow = z * bintov - P.vel;
         const double Us = (vlow + 0.5 * bintov) * P.ibs;
-        const float Y = ufsq * __builtin_amdgcn_rcpf((float)(Us * Us));
+        const float Y = P.ufsq * __builtin_amdgcn_rcpf((float)(Us * Us));
         float S = P.Cw[kWingTerms - 1];
 #pragma unroll
         for (int q = kWingTerms - 2; q >= 0; --q) S = __builtin_fmaf(S, Y, P.Cw[q]);
@@ -1003,7 +1018,7 @@ __device__ inline int near_step(const DepositArgs &A, const PairRec &P, float *s
         // Sub-sample m of the step, in increasing velocity: sub-sample m mod
         // (np-1) of its pixel (singleabs.h:118-121) up to the rounding of m dv
         // against the pixel's own vlow, or (np = 1) pixel m's centre
-        // (singleabs.h:113); positions as kUScale v / b.
+        // (singleabs.h:113); positions in u's scale.
         const int nsub = nm1 == 0 ? pcount : pcount * nm1 + 1;
         const double dss = P.dss;
         double sv = vf * P.ibs;
@@ -1171,12 +1186,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             if (needing) {
                 const int nneed = __popcll(needing);
                 if (more && __popc(take_full ? full : light) < nneed && __popc(free) >= kRefillRoom) {
-                    // claim up to the free records, fewer near the end of the item so
-                    // that the block's wavefronts finish together
-                    const long long rem = (long long)w.p1 - (long long)__atomic_load_n(&s_next, __ATOMIC_RELAXED);
-                    const long long share = rem / (2 * kWavesPerBlock);
-                    int want = __popc(free);
-                    if (share < want) want = (int)(share > 2 * kGroupsPerWave ? share : 2 * kGroupsPerWave);
+                    int want = pairs_wanted((long long)w.p1 - (long long)__atomic_load_n(&s_next, __ATOMIC_RELAXED),
+                                            kWavesPerBlock, kGroupsPerWave, __popc(free));
                     if (A.claim < want) want = A.claim;
                     if (want < 1) want = 1;
                     want = __builtin_amdgcn_readfirstlane(want);
@@ -1208,7 +1219,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             // walk there, one such walk of the wavefront after the other
             const int zf = z0 + dir * c;
             const double vf = zf * bintov - P.vel;   // absorption.cpp:252
-            const bool far = walking && fabs((vf + 0.5 * bintov) * P.ibs) >= (double)P.ufs;
+            const double uc = (vf + 0.5 * bintov) * P.ibs;
+            const bool far = walking && uc * uc >= (double)P.ufsq;
             int n = 0, adv = 0;
             for (unsigned long long fm = __ballot(far) & leaders; fm; fm &= fm - 1ull) {
                 const int src = __builtin_ctzll(fm);
@@ -1345,26 +1357,11 @@ __global__ __launch_bounds__(kThreads) void tau_fixup_kernel(DepositArgs A, cons
 // With g(z) = dL/dtau at the pixel:
 //   dL/d dens = sum_z g scale/dens S
 //   dL/d vel  = sum_z g scale/b SU,          SU = sum t W dH/du
-//   dL/d T    = -sum_z g scale/(2T) (S + SF), SF = sum t W (u dH/du + a dH/da)
+//   dL/d T    = -sum_z g scale/(2T) ST,      ST = sum t W (H + u dH/du + a dH/da)
 // over exactly the pixels the forward deposited (recorded windows); the
 // discrete choices (window ends, pixel index, sub-sample count) are held
 // fixed.  Far-wing pixels use the same moment expansion as the forward, with
-// a second coefficient set for SF and the derivative of the first for SU.
-
-__device__ inline void adj_inner32(const PairTau &P, double vouter, const float *gtab, float &S, float &SU,
-                                   float &SF)
-{
-    const double s = vouter * P.ibs;
-    const VoigtA va = P.va;
-#pragma unroll  // full: the adjoint kernel 6% faster than unrolling by 2 at 128^3
-    for (int j = -3; j <= 3; ++j) {
-        const VoigtGrad g = voigt32_grad(va, (float)(1 / kUScale) * sample_us(P.qs, j, s), gtab);
-        const float w = P.W[j < 0 ? -j : j];
-        S = __builtin_fmaf(w, g.H, S);
-        SU = __builtin_fmaf(w, g.Hu, SU);
-        SF = __builtin_fmaf(w, g.F, SF);
-    }
-}
+// a second coefficient set for ST and the derivative of the first for SU.
 
 // The same three sums with the FP64 Faddeeva function and FP64 kernel weights,
 // for the pairs the forward evaluates in FP64 (damping parameter above
@@ -1414,152 +1411,280 @@ __device__ inline void adj_pixel64(const PairTau &P, double vlow, double bintov,
     SF *= inv;
 }
 
-// Far-wing pixel (|U| >= ufar) of the adjoint: S, SU and SF by the moment
-// expansion of the forward and its derivative.
-__device__ inline void adj_far(const PairTau &P, double vlow, double bintov, double &S, double &SU, double &SF)
+// A pair of the adjoint: its window's pixels zlo .. zlo + n - 1, of which the first
+// nfl and the last n - nfl - nn lie in the far wing (|U| >= ufar).
+struct AdjRec {
+    double s0;        // the lower end of pixel zlo over b, in u's scale
+    double ibs, dss, qs;   // as PairRec
+    float W[4];
+    double scale_nd;  // amp * dvk / velfac (scale without the density)
+    double inv_nm1;   // 1 / max(np - 1, 1)
+    float Cw[kWingTerms], CwT[kWingTerms];
+    VoigtP vp;
+    float a2, ufsq, dens, temp;
+    int zlo, n, nfl, nn, nm1, part;
+};
+static_assert(sizeof(AdjRec) == 208, "AdjRec layout: W on a 16-byte boundary");
+
+constexpr int kAdjThreads = 1024;
+constexpr int kAdjWaves = kAdjThreads / 64;
+
+// Claim `want` pairs for the wavefront and set up those with a window, as
+// refill_wave does for the forward.  FP64 pairs go to the list of
+// tau_adjoint64_kernel.
+__device__ inline void refill_adjoint(const DepositArgs &A, const WorkItem &w, int item, const LineDesc &L,
+                                      const LosInfo &los, unsigned long long *next, AdjRec *recs, int lane, int want,
+                                      unsigned &free, unsigned &light, unsigned &full, bool &more)
 {
-    const double U = (vlow + 0.5 * bintov) * P.inv_b;
-    const float Y = (float)(P.ufar * P.ufar) * __builtin_amdgcn_rcpf((float)(U * U));
-    float s = P.Cw[kWingTerms - 1], d = kWingTerms * P.Cw[kWingTerms - 1], f = P.CwF[kWingTerms - 1];
-#pragma unroll
-    for (int t = kWingTerms - 2; t >= 0; --t) {
-        s = __builtin_fmaf(s, Y, P.Cw[t]);
-        d = __builtin_fmaf(d, Y, (t + 1.0f) * P.Cw[t]);
-        f = __builtin_fmaf(f, Y, P.CwF[t]);
+    unsigned long long base = 0;
+    if (lane == 0) base = atomicAdd(next, (unsigned long long)want);
+    base = (unsigned long long)__shfl((long long)base, 0, 64);
+    const long long kk = (long long)base + lane;
+    const double bintov = A.vbox / A.nbins;
+    bool enq = false;
+    int lf = 0, lb = 0;
+    PairConsts C;
+    if (lane < want && kk < w.p1) {
+        const long long wi = ((long long)w.line * A.npairs + kk) * 2;
+        lf = A.win[wi];
+        lb = A.win[wi + 1];
+        if (lf + lb > 0 && pair_consts(A, w.line, L, los, kk, FSAMD_WING_TMAX, C)) {
+            enq = !C.fp64;
+            if (C.fp64) push_fixup(A, kk, item, 0, 0, 0);
+        }
     }
-    S = (double)(s * Y);
-    SU = 2.0 / U * (double)(d * Y);
-    SF = (double)(f * Y);
+    const unsigned long long m = __ballot(enq);
+    bool used;
+    const int slot = free_record(free, m, lane, used);
+    wave_sync();   // the records' former pairs have been read
+    if (enq) {
+        AdjRec &r = recs[slot];
+        const VoigtP vp = make_voigt_p(C.aa, C.aa <= (double)kA3Drop);
+        r.vp = vp;
+        const double us = voigt_uscale(vp, C.aa), ibs = us * C.inv_b;
+        const double inv_m = C.np > 1 ? 1.0 / (C.np - 1) : 1.0;
+        const int zlo = C.zmax - lb, n = lf + lb;
+        const double s0 = (zlo * bintov - C.vel) * ibs, bxs = bintov * ibs;   // absorption.cpp:252
+        r.s0 = s0;
+        r.ibs = ibs;
+        r.dss = bxs * inv_m;
+        r.qs = 0.25 * C.vhigh * ibs;
+        r.inv_nm1 = inv_m;
+        r.scale_nd = C.scale_nd;
+        r.a2 = (float)(C.aa * C.aa);
+        const double inv_s2 = 1.0 / (C.vsmooth * C.vsmooth);
+        float W[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const double vv = (i + 4) * C.dvk - C.vhigh;
+            W[i] = kernel_weight_q2(A.kernel, (C.vdr2 + vv * vv) * inv_s2);
+        }
+        *(float4 *)r.W = make_float4(W[0], W[1], W[2], W[3]);
+        const float ufar = (float)C.ufar;
+        r.ufsq = (float)((us * ufar) * (us * ufar));
+        const double iu = 1.0 / (double)ufar;
+        wing_coeffs<true>((float)(C.vhigh * C.inv_b * iu), (float)(0.5 * bintov * C.inv_b * iu), C.np - 1, W[0], W[1],
+                          W[2], W[3], (float)C.aa, ufar, r.Cw, r.CwT);
+        // far-wing pixels: those whose centre s0 + (j + 1/2) bxs lies at or beyond +-ufar
+        const double c0 = s0 + 0.5 * bxs, inv_x = 1.0 / bxs, uf = us * ufar;
+        const double jl = floor((-uf - c0) * inv_x) + 1.0, jr = ceil((uf - c0) * inv_x);
+        const int nfl = (int)fmin(fmax(jl, 0.0), (double)n), end = (int)fmin(fmax(jr, (double)nfl), (double)n);
+        r.nfl = nfl;
+        r.nn = end - nfl;
+        r.zlo = zlo;
+        r.n = n;
+        r.nm1 = C.np - 1;
+        r.part = A.pair_part[kk];
+        r.dens = A.rec[r.part].dens[w.line];
+        r.temp = C.temp;
+    }
+    wave_sync();
+    const unsigned mine = (unsigned)__ballot(used);
+    const unsigned a3 = (unsigned)__ballot(used && recs[lane & 31].vp.a3 != 0.0f);
+    free &= ~mine;
+    light |= mine & ~a3;
+    full |= a3;
+    more = (long long)base + want < w.p1;
 }
 
-template <int kG>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void tau_adjoint_kernel(
-    DepositArgs A, const WorkItem *items, int use_queue)
+// One grid point of a pair: the sums (GradSums) of the kernel samples around s.
+template <bool kA3>
+__device__ inline void adj_point(const AdjRec &P, double s, const float *tab, float &S, float &SU, float &ST,
+                                 float &SP)
 {
-    constexpr int kGroups = kThreads / kG;
-    extern __shared__ double grow[];   // dL/dtau of the item's sightline and line
-    __shared__ __attribute__((aligned(16))) float gtab[kGTableSize];
-    __shared__ PairTau pslot[kGroups];
+    const VoigtP vp = P.vp;
+    const double qs = P.qs;
+    const float a2 = P.a2;
+    const float4 w4 = *(const float4 *)P.W;
+    const float W[4] = {w4.x, w4.y, w4.z, w4.w};
+    GradSums g;
+#pragma unroll
+    for (int j = -3; j <= 3; ++j) g.add<kA3>(vp, a2, W[j < 0 ? -j : j], sample_us(qs, j, s), tab);
+    g.finish(vp, a2, S, SU, ST, SP);
+}
+
+// Bound: VALU issue (24 instructions a sample in the light form).  Structured as
+// tau_kernel: pairs set up one per lane into records, walked in place by lane
+// groups, light and full pairs in runs, far-wing pixels by the whole wavefront.
+// Here the windows are known: a group walks the grid points of its pair's near
+// pixels, each once, weighted by the trapezoid weights and dL/dtau of the
+// pixels it belongs to.  One block of 16 wavefronts a CU shares the table of G
+// and K (32 KB) and the row.  kRow: the row of dL/dtau in LDS; a row that does
+// not fit beside the records (above about 3000 pixels) is read where it is.
+// 2M particles, 1024 sightlines of 1024 pixels: 18.6 -> 8.7 ms; 32768 particles
+// and 50 sightlines, forward and adjoint: 1.2 -> 0.9 ms.
+template <int kG, bool kRow>
+__global__ __launch_bounds__(kAdjThreads) __attribute__((amdgpu_waves_per_eu(4))) void tau_adjoint_kernel(
+    DepositArgs A, const WorkItem *items)
+{
+    constexpr int kGroupsPerWave = 64 / kG;
+    extern __shared__ double grow_lds[];   // dL/dtau of the item's sightline and line
+    struct Lds {
+        __attribute__((aligned(16))) float tab[2 * kPTableSize];
+        AdjRec recs[kAdjWaves * kRecs];
+    };
+    __shared__ Lds lds;
     __shared__ int s_item;
     __shared__ unsigned long long s_next;
-    for (int i = threadIdx.x; i < kGTableSize; i += kThreads) gtab[i] = c_gtab[i];
+    for (int i = threadIdx.x; i < kPTableSize / 4; i += kAdjThreads) {
+        reinterpret_cast<float4 *>(lds.tab)[2 * i] = reinterpret_cast<const float4 *>(d_ptab)[i];
+        reinterpret_cast<float4 *>(lds.tab)[2 * i + 1] = reinterpret_cast<const float4 *>(d_dtab)[i];
+    }
+    const float *tab = lds.tab;
     const int lane = threadIdx.x & 63;
     const int glane = lane % kG;
-    const int gid = threadIdx.x / kG;
-    const int gleader = (lane / kG) * kG;
-    PairTau &P = pslot[gid];
-    const double bintov = A.vbox / A.nbins;
-    int it = use_queue ? 0 : blockIdx.x;
+    AdjRec *recs = lds.recs + (threadIdx.x / 64) * kRecs;
+    const unsigned long long leaders = kG == 64 ? 1ull : (kG == 32 ? 0x0000000100000001ull : 0x0001000100010001ull);
     for (;;) {
-        int item;
         __syncthreads();
-        if (use_queue) {
-            if (threadIdx.x == 0) s_item = atomicAdd(A.queue, 1);
-            __syncthreads();
-            item = s_item;
-        } else {
-            item = it;
-            it += gridDim.x;
-        }
+        if (threadIdx.x == 0) s_item = atomicAdd(A.queue, 1);
+        __syncthreads();
+        const int item = s_item;
         if (item >= A.nitems) break;
         const WorkItem w = items[item];
         const LineDesc L = line_of(A, w.line);
         const double *grad_row = L.out + (size_t)w.los * A.nbins;
-        for (int j = threadIdx.x; j < A.nbins; j += kThreads) grow[j] = grad_row[j];
+        if (kRow)
+            for (int j = threadIdx.x; j < A.nbins; j += kAdjThreads) grow_lds[j] = grad_row[j];
+        const double *grow = kRow ? grow_lds : grad_row;
         if (threadIdx.x == 0) s_next = (unsigned long long)w.p0;
         __syncthreads();
         const LosInfo los = los_info(A, w.los);
+        // group state: 0 needs a pair, 1 walks rec's grid points from c on, 2 no pairs left
+        int state = 0, c = 0, rec = 0;
+        double aS = 0, aU = 0, aT = 0, aP = 0;   // aU, aP: without 1 / scale and 1 / scale^2 (GradSums)
+        unsigned free = ~0u, light = 0, full = 0;
+        bool more = true, take_full = false;
         for (;;) {
-            unsigned long long kk = 0;
-            if (glane == 0) kk = atomicAdd(&s_next, 1ull);
-            kk = (unsigned long long)__shfl((long long)kk, gleader, 64);
-            const bool have = (long long)kk < w.p1;
-            if (!__ballot(have)) break;
-            if (!have) continue;
-            const long long k = (long long)kk;
-            if (!setup_pair<kG>(A, w.line, L, los, k, P, glane)) continue;
-            const long long wi = ((long long)w.line * A.npairs + k) * 2;
-            const int lf = A.win[wi], lb = A.win[wi + 1];
-            const int n = lf + lb;
-            const int zlo = P.zmax - lb;   // the window: pixels zlo .. zlo + n - 1
-            double aS = 0, aU = 0, aF = 0;
-            if (P.fp64) {
-                // the forward walked this pair with the FP64 profile, pixel by
-                // pixel: tau_adjoint64_kernel does the same (the FP64 Faddeeva
-                // code stays out of this kernel's registers)
-                if (glane == 0 && n > 0) push_fixup(A, k, item, 0, 0, 0);
-                continue;
-            }
-            // far-wing pixels (|U| >= ufar) sit at the two ends of the window
-            int nfl = 0, nfr = 0;
-            for (int c = 0; c < n; c += kG) {
-                const int j = c + glane;
-                const double U = ((zlo + j) * bintov - P.vel + 0.5 * bintov) * P.inv_b;
-                const bool far = j < n && fabs(U) >= P.ufar;
-                nfl += __popcll(group_bits<kG>(__ballot(far && U < 0), lane));
-                nfr += __popcll(group_bits<kG>(__ballot(far && U > 0), lane));
-            }
-            if (nfl + nfr > 0) {
-                if (!P.wing_ready) {
-                    wing_setup<kG, true>(P, bintov, glane);
-                    if (glane == 0) P.wing_ready = 1;
-                    wave_sync();
+            const unsigned long long needing = __ballot(state == 0) & leaders;
+            if (needing) {
+                if (more && __popc(take_full ? full : light) < __popcll(needing) && __popc(free) >= kRefillRoom) {
+                    int want = pairs_wanted((long long)w.p1 - (long long)__atomic_load_n(&s_next, __ATOMIC_RELAXED),
+                                            kAdjWaves, kGroupsPerWave, __popc(free));
+                    want = __builtin_amdgcn_readfirstlane(want < 1 ? 1 : want);
+                    refill_adjoint(A, w, item, L, los, &s_next, recs, lane, want, free, light, full, more);
                 }
-                for (int c = 0; c < nfl + nfr; c += kG) {
-                    const int f = c + glane;
-                    if (f < nfl + nfr) {
-                        const int z = zlo + (f < nfl ? f : n - nfr + (f - nfl));
-                        double S, SU, SF;
-                        adj_far(P, z * bintov - P.vel, bintov, S, SU, SF);
-                        const double g = grow[wrap_pixel(z, A.nbins)];
-                        aS += g * S;
-                        aU += g * SU;
-                        aF += g * SF;
+                if ((take_full ? full : light) == 0) take_full = !take_full;
+                for (unsigned long long nm = needing; nm && (light | full); nm &= nm - 1ull) {
+                    const bool f = light == 0 || (take_full && full != 0);
+                    const int at = __builtin_ctz(f ? full : light);
+                    if (f)
+                        full &= full - 1u;
+                    else
+                        light &= light - 1u;
+                    if (lane / kG == __builtin_ctzll(nm) / kG) {
+                        rec = at;
+                        state = 1;
+                        c = 0;
+                        aS = aU = aT = aP = 0;
                     }
                 }
+                if (state == 0 && !more) state = 2;
             }
-            // the other pixels on the shared sub-sample grid of tau_kern_outer
-            // (singleabs.h:110-125): each grid point once, weighted by the
-            // trapezoid weights and dL/dtau of the pixels it belongs to
-            const int j0 = nfl, nn = n - nfl - nfr;
-            if (nn > 0) {
-                const int nm1 = P.np - 1;
-                const int npts = nm1 == 0 ? nn : nn * nm1 + 1;
-                for (int m = glane; m < npts; m += kG) {
-                    double v, wgt;
-                    if (nm1 == 0) {
-                        const int z = zlo + j0 + m;
-                        const double vlow = z * bintov - P.vel;   // absorption.cpp:252
-                        v = ((vlow + bintov) + vlow) / 2.;        // singleabs.h:113
-                        wgt = grow[wrap_pixel(z, A.nbins)];
-                    } else {
-                        const int jj = m / nm1, kk = m - jj * nm1;
-                        const int z = zlo + j0 + jj;
-                        const double vlow = z * bintov - P.vel;
-                        v = kk == 0 ? vlow : kk * P.dv + vlow;    // singleabs.h:118-121
-                        if (kk == 0) {
-                            const double gl = jj > 0 ? grow[wrap_pixel(z - 1, A.nbins)] : 0.0;
-                            const double gr = jj < nn ? grow[wrap_pixel(z, A.nbins)] : 0.0;
-                            wgt = 0.5 * (gl + gr) * P.inv_nm1;
-                        } else {
-                            wgt = grow[wrap_pixel(z, A.nbins)] * P.inv_nm1;
-                        }
+            if (!__ballot(state != 2)) break;
+            const AdjRec &P = recs[rec];
+            const int nm1 = P.nm1;
+            const int npts = state != 1 || P.nn == 0 ? 0 : nm1 == 0 ? P.nn : P.nn * nm1 + 1;
+            const bool a3 = __ballot(state == 1 && P.vp.a3 != 0.0f) != 0ull;
+            const int m = c + glane;
+            if (m < npts) {
+                // grid point m: sub-sample kk of near pixel jj (singleabs.h:110-125)
+                const int jj = nm1 == 0 ? m : (int)((m + 0.5) * P.inv_nm1);
+                const int kk = nm1 == 0 ? 1 : m - jj * nm1;
+                const int z = P.zlo + P.nfl + jj;
+                double wgt = jj < P.nn ? grow[wrap_pixel(z, A.nbins)] : 0.0;
+                if (kk == 0) wgt = 0.5 * (wgt + (jj > 0 ? grow[wrap_pixel(z - 1, A.nbins)] : 0.0));
+                const double dss = P.dss;
+                const double s = __builtin_fma((double)P.nfl * (nm1 == 0 ? 1 : nm1) + m + (nm1 == 0 ? 0.5 : 0.0), dss, P.s0);
+                float S, SU, ST, SP;
+                if (a3)
+                    adj_point<true>(P, s, tab, S, SU, ST, SP);
+                else
+                    adj_point<false>(P, s, tab, S, SU, ST, SP);
+                aS = __builtin_fma(wgt, (double)S, aS);
+                aU = __builtin_fma(wgt, (double)SU, aU);
+                aT = __builtin_fma(wgt, (double)ST, aT);
+                aP = __builtin_fma(wgt, (double)SP, aP);
+            }
+            c += kG;
+            const bool ended = state == 1 && c >= npts;
+            const unsigned long long em = __ballot(ended) & leaders;
+            if (!em) continue;
+            if (ended) {
+                // the trapezoid's weights, and the scale (voigt_uscale) from l1
+                const double k2 = (double)P.vp.l1 * (-1.0 / kLog2E) / (1.0 + 2.0 * (double)P.a2);   // 1 / scale^2
+                const double k1 = kUScale * (0.5 * k2 + 0.5 / (kUScale * kUScale));   // its root, next to 1 / kUScale
+                aS *= P.inv_nm1;
+                aU *= P.inv_nm1 * k1;
+                aT = P.inv_nm1 * __builtin_fma(k2, aP, aT);
+            }
+            for (unsigned long long fm = em; fm; fm &= fm - 1ull) {
+                const int src = __builtin_ctzll(fm);
+                const int at = __builtin_amdgcn_readlane(rec, src);
+                const AdjRec &Q = recs[at];
+                free |= 1u << at;   // its reads below come before the next set-up
+                const int nfar = Q.n - Q.nn;
+                if (nfar == 0) continue;
+                const double bxs = Q.dss * (Q.nm1 == 0 ? 1 : Q.nm1);
+                double fS = 0, fU = 0, fT = 0;
+                for (int i = lane; i < nfar; i += 64) {
+                    const int j = i < Q.nfl ? i : i + Q.nn;
+                    const double Us = __builtin_fma((double)j + 0.5, bxs, Q.s0);
+                    const float Y = Q.ufsq * __builtin_amdgcn_rcpf((float)(Us * Us));
+                    float s = Q.Cw[kWingTerms - 1], d = kWingTerms * Q.Cw[kWingTerms - 1], f = Q.CwT[kWingTerms - 1];
+#pragma unroll
+                    for (int t = kWingTerms - 2; t >= 0; --t) {
+                        s = __builtin_fmaf(s, Y, Q.Cw[t]);
+                        d = __builtin_fmaf(d, Y, (t + 1.0f) * Q.Cw[t]);
+                        f = __builtin_fmaf(f, Y, Q.CwT[t]);
                     }
-                    float s = 0, su = 0, sf = 0;
-                    adj_inner32(P, v, gtab, s, su, sf);
-                    aS += wgt * s;
-                    aU += wgt * su;
-                    aF += wgt * sf;
+                    const double g = grow[wrap_pixel(Q.zlo + j, A.nbins)] * (double)Y;
+                    fS = __builtin_fma(g, (double)s, fS);
+                    fU = __builtin_fma(g * (2.0 * kUScale) / Us, (double)d, fU);
+                    fT = __builtin_fma(g, (double)f, fT);
+                }
+                // each lane of the pair's group takes the lanes of its number
+#pragma unroll
+                for (int o = 32; o >= kG; o >>= 1) {
+                    fS += __shfl_xor(fS, o, 64);
+                    fU += __shfl_xor(fU, o, 64);
+                    fT += __shfl_xor(fT, o, 64);
+                }
+                if (lane / kG == src / kG) {
+                    aS += fS;
+                    aU += fU;
+                    aT += fT;
                 }
             }
-            aS = group_sum<kG>(aS);
-            aU = group_sum<kG>(aU);
-            aF = group_sum<kG>(aF);
-            if (glane == 0 && n > 0) {
-                const int p = P.part;
-                unsafeAtomicAdd(&L.grad_dens[p], P.scale_nd * aS);
-                unsafeAtomicAdd(&A.grad_vel[3 * (size_t)p + los.ax - 1], P.scale * P.inv_b * aU);
-                unsafeAtomicAdd(&A.grad_temp[p], -P.scale / (2.0 * P.temp) * (aS + aF));
+            const double tS = group_sum<kG>(aS), tU = group_sum<kG>(aU), tT = group_sum<kG>(aT);
+            if (ended) {
+                if (glane == 0) {
+                    const double scale = P.scale_nd * (double)P.dens;
+                    unsafeAtomicAdd(&L.grad_dens[P.part], P.scale_nd * tS);
+                    unsafeAtomicAdd(&A.grad_vel[3 * (size_t)P.part + los.ax - 1], scale * P.ibs * (1 / kUScale) * tU);
+                    unsafeAtomicAdd(&A.grad_temp[P.part], -scale / (2.0 * (double)P.temp) * tT);
+                }
+                state = 0;
             }
         }
     }
@@ -1617,35 +1742,27 @@ int launch_tau_adjoint64(const DepositArgs &A, const WorkItem *items, int nblock
     return FSAMD_OK;
 }
 
-int launch_tau_adjoint(int gsize, const DepositArgs &A, const WorkItem *items, int nblocks, hipStream_t s)
+// Whether the adjoint keeps its row in LDS beside its records and table.
+bool adjoint_row_in_lds(int nbins) { return deposit_lds_bytes(nbins) + adjoint_static_lds(16) <= 160 * 1024; }
+
+template <int kG, bool kRow>
+static int launch_adjoint(const DepositArgs &A, const WorkItem *items, int nblocks, hipStream_t s)
 {
-    const size_t shm = deposit_lds_bytes(A.nbins);
-    if (gsize == 16) {
-        if (int rc = raise_lds_limit((const void *)tau_adjoint_kernel<16>, shm)) return rc;
-        tau_adjoint_kernel<16><<<nblocks, kThreads, shm, s>>>(A, items, 1);
-    } else if (gsize == 32) {
-        if (int rc = raise_lds_limit((const void *)tau_adjoint_kernel<32>, shm)) return rc;
-        tau_adjoint_kernel<32><<<nblocks, kThreads, shm, s>>>(A, items, 1);
-    } else {
-        if (int rc = raise_lds_limit((const void *)tau_adjoint_kernel<64>, shm)) return rc;
-        tau_adjoint_kernel<64><<<nblocks, kThreads, shm, s>>>(A, items, 1);
-    }
+    const size_t shm = kRow ? deposit_lds_bytes(A.nbins) : 0;
+    if (int rc = raise_lds_limit((const void *)tau_adjoint_kernel<kG, kRow>, shm)) return rc;
+    tau_adjoint_kernel<kG, kRow><<<nblocks, kAdjThreads, shm, s>>>(A, items);
     FSAMD_HIP(hipGetLastError());
     return FSAMD_OK;
 }
 
-int adjoint_blocks_per_cu(int gsize, int nbins)
+int launch_tau_adjoint(int gsize, const DepositArgs &A, const WorkItem *items, int nblocks, hipStream_t s)
 {
-    int nb = 0;
-    const size_t shm = deposit_lds_bytes(nbins);
-    hipError_t e = gsize == 16 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, tau_adjoint_kernel<16>, kThreads, shm)
-                 : gsize == 32 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, tau_adjoint_kernel<32>, kThreads, shm)
-                               : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, tau_adjoint_kernel<64>, kThreads, shm);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        nb = 1;
-    }
-    return nb < 1 ? 1 : nb;
+    const bool row = adjoint_row_in_lds(A.nbins);
+    if (gsize == 16)
+        return row ? launch_adjoint<16, true>(A, items, nblocks, s) : launch_adjoint<16, false>(A, items, nblocks, s);
+    if (gsize == 32)
+        return row ? launch_adjoint<32, true>(A, items, nblocks, s) : launch_adjoint<32, false>(A, items, nblocks, s);
+    return row ? launch_adjoint<64, true>(A, items, nblocks, s) : launch_adjoint<64, false>(A, items, nblocks, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1964,8 +2081,8 @@ size_t deposit_static_lds(bool tau, int gsize, int waves)
 
 size_t adjoint_static_lds(int gsize)
 {
-    return static_lds(gsize == 16 ? (const void *)tau_adjoint_kernel<16>
-                      : gsize == 32 ? (const void *)tau_adjoint_kernel<32> : (const void *)tau_adjoint_kernel<64>);
+    return static_lds(gsize == 16 ? (const void *)tau_adjoint_kernel<16, true>
+                      : gsize == 32 ? (const void *)tau_adjoint_kernel<32, true> : (const void *)tau_adjoint_kernel<64, true>);
 }
 
 int raise_lds_limit(const void *fn, size_t shm)

@@ -32,13 +32,11 @@
 //   otherwise: Taylor series in y about the real axis.
 #pragma once
 #include <hip/hip_runtime.h>
-#include "dawson_table.h"
 #include "profile_table.h"
 #include "dawson64_table.h"
 
 namespace fsamd {
 
-constexpr float kVoigtCoreMax = 7.0f;
 constexpr float kA32Max = 0.04f;
 constexpr float kTwoOverSqrtPiF = 1.12837916709551257390f;
 constexpr float kInvSqrtPiF = 0.56418958354775628695f;
@@ -46,34 +44,6 @@ constexpr double kSqrtPi = 1.77245385090551602729;
 constexpr double kTwoOverSqrtPi = 1.12837916709551257390;
 constexpr double kLog2E = 1.44269504088896340736;
 constexpr float kLog2EF = 1.44269504088896340736f;
-constexpr int kGTableSize = FSAMD_G_NROW * FSAMD_G_STRIDE;
-
-// (2n+1)!!/2^n, n = 0..8
-#define FSAMD_WING_P {1.0f, 1.5f, 3.75f, 13.125f, 59.0625f, 324.84375f, 2111.484375f, 15836.1328125f, 134607.12890625f}
-// C(2n+3,3) (2n-1)!!/2^n, n = 0..2
-#define FSAMD_WING_Q {1.0f, 5.0f, 26.25f}
-
-// Per-pair constants of the FP32 profile's derivatives (voigt32_grad).
-struct VoigtA {
-    float a;            // damping parameter
-    float a2;           // a^2
-    float a2_6;         // a^2 / 6
-    float two_a_sqpi;   // 2a/sqrt(pi)
-    float a_sqpi;       // a/sqrt(pi)
-    float a2_log2e;     // a^2 log2(e)
-};
-
-__device__ inline VoigtA make_voigt_a(double a)
-{
-    VoigtA v;
-    v.a = (float)a;
-    v.a2 = (float)(a * a);
-    v.a2_6 = (float)(a * a * (1.0 / 6.0));
-    v.two_a_sqpi = (float)(a * kTwoOverSqrtPi);
-    v.a_sqpi = (float)(a * (1.0 / kSqrtPi));
-    v.a2_log2e = (float)(a * a * kLog2E);
-    return v;
-}
 
 // Damping parameters up to which the deposit uses the light form of the
 // profile: without the a^3 term and with the Gaussian exponent cut to
@@ -81,6 +51,9 @@ __device__ inline VoigtA make_voigt_a(double a)
 // most 5.5e-7 relative over all u (the a^3 term at u ~ 3.2; measured against
 // scipy.special.wofz).
 constexpr float kA3Drop = 2e-3f;
+
+// The profile takes kUScale u, so that t is one fma.
+constexpr double kUScale = 4.0;
 
 // Per-pair constants of the FP32 profile.
 struct VoigtP {
@@ -108,8 +81,16 @@ __device__ inline VoigtP make_voigt_p(double a, bool light)
     return v;
 }
 
-// The profile takes kUScale u, so that t is one fma.
-constexpr double kUScale = 4.0;
+// The scale that pair's offsets carry: kUScale up to the rounding of l1, which it
+// takes up, so that the Gaussian's exponent l1 t has none of it (it would cost
+// up to 6e-8 u^2 of the Gaussian; the table's argument is off by 6e-8 instead, which
+// costs G no more than that).
+__device__ inline double voigt_uscale(const VoigtP &v, double a)
+{
+    const double exact = -(1.0 + 2.0 * a * a) * (kLog2E / 16.0);
+    return kUScale - 0.5 * kUScale * (16.0 / kLog2E) * (exact - (double)v.l1);   // (exact / l1)^(1/2) kUScale
+}
+
 // Largest |u| whose t lies in the table, and the floats the table takes.
 constexpr double kVoigtUMax = 2.3e4;
 constexpr int kPTableSize = FSAMD_P_OCTAVES * FSAMD_P_BINS * 4;
@@ -158,86 +139,81 @@ __device__ inline float voigt32(const VoigtP &v, float u, const float *tab)
 }
 
 // ---------------------------------------------------------------------------
-// Profile derivatives for the adjoint, FP32.  With z = u + ia, w' = -2zw + 2i/sqrt(pi):
-//   dH/du = Re w' = -2(uH - aL),   dH/da = -Im w' = 2(uL + aH) - 2/sqrt(pi),
-// L = Im w.  The adjoint needs H, Hu = dH/du and F = u dH/du + a dH/da
-// (the response to the thermal width b, all sample offsets scaling as 1/b):
-//   F = -2(u^2 - a^2) H + 4 a u L - 2a/sqrt(pi).
-// Core |u| < 7: L = -exp(a^2-u^2) sin(2au) + (2/sqrt(pi)) [D(u) - (a^2/2) D''(u)],
-// D = (1 - G)/(2u), D'' = -2D - 2uG.  Wing |u| >= 7: the asymptotic series
-// H = (a/sqrt(pi)) sum p_k u^(-2k-2) gives Hu and F termwise, without the
-// cancellation of the closed forms (a^2-relative corrections dropped there).
-struct VoigtGrad {
-    float H, Hu, F;
-};
+// Profile derivatives for the adjoint, FP32.  Besides H the adjoint needs Hu =
+// dH/du and F = u dH/du + a dH/da (the response to the thermal width b: all
+// sample offsets and a scale as 1/b).  With C = exp(a^2 - u^2) cos(2au), G =
+// D'(u), K = dG/d(u^2), x = 2au and T = tan(x)/x - 1:
+//   H  = C - (2a/sqrt(pi)) (G - (a^2/6) D''')
+//   Hu = -2u [C (1 + 2a^2 (1 + T)) + (2a/sqrt(pi)) (K - (a^2/12) D''''/u)]
+//   F  = -2u^2 C (1 + 4a^2 (1 + T)) + 2a^2 C
+//        - (2a/sqrt(pi)) [2u^2 (K - (a^2/12) D''''/u) + G - (a^2/2) D''']
+// with D''' = (4u^2 - 6) G + 2, D''''/u = -2 D''' - 12 K, beyond u = 20 -12 G^2 and
+// -48 G K.  G and K are rows of one index (profile_table.h): no branch on u.
+// The light form (a <= kA3Drop) leaves out T, D''' and D''''.  The table holds K
+// times kKScale, which keeps its coefficients normal numbers.
+//
+// Sums over samples of weight w, in u' = kUScale u: every factor that depends
+// on the pair alone is applied once, by finish().
+constexpr float kKScale = (float)(1ull << FSAMD_P_DSCALE);
 
-__device__ inline VoigtGrad voigt32_grad(const VoigtA &v, float u, const float *gtab)
-{
-    const float sgn = u < 0 ? -1.0f : 1.0f;
-    const float uh = __builtin_fabsf(u);
-    VoigtGrad r;
-    if (uh >= kVoigtCoreMax) {
-        const float x = __builtin_amdgcn_rcpf(uh * uh);
-        const float P[9] = FSAMD_WING_P;
-        const float Q[3] = FSAMD_WING_Q;
-        float s = P[8], d = 18.0f * P[8], f = -17.0f * P[8];
-#pragma unroll
-        for (int k = 7; k >= 0; --k) {
-            s = __builtin_fmaf(s, x, P[k]);
-            d = __builtin_fmaf(d, x, (2.0f * k + 2.0f) * P[k]);
-            f = __builtin_fmaf(f, x, -(2.0f * k + 1.0f) * P[k]);
+struct GradSums {
+    float cC = 0, cG = 0, uC = 0, uK = 0, pC = 0, pK = 0;   // w C, w G, w u' C, w u' K, w u'^2 C, w u'^2 K
+    float cD = 0, uT = 0, pT = 0;                           // full form: w D''', w u' C T, w u'^2 C T
+
+    // tab: 8 floats a row, G's cubic and K's
+    template <bool kA3>
+    __device__ inline void add(const VoigtP &v, float a2, float w, float us, const float *tab)
+    {
+        const float t = __builtin_fmaf(us, us, 2.0f);
+        float y = __builtin_fmaf(t, v.l1, v.l0);
+        if (kA3) {
+            const float p = __builtin_fmaf(t, 0.0625f, -0.125f);
+            y = __builtin_fmaf(p * p, __builtin_fmaf(p, v.l3, v.l2), y);
         }
-        float q = __builtin_fmaf(Q[2], x, Q[1]);
-        q = __builtin_fmaf(q, x, Q[0]);
-        r.H = v.a_sqpi * x * __builtin_fmaf(-v.a2 * x, q, s);
-        r.Hu = -sgn * v.a_sqpi * x * d * __builtin_amdgcn_rcpf(uh);
-        r.F = v.a_sqpi * x * f;
-        return r;
+        const float C = __builtin_amdgcn_exp2f(y);
+        const unsigned edge = __float_as_uint(t) & 0xfffc0000u;
+        const float d = t - __uint_as_float(edge);
+        const float4 *row = (const float4 *)((const char *)tab + 2 * __builtin_amdgcn_ubfe(edge, 14, 14));
+        const float4 g = row[0], k = row[1];
+        float G = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(g.w, d, g.z), d, g.y), d, g.x);
+        float K = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(k.w, d, k.z), d, k.y), d, k.x);
+        const float wC = w * C, xC = us * wC;
+        if (kA3) {
+            const bool far = t > 6402.0f;
+            const float D = far ? G * (G * -12.0f) : __builtin_fmaf(__builtin_fmaf(t, 0.25f, -6.5f), G, 2.0f);
+            // D''''/u times kKScale
+            const float D4 = far ? G * (K * -48.0f) : __builtin_fmaf(-12.0f, K, (-2.0f * kKScale) * D);
+            K = __builtin_fmaf(0.5f * v.a3, D4, K);
+            G = __builtin_fmaf(v.a3, D, G);
+            cD = __builtin_fmaf(w, D, cD);
+            // x^2 = a^2 u'^2 / 4
+            const float x2 = 0.25f * a2 * (t - 2.0f);
+            const float xT = xC * (x2 * __builtin_fmaf(x2, 2.0f / 15.0f, 1.0f / 3.0f));
+            uT += xT;
+            pT = __builtin_fmaf(us, xT, pT);
+        }
+        cC += wC;
+        uC += xC;
+        pC = __builtin_fmaf(us, xC, pC);
+        cG = __builtin_fmaf(w, G, cG);
+        const float xK = us * (w * K);
+        uK += xK;
+        pK = __builtin_fmaf(us, xK, pK);
     }
-    // exp(a^2 - u^2)
-    const float p = uh * uh;
-    const float E = __builtin_amdgcn_exp2f(__builtin_fmaf(p, -kLog2EF, v.a2_log2e));
-    const float c = 2.0f * v.a * uh;
-    const float c2 = c * c;
-    float cs = __builtin_fmaf(c2, -1.0f / 40320.0f, 1.0f / 720.0f);
-    cs = __builtin_fmaf(c2, -cs, 1.0f / 24.0f);
-    cs = __builtin_fmaf(c2, -cs, 0.5f);
-    cs = __builtin_fmaf(c2, -cs, 1.0f);
-    float sn = __builtin_fmaf(c2, -1.0f / 5040.0f, 1.0f / 120.0f);
-    sn = __builtin_fmaf(c2, sn, -1.0f / 6.0f);
-    sn = c * __builtin_fmaf(c2, sn, 1.0f);
-    // G from the piece's row (two 16-byte reads), in the fractional part of u/width
-    const float q = uh * (1.0f / FSAMD_G_WIDTH);
-    const int idx = min((int)q, FSAMD_G_NPIECE - 1);
-    const float var = q - (float)idx;
-    const float *row = gtab + idx * FSAMD_G_STRIDE;
-    const float4 lo = *(const float4 *)row;
-    const float4 hi = *(const float4 *)(row + 4);
-    float G = __builtin_fmaf(hi.z, var, hi.y);
-    G = __builtin_fmaf(G, var, hi.x);
-    G = __builtin_fmaf(G, var, lo.w);
-    G = __builtin_fmaf(G, var, lo.z);
-    G = __builtin_fmaf(G, var, lo.y);
-    G = __builtin_fmaf(G, var, lo.x);
-    float D;
-    if (uh < 0.25f) {
-        // D(u) = u - 2u^3/3 + 4u^5/15 - 8u^7/105 + 16u^9/945
-        float t = __builtin_fmaf(p, 16.0f / 945.0f, -8.0f / 105.0f);
-        t = __builtin_fmaf(p, t, 4.0f / 15.0f);
-        t = __builtin_fmaf(p, t, -2.0f / 3.0f);
-        D = uh * __builtin_fmaf(p, t, 1.0f);
-    } else {
-        D = (1.0f - G) * 0.5f * __builtin_amdgcn_rcpf(uh);
+    // S = sum w H; SU with sum w Hu = SU / scale; ST and SP with sum w (H + F) = ST +
+    // SP / scale^2, scale the pair's voigt_uscale.  H and F cancel to the next
+    // order in the wings, so their sum is formed before it is rounded; and
+    // H + F integrates to nearly zero over the profile, so the scale, whose
+    // rounding would not average out, is left to the caller.
+    __device__ inline void finish(const VoigtP &v, float a2, float &S, float &SU, float &ST, float &SP) const
+    {
+        const float A = v.two_a_sqpi;
+        S = __builtin_fmaf(-A, cG, cC);
+        SU = -2.0f * (__builtin_fmaf(2.0f * a2, uC + uT, uC) + A * ((1.0f / kKScale) * uK));
+        ST = __builtin_fmaf(2.0f * a2, cC, cC) - 2.0f * A * (cG + v.a3 * cD);
+        SP = -2.0f * __builtin_fmaf((1.0f / kKScale) * A, pK, __builtin_fmaf(4.0f * a2, pC + pT, pC));
     }
-    const float D2 = -2.0f * D - 2.0f * uh * G;
-    const float D3 = __builtin_fmaf(__builtin_fmaf(4.0f, p, -6.0f), G, 2.0f);
-    const float H = __builtin_fmaf(-v.two_a_sqpi, __builtin_fmaf(-v.a2_6, D3, G), E * cs);
-    const float L = __builtin_fmaf(kTwoOverSqrtPiF, __builtin_fmaf(-0.5f * v.a2, D2, D), -E * sn);
-    r.H = H;
-    r.Hu = sgn * (-2.0f * __builtin_fmaf(uh, H, -v.a * L));
-    r.F = __builtin_fmaf(-2.0f * (p - v.a2), H, __builtin_fmaf(4.0f * v.a * uh, L, -v.two_a_sqpi));
-    return r;
-}
+};
 
 // ---------------------------------------------------------------------------
 // FP64 Faddeeva w(z), y >= 0.

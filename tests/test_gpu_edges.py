@@ -137,3 +137,44 @@ def test_split_rows(oracle, n, nlos, nbins, hfrac):
     if total.item() > 0:
         total.backward()
         assert float((d.grad.double() * d.detach().double()).sum()) == pytest.approx(total.item(), rel=1e-5)
+
+
+# windows of no, one and many pixels, midpoints and many sub-samples, far wings
+# (strong damping), light and full profiles side by side, rows beyond the
+# adjoint's LDS and rows it refuses
+@pytest.mark.parametrize("nbins,kernel,dscale,tscale,gscale", [(8, 1, 1.0, 1.0, 1.0), (64, 3, 1e3, 1e-2, 1.0),
+                                                               (300, 0, 1e6, 1.0, 10.0), (1024, 1, 1e4, 1.0, 20.0),
+                                                               (3200, 1, 1.0, 1.0, 1.0), (129, 1, 1e-9, 1.0, 1.0)])
+def test_adjoint_against_fp64(nbins, kernel, dscale, tscale, gscale):
+    """Gradients of sum(tau * weights) by the FP32 adjoint against the same
+    windows by the FP64 one (fsamd_set_fp64, pinned to the torch reference):
+    1e-5 of the largest of each gradient, the stated tolerance of tau."""
+    import torch
+    args = list(small_gas(150, 700.0, 3, nbins, kernel, 0.15))
+    dens, temp = (args[13] * dscale).astype(np.float32), (args[14] * tscale).astype(np.float32)
+    line = (args[6], args[7] * gscale, args[8], args[9])
+    plan = SP.Plan(args[3], dev(args[11]), dev(args[15]), dev(args[16]), dev(args[17]))
+    plan.keep_windows(True)
+    g = dev(np.random.default_rng(2).standard_normal((3, nbins)))
+    out = {}
+    for fp64 in (False, True):
+        SP.set_fp64(fp64)
+        try:
+            SP.tau(plan, nbins, kernel, args[4], dev(args[12]), dev(temp), [line], [dev(dens)])
+            gd, gT, gv = SP.tau_adjoint(plan, nbins, kernel, args[4], dev(args[12]), dev(temp), [line], [dev(dens)], [g])
+        finally:
+            SP.set_fp64(False)
+        out[fp64] = [gd[0], gT, gv]
+    for a, b in zip(out[False], out[True]):
+        assert torch.isfinite(a).all()
+        assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max())
+
+
+def test_adjoint_refuses_long_rows():
+    args = small_gas(20, 700.0, 1, 20000, 1, 0.2)
+    plan = SP.Plan(args[3], dev(args[11]), dev(args[15]), dev(args[16]), dev(args[17]))
+    plan.keep_windows(True)
+    line, vel, temp, dens = args[6:10], dev(args[12]), dev(args[14]), dev(args[13])
+    t = SP.tau(plan, 20000, 1, args[4], vel, temp, [line], [dens])[0]
+    with pytest.raises(Exception, match="nbins too large"):
+        SP.tau_adjoint(plan, 20000, 1, args[4], vel, temp, [line], [dens], [t])
