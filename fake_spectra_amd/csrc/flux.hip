@@ -2,6 +2,7 @@
 // (py_module.cpp:235-262, fluxstatistics.py:26-39), spectrograph smoothing
 // (spec_utils.py:5-25), the 1D flux power (fluxstatistics.py:71-108) and the
 // flux PDF (fluxstatistics.py:41-49).  All FP64, HBM-bound streaming kernels.
+#include "exp_table.h"
 #include "fsamd_internal.h"
 
 #include <algorithm>
@@ -43,24 +44,136 @@ __device__ inline void block_sum(double (&v)[kN])
     __syncthreads();
 }
 
-// Per-block partial sums of exp(-s tau), tau exp(-s tau) and the count of
-// pixels with tau <= thresh (py_module.cpp:242-251).
+__device__ const __attribute__((aligned(16))) double d_exp[2 * FSAMD_EXP_N] = FSAMD_EXP_INIT;
+
+// exp(x), |x| cut at 800 where it is 0 or infinite; kNeg: for x <= 0, where one
+// fmax cuts (it drops a NaN, which the callers' x cannot be or which they keep):
+// table of 2^(j/128) as hi + lo in LDS, polynomial of degree 6 in the rest
+// |r| <= ln 2 / 256 (truncation 5e-19); the last addition's rounding is all but
+// 0.01 of the 0.51 ulp of its error.  17 instructions where the math library's
+// takes 36, which bounded the kernels below instead of HBM.
+template <bool kNeg>
+__device__ inline double flux_exp(double x, const double2 *tab)
+{
+    x = kNeg ? fmax(x, -800.0) : x < -800.0 ? -800.0 : x > 800.0 ? 800.0 : x;
+    constexpr double kRound = 6755399441055744.0;   // 1.5 2^52: the sum's low bits are rint
+    const double kd = __builtin_fma(x, FSAMD_EXP_INV, kRound);
+    const int k = __double2loint(kd);
+    const double kf = kd - kRound;
+    const double r = __builtin_fma(kf, -FSAMD_EXP_STEP_LO, __builtin_fma(kf, -FSAMD_EXP_STEP_HI, x));
+    const double2 T = tab[k & (FSAMD_EXP_N - 1)];
+    double q = __builtin_fma(r, 1.0 / 120, 1.0 / 24);
+    q = __builtin_fma(r, q, 1.0 / 6);
+    q = __builtin_fma(r, q, 0.5);
+    q = __builtin_fma(r * r, q, r);
+    return ldexp(T.x + __builtin_fma(T.x, q, T.y), k >> FSAMD_EXP_LOG2N);
+}
+
+__device__ inline void load_exp_table(double2 *tab)
+{
+    for (int i = threadIdx.x; i < FSAMD_EXP_N; i += blockDim.x) tab[i] = reinterpret_cast<const double2 *>(d_exp)[i];
+}
+
+// Sums of t^j exp(-s t), j = 0 .. kMoments, the count of pixels with tau <=
+// thresh that they are over (py_module.cpp:242-251), and of those the count
+// with t < 0: [kSums][gridDim.x] partial sums.
+//
+// Bound: FP64 issue, 51 instructions a pixel, close above HBM (one read of the
+// field).  The higher moments (two instructions each) let a pass serve the later
+// steps of the iteration too (see taylor_step): 4 -> 2 passes for a forest of
+// mean flux 0.68, 6 -> 4 for 0.8.  82M pixels: 218 us a pass with three sums and the
+// math library's exp, 163 us now (a batch of 4 and 2048 blocks 167; moments to
+// the 8th only 153, but a pass more in half of the cases).
+constexpr int kMoments = 12;
+constexpr int kSums = kMoments + 3;
+constexpr int kMomentBlocks = 1536;   // 6 blocks a CU
+constexpr int kMomentBatch = 2;       // pixels a thread loads before the first is used
+
 __global__ __launch_bounds__(kFluxThreads) void flux_moments_kernel(const double *tau, long long n, double scale,
                                                                    double thresh, double *partial)
 {
-    double v[3] = {0, 0, 0};
+    __shared__ double2 etab[FSAMD_EXP_N];
+    load_exp_table(etab);
+    __syncthreads();
+    double v[kSums] = {};
+    int used = 0;
+    const auto add = [&](double t, double e) {
+#pragma unroll
+        for (int j = 0; j <= kMoments; ++j) {
+            v[j] += e;
+            e *= t;
+        }
+    };
+    const auto add_any = [&](double t) {
+        if (t > thresh) return;
+        ++used;
+        v[kMoments + 2] += t < 0.0 ? 1.0 : 0.0;
+        add(t, flux_exp<false>(-scale * t, etab));
+    };
     const long long stride = (long long)gridDim.x * kFluxThreads;
-    for (long long i = blockIdx.x * (long long)kFluxThreads + threadIdx.x; i < n; i += stride) {
-        const double t = tau[i];
-        if (t > thresh) continue;
-        const double e = exp(-scale * t);
-        v[0] += e;
-        v[1] += e * t;
-        v[2] += 1.0;
+    long long i = blockIdx.x * (long long)kFluxThreads + threadIdx.x;
+    const auto load = [&](double *t) {
+#pragma unroll
+        for (int q = 0; q < kMomentBatch; ++q) t[q] = tau[i + q * stride];
+    };
+    double next[kMomentBatch];   // the next batch is in flight while one is summed
+    bool more = i + (kMomentBatch - 1) * stride < n;
+    if (more) load(next);
+    while (more) {
+        double t[kMomentBatch];
+        bool plain = true;
+#pragma unroll
+        for (int q = 0; q < kMomentBatch; ++q) t[q] = next[q];
+        i += kMomentBatch * stride;
+        more = i + (kMomentBatch - 1) * stride < n;
+        if (more) load(next);
+#pragma unroll
+        for (int q = 0; q < kMomentBatch; ++q) plain = plain && t[q] >= 0.0 && t[q] <= thresh;
+        if (plain) {
+            used += kMomentBatch;
+#pragma unroll
+            for (int q = 0; q < kMomentBatch; ++q) add(t[q], flux_exp<true>(-scale * t[q], etab));
+        } else {
+            for (int q = 0; q < kMomentBatch; ++q) add_any(t[q]);
+        }
     }
-    block_sum<3>(v);
+    for (; i < n; i += stride) add_any(tau[i]);
+    v[kMoments + 1] = used;
+    block_sum<kSums>(v);
     if (threadIdx.x == 0)
-        for (int i = 0; i < 3; ++i) partial[3 * blockIdx.x + i] = v[i];
+        for (int j = 0; j < kSums; ++j) partial[(size_t)j * gridDim.x + blockIdx.x] = v[j];
+}
+
+// One block a row: out[row] = sum of in[row][0 .. n)
+__global__ __launch_bounds__(kFluxThreads) void row_sum_kernel(const double *in, int n, double *out)
+{
+    double v[1] = {0.0};
+    for (int i = threadIdx.x; i < n; i += kFluxThreads) v[0] += in[(size_t)blockIdx.x * n + i];
+    block_sum<1>(v);
+    if (threadIdx.x == 0) out[blockIdx.x] = v[0];
+}
+
+// F(z) = sum exp(-z t) and G(z) = -F'(z) from the moments at c, by their Taylor
+// polynomials.  For t >= 0 a pixel's remainder is at most
+// max_t t^J exp(-x t) |z - c|^J / J! <= r^J / sqrt(2 pi J), r = |z - c| / x,
+// x = min(z, c), with J = kMoments + 1 for F and (J / x) times that of |z - c|^(J-1)
+// for G.  False where the Newton step (F - target) / G would be off by more than
+// 1e-14 z: then the field has to be summed at z.
+static bool taylor_step(const double *sum, double c, double z, double target, double &F, double &G)
+{
+    const double used = sum[kMoments + 1], d = z - c, x = std::min(z, c), r = std::fabs(d) / x;
+    if (sum[kMoments + 2] != 0 || !(r < 0.5)) return false;
+    F = G = 0;
+    double f = 1;   // (-d)^j / j!
+    for (int j = 0; j <= kMoments; ++j) {
+        F += f * sum[j];
+        if (j < kMoments) G += f * sum[j + 1];
+        f *= -d / (j + 1);
+    }
+    if (!std::isfinite(F) || !std::isfinite(G)) return false;
+    constexpr double J = kMoments + 1;
+    const double rem = used * std::pow(r, J - 1) / std::sqrt(2 * M_PI * J);
+    return rem * r + std::fabs((F - target) / G) * rem * J / x <= 1e-14 * z * G;
 }
 
 // Gaussian smoothing along rows with periodic wrap, weights w[0..2r]
@@ -339,31 +452,31 @@ int fsamd_mean_flux_scale(const double *tau, long long n, double mean_flux_desir
         return FSAMD_OK;
     }
     hipStream_t s = (hipStream_t)stream;
-    const int nblocks = (int)std::min<long long>(1024, (n + kFluxThreads - 1) / kFluxThreads);
+    const int nblocks = (int)std::min<long long>(kMomentBlocks, (n + kFluxThreads - 1) / kFluxThreads);
     double *partial = nullptr;
-    FSAMD_HIP(hipMalloc(&partial, sizeof(double) * 3 * nblocks));
-    std::vector<double> host(3 * nblocks);
-    double scale, newscale = 1;
+    FSAMD_HIP(hipMalloc(&partial, sizeof(double) * kSums * (nblocks + 1)));
+    double *total = partial + (size_t)kSums * nblocks;
+    double sum[kSums], centre = 0, scale, newscale = 1;
     int rc = FSAMD_OK;
     for (int it = 0; it < 1000; ++it) {
         scale = newscale;
-        flux_moments_kernel<<<nblocks, kFluxThreads, 0, s>>>(tau, n, scale, thresh, partial);
-        hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = hipMemcpyAsync(host.data(), partial, sizeof(double) * 3 * nblocks,
-                                                hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) {
-            rc = fail(FSAMD_ERR_HIP, std::string("flux moments: ") + hipGetErrorString(e));
-            break;
-        }
-        double mf = 0, tmf = 0, used = 0;
-        for (int b = 0; b < nblocks; ++b) {
-            mf += host[3 * b];
-            tmf += host[3 * b + 1];
-            used += host[3 * b + 2];
+        double F, G;
+        if (it == 0 || !taylor_step(sum, centre, scale, mean_flux_desired * sum[kMoments + 1], F, G)) {
+            flux_moments_kernel<<<nblocks, kFluxThreads, 0, s>>>(tau, n, scale, thresh, partial);
+            row_sum_kernel<<<kSums, kFluxThreads, 0, s>>>(partial, nblocks, total);
+            hipError_t e = hipGetLastError();
+            if (e == hipSuccess) e = hipMemcpyAsync(sum, total, sizeof(sum), hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = hipStreamSynchronize(s);
+            if (e != hipSuccess) {
+                rc = fail(FSAMD_ERR_HIP, std::string("flux moments: ") + hipGetErrorString(e));
+                break;
+            }
+            centre = scale;
+            F = sum[0];
+            G = sum[1];
         }
         // Newton-Raphson on <exp(-s tau)> = mean_flux_desired (py_module.cpp:252-257)
-        newscale = scale + (mf - mean_flux_desired * used) / tmf;
+        newscale = scale + (F - mean_flux_desired * sum[kMoments + 1]) / G;
         if (newscale <= 0) newscale = 1e-10;
         if (!(fabs(newscale - scale) > tol * newscale)) break;
         if (it == 999) rc = fail(FSAMD_ERR_ARG, "mean flux rescale did not converge");
