@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 namespace fsamd {
@@ -196,66 +197,48 @@ __global__ __launch_bounds__(kFluxThreads) void res_corr_kernel(const double *in
     }
 }
 
-// Direct-sum power spectrum, kept for npix too large for the FFT's LDS
-// buffers: power[row][k] = |sum_j d_j exp(-2 pi i j k / npix)|^2 with
-// d = exp(-s tau)/mean - 1, over an LDS twiddle table.  One block per
-// sightline, O(npix^2).
-__global__ __launch_bounds__(kFluxThreads) void flux_dft_kernel(const double *tau, int nlos, int npix, double scale,
-                                                               double inv_mean, double *power)
-{
-    extern __shared__ double sh[];
-    double *d = sh;                 // [npix]
-    double *cs = sh + npix;         // [npix] cos(2 pi m / npix)
-    double *sn = sh + 2 * npix;     // [npix] sin(2 pi m / npix)
-    for (int m = threadIdx.x; m < npix; m += kFluxThreads) {
-        double s, c;
-        sincospi(2.0 * m / npix, &s, &c);
-        cs[m] = c;
-        sn[m] = s;
-    }
-    const int nk = npix / 2 + 1;
-    for (int row = blockIdx.x; row < nlos; row += gridDim.x) {
-        __syncthreads();
-        for (int j = threadIdx.x; j < npix; j += kFluxThreads)
-            d[j] = exp(-scale * tau[(size_t)row * npix + j]) * inv_mean - 1.0;
-        __syncthreads();
-        for (int k = threadIdx.x; k < nk; k += kFluxThreads) {
-            double re = 0, im = 0;
-            unsigned int m = 0;        // j k mod npix
-            for (int j = 0; j < npix; ++j) {
-                re += d[j] * cs[m];
-                im -= d[j] * sn[m];
-                m += (unsigned int)k;
-                if (m >= (unsigned int)npix) m -= npix;
-            }
-            power[(size_t)row * nk + k] = re * re + im * im;
-        }
-    }
-}
-
 // ---- mixed-radix FFT power spectrum ---------------------------------------
 // Self-sorting (Stockham) decimation-in-time FFT of length n = R_1 R_2 ...
-// R_S in LDS, two buffers ping-ponged.  Stage s with radix R, after the
-// transforms of length p = R_1 ... R_{s-1}: for i in [0, n/R), k = i mod p,
-//   u_r = a[i + r n/R] W_n^{r k n/(p R)},   b[(i - k) R + k + q p] = sum_r u_r W_R^{r q}.
+// R_S in one LDS buffer.  Stage s with radix R, after the transforms of length
+// p = R_1 ... R_{s-1}: for i in [0, n/R), k = i mod p,
+//   u_r = a[i + r n/R] W_n^{r k n/(p R)},   a'[(i - k) R + k + q p] = sum_r u_r W_R^{r q};
+// a thread holds its values of a stage in registers between the barriers.
 // Two real sightlines a, b share one complex transform Z of a + i b; the sum
 // of their powers at mode k is (|Z_k|^2 + |Z_{n-k}|^2) / 2, which is all the
 // flux power needs (it averages the power over sightlines).
+//
+// Bound: LDS traffic and FP64 issue.  Radix 8 with a block of n/8 threads: four
+// stages for 2048 pixels; the first reads the sightlines and stores at stride 8,
+// which the swizzle spreads over the banks.  One buffer, the sums of the power
+// in registers: 34 KB a block of 2048 pixels, four blocks a CU.  Powers of two
+// have the next pair's pixels on their way over a pair's later stages: 395 -> 280
+// us for 40000 sightlines of 2048 (598 with radix 4 and two buffers).  Other
+// lengths: 13333 of 1500 510 -> 175 us, 4000 of 5000 (a direct sum before) 48 ->
+// 0.20 ms, the prime 2003 6.6 -> 1.4 ms for 2000.
 
 constexpr int kFftMaxStages = 40;
+constexpr int kFftPoints = 8;          // values a thread holds, n <= kFftPoints * threads
+constexpr int kFftMaxThreads = 896;
 struct FftPlan {
     int nst;
-    int radix[kFftMaxStages];
+    int twiddle[kFftMaxStages];   // where the stage's twiddles start in the table
+    unsigned char any;            // a radix without a stage of its own
+    short radix[kFftMaxStages];
 };
 
-// Radices 4, 2, 3, 5, 7 first, then any remaining prime factors.
+// Radices 8, 4, 2, 3, 5, 7 first, then any remaining prime factors.
 static FftPlan fft_plan(int n)
 {
     FftPlan f{};
-    for (int r : {4, 2, 3, 5, 7})
-        while (n % r == 0) { f.radix[f.nst++] = r; n /= r; }
+    for (int r : {8, 4, 2, 3, 5, 7})
+        while (n % r == 0) { f.radix[f.nst++] = (short)r; n /= r; }
     for (int q = 11; n > 1; q += 2)
-        while (n % q == 0) { f.radix[f.nst++] = q; n /= q; }
+        while (n % q == 0) { f.radix[f.nst++] = (short)q; n /= q; f.any = 1; }
+    int p = 1;
+    for (int st = 0; st < f.nst; ++st) {
+        f.twiddle[st] = p - 1;    // (R - 1) p a stage, sum over the stages before
+        p *= f.radix[st];
+    }
     return f;
 }
 
@@ -265,129 +248,379 @@ __device__ inline double2 cmul(double2 a, double2 b)
 }
 __device__ inline double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
 __device__ inline double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
+__device__ inline double2 cmul_mi(double2 a) { return make_double2(a.y, -a.x); }   // -i a
 
-// One stage of radix R (compile-time), tw[m] = W_n^m = exp(-2 pi i m / n).
-template <int R>
-__device__ inline void fft_stage(const double2 *a, double2 *b, const double2 *tw, int n, int p)
+// exp(-2 pi i m / n)
+__device__ inline double2 unit_root(int m, int n)
 {
-    const int m = n / R;
-    const int tstep = n / (p * R);
-    for (int i = threadIdx.x; i < m; i += kFluxThreads) {
-        const int k = i % p;
-        double2 u[R];
-        u[0] = a[i];
-#pragma unroll
-        for (int r = 1; r < R; ++r) u[r] = cmul(a[i + r * m], tw[r * k * tstep]);  // r k tstep < n
-        const int j = (i - k) * R + k;
-        if constexpr (R == 2) {
-            b[j] = cadd(u[0], u[1]);
-            b[j + p] = csub(u[0], u[1]);
-        } else if constexpr (R == 4) {
-            // W_4 = -i
-            const double2 s02 = cadd(u[0], u[2]), d02 = csub(u[0], u[2]);
-            const double2 s13 = cadd(u[1], u[3]), d13 = csub(u[1], u[3]);
-            b[j] = cadd(s02, s13);
-            b[j + p] = make_double2(d02.x + d13.y, d02.y - d13.x);       // d02 - i d13
-            b[j + 2 * p] = csub(s02, s13);
-            b[j + 3 * p] = make_double2(d02.x - d13.y, d02.y + d13.x);   // d02 + i d13
-        } else {
-            const int wstep = n / R;
-#pragma unroll
-            for (int q = 0; q < R; ++q) {
-                double2 acc = u[0];
-#pragma unroll
-                for (int r = 1; r < R; ++r) acc = cadd(acc, cmul(u[r], tw[((r * q) % R) * wstep]));
-                b[j + q * p] = acc;
-            }
-        }
-    }
-}
-
-// A stage of any radix R: one output per thread iteration, O(R) terms each.
-__device__ inline void fft_stage_any(const double2 *a, double2 *b, const double2 *tw, int n, int p, int R)
-{
-    const int m = n / R;
-    const int tstep = n / (p * R);
-    const int wstep = n / R;
-    for (int o = threadIdx.x; o < n; o += kFluxThreads) {
-        const int q = o / m, i = o - q * m;
-        const int k = i % p;
-        double2 acc = make_double2(0.0, 0.0);
-        for (int r = 0; r < R; ++r) {
-            int t = r * k * tstep + ((r * q) % R) * wstep;   // both terms < n
-            if (t >= n) t -= n;
-            acc = cadd(acc, cmul(a[i + r * m], tw[t]));
-        }
-        b[(i - k) * R + k + q * p] = acc;
-    }
-}
-
-__global__ void fft_twiddle_kernel(double2 *tw, int n)
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= n) return;
     double s, c;
     sincospi(2.0 * m / n, &s, &c);
-    tw[m] = make_double2(c, -s);
+    return make_double2(c, -s);
+}
+
+// In place: v_q = sum_r u_r W_R^{r q}
+template <int R>
+__device__ inline void dft(double2 (&u)[R])
+{
+    if constexpr (R == 2) {
+        const double2 a = u[0];
+        u[0] = cadd(a, u[1]);
+        u[1] = csub(a, u[1]);
+    } else if constexpr (R == 4) {
+        const double2 s02 = cadd(u[0], u[2]), d02 = csub(u[0], u[2]);
+        const double2 s13 = cadd(u[1], u[3]), d13 = cmul_mi(csub(u[1], u[3]));
+        u[0] = cadd(s02, s13);
+        u[1] = cadd(d02, d13);
+        u[2] = csub(s02, s13);
+        u[3] = csub(d02, d13);
+    } else if constexpr (R == 8) {
+        double2 e[4] = {u[0], u[2], u[4], u[6]}, o[4] = {u[1], u[3], u[5], u[7]};
+        dft<4>(e);
+        dft<4>(o);
+        constexpr double h = 0.70710678118654752440;
+        o[1] = make_double2(h * (o[1].x + o[1].y), h * (o[1].y - o[1].x));
+        o[2] = cmul_mi(o[2]);
+        o[3] = make_double2(h * (o[3].y - o[3].x), -h * (o[3].x + o[3].y));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            u[q] = cadd(e[q], o[q]);
+            u[q + 4] = csub(e[q], o[q]);
+        }
+    } else {
+        // cos and sin of 2 pi m / R
+        constexpr double c3[] = {1.0, -0.5, -0.5}, s3[] = {0.0, 0.86602540378443864676, -0.86602540378443864676};
+        constexpr double c5[] = {1.0, 0.30901699437494742410, -0.80901699437494742410, -0.80901699437494742410,
+                                 0.30901699437494742410};
+        constexpr double s5[] = {0.0, 0.95105651629515357212, 0.58778525229247312917, -0.58778525229247312917,
+                                 -0.95105651629515357212};
+        constexpr double c7[] = {1.0, 0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624,
+                                 -0.90096886790241912624, -0.22252093395631440429, 0.62348980185873353053};
+        constexpr double s7[] = {0.0, 0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048,
+                                 -0.43388373911755812048, -0.97492791218182360702, -0.78183148246802980871};
+        double2 v[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            v[q] = u[0];
+#pragma unroll
+            for (int r = 1; r < R; ++r) {
+                const int m = (r * q) % R;
+                const double c = R == 3 ? c3[m % 3] : R == 5 ? c5[m % 5] : c7[m % 7];
+                const double s = R == 3 ? s3[m % 3] : R == 5 ? s5[m % 5] : s7[m % 7];
+                v[q] = cadd(v[q], cmul(u[r], make_double2(c, -s)));
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < R; ++q) u[q] = v[q];
+    }
+}
+
+// threadIdx.x as a value of its own at each use: a stage's addresses, the same
+// for every pair, are computed where they are used instead of all being kept
+// (and spilled) over the loop.
+__device__ inline int fft_thread()
+{
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+
+__device__ inline int fft_swizzle(int j, int mask) { return j ^ ((j >> 3) & mask); }
+
+// What a plan's kernel holds: the stages of radices 8, 4 and 2 and the next
+// pair's pixels on their way; all stages with a radix of their own; any.
+enum FftKind { kFftPow2, kFftSmall, kFftAny };
+
+// The two sightlines' optical depths at z + r m, r < R; row1 is NULL for the
+// odd one out, whose partner is zero.
+template <int R>
+__device__ inline void load_pair(const double *row0, const double *row1, int z, int m, double2 (&u)[R])
+{
+#pragma unroll
+    for (int r = 0; r < R; ++r) u[r] = make_double2(row0[z + r * m], row1 ? row1[z + r * m] : 0.0);
+}
+
+// In place: exp(-s tau) / mean - 1
+template <int R, bool kTable>
+__device__ inline void pair_flux(double2 (&u)[R], bool two, double scale, double inv_mean, const double2 *etab)
+{
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const double x = -scale * u[r].x, y = -scale * u[r].y;
+        u[r].x = (kTable ? flux_exp<false>(x, etab) : exp(x)) * inv_mean - 1.0;
+        u[r].y = two ? (kTable ? flux_exp<false>(y, etab) : exp(y)) * inv_mean - 1.0 : 0.0;
+        if (r % 2 == 1) __builtin_amdgcn_sched_barrier(0);   // four at a time, not all in registers at once
+    }
+}
+
+// The first stage for radix 8, one butterfly a thread, on pixels already loaded
+__device__ inline void fft_first8(double2 *a, double2 (&u)[8], bool two, int n, double scale, double inv_mean,
+                                  const double2 *etab)
+{
+    const int i = fft_thread();
+    if (i < n / 8) {
+        pair_flux<8, true>(u, two, scale, inv_mean, etab);
+        dft<8>(u);
+    }
+    __syncthreads();
+    if (i < n / 8) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) a[fft_swizzle(i * 8 + q, 7)] = u[q];
+    }
+    __syncthreads();
+}
+
+// One stage of radix R; the first one (kFirst) reads the sightlines.  mask_in,
+// mask_out: the swizzle of the buffer as it is read and as it is left.
+template <int R, bool kFirst, bool kTable>
+__device__ inline void fft_stage(double2 *a, const double2 *tw, int n, int p, int mask_in, int mask_out,
+                                 const double *row0, const double *row1, double scale, double inv_mean,
+                                 const double2 *etab)
+{
+    constexpr int kC = (kFftPoints + R - 1) / R;
+    const int m = n / R;
+    const float inv_p = 1.0f / p;
+    const int tid = fft_thread();
+    double2 u[kC][R];
+#pragma unroll
+    for (int c = 0; c < kC; ++c) {
+        const int i = tid + c * blockDim.x;
+        if (i >= m) continue;
+        if (kFirst) {
+            load_pair<R>(row0, row1, i, m, u[c]);
+            pair_flux<R, kTable>(u[c], row1, scale, inv_mean, etab);
+        } else {
+            const int k = i - p * (int)((i + 0.5f) * inv_p);
+            u[c][0] = a[fft_swizzle(i, mask_in)];
+#pragma unroll
+            for (int r = 1; r < R; ++r) u[c][r] = cmul(a[fft_swizzle(i + r * m, mask_in)], tw[(r - 1) * p + k]);
+        }
+        dft<R>(u[c]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < kC; ++c) {
+        const int i = tid + c * blockDim.x;
+        if (i >= m) continue;
+        const int k = kFirst ? 0 : i - p * (int)((i + 0.5f) * inv_p);
+        const int j = (i - k) * R + k;
+#pragma unroll
+        for (int q = 0; q < R; ++q) a[fft_swizzle(j + q * p, mask_out)] = u[c][q];
+    }
+    __syncthreads();
+}
+
+// exp(-2 pi i t / n), 0 <= t < n, from a table of t <= n/2
+__device__ inline double2 half_root(const double2 *half, int t, int n)
+{
+    double2 w = half[min(t, n - t)];
+    w.y = 2 * t > n ? -w.y : w.y;
+    return w;
+}
+
+// A stage of any odd radix R, O(R) terms an output: outputs q and R - q share
+// the sums C = sum u_r cos and S = sum u_r sin of 2 pi r q / R, C -+ i S.
+__device__ inline void fft_stage_any(double2 *a, const double2 *half, int n, int p, int R, int mask_in)
+{
+    constexpr int kC = (kFftPoints * 12 / 11 + 1) / 2 + 1;   // m (R + 1) / 2 <= (n + n/11) / 2 sums over n/8 threads
+    const int m = n / R, nsum = m * ((R + 1) / 2);
+    const int tstep = n / (p * R), tid = fft_thread(), T = blockDim.x;
+    if (p > 1) {
+        for (int j = tid; j < n; j += T) {
+            const int r = j / m, k = (j - r * m) % p;
+            double2 &v = a[fft_swizzle(j, mask_in)];
+            v = cmul(v, half_root(half, r * k * tstep, n));
+        }
+        __syncthreads();
+    }
+    double2 C[kC], S[kC];
+#pragma unroll
+    for (int c = 0; c < kC; ++c) {
+        const int o = tid + c * T;
+        C[c] = S[c] = make_double2(0.0, 0.0);
+        if (o >= nsum) continue;
+        const int q = o / m, i = o - q * m;
+        int t = 0;
+        for (int r = 0; r < R; ++r) {
+            const double2 w = half_root(half, t, n), u = a[fft_swizzle(i + r * m, mask_in)];
+            C[c] = make_double2(fma(u.x, w.x, C[c].x), fma(u.y, w.x, C[c].y));
+            S[c] = make_double2(fma(u.x, -w.y, S[c].x), fma(u.y, -w.y, S[c].y));
+            t += q * m;
+            t -= t >= n ? n : 0;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < kC; ++c) {
+        const int o = tid + c * T;
+        if (o >= nsum) continue;
+        const int q = o / m, i = o - q * m;
+        const int k = i % p, j = (i - k) * R + k;
+        const double2 is = cmul_mi(S[c]);   // -i S
+        a[j + q * p] = cadd(C[c], is);
+        if (q > 0) a[j + (R - q) * p] = csub(C[c], is);
+    }
+    __syncthreads();
+}
+
+// The stages' twiddles: of stage s, radix R, tw[twiddle[s] + (r - 1) p + k] = W_n^{r k n/(p R)}.
+__global__ void fft_twiddle_kernel(double2 *tw, FftPlan fp)
+{
+    const int at = blockIdx.x * blockDim.x + threadIdx.x;
+    int p = 1;
+    for (int st = 0; st < fp.nst; ++st) {
+        const int R = fp.radix[st], e = at - fp.twiddle[st];
+        if (e < (R - 1) * p) {
+            if (e >= 0) tw[at] = unit_root((e / p + 1) * (e % p), p * R);
+            return;
+        }
+        p *= R;
+    }
 }
 
 // Each block transforms sightline pairs blockIdx.x, blockIdx.x + gridDim.x, ...
 // and writes the sum of their powers to part[blockIdx.x][k]; the blocks'
 // rows are then summed in block order, so the result does not depend on
-// scheduling.  LDS: two complex buffers of n and the accumulator of n/2 + 1.
-__global__ __launch_bounds__(kFluxThreads) void flux_fft_kernel(const double *tau, int nlos, int npix, double scale,
-                                                               double inv_mean, const double2 *tw, FftPlan fp,
-                                                               double *part)
+// scheduling.
+template <FftKind kKind>
+__global__ __launch_bounds__(kFftMaxThreads) void flux_fft_kernel(const double *tau, int nlos, int npix, double scale,
+                                                                 double inv_mean, const double2 *tw, FftPlan fp,
+                                                                 double *part)
 {
+    constexpr bool kTable = kKind != kFftAny;   // whose sums are far longer than the exponentials
     extern __shared__ double2 shc[];
-    double2 *A = shc, *B = shc + npix;
-    double *acc = reinterpret_cast<double *>(shc + 2 * npix);
-    const int nk = npix / 2 + 1;
-    for (int k = threadIdx.x; k < nk; k += kFluxThreads) acc[k] = 0.0;
+    double2 *a = shc, *half = shc + npix, *etab = half;   // one of the two tables
+    constexpr int kModes = kFftPoints / 2 + 1;   // npix/2 + 1 modes over npix/8 threads
+    double acc[kModes] = {};
+    const int nk = npix / 2 + 1, T = blockDim.x;
+    if (kTable)
+        load_exp_table(etab);
+    else
+        for (int m = threadIdx.x; m < nk; m += T) half[m] = unit_root(m, npix);
+    __syncthreads();
     const int npair = (nlos + 1) / 2;
+    double2 next[8];   // kFftPow2: this thread's pixels of the pair to come
+    const auto load_next = [&](int pr) {
+        const int i = fft_thread();
+        if (i >= npix / 8) return;
+        const double *row = tau + 2 * (size_t)pr * npix;
+        load_pair<8>(row, 2 * pr + 1 < nlos ? row + npix : nullptr, i, npix / 8, next);
+    };
+    if (kKind == kFftPow2 && (int)blockIdx.x < npair) load_next(blockIdx.x);
     for (int pr = blockIdx.x; pr < npair; pr += gridDim.x) {
         const size_t r0 = 2 * (size_t)pr;
-        const bool two = r0 + 1 < (size_t)nlos;
-        __syncthreads();   // the last pair's power reads are done
-        for (int j = threadIdx.x; j < npix; j += kFluxThreads) {
-            const double x = exp(-scale * tau[r0 * npix + j]) * inv_mean - 1.0;
-            const double y = two ? exp(-scale * tau[(r0 + 1) * npix + j]) * inv_mean - 1.0 : 0.0;
-            A[j] = make_double2(x, y);
+        const double *row0 = tau + r0 * npix, *row1 = r0 + 1 < (size_t)nlos ? row0 + npix : nullptr;
+        int p = 1, mask = 0, st = 0;
+        if (kKind == kFftPow2) {
+            fft_first8(a, next, row1, npix, scale, inv_mean, etab);
+            if (pr + (int)gridDim.x < npair) load_next(pr + gridDim.x);
+            st = 1;
+            p = 8;
+            mask = 7;
         }
-        double2 *src = A, *dst = B;
-        int p = 1;
-        for (int st = 0; st < fp.nst; ++st) {
-            __syncthreads();
+        for (; st < fp.nst; ++st) {
             const int R = fp.radix[st];
-            switch (R) {
-            case 2: fft_stage<2>(src, dst, tw, npix, p); break;
-            case 3: fft_stage<3>(src, dst, tw, npix, p); break;
-            case 4: fft_stage<4>(src, dst, tw, npix, p); break;
-            case 5: fft_stage<5>(src, dst, tw, npix, p); break;
-            case 7: fft_stage<7>(src, dst, tw, npix, p); break;
-            default: fft_stage_any(src, dst, tw, npix, p, R); break;
+            const double2 *ts = tw + fp.twiddle[st];
+            if (st == 0) {
+                mask = npix % 8 == 0 ? 7 : 0;   // whole groups of 8
+                const auto stage = [&](auto radix) {
+                    fft_stage<decltype(radix)::value, true, kTable>(a, ts, npix, p, 0, mask, row0, row1, scale,
+                                                                   inv_mean, etab);
+                };
+                switch (R) {
+                case 2: stage(std::integral_constant<int, 2>()); break;
+                case 3: stage(std::integral_constant<int, 3>()); break;
+                case 4: stage(std::integral_constant<int, 4>()); break;
+                case 5: stage(std::integral_constant<int, 5>()); break;
+                case 7: stage(std::integral_constant<int, 7>()); break;
+                case 8: stage(std::integral_constant<int, 8>()); break;
+                default:
+                    if (kKind != kFftAny) break;
+                    __syncthreads();   // the last pair's power has been read
+                    for (int j = threadIdx.x; j < npix; j += T) {
+                        double2 u[1];
+                        load_pair<1>(row0, row1, j, 0, u);
+                        pair_flux<1, false>(u, row1, scale, inv_mean, etab);
+                        a[j] = u[0];
+                    }
+                    mask = 0;
+                    __syncthreads();
+                    fft_stage_any(a, half, npix, p, R, 0);
+                }
+            } else {
+                const auto stage = [&](auto radix) {
+                    fft_stage<decltype(radix)::value, false, kTable>(a, ts, npix, p, mask, 0, row0, row1, scale,
+                                                                    inv_mean, etab);
+                };
+                if (kKind == kFftPow2) {
+                    if (R == 8)
+                        stage(std::integral_constant<int, 8>());
+                    else if (R == 4)
+                        stage(std::integral_constant<int, 4>());
+                    else
+                        stage(std::integral_constant<int, 2>());
+                } else {
+                    switch (R) {
+                    case 2: stage(std::integral_constant<int, 2>()); break;
+                    case 3: stage(std::integral_constant<int, 3>()); break;
+                    case 4: stage(std::integral_constant<int, 4>()); break;
+                    case 5: stage(std::integral_constant<int, 5>()); break;
+                    case 7: stage(std::integral_constant<int, 7>()); break;
+                    case 8: stage(std::integral_constant<int, 8>()); break;
+                    default:
+                        if (kKind == kFftAny) fft_stage_any(a, half, npix, p, R, mask);
+                    }
+                }
+                mask = 0;
             }
-            double2 *t = src; src = dst; dst = t;
             p *= R;
         }
-        __syncthreads();
-        // each thread owns modes k = threadIdx.x + c kFluxThreads of acc
-        for (int k = threadIdx.x; k < nk; k += kFluxThreads) {
-            const double2 z = src[k], w = src[k == 0 ? 0 : npix - k];
-            acc[k] += 0.5 * ((z.x * z.x + z.y * z.y) + (w.x * w.x + w.y * w.y));
+        if (fp.nst == 0) {   // one pixel
+            double2 u[1];
+            __syncthreads();
+            load_pair<1>(row0, row1, 0, 0, u);
+            pair_flux<1, false>(u, row1, scale, inv_mean, etab);
+            if (threadIdx.x == 0) a[0] = u[0];
+            __syncthreads();
+        }
+        // each thread owns modes threadIdx.x + c T
+        const int tid = fft_thread();
+#pragma unroll
+        for (int c = 0; c < kModes; ++c) {
+            const int k = tid + c * T;
+            if (k >= nk) continue;
+            const double2 z = a[fft_swizzle(k, mask)], w = a[fft_swizzle(k == 0 ? 0 : npix - k, mask)];
+            acc[c] += 0.5 * ((z.x * z.x + z.y * z.y) + (w.x * w.x + w.y * w.y));
         }
     }
-    for (int k = threadIdx.x; k < nk; k += kFluxThreads) part[(size_t)blockIdx.x * nk + k] = acc[k];
+#pragma unroll
+    for (int c = 0; c < kModes; ++c) {
+        const int k = threadIdx.x + c * T;
+        if (k < nk) part[(size_t)blockIdx.x * nk + k] = acc[c];
+    }
 }
 
-// sum over rows of power[row][k], in row order (deterministic)
-__global__ void column_sum_kernel(const double *power, int nrow, int nk, double *out)
+// out[k] = norm * sum over rows of part[row][k], in a fixed order: a block has
+// 16 columns (128 bytes of a row), its 16 groups of threads each a run of rows.
+// One thread a column took 337 us for 1024 rows of 1025, this 6.
+constexpr int kSumCols = 16;
+__global__ __launch_bounds__(kFluxThreads) void column_sum_kernel(const double *part, int nrow, int nk, double norm,
+                                                                 double *out)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nk) return;
+    constexpr int kRuns = kFluxThreads / kSumCols;
+    __shared__ double sums[kRuns][kSumCols];
+    const int col = threadIdx.x % kSumCols, run = threadIdx.x / kSumCols;
+    const int k = blockIdx.x * kSumCols + col;
+    const int len = (nrow + kRuns - 1) / kRuns, end = min(nrow, (run + 1) * len);
     double s = 0;
-    for (int r = 0; r < nrow; ++r) s += power[(size_t)r * nk + k];
-    out[k] = s;
+    if (k < nk)
+#pragma unroll 8
+        for (int r = run * len; r < end; ++r) s += part[(size_t)r * nk + k];
+    sums[run][col] = s;
+    __syncthreads();
+    if (run == 0 && k < nk) {
+        for (int i = 1; i < kRuns; ++i) s += sums[i][col];
+        out[k] = s * norm;
+    }
 }
 
 // Histogram of exp(-s tau) over nb equal bins of [0, 1], bin edges e_k =
@@ -518,56 +751,35 @@ int fsamd_flux_power(const double *tau, int nlos, int npix, double scale, double
 {
     if (nlos < 1 || npix < 1 || !tau || !power || !(mean_flux != 0))
         return fail(FSAMD_ERR_ARG, "bad arguments to fsamd_flux_power");
+    // a pair's row with the half table of roots beside it
     constexpr size_t kLdsBytes = 160 * 1024;
+    if (sizeof(double) * 3 * (size_t)npix > kLdsBytes)
+        return fail(FSAMD_ERR_UNSUPPORTED, "flux power: npix too large for the LDS buffers");
     hipStream_t s = (hipStream_t)stream;
     const int nk = npix / 2 + 1;
-    const size_t fft_shm = sizeof(double2) * 2 * (size_t)npix + sizeof(double) * (size_t)nk;
-    const size_t dft_shm = sizeof(double) * 3 * (size_t)npix;
-    const bool use_fft = fft_shm <= kLdsBytes;
-    if (!use_fft && dft_shm > kLdsBytes)
-        return fail(FSAMD_ERR_UNSUPPORTED, "flux power: npix too large for the LDS buffers");
-    // FFT: one partial row per block (at most 1024 blocks), DFT: one per sightline
-    const int npair = (nlos + 1) / 2;
-    const int nblk = use_fft ? std::min(npair, 1024) : nlos;
-    const size_t nrow = (size_t)nblk;
-    double *per = nullptr;
-    FSAMD_HIP(hipMalloc(&per, sizeof(double) * nrow * nk + (use_fft ? sizeof(double2) * (size_t)npix : 0)));
-    hipError_t e = hipSuccess;
-    if (use_fft) {
-        double2 *tw = reinterpret_cast<double2 *>(per + nrow * nk);
-        if (int rc = raise_lds_limit((const void *)flux_fft_kernel, fft_shm)) {
-            (void)hipFree(per);
-            return rc;
-        }
-        fft_twiddle_kernel<<<(npix + 255) / 256, 256, 0, s>>>(tw, npix);
-        e = hipGetLastError();
-        if (e == hipSuccess) {
-            flux_fft_kernel<<<nblk, kFluxThreads, fft_shm, s>>>(tau, nlos, npix, scale, 1.0 / mean_flux, tw,
-                                                               fft_plan(npix), per);
-            e = hipGetLastError();
-        }
-    } else {
-        if (int rc = raise_lds_limit((const void *)flux_dft_kernel, dft_shm)) {
-            (void)hipFree(per);
-            return rc;
-        }
-        flux_dft_kernel<<<std::min(nlos, 65536), kFluxThreads, dft_shm, s>>>(tau, nlos, npix, scale,
-                                                                            1.0 / mean_flux, per);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) {
-        column_sum_kernel<<<(nk + 255) / 256, 256, 0, s>>>(per, (int)nrow, nk, power);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(per);
-    if (e != hipSuccess) return fail(FSAMD_ERR_HIP, std::string("flux power: ") + hipGetErrorString(e));
+    const FftPlan fp = fft_plan(npix);
+    const size_t shm = sizeof(double2) * ((size_t)npix + (fp.any ? nk : FSAMD_EXP_N));
+    const bool pow2 = npix % 8 == 0 && (npix & (npix - 1)) == 0;
+    const auto kernel = fp.any ? flux_fft_kernel<kFftAny> : pow2 ? flux_fft_kernel<kFftPow2> : flux_fft_kernel<kFftSmall>;
+    const int threads = ((npix + kFftPoints - 1) / kFftPoints + 63) / 64 * 64;
+    if (int rc = raise_lds_limit((const void *)kernel, shm)) return rc;
+    int dev = 0, ncu = 0, percu = 0;
+    FSAMD_HIP(hipGetDevice(&dev));
+    FSAMD_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    FSAMD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&percu, kernel, threads, shm));
+    const int nblk = std::min((nlos + 1) / 2, std::max(1, percu) * ncu);
+    double *part = nullptr;
+    FSAMD_HIP(hipMalloc(&part, sizeof(double) * (size_t)nblk * nk + sizeof(double2) * (size_t)npix));
+    double2 *tw = reinterpret_cast<double2 *>(part + ((size_t)nblk * nk + 1) / 2 * 2);
+    fft_twiddle_kernel<<<(npix + 255) / 256, 256, 0, s>>>(tw, fp);
+    kernel<<<nblk, threads, shm, s>>>(tau, nlos, npix, scale, 1.0 / mean_flux, tw, fp, part);
     // mean over sightlines of vmax |F_k|^2 / npix^2 (fluxstatistics.py:49-56, 95-102)
-    std::vector<double> h(nk);
-    FSAMD_HIP(hipMemcpy(h.data(), power, sizeof(double) * nk, hipMemcpyDeviceToHost));
     const double norm = vmax / ((double)npix * (double)npix) / nlos;
-    for (double &x : h) x *= norm;
-    FSAMD_HIP(hipMemcpy(power, h.data(), sizeof(double) * nk, hipMemcpyHostToDevice));
+    column_sum_kernel<<<(nk + kSumCols - 1) / kSumCols, kFluxThreads, 0, s>>>(part, nblk, nk, norm, power);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    (void)hipFree(part);
+    if (e != hipSuccess) return fail(FSAMD_ERR_HIP, std::string("flux power: ") + hipGetErrorString(e));
     return FSAMD_OK;
 }
 

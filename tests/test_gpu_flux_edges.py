@@ -1,4 +1,5 @@
-"""Flux statistics at the sizes where the kernels' splits change: the mean-flux
+"""Flux statistics at the sizes where the kernels' splits change: transforms of
+every radix the plan knows and of primes, the column sums, the mean-flux
 iteration on fields with excluded, negative and deep pixels."""
 import math
 
@@ -18,6 +19,40 @@ def _field(nlos, npix, seed):
     t[r.random(t.shape) < 0.05] = 0.0
     t[r.random(t.shape) < 0.01] = 1e5     # no flux left
     return t
+
+
+# 8s alone (8, 64, 512, 4096), with 4 and 2 (16, 32, 2048), odd radices, all of
+# them (840), primes and their multiples, one thread's last value (513), the
+# largest size before and behind the root table's, the longest that is taken
+@pytest.mark.parametrize("npix", [1, 2, 3, 4, 5, 7, 8, 9, 11, 13, 16, 22, 32, 49, 64, 121, 505, 512, 513, 840, 1001, 1023,
+                                  2048, 2187, 3125, 4096, 4551, 4552, 5120, 6561, 6826])
+@pytest.mark.parametrize("nlos", [1, 2, 5])
+def test_power_of_all_radices(npix, nlos):
+    """Amplitudes (roots of the power, rms over the rows): a mode of the FP64
+    transform is off by some eps log2(n) |d| (a direct sum over a prime: by
+    eps sqrt(n) |d|; 40 + n/8 covers both), and d itself by 4 ulp of flux / mean."""
+    t = _field(nlos, npix, npix)
+    _, got = GF.flux_power(torch.from_numpy(t).cuda(), 100.0, mean_flux_desired=None)
+    f = np.exp(-t) / np.exp(-t).mean()
+    ref = (np.abs(np.fft.rfft(f - 1, axis=1)) ** 2).mean(0) * 100.0 / npix ** 2
+    off = 2.3e-16 * (40 + npix / 8) * np.sqrt(((f - 1) ** 2).sum(1).mean()) + 1e-15 * npix * f.max()
+    assert np.all(np.abs(np.sqrt(got) - np.sqrt(ref)) <= off * 10.0 / npix)
+
+
+def test_power_refuses_longer_rows():
+    with pytest.raises(Exception, match="npix too large"):
+        GF.flux_power(torch.zeros((1, 6827), dtype=torch.float64, device="cuda"), 1.0)
+
+
+@pytest.mark.parametrize("nlos,npix", [(1, 300), (31, 33), (1279, 14), (5000, 32), (20000, 8)])
+def test_power_of_many_rows(nlos, npix):
+    """Blocks with no, one and several pairs; rows of partial sums that do not
+    fill the column sum's runs: sums of like-signed terms, eps sqrt(rows) off."""
+    t = _field(nlos, npix, nlos)
+    _, got = GF.flux_power(torch.from_numpy(t).cuda(), 7.0)
+    d = np.exp(-t) / np.exp(-t).mean() - 1
+    ref = (np.abs(np.fft.rfft(d, axis=1)) ** 2).mean(0) * 7.0 / npix ** 2
+    assert np.all(np.abs(got - ref) <= 1e-12 * ref.max())
 
 
 @pytest.mark.parametrize("n", [1, 2, 255, 257, 1536 * 256 - 1, 1536 * 256 * 2, 1536 * 256 * 5 + 77])
