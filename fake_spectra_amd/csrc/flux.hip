@@ -177,23 +177,96 @@ static bool taylor_step(const double *sum, double c, double z, double target, do
     return rem * r + std::fabs((F - target) / G) * rem * J / x <= 1e-14 * z * G;
 }
 
-// Gaussian smoothing along rows with periodic wrap, weights w[0..2r]
+// Gaussian smoothing along rows with periodic wrap, weights w[0 .. nw), nw = 2r + 1
 // (the correlation of scipy.ndimage.gaussian_filter1d, mode 'wrap').
-__global__ __launch_bounds__(kFluxThreads) void res_corr_kernel(const double *in, double *out, int nrow, int ncol,
-                                                               const double *w, int r)
+//
+// Bound: HBM, a read and a write.  A block stages a stretch of `cols` columns
+// of a row with its taps' margin (of several rows where they are short) and the
+// weights in LDS, kResTaps taps at a time; a thread has kResOut neighbouring
+// outputs, so that two pixels and two weights read feed eight multiply-adds.
+// 40000 rows of 2048, 9 taps: 900 -> 270 us (4.9 TB/s);
+// 9765 of 2048, 57 taps, a call: 1060 -> 131 us.
+constexpr int kResOut = 4;
+constexpr int kResCols = kResOut * kFluxThreads;
+constexpr int kResTaps = 256;   // even: only the last stretch of taps has an odd one
+constexpr int kResLds = 2560;   // doubles of short rows in a block: 20 KB, eight blocks a CU
+
+struct ResTile {
+    int cols, rows, nchunk;     // a block's part: cols columns of rows rows; nchunk parts a row
+    int stride;                 // of a staged row, a multiple of kResOut
+};
+
+static ResTile res_tile(int ncol, int nw)
 {
-    for (int row = blockIdx.x; row < nrow; row += gridDim.x) {
-        const double *src = in + (size_t)row * ncol;
-        double *dst = out + (size_t)row * ncol;
-        for (int i = threadIdx.x; i < ncol; i += kFluxThreads) {
-            double acc = 0;
-            for (int k = -r; k <= r; ++k) {
-                int j = (i + k) % ncol;
-                if (j < 0) j += ncol;
-                acc += w[k + r] * src[j];
+    ResTile t;
+    t.cols = std::min(ncol, kResCols);
+    t.nchunk = (ncol + t.cols - 1) / t.cols;
+    t.stride = (t.cols + kResOut - 1) / kResOut * kResOut + (std::min(nw, kResTaps) + kResOut) / kResOut * kResOut;
+    const int groups = (t.cols + kResOut - 1) / kResOut;
+    t.rows = std::max(1, std::min(kFluxThreads / groups, kResLds / t.stride));
+    return t;
+}
+
+__global__ __launch_bounds__(kFluxThreads) void res_corr_kernel(const double *in, double *out, int nrow, int ncol,
+                                                               const double *w, int nw, ResTile tile, long long nparts)
+{
+    extern __shared__ double2 shc[];
+    double *taps = reinterpret_cast<double *>(shc), *pix = taps + (min(nw, kResTaps) + 1) / 2 * 2;
+    const int groups = (tile.cols + kResOut - 1) / kResOut;
+    const int myrow = threadIdx.x / groups, at = threadIdx.x % groups * kResOut;
+    double *mine = pix + myrow * tile.stride + at;
+    // a short row is loaded by a wavefront, a long one by the block
+    const int lrow = tile.rows > 1 ? threadIdx.x / 64 : 0, lrows = tile.rows > 1 ? kFluxThreads / 64 : 1;
+    const int lcol = tile.rows > 1 ? threadIdx.x % 64 : threadIdx.x, lcols = tile.rows > 1 ? 64 : kFluxThreads;
+    for (long long part = blockIdx.x; part < nparts; part += gridDim.x) {
+        const int row0 = (int)(part / tile.nchunk) * tile.rows, col0 = (int)(part % tile.nchunk) * tile.cols;
+        const int rows = min(tile.rows, nrow - row0), cols = min(tile.cols, ncol - col0);
+        double acc[kResOut] = {};
+        for (int k0 = 0; k0 < nw; k0 += kResTaps) {
+            const int nk = min(kResTaps, nw - k0), width = cols + nk - 1;
+            int first = (col0 - nw / 2 + k0) % ncol;
+            if (first < 0) first += ncol;
+            __syncthreads();
+            for (int k = threadIdx.x; k < nk; k += kFluxThreads) taps[k] = w[k0 + k];
+            for (int r = lrow; r < rows; r += lrows) {
+                const double *src = in + (size_t)(row0 + r) * ncol;
+                for (int x = lcol; x < width; x += lcols) {
+                    int j = first + x;
+                    if (j >= ncol) j -= ncol;
+                    if (j >= ncol) j %= ncol;   // more taps than columns
+                    pix[r * tile.stride + x] = src[j];
+                }
             }
-            dst[i] = acc;
+            __syncthreads();
+            if (myrow >= rows) continue;
+            double2 s0 = *(const double2 *)mine, s1 = *(const double2 *)(mine + 2);
+            for (int k = 0; k + 1 < nk; k += 2) {
+                const double2 s2 = *(const double2 *)(mine + k + 4), t = *(const double2 *)(taps + k);
+                acc[0] = fma(t.y, s0.y, fma(t.x, s0.x, acc[0]));
+                acc[1] = fma(t.y, s1.x, fma(t.x, s0.y, acc[1]));
+                acc[2] = fma(t.y, s1.y, fma(t.x, s1.x, acc[2]));
+                acc[3] = fma(t.y, s2.x, fma(t.x, s1.y, acc[3]));
+                s0 = s1;
+                s1 = s2;
+            }
+            if (nk & 1) {
+                const double t = taps[nk - 1];
+                acc[0] = fma(t, s0.x, acc[0]);
+                acc[1] = fma(t, s0.y, acc[1]);
+                acc[2] = fma(t, s1.x, acc[2]);
+                acc[3] = fma(t, s1.y, acc[3]);
+            }
         }
+        // through LDS, for whole lines
+        __syncthreads();
+        if (myrow < rows) {
+            *(double2 *)mine = make_double2(acc[0], acc[1]);
+            *(double2 *)(mine + 2) = make_double2(acc[2], acc[3]);
+        }
+        __syncthreads();
+        for (int r = lrow; r < rows; r += lrows)
+            for (int x = lcol; x < cols; x += lcols)
+                out[(size_t)(row0 + r) * ncol + col0 + x] = pix[r * tile.stride + x];
     }
 }
 
@@ -625,49 +698,64 @@ __global__ __launch_bounds__(kFluxThreads) void column_sum_kernel(const double *
 
 // Histogram of exp(-s tau) over nb equal bins of [0, 1], bin edges e_k =
 // k / nb as numpy.histogram places them (searchsorted on the edges, the last
-// bin closed); values outside [0, 1] are not counted.
+// bin closed); values outside [0, 1] are not counted.  f nb is within 2e-11 of
+// its value (nb <= 40960), so the edges decide only next to a whole number.
 __device__ inline int flux_bin(double f, int nb)
 {
-    int b = (int)(f * nb);
-    b = b < 0 ? 0 : (b > nb - 1 ? nb - 1 : b);
-    if (f < (double)b / (double)nb && b > 0) --b;
-    if (b < nb - 1 && f >= (double)(b + 1) / (double)nb) ++b;
+    const double x = f * nb, e = rint(x);
+    int b = min((int)x, nb - 1);
+    if (fabs(x - e) < 1e-9 && e > 0.0 && e < (double)nb) b = f < e / (double)nb ? (int)e - 1 : (int)e;
     return b;
 }
 
 // Counts are kept per block in LDS and added to the global bins once per
-// block: nb <= kFluxPrivBins bins get one private row per thread (no atomics;
-// a flux field piles up in few bins, which would serialize atomics), larger
-// nb one shared row with LDS atomics.
-constexpr int kFluxPrivBins = 32;
+// block: as many copies of a bin as there is room for, up to one a thread (a
+// flux field piles up in few bins, which would serialize the atomics).
+//
+// Bound: HBM, one read of the field.  82M pixels, 20 bins: 230 -> 145 us, with
+// the two divides a pixel and the 256 copies read by one thread a bin gone; 50
+// bins, one copy before, a call on 20M pixels: 140 -> 105 us.
+constexpr int kHistCounts = 10240;   // 40 KB: four blocks a CU
+constexpr int kHistBatch = 4;
 
+// kTable: exp by flux_exp's table, where the LDS holds it beside the bins
+template <bool kTable>
 __global__ __launch_bounds__(kFluxThreads) void flux_hist_kernel(const double *tau, long long n, double scale, int nb,
-                                                                unsigned long long *counts)
+                                                                int copies, unsigned long long *counts)
 {
-    extern __shared__ unsigned int hist[];   // [nb][kFluxThreads] private rows, or [nb] shared
-    const bool priv = nb <= kFluxPrivBins;
-    const int rows = priv ? nb * kFluxThreads : nb;
-    for (int i = threadIdx.x; i < rows; i += kFluxThreads) hist[i] = 0;
+    extern __shared__ double2 shc[];
+    double2 *etab = shc;
+    unsigned int *hist = reinterpret_cast<unsigned int *>(shc + (kTable ? FSAMD_EXP_N : 0));   // [nb][copies]
+    if (kTable) load_exp_table(etab);
+    for (int i = threadIdx.x; i < nb * copies; i += kFluxThreads) hist[i] = 0;
     __syncthreads();
+    const int copy = threadIdx.x & (copies - 1);
+    const auto add = [&](double t) {
+        const double f = kTable ? flux_exp<false>(-scale * t, etab) : exp(-scale * t);
+        if (f >= 0.0 && f <= 1.0) atomicAdd(&hist[flux_bin(f, nb) * copies + copy], 1u);
+    };
     const long long stride = (long long)gridDim.x * kFluxThreads;
-    for (long long i = blockIdx.x * (long long)kFluxThreads + threadIdx.x; i < n; i += stride) {
-        const double f = exp(-scale * tau[i]);
-        if (!(f >= 0.0 && f <= 1.0)) continue;
-        const int b = flux_bin(f, nb);
-        if (priv)
-            ++hist[b * kFluxThreads + threadIdx.x];
-        else
-            atomicAdd(&hist[b], 1u);
+    long long i = blockIdx.x * (long long)kFluxThreads + threadIdx.x;
+    for (; i + (kHistBatch - 1) * stride < n; i += kHistBatch * stride) {
+        double t[kHistBatch];
+#pragma unroll
+        for (int q = 0; q < kHistBatch; ++q) t[q] = tau[i + q * stride];
+#pragma unroll
+        for (int q = 0; q < kHistBatch; ++q) add(t[q]);
+    }
+    for (; i < n; i += stride) add(tau[i]);
+    __syncthreads();
+    // min(copies, 64) lanes a bin
+    const int lanes = min(copies, 64), sub = threadIdx.x & (lanes - 1);
+    for (int b = threadIdx.x / lanes; b < nb; b += kFluxThreads / lanes) {
+        unsigned int c = 0;
+        for (int k = sub; k < copies; k += lanes) c += hist[b * copies + k];
+        for (int o = lanes / 2; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+        if (sub == 0) hist[b * copies] = c;
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < nb; b += kFluxThreads) {
-        unsigned long long c = 0;
-        if (priv)
-            for (int t = 0; t < kFluxThreads; ++t) c += hist[b * kFluxThreads + t];
-        else
-            c = hist[b];
-        if (c) atomicAdd(&counts[b], c);
-    }
+    for (int b = threadIdx.x; b < nb; b += kFluxThreads)   // neighbouring bins in one instruction
+        if (const unsigned int c = hist[b * copies]) atomicAdd(&counts[b], (unsigned long long)c);
 }
 
 }  // namespace fsamd
@@ -737,7 +825,11 @@ int fsamd_res_corr(const double *in, double *out, int nrow, int ncol, double sig
     FSAMD_HIP(hipMalloc(&dw, sizeof(double) * w.size()));
     hipError_t e = hipMemcpyAsync(dw, w.data(), sizeof(double) * w.size(), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
-        res_corr_kernel<<<std::min(nrow, 65536), kFluxThreads, 0, s>>>(in, out, nrow, ncol, dw, r);
+        const ResTile t = res_tile(ncol, 2 * r + 1);
+        const long long nparts = ((long long)nrow + t.rows - 1) / t.rows * t.nchunk;
+        const size_t shm = sizeof(double) * ((size_t)t.rows * t.stride + (std::min(2 * r + 1, kResTaps) + 1) / 2 * 2);
+        res_corr_kernel<<<(int)std::min<long long>(nparts, 4096), kFluxThreads, shm, s>>>(in, out, nrow, ncol, dw,
+                                                                                             2 * r + 1, t, nparts);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -790,11 +882,19 @@ int fsamd_flux_hist(const double *tau, long long n, double scale, int nbins, uns
     hipStream_t s = (hipStream_t)stream;
     FSAMD_HIP(hipMemsetAsync(counts, 0, sizeof(unsigned long long) * nbins, s));
     if (n > 0) {
-        const int nblocks = (int)std::min<long long>(4096, (n + kFluxThreads - 1) / kFluxThreads);
-        const size_t shm = sizeof(unsigned int) * (size_t)(nbins <= kFluxPrivBins ? nbins * kFluxThreads : nbins);
-        if (shm > 160 * 1024) return fail(FSAMD_ERR_UNSUPPORTED, "flux histogram: too many bins for the LDS");
-        if (int rc = raise_lds_limit((const void *)flux_hist_kernel, shm)) return rc;
-        flux_hist_kernel<<<nblocks, kFluxThreads, shm, s>>>(tau, n, scale, nbins, counts);
+        constexpr size_t kLdsBytes = 160 * 1024, kTabBytes = sizeof(double2) * FSAMD_EXP_N;
+        size_t shm = sizeof(unsigned int) * (size_t)nbins;
+        if (shm > kLdsBytes) return fail(FSAMD_ERR_UNSUPPORTED, "flux histogram: too many bins for the LDS");
+        const int nblocks = (int)std::min<long long>(1024, (n + kFluxThreads - 1) / kFluxThreads);
+        // no more counts than a block has pixels: they are cleared and added up
+        const long long room = std::min<long long>(kHistCounts, n / nblocks);
+        int copies = 1;
+        while (copies < kFluxThreads && 2LL * copies * nbins <= room) copies *= 2;
+        const bool table = shm + kTabBytes <= kLdsBytes;
+        shm = shm * copies + (table ? kTabBytes : 0);
+        const auto kernel = table ? flux_hist_kernel<true> : flux_hist_kernel<false>;
+        if (int rc = raise_lds_limit((const void *)kernel, shm)) return rc;
+        kernel<<<nblocks, kFluxThreads, shm, s>>>(tau, n, scale, nbins, copies, counts);
         FSAMD_HIP(hipGetLastError());
     }
     FSAMD_HIP(hipStreamSynchronize(s));

@@ -1,6 +1,7 @@
 """Flux statistics at the sizes where the kernels' splits change: transforms of
 every radix the plan knows and of primes, the column sums, the mean-flux
-iteration on fields with excluded, negative and deep pixels."""
+iteration on fields with excluded, negative and deep pixels, smoothing in one
+and several stretches, histograms of few and many bins."""
 import math
 
 import numpy as np
@@ -77,3 +78,43 @@ def test_mean_flux_excluded_and_negative_pixels():
         assert abs(got - FS.mean_flux_scale(t, 0.5, 1e-8, thresh=thresh)) <= 1e-12 * got
     t[11] = np.nan
     assert math.isnan(GF.mean_flux(torch.from_numpy(t).cuda(), 0.5))
+
+
+# one chunk of columns or several, several rows a block, taps in one stretch and
+# in several, more taps than columns, a single column
+@pytest.mark.parametrize("nrow,ncol", [(1, 1), (3, 2), (700, 5), (37, 64), (5, 255), (9, 1023), (4, 1024), (3, 1025), (2, 2049),
+                                       (1, 5000)])
+@pytest.mark.parametrize("sigma", [0.1, 1.04, 31.9, 40.0, 300.0])
+def test_smoothing_of_all_splits(nrow, ncol, sigma):
+    """A weighted mean of nw pixels: eps sqrt(nw) of the largest, with 4 ulp for
+    the weights."""
+    x = np.random.default_rng(ncol).random((nrow, ncol))
+    dvbin = 8 / (2 * np.sqrt(2 * np.log(2))) / sigma
+    got = GF.res_corr(torch.from_numpy(x).cuda(), dvbin, 8).cpu().numpy()
+    nw = 8 * sigma + 1
+    assert np.max(np.abs(got - FS.res_corr(x, dvbin, 8))) <= 2.3e-16 * (4 + np.sqrt(nw)) * 2
+
+
+@pytest.mark.parametrize("nbins", [1, 2, 20, 40, 41, 50, 1000, 10241, 40448, 40960])
+@pytest.mark.parametrize("n", [3, 255, 2048 * 256 * 4 + 11])
+def test_histogram_of_all_bin_counts(nbins, n):
+    """Pixels inside their bins (a tenth of its width from the edges), at no and
+    all of the flux, and some that are not counted: the counts are exact."""
+    r = np.random.default_rng(nbins)
+    k = r.integers(0, nbins, n)
+    k[: n // 2] //= 3
+    t = -np.log((k + r.uniform(0.1, 0.9, n)) / nbins)
+    t[::5], k[::5] = 0.0, nbins - 1
+    t[1::7], k[1::7] = 1e5, 0
+    t[2::11], k[2::11] = np.nan, -1
+    if n > 100:
+        t[3::13], k[3::13] = -0.5, -1
+        t[4::17], k[4::17] = np.inf, 0
+    counts = np.bincount(k[k >= 0], minlength=nbins)
+    _, pdf = GF.flux_pdf(torch.from_numpy(t).cuda(), nbins)
+    np.testing.assert_array_equal(np.rint(pdf * counts.sum() / nbins), counts)
+
+
+def test_histogram_refuses_too_many_bins():
+    with pytest.raises(Exception, match="too many bins"):
+        GF.flux_pdf(torch.zeros(4, dtype=torch.float64, device="cuda"), 40961)
