@@ -445,6 +445,14 @@ static_assert(64 * kRoundsMax < (1 << 16) && kRoundsMax < (1 << 8), "StepShape::
 
 __device__ inline StepShape unpack_shape(int s) { return StepShape{s & 0xffff, (s >> 16) & 0xff, s >> 24}; }
 
+// A step's work beside its sums (the pair's state, trapezoid, tail cut, deposit)
+// costs as much as one and a half rounds of sums, so groups of 16 and 32 lanes
+// take two rounds where pixels have several sub-samples: 16 lanes 15 pixels of 3
+// in place of 7, 7 of 5 in place of 3.  256^3 x 5000 x 2048, two lines, 89.9 ->
+// 85.1 ms; with metals (12288 x 1024) 268 -> 206; top-hat, 512^3, 193 -> 153.
+// Three or four rounds cost more past the cut than they save (214 and 225 with
+// metals), and so do two of 64 lanes (323 -> 362).  Wider grids: as many rounds
+// as two pixels take.
 __device__ inline StepShape step_shape(int np, int kg)
 {
     StepShape sh;
@@ -452,12 +460,9 @@ __device__ inline StepShape step_shape(int np, int kg)
     if (sh.nm1 == 0) {
         sh.rounds = 1;
         sh.pstep = kg;
-    } else if (sh.nm1 < kg) {
-        sh.rounds = 1;
-        sh.pstep = (kg - 1) / sh.nm1;
     } else {
-        sh.rounds = min(kRoundsMax, (2 * sh.nm1 + kg) / kg);
-        sh.pstep = (kg * sh.rounds - 1) / sh.nm1;
+        sh.rounds = sh.nm1 >= kg ? min(kRoundsMax, (2 * sh.nm1 + kg) / kg) : kg < 64 ? 2 : 1;
+        sh.pstep = min(kg, (kg * sh.rounds - 1) / sh.nm1);
     }
     return sh;
 }

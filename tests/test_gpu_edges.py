@@ -178,3 +178,30 @@ def test_adjoint_refuses_long_rows():
     t = SP.tau(plan, 20000, 1, args[4], vel, temp, [line], [dens])[0]
     with pytest.raises(Exception, match="nbins too large"):
         SP.tau_adjoint(plan, 20000, 1, args[4], vel, temp, [line], [dens], [t])
+
+
+# pixels of 1 to 129 sub-samples, around the counts where a lane group of 16, 32
+# or 64 takes another number of rounds, pixels or none (FP64), in narrow and
+# wide supports; rows of less than a step and of many
+@pytest.mark.parametrize("group", [16, 32, 64])
+@pytest.mark.parametrize("nbins,hfrac,kernel", [(200, 0.004, 1), (200, 0.05, 3), (9, 0.1, 1), (2048, 0.002, 0)])
+def test_walks_of_all_sample_counts(oracle, group, nbins, hfrac, kernel):
+    nm1 = np.array([0, 2, 4, 6, 8, 10, 14, 16, 20, 30, 32, 34, 62, 64, 66, 128] * 12)
+    velfac = synth.Cosmology().velfac()
+    args = list(small_gas(nm1.size, 20.0 * nbins / velfac, 4, nbins, kernel, hfrac))
+    # a pixel is 20 km/s: b so that it has nm1 + 1 sub-samples (2 ceil(20 / b) + 1, one below b = 40)
+    b = np.where(nm1 == 0, 50.0, 20.0 / (nm1 / 2 - 0.4))
+    args[14] = (1e4 * (b / 12.85) ** 2).astype(np.float32)
+    args[15] = np.maximum(args[15], np.float32(2.0 / velfac))
+    args[16] = (1 + np.arange(4) % 3).astype(np.int32)
+    rng = np.random.default_rng(7)
+    args[17] = args[11][rng.integers(0, nm1.size, 4)].astype(np.float64) + 1e-3
+    ref = oracle.interpolate(*args)
+    from fake_spectra_amd import _native as N
+    N.set_group_size(group)
+    try:
+        got = SP._Particle_Interpolate(*args)
+    finally:
+        N.set_group_size(16)
+    assert np.max(ref) > 0
+    assert_tau_close(got, ref, "sub-sample counts")
