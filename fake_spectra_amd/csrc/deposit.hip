@@ -437,13 +437,12 @@ constexpr int kRoundsMax = 4;
 
 struct StepShape {
     int nm1;      // np - 1 (0: midpoint)
-    int rounds;   // lane rounds per step
     int pstep;    // pixels per step
-    __device__ inline int packed() const { return nm1 | (rounds << 16) | (pstep << 24); }
+    __device__ inline int packed() const { return nm1 | (pstep << 16); }
 };
-static_assert(64 * kRoundsMax < (1 << 16) && kRoundsMax < (1 << 8), "StepShape::packed");
+static_assert(64 * kRoundsMax < (1 << 16), "StepShape::packed");
 
-__device__ inline StepShape unpack_shape(int s) { return StepShape{s & 0xffff, (s >> 16) & 0xff, s >> 24}; }
+__device__ inline StepShape unpack_shape(int s) { return StepShape{s & 0xffff, s >> 16}; }
 
 // A step's work beside its sums (the pair's state, trapezoid, tail cut, deposit)
 // costs as much as one and a half rounds of sums, so groups of 16 and 32 lanes
@@ -457,12 +456,10 @@ __device__ inline StepShape step_shape(int np, int kg)
 {
     StepShape sh;
     sh.nm1 = np - 1;
-    if (sh.nm1 == 0) {
-        sh.rounds = 1;
-        sh.pstep = kg;
-    } else {
-        sh.rounds = sh.nm1 >= kg ? min(kRoundsMax, (2 * sh.nm1 + kg) / kg) : kg < 64 ? 2 : 1;
-        sh.pstep = min(kg, (kg * sh.rounds - 1) / sh.nm1);
+    sh.pstep = kg;
+    if (sh.nm1 > 0) {
+        const int rounds = sh.nm1 >= kg ? min(kRoundsMax, (2 * sh.nm1 + kg) / kg) : kg < 64 ? 2 : 1;
+        sh.pstep = min(kg, (kg * rounds - 1) / sh.nm1);
     }
     return sh;
 }
@@ -658,16 +655,22 @@ __device__ inline bool setup_pair(const DepositArgs &A, int line, const LineDesc
 // weights and the ten far-wing coefficients) runs on up to kRecs lanes at once
 // instead of on the few lanes of one lane group.  A group walks its pair in
 // the record where it lies.  Which records are free, and which hold pairs of
-// the light and of the full profile, are three masks of the wavefront: the
-// groups take pairs of one class as long as there are some, so that the near
-// steps of the wavefront mostly run the light code (a step runs the full code,
-// 180 instead of 85 instructions a sum, if any of its groups needs it).  Against
-// a ring in claim order whose records were copied to a slot per group: 99.3 ->
-// 89.6 ms at 256^3 x 5000 x 2048, two lines; 301 -> 269 with a metal line (half
-// of its pairs full) at 12288 x 1024.
+// either class, are three masks of the wavefront: the groups take pairs of one
+// class as long as there are some, so that the near steps of the wavefront
+// mostly run the light code (a step runs the full code, 180 instead of 85
+// instructions a sum, if any of its groups needs it) and its four groups the
+// same number of rounds.  The one class is the light profile on several
+// sub-samples; the other the full profile, and midpoint pixels: fields have few of
+// one or of the other, and a class of each costs more in refills than it
+// saves.  Against a ring in claim order whose records were copied to a slot per
+// group: 99.3 -> 89.6 ms at 256^3 x 5000 x 2048, two lines; 301 -> 269 with a metal
+// line (half of its pairs full) at 12288 x 1024; midpoint pixels apart 84.2 -> 80.5
+// and 202.5 -> 203.2.
 constexpr int kRecs = kWaveClaim;
 static_assert(kRecs == 32, "the record masks are 32-bit");
-constexpr int kRefillRoom = 12;   // fewest free records worth a set-up while others wait
+// Fewest free records worth a set-up, whose cost hardly depends on their number,
+// while others wait: 12 -> 24 82.2 -> 80.5 and 208.5 -> 203.2 ms; 28 the same.
+constexpr int kRefillRoom = 24;
 
 // The far-wing coefficients of wing_setup for one pair, all ten on one lane
 // (the batched set-up of the main kernel), in FP32: every term is positive,
@@ -843,10 +846,11 @@ __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int 
     }
     wave_sync();
     const unsigned mine = (unsigned)__ballot(used);
-    const unsigned a3 = (unsigned)__ballot(used && recs[lane & 31].vp.a3 != 0.0f);
+    const PairRec &mr = recs[lane & 31];
+    const unsigned other = (unsigned)__ballot(used && (mr.vp.a3 != 0.0f || unpack_shape(mr.shape).nm1 == 0));
     free &= ~mine;
-    light |= mine & ~a3;
-    full |= a3;
+    light |= mine & ~other;
+    full |= other;
     more = (long long)base + want < w.p1;
 }
 
@@ -1024,18 +1028,15 @@ __device__ inline int near_step(const DepositArgs &A, const PairRec &P, float *s
         // (np-1) of its pixel (singleabs.h:118-121) up to the rounding of m dv
         // against the pixel's own vlow, or (np = 1) pixel m's centre
         // (singleabs.h:113); positions in u's scale.
-        const int nsub = nm1 == 0 ? pcount : pcount * nm1 + 1;
+        const int nsub = nm1 == 0 ? pcount : __mul24(pcount, nm1) + 1;
         const double dss = P.dss;
         double sv = vf * P.ibs;
         if (nm1 == 0) sv = __builtin_fma(0.5, dss, sv);
-        if (dir < 0) sv = __builtin_fma((double)((1 - pcount) * max(nm1, 1)), dss, sv);   // its lowest pixel
-        for (int r = 0; r < sh.rounds; ++r) {
-            const int m = glane + r * kG;
-            if (m < nsub) {
-                const double at = __builtin_fma((double)m, dss, sv);
-                sbuf[m] = a3 ? inner32<true>(P, at, ptab) : inner32<false>(P, at, ptab);
-                if (kStats) st.sums++;
-            }
+        if (dir < 0) sv = __builtin_fma((double)__mul24(1 - pcount, max(nm1, 1)), dss, sv);   // its lowest pixel
+        for (int m = glane; m < nsub; m += kG) {
+            const double at = __builtin_fma((double)m, dss, sv);
+            sbuf[m] = a3 ? inner32<true>(P, at, ptab) : inner32<false>(P, at, ptab);
+            if (kStats) st.sums++;
         }
     }
     wave_sync();
@@ -1045,7 +1046,7 @@ __device__ inline int near_step(const DepositArgs &A, const PairRec &P, float *s
         // trapezoid over the pixel's sub-samples (singleabs.h:116-125); np = 1:
         // both ends are the one sample
         const int j = dir > 0 ? glane : pcount - 1 - glane;
-        const float *sp = sbuf + (nm1 == 0 ? j : j * nm1);
+        const float *sp = sbuf + (nm1 == 0 ? j : __mul24(j, nm1));
         double tot = 0.5 * ((double)sp[0] + (double)sp[nm1]);
         for (int kk = 1; kk < nm1; ++kk) tot += (double)sp[kk];
         t = P.snear * tot;
@@ -1175,7 +1176,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         // group state: dir 0 = needs a pair, +1/-1 = walking, 2 = no pairs left;
         // rec: its record; c: pixels walked in this direction
         int dir = 0, c = 0, z0 = 0, rec = 0;
-        // the wavefront's records, and the class it takes pairs from
+        // the wavefront's records: free, waiting by class (full: the other class,
+        // see kRecs), and the class it takes pairs from
         unsigned free = ~0u, light = 0, full = 0;
         bool more = half > 0, take_full = false;   // a row of one pixel has no window (absorption.cpp:249-279)
         for (;;) {
