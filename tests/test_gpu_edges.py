@@ -205,3 +205,26 @@ def test_walks_of_all_sample_counts(oracle, group, nbins, hfrac, kernel):
         N.set_group_size(16)
     assert np.max(ref) > 0
     assert_tau_close(got, ref, "sub-sample counts")
+
+
+# supports that cross the box on either side of either axis, narrower than a
+# cell, as wide as the box and wider; positions on its edges, outside it, far
+# outside it and no numbers
+@pytest.mark.parametrize("nlos", [1, 5, 40, 900])
+@pytest.mark.parametrize("hfrac", [1e-4, 0.02, 0.3, 0.7, 3.0])
+def test_windows_of_cells(oracle, nlos, hfrac):
+    box = 1000.0
+    args = small_gas(300, box, nlos, 8, 1, hfrac)
+    pos, h, axis, cofm = args[11], args[15], args[16], args[17]
+    edge = np.array([0.0, 0.3, np.nextafter(np.float32(box), np.float32(0)), 999.7, 500.0], dtype=np.float32)
+    pos[:125] = np.stack(np.meshgrid(edge, edge, edge), -1).reshape(-1, 3)
+    cofm[: nlos // 2] = np.where(cofm[: nlos // 2] < 500.0, 0.01 * cofm[: nlos // 2], 1000.0 - 0.01 * (1000.0 - cofm[: nlos // 2]))
+    pos[130] = [-3.0, 1001.0, 500.0]
+    pos[131] = [-2000.5, 0.1, 4000.5]
+    pos[132] = [1e20, -1e20, 5.0]
+    pos[133] = [np.nan, 10.0, 20.0]
+    _, parts, _ = oracle.near_particles(box, pos, h, axis, cofm)
+    assert np.array_equal(SP._near_lines(box, pos, h, axis, cofm), np.unique(parts))
+    plan = SP.Plan(box, dev(pos), dev(h), dev(axis), dev(cofm))
+    assert plan.npairs == len(parts)
+    plan.close()
