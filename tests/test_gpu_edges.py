@@ -228,3 +228,24 @@ def test_windows_of_cells(oracle, nlos, hfrac):
     plan = SP.Plan(box, dev(pos), dev(h), dev(axis), dev(cofm))
     assert plan.npairs == len(parts)
     plan.close()
+
+
+# grids of one block: fewer sightlines than its threads, as many, more; cells
+# up to its limit (8192: 90 x 90 on one axis) and beyond; a sightline at
+# infinity
+@pytest.mark.parametrize("nlos,axes", [(1, 1), (2, 3), (1023, 3), (1025, 1), (4099, 3), (8100, 1), (8101, 1), (8400, 3)])
+def test_grid_of_one_block(oracle, nlos, axes):
+    box = 1000.0
+    args = small_gas(200, box, nlos, 8, 1, 0.02)
+    pos, h, axis, cofm = args[11], args[15], args[16], args[17]
+    axis[:] = 1 + np.arange(nlos) % axes
+    if nlos > 1000:
+        cofm[17] = np.inf
+        cofm[18, :] = cofm[19, :]
+        cofm[20, :] = 0.0
+        cofm[21, :] = box
+    off, parts, _ = oracle.near_particles(box, pos, h, axis, cofm)
+    plan = SP.Plan(box, dev(pos), dev(h), dev(axis), dev(cofm))
+    got_off, got_parts = plan.pairs()
+    assert np.array_equal(got_off.cpu().numpy(), off) and np.array_equal(got_parts.cpu().numpy(), parts)
+    plan.close()
