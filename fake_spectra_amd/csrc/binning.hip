@@ -359,6 +359,27 @@ __global__ __launch_bounds__(kGridThreads) void grid_small_kernel(const int *axi
     }
 }
 
+// The plan's copies of few sightlines and their number on each axis, by one
+// block (2 us for 64) in place of two copies, a memset and los_axis_count_kernel,
+// 4 to 5 us each to the host.
+constexpr int kIntakeMax = kGridSmallCells;
+
+__global__ __launch_bounds__(kGridThreads) void los_intake_kernel(const int *axis, const double *cofm, int nlos,
+                                                                  int *axis_out, double *cofm_out, int *counts3)
+{
+    __shared__ int c[3];
+    if (threadIdx.x < 3) c[threadIdx.x] = 0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < nlos; i += kGridThreads) {
+        const int a = axis[i];
+        axis_out[i] = a;
+        if (a >= 1 && a <= 3) atomicAdd(&c[a - 1], 1);
+    }
+    for (int i = threadIdx.x; i < 3 * nlos; i += kGridThreads) cofm_out[i] = cofm[i];
+    __syncthreads();
+    if (threadIdx.x < 3) counts3[threadIdx.x] = c[threadIdx.x];
+}
+
 __global__ void los_cell_kernel(const int *axis, const double *cofm, int nlos, double box, LosGrid g,
                                 int *cell_of, int *cell_count)
 {
@@ -1284,20 +1305,22 @@ static int grid_build(fsamd_plan *P, double box, const int *axis, const double *
     P->nlos = nlos;
     if ((rc = P->axis.alloc(sizeof(int) * (size_t)nlos, P->arena))) return rc;
     if ((rc = P->cofm.alloc(sizeof(double) * 3 * (size_t)nlos, P->arena))) return rc;
-    if (nlos > 0) {
-        FSAMD_HIP(hipMemcpyAsync(P->axis.ptr, axis, sizeof(int) * nlos, hipMemcpyDeviceToDevice, s));
-        FSAMD_HIP(hipMemcpyAsync(P->cofm.ptr, cofm, sizeof(double) * 3 * nlos, hipMemcpyDeviceToDevice, s));
-    }
-    // --- sightline grid
     DevBuf counts3;
     if ((rc = counts3.alloc(sizeof(int) * 4, P->arena))) return rc;
-    FSAMD_HIP(hipMemsetAsync(counts3.ptr, 0, sizeof(int) * 4, s));
-    if (nlos > 0) {
+    if (nlos <= kIntakeMax) {
+        los_intake_kernel<<<1, kGridThreads, 0, s>>>(axis, cofm, nlos, P->axis.as<int>(), P->cofm.as<double>(),
+                                                     counts3.as<int>());
+        FSAMD_HIP(hipGetLastError());
+    } else {
+        FSAMD_HIP(hipMemcpyAsync(P->axis.ptr, axis, sizeof(int) * nlos, hipMemcpyDeviceToDevice, s));
+        FSAMD_HIP(hipMemcpyAsync(P->cofm.ptr, cofm, sizeof(double) * 3 * nlos, hipMemcpyDeviceToDevice, s));
+        FSAMD_HIP(hipMemsetAsync(counts3.ptr, 0, sizeof(int) * 4, s));
         los_axis_count_kernel<<<std::min((nlos + 255) / 256, kAxisBlocks), 256, 0, s>>>(P->axis.as<int>(), nlos, counts3.as<int>());
         FSAMD_HIP(hipGetLastError());
     }
+    // --- sightline grid
     int hc[4] = {0, 0, 0, 0};
-    FSAMD_HIP(hipMemcpyAsync(hc, counts3.ptr, sizeof(int) * 4, hipMemcpyDeviceToHost, s));
+    FSAMD_HIP(hipMemcpyAsync(hc, counts3.ptr, sizeof(int) * 3, hipMemcpyDeviceToHost, s));
     FSAMD_HIP(hipStreamSynchronize(s));
     LosGrid &g = P->grid;
     int ncells = 0;
@@ -1450,9 +1473,6 @@ int plan_build(fsamd_plan *P, double box, const float *pos, const float *h, long
             return off[a + 1] - off[a] > off[b + 1] - off[b];
         });
     }
-    if ((rc = P->order.alloc(sizeof(int) * (size_t)std::max(nlos, 1), P->arena))) return rc;
-    if (nlos > 0)
-        FSAMD_HIP(hipMemcpy(P->order.ptr, order.data(), sizeof(int) * nlos, hipMemcpyHostToDevice));
     P->order_host = std::move(order);
     P->off_host = std::move(off);
     return FSAMD_OK;

@@ -89,10 +89,9 @@ struct fsamd_plan {
     fsamd::DevBuf poff;                   // [npart+1] particle-major pair offsets
     fsamd::DevBuf line_off;               // [nlos+1]
     fsamd::DevBuf pair_part;              // [npairs]
-    fsamd::DevBuf order;                  // sightlines by descending pair count
     fsamd::DevBuf seg;                    // [npairs] float2 Voronoi segment ends (kernel 2)
     bool seg_ready = false;
-    std::vector<int> order_host;
+    std::vector<int> order_host;          // sightlines by descending pair count
     std::vector<long long> off_host;
     // Deposit launch state, reused across calls so that a call allocates,
     // copies and synchronizes nothing once warm (and can be graph-captured).
@@ -147,7 +146,7 @@ struct fsamd_plan {
         if (d != cur) (void)hipSetDevice(d);
         (void)hipDeviceSynchronize();
         for (fsamd::DevBuf *b : {&axis, &cofm, &cell_start, &cell_ids, &cell_kl, &poff, &line_off, &pair_part,
-                                 &order, &seg, &queue, &eager_lines.buf, &stats, &rec, &fix, &fix_count, &win})
+                                 &seg, &queue, &eager_lines.buf, &stats, &rec, &fix, &fix_count, &win})
             b->recycle();
         for (auto &it : item_sets) it->buf.recycle();
         for (auto &t : pinned_lines) t->buf.recycle();
