@@ -155,11 +155,18 @@ __global__ void scan_reduce_kernel(const T *in, long long n, long long *sums)
     if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
 
-// out[i] = tile_off[tile] + exclusive prefix within the tile; out may alias in
-template <typename T>
+// out[i] = the tile's offset + exclusive prefix within the tile; out may alias
+// in.  kSums: tile_off holds the tiles' sums as scan_reduce_kernel left them, at
+// most kScanThreads of them, which each block adds up itself.  kEnd: out[n] = total.
+template <typename T, bool kSums, bool kEnd>
 __global__ void scan_apply_kernel(const T *in, long long *out, long long n, const long long *tile_off)
 {
     __shared__ long long lds4[kScanThreads / 64];
+    long long first = 0;
+    if (kSums)
+        block_excl_scan(threadIdx.x < blockIdx.x ? tile_off[threadIdx.x] : 0, lds4, &first);
+    else if (tile_off)
+        first = tile_off[blockIdx.x];
     const long long base = (long long)blockIdx.x * kScanTile + (long long)threadIdx.x * kScanItems;
     long long v[kScanItems];
     long long s = 0;
@@ -169,12 +176,13 @@ __global__ void scan_apply_kernel(const T *in, long long *out, long long n, cons
         s += v[i];
     }
     long long tot;
-    long long off = block_excl_scan(s, lds4, &tot) + (tile_off ? tile_off[blockIdx.x] : 0);
+    long long off = block_excl_scan(s, lds4, &tot) + first;
 #pragma unroll
     for (int i = 0; i < kScanItems; ++i) {
         if (base + i < n) out[base + i] = off;
         off += v[i];
     }
+    if (kEnd && base < n && base + kScanItems >= n) out[n] = off;
 }
 
 size_t exclusive_scan_ws_bytes(long long n)
@@ -196,7 +204,7 @@ static int scan_i64_rec(long long *data, long long n, char *ws, size_t ws_bytes,
     if (n <= 0) return FSAMD_OK;
     long long nt = (n + kScanTile - 1) / kScanTile;
     if (nt == 1) {
-        scan_apply_kernel<long long><<<1, kScanThreads, 0, s>>>(data, data, n, nullptr);
+        scan_apply_kernel<long long, false, false><<<1, kScanThreads, 0, s>>>(data, data, n, nullptr);
         FSAMD_HIP(hipGetLastError());
         return FSAMD_OK;
     }
@@ -205,9 +213,14 @@ static int scan_i64_rec(long long *data, long long n, char *ws, size_t ws_bytes,
     long long *sums = (long long *)ws;
     scan_reduce_kernel<long long><<<(int)nt, kScanThreads, 0, s>>>(data, n, sums);
     FSAMD_HIP(hipGetLastError());
+    if (nt <= kScanThreads) {
+        scan_apply_kernel<long long, true, false><<<(int)nt, kScanThreads, 0, s>>>(data, data, n, sums);
+        FSAMD_HIP(hipGetLastError());
+        return FSAMD_OK;
+    }
     int rc = scan_i64_rec(sums, nt, ws + need, ws_bytes - need, s);
     if (rc) return rc;
-    scan_apply_kernel<long long><<<(int)nt, kScanThreads, 0, s>>>(data, data, n, sums);
+    scan_apply_kernel<long long, false, false><<<(int)nt, kScanThreads, 0, s>>>(data, data, n, sums);
     FSAMD_HIP(hipGetLastError());
     return FSAMD_OK;
 }
@@ -229,15 +242,21 @@ int exclusive_scan_i32_to_i64(const int *in, long long *out, long long n, void *
     size_t need = sizeof(long long) * (size_t)(nt + 1);
     if (need > ws_bytes) return fail(FSAMD_ERR_ARG, "scan workspace too small");
     long long *sums = (long long *)ws;
-    scan_reduce_kernel<int><<<(int)nt, kScanThreads, 0, s>>>(in, n, sums);
+    if (nt > 1) {
+        scan_reduce_kernel<int><<<(int)nt, kScanThreads, 0, s>>>(in, n, sums);
+        FSAMD_HIP(hipGetLastError());
+    }
+    // up to 256 tiles (half a million entries): no scan of the sums between, two
+    // launches in place of three, a memset and a copy (4 to 5 us each to the host)
+    if (nt == 1) {
+        scan_apply_kernel<int, false, true><<<1, kScanThreads, 0, s>>>(in, out, n, nullptr);
+    } else if (nt <= kScanThreads) {
+        scan_apply_kernel<int, true, true><<<(int)nt, kScanThreads, 0, s>>>(in, out, n, sums);
+    } else {
+        if (int rc = scan_i64_rec(sums, nt, (char *)ws + need, ws_bytes - need, s)) return rc;
+        scan_apply_kernel<int, false, true><<<(int)nt, kScanThreads, 0, s>>>(in, out, n, sums);
+    }
     FSAMD_HIP(hipGetLastError());
-    // sums[nt] := 0 so that after the scan sums[nt] holds the grand total
-    FSAMD_HIP(hipMemsetAsync(sums + nt, 0, sizeof(long long), s));
-    int rc = scan_i64_rec(sums, nt + 1, (char *)ws + need, ws_bytes - need, s);
-    if (rc) return rc;
-    scan_apply_kernel<int><<<(int)nt, kScanThreads, 0, s>>>(in, out, n, sums);
-    FSAMD_HIP(hipGetLastError());
-    FSAMD_HIP(hipMemcpyAsync(out + n, sums + nt, sizeof(long long), hipMemcpyDeviceToDevice, s));
     return FSAMD_OK;
 }
 

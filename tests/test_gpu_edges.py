@@ -249,3 +249,21 @@ def test_grid_of_one_block(oracle, nlos, axes):
     got_off, got_parts = plan.pairs()
     assert np.array_equal(got_off.cpu().numpy(), off) and np.array_equal(got_parts.cpu().numpy(), parts)
     plan.close()
+
+
+# offsets of one scan tile of 2048 entries, of several, of the 256 whose
+# sums a block adds up itself, and of more; ends on and next to a tile's
+@pytest.mark.parametrize("n", [1, 255, 2047, 2048, 2049, 524287, 524288, 524289, 1300000])
+def test_offsets_of_all_scan_sizes(n):
+    """One sightline that every second particle reaches: the neighbour list is
+    those particles in order."""
+    rng = np.random.default_rng(n)
+    pos = (rng.random((n, 3)) * 1000.0).astype(np.float32)
+    pos[:, 1:] = 500.0
+    pos[1::2, 2] = 900.0
+    h = np.full(n, 2.0, dtype=np.float32)
+    plan = SP.Plan(1000.0, dev(pos), dev(h), dev(np.ones(1, dtype=np.int32)), dev(np.array([[0.0, 500.5, 500.5]])))
+    off, parts = plan.pairs()
+    want = np.arange(0, n, 2)
+    assert off.cpu().tolist() == [0, want.size] and np.array_equal(parts.cpu().numpy(), want)
+    plan.close()
