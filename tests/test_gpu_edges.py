@@ -267,3 +267,22 @@ def test_offsets_of_all_scan_sizes(n):
     want = np.arange(0, n, 2)
     assert off.cpu().tolist() == [0, want.size] and np.array_equal(parts.cpu().numpy(), want)
     plan.close()
+
+
+# pairs of less than a sort tile (4096), one, one more, several and remainders;
+# sightline ids of 1 to 17 bits, in one to three passes
+@pytest.mark.parametrize("n,nlos", [(1, 1), (5, 2), (63, 65), (64, 64), (17, 241), (128, 64), (300, 257), (1, 4096), (1, 4097),
+                                    (3, 70001), (2, 131072)])
+def test_sorted_pairs_of_all_sizes(n, nlos):
+    """Every particle reaches every sightline: each row holds all of them in
+    order."""
+    rng = np.random.default_rng(n)
+    pos = (500.0 + rng.random((n, 3))).astype(np.float32)
+    cofm = 500.0 + rng.random((nlos, 3))
+    h = np.full(n, 300.0, dtype=np.float32)
+    axis = (1 + np.arange(nlos) % 3).astype(np.int32)
+    plan = SP.Plan(1000.0, dev(pos), dev(h), dev(axis), dev(cofm))
+    off, parts = plan.pairs()
+    assert np.array_equal(off.cpu().numpy(), n * np.arange(nlos + 1))
+    assert np.array_equal(parts.cpu().numpy(), np.tile(np.arange(n), nlos))
+    plan.close()
