@@ -501,6 +501,10 @@ __device__ inline bool cell_window(double x, double hr, double inv, int nc, int 
     return true;
 }
 
+// Supports that reach no sightline: no number, or infinite (los_accept, like the
+// reference's windows, is empty or undefined for them).
+__device__ inline bool finite_support(float hh) { return fabs((double)hh) < 1e300; }
+
 // Visit every sightline accepted for particle p; f(sightline, dr2) returns
 // false to stop the visit early.
 //
@@ -513,8 +517,8 @@ __device__ inline bool cell_window(double x, double hr, double inv, int nc, int 
 template <class F>
 __device__ inline void visit_accepted(const BinArgs &A, const float *p, float hh, F &&f)
 {
+    if (!finite_support(hh)) return;
     const double ah = fabs((double)hh);
-    if (!(ah < 1e300)) return;  // NaN / inf support: the reference's windows are empty or undefined
     for (int ai = 0; ai < 3; ++ai) {
         if (A.grid.nlos_axis[ai] == 0) continue;
         const int ax = ai + 1;
@@ -580,6 +584,7 @@ __global__ void bin_emit_kernel(BinArgs A, const long long *poff, int *keys, int
 // point of the plane accepts it, on any axis.
 __device__ inline bool own_cell_accepts(const BinArgs &A, const float *p, float hh)
 {
+    if (!finite_support(hh)) return false;
     for (int ai = 0; ai < 3; ++ai) {
         if (A.grid.nlos_axis[ai] == 0) continue;
         float first, second;
