@@ -673,70 +673,80 @@ static_assert(kRecs == 32, "the record masks are 32-bit");
 constexpr int kRefillRoom = 24;
 
 // The far-wing coefficients of wing_setup for one pair, all ten on one lane
-// (the batched set-up of the main kernel), in FP32: every term is positive,
-// so the coefficients keep ~4e-7 of the FP64 values and the far-wing sum
-// ~4e-7 (checked against the FP64 computation over sub-sample counts 1..255,
-// kernel extents 0..30 b and a <= 0.04).  c0 = vhigh/b and h = half the
-// pixel width over b, both in units of ufar; W the kernel weights at offsets
-// 0, 1/4, 1/2, 3/4 of vhigh; m1 = sub-samples - 1 (at most FSAMD_WING_TMAX).
+// (the batched set-up), with
+//   C_n = a/(sqrt(pi) ufar^2) sum_(k<=n) (p_k - a^2 q_(k-1)) ufar^(-2k) C(2n+1, 2(n-k)) m_(n-k):
+// every term is positive and the powers of 1/ufar that underflow for wide
+// supports (FP32: k > 4 at 1e4 Doppler widths) are those of negligible terms.  With
+// a/(sqrt(pi)) ufar^(-2n-2) taken first FP32 lost whole coefficients from ufar = 150
+// on: tau was off by 5e-5 at supports of 3000 b, the temperature response of the far
+// wing by 1.4e-5 at 300 b and 1.1e-4 at 1000 b (now 2e-7; the series' own truncation
+// is 7e-7 at |U| = ufar).  c0 = vhigh/b and h = half the pixel
+// width over b, both in units of ufar; W the kernel weights at offsets 0, 1/4, 1/2,
+// 3/4 of vhigh; m1 = sub-samples - 1 (at most FSAMD_WING_TMAX).  Real: float for
+// the optical depth, double for the adjoint (2.1M particles, 1024 sightlines, forward
+// and adjoint 15.1 -> 15.5 ms).
 // kAdj: CwT receives the coefficients of the sum of W (H + u dH/du + a dH/da),
 // from that operator on the term a p_k u^(-2k-2) - a^3 q_(k-1) u^(-2k-2); its
 // leading one is zero.
-template <bool kAdj>
-__device__ __noinline__ void wing_coeffs(float c0, float h, int m1, float W0, float W1, float W2, float W3, float a,
-                                         float ufar, float *Cw, float *CwT)
+template <typename Real, bool kAdj>
+__device__ __noinline__ void wing_coeffs(Real c0, Real h, int m1, float W0, float W1, float W2, float W3, Real a,
+                                         Real ufar, float *Cw, float *CwT)
 {
-    float Y[kWingTerms];
+    Real Y[kWingTerms];
     if (m1 == 0) {
-        Y[0] = 1.0f;
+        Y[0] = 1;
 #pragma unroll
-        for (int n = 1; n < kWingTerms; ++n) Y[n] = 0.0f;
+        for (int n = 1; n < kWingTerms; ++n) Y[n] = 0;
     } else {
-        const float h2 = h * h;
-        float pw = 1.0f;
+        const Real h2 = h * h;
+        Real pw = 1;
 #pragma unroll
         for (int n = 0; n < kWingTerms; ++n) {
-            Y[n] = pw * (float)c_wing_T[m1 * kWingTerms + n];
+            Y[n] = pw * (Real)c_wing_T[m1 * kWingTerms + n];
             pw *= h2;
         }
     }
     // kernel samples at +-(c0/4, c0/2, 3c0/4) and 0
-    const float x1 = 0.0625f * c0 * c0, x2 = 0.25f * c0 * c0, x3 = 0.5625f * c0 * c0;
-    const float w1 = 2.0f * W1, w2 = 2.0f * W2, w3 = 2.0f * W3;
-    float X[kWingTerms];
-    float p1 = 1.0f, p2 = 1.0f, p3 = 1.0f;
+    const Real x1 = (Real)0.0625 * c0 * c0, x2 = (Real)0.25 * c0 * c0, x3 = (Real)0.5625 * c0 * c0;
+    const Real w1 = 2 * (Real)W1, w2 = 2 * (Real)W2, w3 = 2 * (Real)W3;
+    Real X[kWingTerms];
+    Real p1 = 1, p2 = 1, p3 = 1;
 #pragma unroll
     for (int k = 0; k < kWingTerms; ++k) {
-        X[k] = w1 * p1 + w2 * p2 + w3 * p3 + (k == 0 ? W0 : 0.0f);
+        X[k] = fma(w1, p1, fma(w2, p2, k == 0 ? fma(w3, p3, (Real)W0) : w3 * p3));
         p1 *= x1;
         p2 *= x2;
         p3 *= x3;
     }
-    float m[kWingTerms];
+    Real m[kWingTerms];
 #pragma unroll
     for (int n = 0; n < kWingTerms; ++n) {
-        float t = 0.0f;
+        Real t = 0;
 #pragma unroll
-        for (int k = 0; k <= n; ++k) t += (float)c_binom_even[n * kWingTerms + k] * X[k] * Y[n - k];
+        for (int k = 0; k <= n; ++k) t = fma((Real)c_binom_even[n * kWingTerms + k] * X[k], Y[n - k], t);
         m[n] = t;
     }
-    const float iu = 1.0f / ufar, iu2 = iu * iu, u2 = ufar * ufar, a2 = a * a;
-    float lead = a * kInvSqrtPiF * iu2;   // a/sqrt(pi) ufar^(-2n-2) at n = 0
+    const Real iu = 1 / ufar, iu2 = iu * iu, a2 = a * a, lead = a * (Real)(1.0 / kSqrtPi) * iu2;
+    Real g[kWingTerms], gT[kWingTerms];
+    Real pw = 1;   // ufar^(-2k)
+#pragma unroll
+    for (int k = 0; k < kWingTerms; ++k) {
+        const Real pk = (Real)c_wing_p[k], qk = k > 0 ? (Real)c_wing_q[k - 1] : 0;
+        g[k] = pw * (pk - a2 * qk);
+        if (kAdj) gT[k] = pw * ((2 * k - 2) * a2 * qk - 2 * k * pk);
+        pw *= iu2;
+    }
 #pragma unroll
     for (int n = 0; n < kWingTerms; ++n) {
-        float cn = 0.0f, cf = 0.0f, gs = lead;
+        Real cn = 0, cT = 0;
 #pragma unroll
         for (int j = 0; j <= n; ++j) {
-            if (j > 0) gs *= u2;
-            const int k = n - j;
-            const float qk = k > 0 ? (float)c_wing_q[k - 1] : 0.0f;
-            const float bm = gs * (float)c_binom_odd[n * kWingTerms + j] * m[j];
-            cn += ((float)c_wing_p[k] - a2 * qk) * bm;
-            if (kAdj) cf += ((2.0f * k - 2.0f) * a2 * qk - 2.0f * k * (float)c_wing_p[k]) * bm;
+            const Real bm = (Real)c_binom_odd[n * kWingTerms + j] * m[j];
+            cn = fma(g[n - j], bm, cn);
+            if (kAdj) cT = fma(gT[n - j], bm, cT);
         }
-        Cw[n] = cn;
-        if (kAdj) CwT[n] = cf;
-        lead *= iu2;
+        Cw[n] = (float)(lead * cn);
+        if (kAdj) CwT[n] = (float)(lead * cT);
     }
 }
 
@@ -841,7 +851,7 @@ __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int 
         r.shape = sh.packed();
         // far-wing coefficients, in units of that ufar
         const double iu = 1.0 / (double)ufar;
-        wing_coeffs<false>((float)(C.vhigh * C.inv_b * iu), (float)(0.5 * bintov * C.inv_b * iu), sh.nm1, W[0], W[1],
+        wing_coeffs<float, false>((float)(C.vhigh * C.inv_b * iu), (float)(0.5 * bintov * C.inv_b * iu), sh.nm1, W[0], W[1],
                            W[2], W[3], (float)C.aa, ufar, r.Cw, nullptr);
     }
     wave_sync();
@@ -1490,8 +1500,8 @@ __device__ inline void refill_adjoint(const DepositArgs &A, const WorkItem &w, i
         const float ufar = (float)C.ufar;
         r.ufsq = (float)((us * ufar) * (us * ufar));
         const double iu = 1.0 / (double)ufar;
-        wing_coeffs<true>((float)(C.vhigh * C.inv_b * iu), (float)(0.5 * bintov * C.inv_b * iu), C.np - 1, W[0], W[1],
-                          W[2], W[3], (float)C.aa, ufar, r.Cw, r.CwT);
+        wing_coeffs<double, true>(C.vhigh * C.inv_b * iu, 0.5 * bintov * C.inv_b * iu, C.np - 1, W[0], W[1], W[2], W[3],
+                                  C.aa, (double)ufar, r.Cw, r.CwT);
         // far-wing pixels: those whose centre s0 + (j + 1/2) bxs lies at or beyond +-ufar
         const double c0 = s0 + 0.5 * bxs, inv_x = 1.0 / bxs, uf = us * ufar;
         const double jl = floor((-uf - c0) * inv_x) + 1.0, jr = ceil((uf - c0) * inv_x);

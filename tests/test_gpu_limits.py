@@ -2,11 +2,16 @@
 import numpy as np
 import pytest
 
-from fake_spectra_amd import spectra_priv as SP
+from fake_spectra_amd import spectra_priv as SP, synth
+from fake_spectra_amd.lines import HI_1215
 from gpu_util import dev
 from test_gpu_edges import small_gas
+from torch_reference import BOLTZMANN, LIGHT, PROTONMASS, SIGMA_T, kernel_weight
 
 pytestmark = pytest.mark.gpu
+
+VELFAC = synth.Cosmology().velfac()
+
 
 # sightlines in nearly all cells of the search grid, in some, in one
 @pytest.mark.parametrize("nlos", [1, 30, 700])
@@ -24,3 +29,90 @@ def test_near_lines_of_supports_that_are_no_numbers(oracle, nlos):
     assert np.array_equal(plan.near_lines().cpu().numpy(), want)
     assert np.array_equal(SP._near_lines(box, pos, h, axis, cofm), want)
     plan.close()
+
+
+class LoneParticle:
+    """One particle on one sightline in a box of twelve of its supports, a
+    support of `support` Doppler widths (b = 10 km/s) and a damping parameter
+    a; the density is so high that no pixel of the row ends a window."""
+
+    def __init__(self, support, kernel, a):
+        px = min(20.0, support / 50.0)                       # pixel in Doppler widths
+        self.nbins, self.kernel = 2 * int(6 * support / px), kernel
+        b0 = 10.0
+        box = 12.0 * support * b0 / VELFAC
+        pos = np.full((1, 3), 0.5 * box, dtype=np.float32)
+        self.h = np.array([support * b0 / VELFAC], dtype=np.float32)
+        cofm = np.array([[0.0, 0.5 * box + 0.2 * support * b0 / VELFAC, 0.5 * box]])
+        temp = np.array([1e4 * (b0 / 12.85) ** 2], dtype=np.float32)
+        gamma = a * b0 * 4 * np.pi * 1e5 / HI_1215.lambda_cm
+        self.line = (HI_1215.lambda_cm, gamma, HI_1215.fosc, HI_1215.amumass)
+        self.box, self.pos, self.cofm, self.temp = box, pos, cofm, temp
+        self.dens = np.array([1e30], dtype=np.float32)
+        self.plan = SP.Plan(box, dev(pos), dev(self.h), dev(np.array([1], dtype=np.int32)), dev(cofm))
+        self.args = (self.nbins, kernel, VELFAC, dev(np.zeros((1, 3), dtype=np.float32)), dev(temp), [self.line],
+                     [dev(self.dens)])
+        # pixel centres from the particle, in supports
+        self.at = ((np.arange(self.nbins) + 0.5) * box / self.nbins - float(pos[0, 0])) / float(self.h[0])
+
+    def far_gradients(self, weights):
+        """dL/d dens, dL/dT and dL/d vel of L = sum(weights tau) over pixels of the far
+        wing, in FP64: with w(z) = i/sqrt(pi) sum_n c_n z^(-2n-1), z = u + ia, the sums
+        of H = Re w, dH/du = Re w' and H + u dH/du + a dH/da = Re(w + z w') term by term
+        (the last has lost 1/u^2 of its parts, which no difference of them keeps)."""
+        lam, gamma, fosc, amu = self.line
+        T, dens, h = float(self.temp[0]), float(self.dens[0]), float(self.h[0])
+        b = np.sqrt(2 * BOLTZMANN / (amu * PROTONMASS)) / 1e5 * np.sqrt(T)
+        a = gamma * lam / (4 * np.pi) / 1e5 / b
+        amp = np.sqrt(3 * np.pi * SIGMA_T / 8) * lam * fosc / np.sqrt(np.pi) * (LIGHT / 1e5 / b)
+        d2 = (float(self.pos[0, 1]) - self.cofm[0, 1]) ** 2 + (float(self.pos[0, 2]) - self.cofm[0, 2]) ** 2
+        vh = VELFAC * np.sqrt(h * h - d2)
+        dvk = vh / 4
+        vv = np.arange(1, 8) * dvk - vh
+        W = kernel_weight(self.kernel, np.sqrt(VELFAC ** 2 * d2 + vv * vv) / (VELFAC * h))
+        width = self.box * VELFAC / self.nbins
+        npts = 1 if width < b / 2 else int(2 * np.ceil(width / b) + 1)
+        off = np.array([0.5]) if npts == 1 else np.arange(npts) / (npts - 1)
+        t = np.ones(npts)
+        if npts > 1:
+            t[[0, -1]] = 0.5
+            t /= npts - 1
+        S = np.zeros(3)
+        for z in np.nonzero(weights)[0]:
+            v = (z + off) * width - VELFAC * float(self.pos[0, 0])
+            zz = (vv[:, None] - v[None, :]) / b + 1j * a
+            term, c, s = 1 / zz, 1.0, np.zeros((3,) + zz.shape, dtype=complex)
+            for n in range(12):
+                s[0] += c * term
+                s[1] += -2 * n * c * term
+                s[2] += -(2 * n + 1) * c * term / zz
+                term, c = term / (zz * zz), c * (n + 0.5)
+            S += weights[z] * np.einsum("i,j,kij->k", W, t, (1j / np.sqrt(np.pi) * s).real)
+        scale = amp * dvk / VELFAC
+        return S[0] * scale, -S[1] * scale * dens / (2 * T), S[2] * scale * dens / b
+
+    def check(self):
+        """tau everywhere (FP64 path) and the gradients of a side of the far wing
+        alone, to the stated tolerance of tau."""
+        self.plan.keep_windows(True)
+        tau = SP.tau(self.plan, *self.args)[0].cpu().numpy()
+        # the expansion begins near 2.25; the row's last pixel may be the other walk's, one box length off
+        w = np.where((self.at > 2.4) & (self.at < 5.9), 1.0 + 0.3 * np.sin(7.0 * self.at), 0.0)
+        got = SP.tau_adjoint(self.plan, *self.args, [dev(w[None])])
+        SP.set_fp64(True)
+        try:
+            want = SP.tau(self.plan, *self.args)[0].cpu().numpy()
+        finally:
+            SP.set_fp64(False)
+        assert np.all(want > 0) and np.max(np.abs(tau - want) / want) <= 1e-5
+        for name, x, y in zip(("dens", "T", "vel"), (got[0][0][0], got[1][0], got[2][0, 0]), self.far_gradients(w)):
+            assert abs(float(x) - y) <= 1e-5 * abs(y), name
+        self.plan.close()
+
+
+# supports at which powers of the far wing's distance leave the range of FP32
+# numbers one after the other; weights flat and falling
+@pytest.mark.parametrize("kernel", [0, 1])
+@pytest.mark.parametrize("support", [10, 30, 100, 300, 1000, 3000])
+def test_far_wing_of_wide_supports(support, kernel):
+    LoneParticle(support, kernel, 1e-2).check()
