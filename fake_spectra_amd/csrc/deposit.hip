@@ -1476,7 +1476,8 @@ __device__ inline void refill_adjoint(const DepositArgs &A, const WorkItem &w, i
     wave_sync();   // the records' former pairs have been read
     if (enq) {
         AdjRec &r = recs[slot];
-        const VoigtP vp = make_voigt_p(C.aa, C.aa <= (double)kA3Drop);
+        VoigtP vp = make_voigt_p(C.aa, C.aa <= (double)kA3Drop);
+        vp.a3 = (float)(C.aa * C.aa * (-1.0 / 6.0));   // in the short form too (GradSums)
         r.vp = vp;
         const double us = voigt_uscale(vp, C.aa), ibs = us * C.inv_b;
         const double inv_m = C.np > 1 ? 1.0 / (C.np - 1) : 1.0;
@@ -1517,15 +1518,15 @@ __device__ inline void refill_adjoint(const DepositArgs &A, const WorkItem &w, i
     }
     wave_sync();
     const unsigned mine = (unsigned)__ballot(used);
-    const unsigned a3 = (unsigned)__ballot(used && recs[lane & 31].vp.a3 != 0.0f);
+    const unsigned fulls = (unsigned)__ballot(used && recs[lane & 31].vp.l2 != 0.0f);
     free &= ~mine;
-    light |= mine & ~a3;
-    full |= a3;
+    light |= mine & ~fulls;
+    full |= fulls;
     more = (long long)base + want < w.p1;
 }
 
 // One grid point of a pair: the sums (GradSums) of the kernel samples around s.
-template <bool kA3>
+template <bool kFull>
 __device__ inline void adj_point(const AdjRec &P, double s, const float *tab, float &S, float &SU, float &ST,
                                  float &SP)
 {
@@ -1536,20 +1537,21 @@ __device__ inline void adj_point(const AdjRec &P, double s, const float *tab, fl
     const float W[4] = {w4.x, w4.y, w4.z, w4.w};
     GradSums g;
 #pragma unroll
-    for (int j = -3; j <= 3; ++j) g.add<kA3>(vp, a2, W[j < 0 ? -j : j], sample_us(qs, j, s), tab);
+    for (int j = -3; j <= 3; ++j) g.add<kFull>(vp, a2, W[j < 0 ? -j : j], sample_us(qs, j, s), tab);
     g.finish(vp, a2, S, SU, ST, SP);
 }
 
-// Bound: VALU issue (24 instructions a sample in the light form).  Structured as
+// Bound: VALU issue (32 instructions a sample in the short form).  Structured as
 // tau_kernel: pairs set up one per lane into records, walked in place by lane
-// groups, light and full pairs in runs, far-wing pixels by the whole wavefront.
+// groups, pairs of the short and of the full form in runs, far-wing pixels by the
+// whole wavefront.
 // Here the windows are known: a group walks the grid points of its pair's near
 // pixels, each once, weighted by the trapezoid weights and dL/dtau of the
 // pixels it belongs to.  One block of 16 wavefronts a CU shares the table of G
 // and K (32 KB) and the row.  kRow: the row of dL/dtau in LDS; a row that does
 // not fit beside the records (above about 3000 pixels) is read where it is.
-// 2M particles, 1024 sightlines of 1024 pixels: 18.6 -> 8.7 ms; 32768 particles
-// and 50 sightlines, forward and adjoint: 1.2 -> 0.9 ms.
+// 2.1M particles, 1024 sightlines of 1024 pixels, forward and adjoint: 37.9 -> 15.9
+// ms.
 template <int kG, bool kRow>
 __global__ __launch_bounds__(kAdjThreads) __attribute__((amdgpu_waves_per_eu(4))) void tau_adjoint_kernel(
     DepositArgs A, const WorkItem *items)
@@ -1622,7 +1624,7 @@ __global__ __launch_bounds__(kAdjThreads) __attribute__((amdgpu_waves_per_eu(4))
             const AdjRec &P = recs[rec];
             const int nm1 = P.nm1;
             const int npts = state != 1 || P.nn == 0 ? 0 : nm1 == 0 ? P.nn : P.nn * nm1 + 1;
-            const bool a3 = __ballot(state == 1 && P.vp.a3 != 0.0f) != 0ull;
+            const bool any_full = __ballot(state == 1 && P.vp.l2 != 0.0f) != 0ull;
             const int m = c + glane;
             if (m < npts) {
                 // grid point m: sub-sample kk of near pixel jj (singleabs.h:110-125)
@@ -1634,7 +1636,7 @@ __global__ __launch_bounds__(kAdjThreads) __attribute__((amdgpu_waves_per_eu(4))
                 const double dss = P.dss;
                 const double s = __builtin_fma((double)P.nfl * (nm1 == 0 ? 1 : nm1) + m + (nm1 == 0 ? 0.5 : 0.0), dss, P.s0);
                 float S, SU, ST, SP;
-                if (a3)
+                if (any_full)
                     adj_point<true>(P, s, tab, S, SU, ST, SP);
                 else
                     adj_point<false>(P, s, tab, S, SU, ST, SP);

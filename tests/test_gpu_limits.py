@@ -1,6 +1,7 @@
 """Calls at the ends of what the entry points take."""
 import numpy as np
 import pytest
+import torch
 
 from fake_spectra_amd import spectra_priv as SP, synth
 from fake_spectra_amd.lines import HI_1215
@@ -116,3 +117,52 @@ class LoneParticle:
 @pytest.mark.parametrize("support", [10, 30, 100, 300, 1000, 3000])
 def test_far_wing_of_wide_supports(support, kernel):
     LoneParticle(support, kernel, 1e-2).check()
+
+
+# damping parameters up to where the optical depth drops the a^3 term, and beyond;
+# supports of half a Doppler width and of twenty
+@pytest.mark.parametrize("support,peak", [(0.5, 1e4), (3.0, 1e6), (20.0, 1e6)])
+@pytest.mark.parametrize("a", [4e-4, 1.2e-3, 1.95e-3, 2.5e-3])
+def test_saturated_gradients_keep_the_cubic_term(a, support, peak):
+    """Gradients of sum(exp(-2 tau)) through saturated cores come from |u| = 3 to 5
+    alone, where the a^3 term is up to 5.5e-7 of the profile, or from the wings: FP32
+    against FP64, half of the density's are right to an FP32 unit in the last
+    place, 2^-23, and half of the temperature's, a difference, to the stated 1e-5."""
+    errs = [], []
+    b0, n, nlos = 10.0, 300, 60
+    for seed in range(4):
+        rng = np.random.default_rng(seed)
+        b = np.maximum(b0 * np.exp(0.02 * rng.standard_normal(n)), 0.9 * b0)
+        temp = (1e4 * (b / 12.85) ** 2).astype(np.float32)
+        h0 = support * b0 / VELFAC
+        box = max(20 * h0, 40 * b0 / VELFAC)
+        nbins = int(box * VELFAC / 2.5)
+        pos = (rng.random((n, 3)) * box).astype(np.float32)
+        h = (h0 * np.exp(0.2 * rng.standard_normal(n))).astype(np.float32)
+        vel = (10 * rng.standard_normal((n, 3))).astype(np.float32)
+        axis = (1 + np.arange(nlos) % 3).astype(np.int32)
+        cofm = pos[rng.integers(0, n, nlos)].astype(np.float64) + 0.1 * h0
+        line = (HI_1215.lambda_cm, a * b0 * 4 * np.pi * 1e5 / HI_1215.lambda_cm, HI_1215.fosc, HI_1215.amumass)
+        plan = SP.Plan(box, dev(pos), dev(h), dev(axis), dev(cofm))
+        plan.keep_windows(True)
+        dens = np.exp(20 + 0.3 * rng.standard_normal(n)).astype(np.float32)
+        call = (nbins, 1, VELFAC, dev(vel), dev(temp), [line])
+        top = float(SP.tau(plan, *call, [dev(dens)])[0].max())
+        dens = dev((dens * (peak / top)).astype(np.float32))
+        grads, weights = [], None
+        for fp64 in (True, False):
+            SP.set_fp64(fp64)
+            try:
+                tau = SP.tau(plan, *call, [dens])[0]
+                weights = -2 * torch.exp(-2 * tau) if weights is None else weights
+                gd, gt, _ = SP.tau_adjoint(plan, *call, [dens], [weights])
+            finally:
+                SP.set_fp64(False)
+            grads.append((gd[0].cpu().numpy(), gt.cpu().numpy()))
+        for e, want, got in zip(errs, *grads):
+            m = want != 0
+            e.append(np.abs(got - want)[m] / np.abs(want[m]))
+        plan.close()
+    density, temperature = (np.concatenate(e) for e in errs)
+    assert density.size > 200
+    assert np.median(density) <= 2.0 ** -23 and np.median(temperature) <= 1e-5
