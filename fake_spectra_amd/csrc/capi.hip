@@ -622,7 +622,7 @@ int fsamd_plan_overflow(fsamd_plan *plan, int *flag, void *stream)
     unsigned long long fc[2] = {0, 0};
     FSAMD_HIP(hipMemcpyAsync(fc, plan->fix_count.ptr, sizeof(fc), hipMemcpyDeviceToHost, (hipStream_t)stream));
     FSAMD_HIP(hipStreamSynchronize((hipStream_t)stream));
-    *flag = fc[1] != 0;
+    *flag = (fc[1] & 1) != 0;   // (the second bit is the adjoint's)
     return FSAMD_OK;
 }
 
@@ -783,16 +783,21 @@ int fsamd_tau_adjoint(fsamd_plan *P, int nbins, int kernel, double velfac, const
         if ((rc = launch_fill_i32(A.queue, 0, 1, s))) return rc;
         if ((rc = launch_fill_i32((int *)A.fix_count, 0, 4, s))) return rc;
         const int nblocks = std::min(slots, A.nitems);
-        if ((rc = launch_tau_adjoint(gsize, A, set->buf.as<WorkItem>(), nblocks, s))) return rc;
+        if ((rc = launch_tau_adjoint(gsize, false, A, set->buf.as<WorkItem>(), nblocks, s))) return rc;
         if ((rc = launch_tau_adjoint64(A, set->buf.as<WorkItem>(), dev.ncu * 2, s))) return rc;
         unsigned long long fc[2] = {0, 0};
         FSAMD_HIP(hipMemcpyAsync(fc, A.fix_count, sizeof(fc), hipMemcpyDeviceToHost, s));
         FSAMD_HIP(hipStreamSynchronize(s));
         // the forward listed every FP64 pair of the group in this list, so it
         // holds them unless the FP64 setting changed in between
-        if (fc[1])
+        if (fc[1] & 1)
             return fail(FSAMD_ERR_UNSUPPORTED, "adjoint: more FP64 pairs than the forward's fix-up list holds; "
                                                "run the forward with the same fsamd_set_fp64 setting");
+        if (fc[1] & 2) {
+            if ((rc = launch_fill_i32(A.queue, 0, 1, s))) return rc;
+            if ((rc = launch_tau_adjoint(gsize, true, A, set->buf.as<WorkItem>(), nblocks, s))) return rc;
+            FSAMD_HIP(hipStreamSynchronize(s));
+        }
     }
     return FSAMD_OK;
 }

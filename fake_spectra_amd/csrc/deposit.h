@@ -31,7 +31,8 @@ int deposit_blocks_per_cu(bool tau, bool lds, int gsize, int waves, int nbins, i
 // rows a column-density work item takes of nlines
 int colden_fields(int nlines, int nbins);
 int effective_waves(bool lds, bool stats, int waves);
-int launch_tau_adjoint(int gsize, const DepositArgs &A, const WorkItem *items, int nblocks, hipStream_t s);
+// wide: the pass over the pairs that the other one left out (fix_count[1] & 2)
+int launch_tau_adjoint(int gsize, bool wide, const DepositArgs &A, const WorkItem *items, int nblocks, hipStream_t s);
 // one block of the adjoint kernel fills a CU
 bool adjoint_row_in_lds(int nbins);
 // the FP64 pairs tau_adjoint_kernel listed in A.fix (after it, on the same stream)

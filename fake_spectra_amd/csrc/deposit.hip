@@ -219,7 +219,7 @@ struct PairTau : PairRec {
     double scale_nd; // amp * dvk / velfac (scale without the density)
     double temp;     // particle temperature
     int part;        // particle index
-    int fp64;
+    int fp64, wide;
     int np;          // sub-samples per pixel (1 = midpoint)
     int wing_ready;  // Cw computed
     double inv_nm1;  // 1 / (np - 1)
@@ -269,6 +269,23 @@ __device__ inline float inner32(const PairRec &P, double s, const float *ptab)
     return __builtin_fmaf(-vp.two_a_sqpi, sG, sE);
 }
 
+// The same sum for a pair whose samples may lie beyond the profile's table.
+__device__ inline float inner32_wide(const PairRec &P, double s, const float *ptab)
+{
+    const VoigtP vp = P.vp;
+    const double qs = P.qs;
+    float sE = 0.0f, sG = 0.0f;
+#pragma unroll 1
+    for (int j = -3; j <= 3; ++j) {
+        float E, G;
+        voigt_terms<true, true>(vp, sample_us(qs, j, s), ptab, E, G);
+        const float w = P.W[j < 0 ? -j : j];
+        sE = __builtin_fmaf(w, E, sE);
+        sG = __builtin_fmaf(w, G, sG);
+    }
+    return __builtin_fmaf(-vp.two_a_sqpi, sG, sE);
+}
+
 // One sample of that sum (i = 1 .. kNGrid - 1) with the FP64 profile and FP64
 // kernel weights.
 __device__ inline double sample64(const PairTau &P, double vouter, int kernel, int i, const double *gtab64)
@@ -305,7 +322,10 @@ __device__ inline double taulast_pixel(const PairTau &P, double vlow, double bin
             return P.scale * (double)(S * Y);
         }
     }
-    auto inner = [&](double v) { return k64 ? inner64(P, v, kernel, gtab64) : inner32(P, v * P.ibs, ptab); };
+    auto inner = [&](double v) {
+        return k64 ? inner64(P, v, kernel, gtab64)
+               : (double)(P.wide ? inner32_wide(P, v * P.ibs, ptab) : inner32(P, v * P.ibs, ptab));
+    };
     if (width < P.b / 2.) return P.scale * inner((vhighp + vlow) / 2.);
     const int np = 2 * ceil(width / (P.b / 2.) / 2) + 1.;
     const double dv = width / (np - 1);
@@ -464,6 +484,9 @@ __device__ inline StepShape step_shape(int np, int kg)
     return sh;
 }
 
+// A fix-up entry's dir: the direction of a deferred walk, or a whole pair.
+enum { kFixPair64 = 0, kFixPair = 2 };
+
 // Append a walk to the fix-up list.  The counter is 64-bit, so it cannot wrap
 // within a launch; entries past the capacity only raise the overflow flag.
 __device__ inline void push_fixup(const DepositArgs &A, long long k, int item, int z0, int count, int dir)
@@ -518,13 +541,18 @@ struct LaneStats {
 struct PairConsts {
     double vel, b, inv_b, dvk, vhigh, vdr2, vsmooth, aa, scale, scale_nd, ufar;
     float temp;
-    int zmax, np, fp64;
+    int zmax, np, fp64, wide;
 };
 
 // Pair kk (the particle at pair_part[kk]).  Returns false if the particle does
 // not reach the sightline (absorption.cpp:232; on the Voronoi mesh, if it owns
 // no segment of it, absorption.cpp:221-229).  fp64 routes the pair to the
-// FP64 path.
+// FP64 path.  wide: samples of a near step may lie beyond the profile's table
+// (supports of more than 5700 Doppler widths); such a pair is walked in FP32 by the
+// fix-up kernel, and by a launch of its own in the adjoint: their code in the main
+// kernels costs every call 2.4% (256^3 x 5000 x 2048, two lines, 76.5 -> 78.3 ms) and the
+// adjoint's 8%.  In FP64, the other way out, 43 such particles of 32768 took half of
+// a call (1.05 ms, 0.58 so) and 4700 three quarters (8.3 ms, 3.6 so).
 __device__ inline bool pair_consts(const DepositArgs &A, int line, const LineDesc &L, const LosInfo &los,
                                    long long kk, int max_sums, PairConsts &C)
 {
@@ -580,12 +608,12 @@ __device__ inline bool pair_consts(const DepositArgs &A, int line, const LineDes
     const bool grid_edge = fabs(bintov - b / 2.) <= 1e-12 * bintov || (np > 1 && fabs(xs - rint(xs)) <= 1e-12 * xs);
     const double dmax = (vhigh - dvk) * inv_b + (np > 1 ? 0.5 * bintov * inv_b : 0.0);
     C.ufar = fmax(7.0 + dmax, 3.0 * dmax);
-    // pixels wider than max_sums sub-samples do not fit one walk step; samples
-    // of a near step (up to 4 * 64 sub-samples of half a b past ufar) must lie
-    // within the profile's table, which leaves out only supports of thousands
-    // of Doppler widths
+    // pixels wider than max_sums sub-samples do not fit one walk step; a near step
+    // reaches up to 4 * 64 sub-samples of half a b past ufar
+    const double reach = C.ufar + dmax + 130.0;
+    C.wide = !(reach <= kVoigtUMax);
     C.fp64 = A.force_fp64 || !(aa <= (double)kA32Max) || grid_edge || np - 1 > max_sums - 1 ||
-             !(C.ufar + dmax + 130.0 <= kVoigtUMax);
+             !(reach <= kVoigtUWide);
     C.vel = vel;
     C.b = b;
     C.inv_b = inv_b;
@@ -633,6 +661,7 @@ __device__ inline bool setup_pair(const DepositArgs &A, int line, const LineDesc
         P.aa = C.aa;
         P.zmax = C.zmax;
         P.fp64 = C.fp64;
+        P.wide = C.wide;
         P.vp = make_voigt_p(C.fp64 ? 0.0 : C.aa, C.aa <= (double)kA3Drop);
         P.scale = C.scale;
         P.scale_nd = C.scale_nd;
@@ -789,8 +818,8 @@ __device__ inline int pairs_wanted(long long left, int waves, int groups, int nf
 }
 
 // Claim up to `want` (at most the free records) pairs of item w for the
-// wavefront, set them up one per lane and put those walked in FP32 into free
-// records; FP64 pairs go straight to the fix-up list.  Every lane of the
+// wavefront, set them up one per lane and put those of the main kernel into free
+// records; FP64 and wide pairs go straight to the fix-up list.  Every lane of the
 // wavefront calls it; `more` says whether the item has pairs left.
 template <int kG, bool kStats>
 __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int gitem, const LineDesc &L,
@@ -806,9 +835,9 @@ __device__ inline void refill_wave(const DepositArgs &A, const WorkItem &w, int 
     PairConsts C;
     if (lane < want && kk < w.p1 && pair_consts(A, w.line, L, los, kk, kG * kRoundsMax, C)) {
         if (kStats) st.pairs++;
-        if (C.fp64) {
-            if (kStats) st.pairs64++;
-            push_fixup(A, kk, gitem, C.zmax, A.nbins / 2, 0);
+        if (C.fp64 || C.wide) {
+            if (kStats) st.pairs64 += C.fp64;
+            push_fixup(A, kk, gitem, C.zmax, A.nbins / 2, C.fp64 ? kFixPair64 : kFixPair);
         } else {
             enq = true;
         }
@@ -1340,9 +1369,16 @@ __global__ __launch_bounds__(kThreads) void tau_fixup_kernel(DepositArgs A, cons
         double *out_row = L.out + (size_t)w.los * A.nbins;
         const LosInfo los = los_info(A, w.los);
         if (!setup_pair<kFixG>(A, w.line, L, los, f.k, P, glane)) continue;
-        if (f.dir == 0) {
+        if (f.dir == kFixPair64) {
             const int lf = walk_fix<kFixG, kWalkFull64, kStats>(A, P, out_row, ptab, gtab64, P.zmax, 1, half, lane, st);
             const int lb = walk_fix<kFixG, kWalkFull64, kStats>(A, P, out_row, ptab, gtab64, P.zmax - 1, -1, half, lane, st);
+            if (glane == 0) {
+                record_window(A, w.line, f.k, 1, lf);
+                record_window(A, w.line, f.k, -1, lb);
+            }
+        } else if (f.dir == kFixPair) {
+            const int lf = walk_fix<kFixG, kWalkGuarded, kStats>(A, P, out_row, ptab, gtab64, P.zmax, 1, half, lane, st);
+            const int lb = walk_fix<kFixG, kWalkGuarded, kStats>(A, P, out_row, ptab, gtab64, P.zmax - 1, -1, half, lane, st);
             if (glane == 0) {
                 record_window(A, w.line, f.k, 1, lf);
                 record_window(A, w.line, f.k, -1, lb);
@@ -1448,7 +1484,9 @@ constexpr int kAdjWaves = kAdjThreads / 64;
 
 // Claim `want` pairs for the wavefront and set up those with a window, as
 // refill_wave does for the forward.  FP64 pairs go to the list of
-// tau_adjoint64_kernel.
+// tau_adjoint64_kernel.  kWide: the wide pairs alone; without it they are left out
+// and the second bit of fix_count[1] tells that there are some.
+template <bool kWide>
 __device__ inline void refill_adjoint(const DepositArgs &A, const WorkItem &w, int item, const LineDesc &L,
                                       const LosInfo &los, unsigned long long *next, AdjRec *recs, int lane, int want,
                                       unsigned &free, unsigned &light, unsigned &full, bool &more)
@@ -1458,7 +1496,7 @@ __device__ inline void refill_adjoint(const DepositArgs &A, const WorkItem &w, i
     base = (unsigned long long)__shfl((long long)base, 0, 64);
     const long long kk = (long long)base + lane;
     const double bintov = A.vbox / A.nbins;
-    bool enq = false;
+    bool enq = false, left_out = false;
     int lf = 0, lb = 0;
     PairConsts C;
     if (lane < want && kk < w.p1) {
@@ -1466,10 +1504,12 @@ __device__ inline void refill_adjoint(const DepositArgs &A, const WorkItem &w, i
         lf = A.win[wi];
         lb = A.win[wi + 1];
         if (lf + lb > 0 && pair_consts(A, w.line, L, los, kk, FSAMD_WING_TMAX, C)) {
-            enq = !C.fp64;
-            if (C.fp64) push_fixup(A, kk, item, 0, 0, 0);
+            enq = !C.fp64 && (bool)C.wide == kWide;
+            if (!kWide && C.fp64) push_fixup(A, kk, item, 0, 0, kFixPair64);
+            left_out = !kWide && !C.fp64 && C.wide;
         }
     }
+    if (!kWide && __ballot(left_out) && lane == 0) atomicOr(&A.fix_count[1], 2ull);
     const unsigned long long m = __ballot(enq);
     bool used;
     const int slot = free_record(free, m, lane, used);
@@ -1541,6 +1581,19 @@ __device__ inline void adj_point(const AdjRec &P, double s, const float *tab, fl
     g.finish(vp, a2, S, SU, ST, SP);
 }
 
+// The same for a wide pair.
+__device__ inline void adj_point_wide(const AdjRec &P, double s, const float *tab, float &S, float &SU, float &ST,
+                                      float &SP)
+{
+    const VoigtP vp = P.vp;
+    const double qs = P.qs;
+    const float a2 = P.a2;
+    GradSums g;
+#pragma unroll 1
+    for (int j = -3; j <= 3; ++j) g.add<true, true>(vp, a2, P.W[j < 0 ? -j : j], sample_us(qs, j, s), tab);
+    g.finish(vp, a2, S, SU, ST, SP);
+}
+
 // Bound: VALU issue (32 instructions a sample in the short form).  Structured as
 // tau_kernel: pairs set up one per lane into records, walked in place by lane
 // groups, pairs of the short and of the full form in runs, far-wing pixels by the
@@ -1549,10 +1602,11 @@ __device__ inline void adj_point(const AdjRec &P, double s, const float *tab, fl
 // pixels, each once, weighted by the trapezoid weights and dL/dtau of the
 // pixels it belongs to.  One block of 16 wavefronts a CU shares the table of G
 // and K (32 KB) and the row.  kRow: the row of dL/dtau in LDS; a row that does
-// not fit beside the records (above about 3000 pixels) is read where it is.
+// not fit beside the records (above about 3000 pixels) is read where it is.  kWide:
+// the pass over the wide pairs, where a first pass met some.
 // 2.1M particles, 1024 sightlines of 1024 pixels, forward and adjoint: 37.9 -> 15.9
 // ms.
-template <int kG, bool kRow>
+template <int kG, bool kRow, bool kWide>
 __global__ __launch_bounds__(kAdjThreads) __attribute__((amdgpu_waves_per_eu(4))) void tau_adjoint_kernel(
     DepositArgs A, const WorkItem *items)
 {
@@ -1601,7 +1655,7 @@ __global__ __launch_bounds__(kAdjThreads) __attribute__((amdgpu_waves_per_eu(4))
                     int want = pairs_wanted((long long)w.p1 - (long long)__atomic_load_n(&s_next, __ATOMIC_RELAXED),
                                             kAdjWaves, kGroupsPerWave, __popc(free));
                     want = __builtin_amdgcn_readfirstlane(want < 1 ? 1 : want);
-                    refill_adjoint(A, w, item, L, los, &s_next, recs, lane, want, free, light, full, more);
+                    refill_adjoint<kWide>(A, w, item, L, los, &s_next, recs, lane, want, free, light, full, more);
                 }
                 if ((take_full ? full : light) == 0) take_full = !take_full;
                 for (unsigned long long nm = needing; nm && (light | full); nm &= nm - 1ull) {
@@ -1636,7 +1690,9 @@ __global__ __launch_bounds__(kAdjThreads) __attribute__((amdgpu_waves_per_eu(4))
                 const double dss = P.dss;
                 const double s = __builtin_fma((double)P.nfl * (nm1 == 0 ? 1 : nm1) + m + (nm1 == 0 ? 0.5 : 0.0), dss, P.s0);
                 float S, SU, ST, SP;
-                if (any_full)
+                if (kWide)
+                    adj_point_wide(P, s, tab, S, SU, ST, SP);
+                else if (any_full)
                     adj_point<true>(P, s, tab, S, SU, ST, SP);
                 else
                     adj_point<false>(P, s, tab, S, SU, ST, SP);
@@ -1764,24 +1820,25 @@ int launch_tau_adjoint64(const DepositArgs &A, const WorkItem *items, int nblock
 // Whether the adjoint keeps its row in LDS beside its records and table.
 bool adjoint_row_in_lds(int nbins) { return deposit_lds_bytes(nbins) + adjoint_static_lds(16) <= 160 * 1024; }
 
-template <int kG, bool kRow>
+template <int kG, bool kRow, bool kWide>
 static int launch_adjoint(const DepositArgs &A, const WorkItem *items, int nblocks, hipStream_t s)
 {
     const size_t shm = kRow ? deposit_lds_bytes(A.nbins) : 0;
-    if (int rc = raise_lds_limit((const void *)tau_adjoint_kernel<kG, kRow>, shm)) return rc;
-    tau_adjoint_kernel<kG, kRow><<<nblocks, kAdjThreads, shm, s>>>(A, items);
+    if (int rc = raise_lds_limit((const void *)tau_adjoint_kernel<kG, kRow, kWide>, shm)) return rc;
+    tau_adjoint_kernel<kG, kRow, kWide><<<nblocks, kAdjThreads, shm, s>>>(A, items);
     FSAMD_HIP(hipGetLastError());
     return FSAMD_OK;
 }
 
-int launch_tau_adjoint(int gsize, const DepositArgs &A, const WorkItem *items, int nblocks, hipStream_t s)
+int launch_tau_adjoint(int gsize, bool wide, const DepositArgs &A, const WorkItem *items, int nblocks, hipStream_t s)
 {
+    if (wide) return launch_adjoint<16, false, true>(A, items, nblocks, s);
     const bool row = adjoint_row_in_lds(A.nbins);
     if (gsize == 16)
-        return row ? launch_adjoint<16, true>(A, items, nblocks, s) : launch_adjoint<16, false>(A, items, nblocks, s);
+        return row ? launch_adjoint<16, true, false>(A, items, nblocks, s) : launch_adjoint<16, false, false>(A, items, nblocks, s);
     if (gsize == 32)
-        return row ? launch_adjoint<32, true>(A, items, nblocks, s) : launch_adjoint<32, false>(A, items, nblocks, s);
-    return row ? launch_adjoint<64, true>(A, items, nblocks, s) : launch_adjoint<64, false>(A, items, nblocks, s);
+        return row ? launch_adjoint<32, true, false>(A, items, nblocks, s) : launch_adjoint<32, false, false>(A, items, nblocks, s);
+    return row ? launch_adjoint<64, true, false>(A, items, nblocks, s) : launch_adjoint<64, false, false>(A, items, nblocks, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -2100,8 +2157,8 @@ size_t deposit_static_lds(bool tau, int gsize, int waves)
 
 size_t adjoint_static_lds(int gsize)
 {
-    return static_lds(gsize == 16 ? (const void *)tau_adjoint_kernel<16, true>
-                      : gsize == 32 ? (const void *)tau_adjoint_kernel<32, true> : (const void *)tau_adjoint_kernel<64, true>);
+    return static_lds(gsize == 16 ? (const void *)tau_adjoint_kernel<16, true, false>
+                      : gsize == 32 ? (const void *)tau_adjoint_kernel<32, true, false> : (const void *)tau_adjoint_kernel<64, true, false>);
 }
 
 int raise_lds_limit(const void *fn, size_t shm)

@@ -93,6 +93,10 @@ __device__ inline double voigt_uscale(const VoigtP &v, double a)
 
 // Largest |u| whose t lies in the table, and the floats the table takes.
 constexpr double kVoigtUMax = 2.3e4;
+// Beyond it (the wide forms below) G = -1/(2u^2), exact to 3e-9, up to where u^4 a^4
+// leaves the range of FP32 numbers.
+constexpr float kVoigtTMax = (float)(2ull << FSAMD_P_OCTAVES);
+constexpr double kVoigtUWide = 1e8;
 constexpr int kPTableSize = FSAMD_P_OCTAVES * FSAMD_P_BINS * 4;
 static_assert(FSAMD_P_BINS == 32 && kUScale * kUScale * kVoigtUMax * kVoigtUMax + 2.0 < (double)(2ull << FSAMD_P_OCTAVES),
               "profile_table.h");
@@ -104,8 +108,9 @@ static_assert(FSAMD_P_OCTAVES == 32, "a row for every value of the five exponent
 // mantissa's first 5 bits and exponent name the row, its remaining bits are
 // the cubic's variable.  14 VALU instructions and one 16-byte LDS read a
 // sample in the light form (kA3 = false; 22 and two reads with a table in u and
-// a selected wing row), 22 in the full one (35).
-template <bool kA3 = true>
+// a selected wing row), 22 in the full one (35).  kWide: any |u| <= kVoigtUWide, with
+// the same values in the table's range.
+template <bool kA3 = true, bool kWide = false>
 __device__ inline void voigt_terms(const VoigtP &v, float us, const float *tab, float &E, float &G)
 {
     const float t = __builtin_fmaf(us, us, 2.0f);
@@ -119,6 +124,7 @@ __device__ inline void voigt_terms(const VoigtP &v, float us, const float *tab, 
     const float d = t - __uint_as_float(edge);
     const float4 c = *(const float4 *)((const char *)tab + __builtin_amdgcn_ubfe(edge, 14, 14));
     G = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(c.w, d, c.z), d, c.y), d, c.x);
+    if (kWide && t >= kVoigtTMax) G = -8.0f * __builtin_amdgcn_rcpf(t);
     if (kA3) {
         // -(a^2/6) D''': (4u^2 - 6) G + 2 loses its digits as 1/u^4, where G -> -1/(2u^2)
         const float D = t > 6402.0f ? G * (G * -12.0f) : __builtin_fmaf(__builtin_fmaf(t, 0.25f, -6.5f), G, 2.0f);
@@ -167,8 +173,8 @@ struct GradSums {
     float cD = 0;                                           // w D'''
     float uT = 0, pT = 0;                                   // full form: w u' C T, w u'^2 C T
 
-    // tab: 8 floats a row, G's cubic and K's
-    template <bool kFull>
+    // tab: 8 floats a row, G's cubic and K's.  kWide: as in voigt_terms.
+    template <bool kFull, bool kWide = false>
     __device__ inline void add(const VoigtP &v, float a2, float w, float us, const float *tab)
     {
         const float t = __builtin_fmaf(us, us, 2.0f);
@@ -184,6 +190,10 @@ struct GradSums {
         const float4 g = row[0], k = row[1];
         float G = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(g.w, d, g.z), d, g.y), d, g.x);
         float K = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(k.w, d, k.z), d, k.y), d, k.x);
+        if (kWide && t >= kVoigtTMax) {
+            G = -8.0f * __builtin_amdgcn_rcpf(t);
+            K = (2.0f * kKScale * G) * G;
+        }
         const float wC = w * C, xC = us * wC;
         const bool far = t > 6402.0f;
         float D = __builtin_fmaf(__builtin_fmaf(t, 0.25f, -6.5f), G, 2.0f);

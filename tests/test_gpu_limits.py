@@ -3,9 +3,9 @@ import numpy as np
 import pytest
 import torch
 
-from fake_spectra_amd import spectra_priv as SP, synth
+from fake_spectra_amd import _native as N, spectra_priv as SP, synth
 from fake_spectra_amd.lines import HI_1215
-from gpu_util import dev
+from gpu_util import assert_tau_close, dev
 from test_gpu_edges import small_gas
 from torch_reference import BOLTZMANN, LIGHT, PROTONMASS, SIGMA_T, kernel_weight
 
@@ -166,3 +166,58 @@ def test_saturated_gradients_keep_the_cubic_term(a, support, peak):
     density, temperature = (np.concatenate(e) for e in errs)
     assert density.size > 200
     assert np.median(density) <= 2.0 ** -23 and np.median(temperature) <= 1e-5
+
+
+def fp64_pairs(call):
+    """A tau call's result and the pairs it walked in FP64."""
+    N.check(N.lib().fsamd_set_stats(1))
+    try:
+        out = call()
+        st = SP.last_stats()
+    finally:
+        N.check(N.lib().fsamd_set_stats(0))
+    assert st["pairs"] > 0
+    return out, st["fp64_pairs"]
+
+
+# supports whose samples leave the profile's table (near 7600 Doppler widths), by
+# little and by much
+@pytest.mark.parametrize("kernel", [0, 1])
+@pytest.mark.parametrize("support", [7600, 8000, 30000])
+def test_far_wing_beyond_the_profile_table(support, kernel):
+    lone = LoneParticle(support, kernel, 1e-2)
+    assert fp64_pairs(lambda: SP.tau(lone.plan, *lone.args))[1] == 0
+    lone.check()
+
+
+# and beside narrow supports of the same rows; light and full profiles
+@pytest.mark.parametrize("group", [16, 64])
+@pytest.mark.parametrize("kernel", [0, 1, 3])
+@pytest.mark.parametrize("a", [1e-4, 1e-2])
+def test_supports_beyond_the_profile_table(oracle, a, kernel, group):
+    n, nlos, nbins = 120, 6, 3000
+    args = list(small_gas(n, 60000.0 / VELFAC, nlos, nbins, kernel, 0.02))
+    args[14][:] = 1e4 * (30.0 / 12.85) ** 2
+    args[14][::4] = 1e4 * (1.0 / 12.85) ** 2             # b = 1 km/s, pixels of 20
+    args[15][::8] = 12000.0 / VELFAC
+    args[7] = a * 4 * np.pi * 1e5 / HI_1215.lambda_cm     # a at b = 1 km/s
+    args[13] = (args[13] * 1e6).astype(np.float32)
+    plan = SP.Plan(args[3], dev(args[11]), dev(args[15]), dev(args[16]), dev(args[17]))
+    call = (nbins, kernel, VELFAC, dev(args[12]), dev(args[14]), [tuple(args[6:10])], [dev(args[13])])
+    N.set_group_size(group)
+    try:
+        plan.keep_windows(True)
+        got, handed = fp64_pairs(lambda: SP.tau(plan, *call)[0])
+        weights = torch.exp(-1e-6 * got) + 0.5
+        grads = SP.tau_adjoint(plan, *call, [weights])
+        SP.set_fp64(True)
+        SP.tau(plan, *call)
+        want = SP.tau_adjoint(plan, *call, [weights])
+    finally:
+        SP.set_fp64(False)
+        N.set_group_size(16)
+    assert handed == 0
+    assert_tau_close(got.cpu().numpy(), oracle.interpolate(*args), "wide supports")
+    for x, y in zip((grads[0][0], grads[1], grads[2]), (want[0][0], want[1], want[2])):
+        assert float((x - y).abs().max()) <= 1e-5 * float(y.abs().max())
+    plan.close()
