@@ -59,11 +59,20 @@ static void line_consts(const fsamd_line &l, LineDesc &d)
     d.out = l.out;
 }
 
-static bool find_item_set(const fsamd_plan *P, int K, long long chunk, int slots, long long unit)
+static fsamd_plan::ItemSet *find_item_set(const fsamd_plan *P, int K, long long chunk, int slots, long long unit)
 {
     for (auto &it : P->item_sets)
-        if (it->K == K && it->chunk == chunk && it->slots == slots && it->unit == unit) return true;
-    return false;
+        if (it->K == K && it->chunk == chunk && it->slots == slots && it->unit == unit) return it.get();
+    return nullptr;
+}
+
+// A set of the same sightlines for K lines (or parts of the fields), cut up for
+// whatever launch shape: every launch can work from it.
+static fsamd_plan::ItemSet *any_item_set(const fsamd_plan *P, int K, long long chunk)
+{
+    for (auto &it : P->item_sets)
+        if (it->K == K && it->chunk == chunk) return it.get();
+    return nullptr;
 }
 
 static long long tune_key(int nbins, int nlines, int kernel)
@@ -92,11 +101,7 @@ constexpr int kAdjointMaxBins = 19536;
 // 3.4 -> 1.2 ms).  Cached.
 static int item_set(fsamd_plan *P, int K, long long chunk, int slots, long long unit, fsamd_plan::ItemSet **out)
 {
-    for (auto &it : P->item_sets)
-        if (it->K == K && it->chunk == chunk && it->slots == slots && it->unit == unit) {
-            *out = it.get();
-            return FSAMD_OK;
-        }
+    if ((*out = find_item_set(P, K, chunk, slots, unit))) return FSAMD_OK;
     auto set = std::make_unique<fsamd_plan::ItemSet>();
     set->K = K;
     set->chunk = chunk;
@@ -325,9 +330,16 @@ static int run_deposit(bool tau, fsamd_plan *P, int nbins, int kernel, double ve
                                                                       nbins, A.fields);
         const long long unit = tau ? kTauPart : kColdenPart;
         fsamd_plan::ItemSet *set = nullptr;
-        if (capturing && !find_item_set(P, parts, chunk_key, slots, unit))
-            return fail(FSAMD_ERR_ARG, "run one uncaptured fsamd_tau call before capturing");
-        if ((rc = item_set(P, parts, chunk_key, slots, unit, &set))) return rc;
+        if (capturing) {
+            // a capture cannot allocate: where the eager call was of another launch
+            // shape, or of the optical depth (one line an item), its items serve
+            set = find_item_set(P, parts, chunk_key, slots, unit);
+            if (!set) set = any_item_set(P, parts, chunk_key);
+            if (!set && (set = any_item_set(P, K, chunk_key))) A.fields = 1;
+            if (!set) return fail(FSAMD_ERR_ARG, "run one uncaptured fsamd_tau call before capturing");
+        } else if ((rc = item_set(P, parts, chunk_key, slots, unit, &set))) {
+            return rc;
+        }
         const std::vector<WorkItem> &items = set->host;
         for (int attempt = 0;; ++attempt) {
             A.fix = P->fix.as<Fixup>();

@@ -221,3 +221,85 @@ def test_supports_beyond_the_profile_table(oracle, a, kernel, group):
     for x, y in zip((grads[0][0], grads[1], grads[2]), (want[0][0], want[1], want[2])):
         assert float((x - y).abs().max()) <= 1e-5 * float(y.abs().max())
     plan.close()
+
+
+def replays_match(graph, outs, again):
+    """Three replays, each against an eager call (into tensors of its own) in
+    the shape that was captured."""
+    for _ in range(3):
+        for o in outs:
+            o.fill_(-1.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for o, e in zip(outs, again()):
+            assert torch.allclose(o, e, rtol=1e-12, atol=0)
+
+
+def test_capture_in_another_launch_shape():
+    """One uncaptured call with the same plan, lines and sizes is all that a
+    capture needs, whatever lane-group width and wavefronts it then uses."""
+    args = small_gas(4000, 900.0, 12, 256, 1, 0.1)
+    plan = SP.Plan(args[3], dev(args[11]), dev(args[15]), dev(args[16]), dev(args[17]))
+    call = (dev(args[12]), dev(args[14]), [HI_1215], [dev(args[13])])
+    outs = SP.tau(plan, 256, 1, VELFAC, *call)
+    eager = outs[0].cpu().numpy().copy()
+    graphs = []
+    try:
+        for group, waves in ((64, 4), (32, 2), (16, 8)):
+            N.set_group_size(group)
+            N.set_block_waves(waves)
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                SP.tau(plan, 256, 1, VELFAC, *call, out=outs)
+            graphs.append((group, waves, graph))
+        for group, waves, graph in graphs:
+            N.set_group_size(group)
+            N.set_block_waves(waves)
+            replays_match(graph, outs, lambda: SP.tau(plan, 256, 1, VELFAC, *call))
+            assert_tau_close(outs[0].cpu().numpy(), eager, "captured")
+    finally:
+        N.set_group_size(16)
+        N.set_block_waves(8)
+
+
+def test_capture_after_autotune():
+    """Many sightlines, of which the autotuner times every second one; the
+    width it chose is captured after an eager call of another shape."""
+    nlos, nbins = 33000, 16
+    args = small_gas(300, 900.0, nlos, nbins, 1, 0.02)
+    plan = SP.Plan(args[3], dev(args[11]), dev(args[15]), dev(args[16]), dev(args[17]))
+    call = (dev(args[12]), dev(args[14]), [HI_1215], [dev(args[13])])
+    SP.autotune(plan, nbins, 1, VELFAC, *call)
+    N.check(N.lib().fsamd_set_stats(1))                  # 4 wavefronts, with counters
+    try:
+        outs = SP.tau(plan, nbins, 1, VELFAC, *call)
+    finally:
+        N.check(N.lib().fsamd_set_stats(0))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        SP.tau(plan, nbins, 1, VELFAC, *call, out=outs)
+    replays_match(graph, outs, lambda: SP.tau(plan, nbins, 1, VELFAC, *call))
+
+
+def test_capture_of_column_density_after_tau():
+    """The eager call with the same lines may be the other of the two."""
+    args = small_gas(3000, 900.0, 9, 300, 1, 0.1)
+    plan = SP.Plan(args[3], dev(args[11]), dev(args[15]), dev(args[16]), dev(args[17]))
+    vel, temp = dev(args[12]), dev(args[14])
+    dens = [dev(args[13]), dev((args[13] * 2).astype(np.float32)), dev((args[13] * 3).astype(np.float32))]
+    want = [o.clone() for o in SP.colden(plan, 300, 1, VELFAC, dens)]
+    plan.close()
+    plan = SP.Plan(args[3], dev(args[11]), dev(args[15]), dev(args[16]), dev(args[17]))
+    outs = [torch.empty((9, 300), dtype=torch.float64, device="cuda") for _ in dens]
+    quad = (HI_1215.lambda_cm, HI_1215.gamma, HI_1215.fosc, HI_1215.amumass)
+    SP.tau(plan, 300, 1, VELFAC, vel, temp, [quad] * 3, dens, out=outs)
+    torch.cuda.synchronize()
+    arr = SP._line_structs([quad] * 3, dens, outs)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        N.check(N.lib().fsamd_colden(plan.handle, 300, 1, VELFAC, SP._ptr(plan.pos), SP._ptr(plan.h), arr, 3,
+                                     SP._stream()))
+    replays_match(graph, outs, lambda: want)
