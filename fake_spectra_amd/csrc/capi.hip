@@ -87,8 +87,12 @@ static long long tune_key(int nbins, int nlines, int kernel)
 constexpr long long kTauPart = 128;
 constexpr long long kAdjointPart = 256;
 constexpr long long kColdenPart = kColThreads;
-// Longest row fsamd_tau_adjoint takes.
-constexpr int kAdjointMaxBins = 19536;
+// Longest row fsamd_tau_adjoint takes.  The kernel reads a row that does not fit LDS
+// where it is, so nothing in it needs a limit: these are the rows the entry has
+// always taken and refused, those that fitted a CU's LDS beside a 1408-byte table and
+// the 384-byte pair slots of a block's 256 / g lane groups (19536, 19920 and 20112
+// pixels for g = 16, 32 and 64).
+static int adjoint_max_bins(int g) { return (160 * 1024 - 1408 - 384 * (256 / g)) / (int)sizeof(double); }
 
 // Work items for K lines (or parts of the fields) in the plan's heaviest-first
 // order; a sightline with more than `chunk` pairs is split into non-direct
@@ -726,8 +730,9 @@ int fsamd_tau_adjoint(fsamd_plan *P, int nbins, int kernel, double velfac, const
     static thread_local DeviceInfo dev;
     int rc;
     if (dev.ncu == 0 && (rc = device_info(dev))) return rc;
-    if (nbins > kAdjointMaxBins)
-        return fail(FSAMD_ERR_UNSUPPORTED, "the adjoint takes rows of at most " + std::to_string(kAdjointMaxBins) +
+    const int gsize = g_group_size.load(std::memory_order_relaxed);
+    if (nbins > adjoint_max_bins(gsize))
+        return fail(FSAMD_ERR_UNSUPPORTED, "the adjoint takes rows of at most " + std::to_string(adjoint_max_bins(gsize)) +
                                                " pixels (nbins too large)");
     std::vector<LineDesc> ld(nlines);
     for (int i = 0; i < nlines; ++i) {
@@ -753,7 +758,6 @@ int fsamd_tau_adjoint(fsamd_plan *P, int nbins, int kernel, double velfac, const
     // the list of pairs for the FP64 adjoint kernel (the forward's fix-up list)
     if (!P->fix_count.ptr && (rc = P->fix_count.alloc(sizeof(unsigned long long) * 2, P->arena))) return rc;
     if (P->fix_cap < 65536 && (rc = grow_fixups(P, 65536, s))) return rc;
-    const int gsize = g_group_size.load(std::memory_order_relaxed);
     for (int g = 0; g < ngroups; ++g) {
         const int k0 = g * kMaxLines;
         const int K = std::min(kMaxLines, nlines - k0);

@@ -303,3 +303,31 @@ def test_capture_of_column_density_after_tau():
         N.check(N.lib().fsamd_colden(plan.handle, 300, 1, VELFAC, SP._ptr(plan.pos), SP._ptr(plan.h), arr, 3,
                                      SP._stream()))
     replays_match(graph, outs, lambda: want)
+
+
+# the longest rows of each lane-group width, and one pixel more
+@pytest.mark.parametrize("group,most", [(16, 19536), (32, 19920), (64, 20112)])
+def test_longest_adjoint_rows(group, most):
+    args = small_gas(30, 700.0, 2, most, 1, 0.2)
+    plan = SP.Plan(args[3], dev(args[11]), dev(args[15]), dev(args[16]), dev(args[17]))
+    plan.keep_windows(True)
+    call = (dev(args[12]), dev(args[14]), [tuple(args[6:10])], [dev(args[13])])
+    weights = dev(np.random.default_rng(4).standard_normal((2, most)))
+    grads = []
+    N.set_group_size(group)
+    try:
+        for fp64 in (False, True):
+            SP.set_fp64(fp64)
+            SP.tau(plan, most, 1, VELFAC, *call)
+            gd, gt, gv = SP.tau_adjoint(plan, most, 1, VELFAC, *call, [weights])
+            grads.append((gd[0], gt, gv))
+        SP.set_fp64(False)
+        t = SP.tau(plan, most + 1, 1, VELFAC, *call)[0]
+        with pytest.raises(Exception, match="nbins too large"):
+            SP.tau_adjoint(plan, most + 1, 1, VELFAC, *call, [t])
+    finally:
+        SP.set_fp64(False)
+        N.set_group_size(16)
+    for x, y in zip(*grads):
+        assert float((x - y).abs().max()) <= 1e-5 * float(y.abs().max())
+    plan.close()
