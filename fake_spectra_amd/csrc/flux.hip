@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <numeric>
 #include <type_traits>
 #include <vector>
 
@@ -89,6 +90,13 @@ constexpr int kMoments = 12;
 constexpr int kSums = kMoments + 3;
 constexpr int kMomentBlocks = 1536;   // 6 blocks a CU
 constexpr int kMomentBatch = 2;       // pixels a thread loads before the first is used
+// Pixels a thread has at least: a block's 15 sums over its threads cost as much as
+// some 16 pixels (600000 pixels, Newton steps that each need a pass: 156 us a call
+// with one, 121 with 8 and 16, 132 with 32; 3M 163, 163, 142 and 144; with three
+// sums a pass it was 130 and 144).
+constexpr int kMomentPixels = 16;
+// Blocks whose sums the host adds up, a launch less a pass (1000 pixels 108 -> 100 us).
+constexpr int kMomentFew = 32;
 
 __global__ __launch_bounds__(kFluxThreads) void flux_moments_kernel(const double *tau, long long n, double scale,
                                                                    double thresh, double *partial)
@@ -775,7 +783,10 @@ int fsamd_mean_flux_scale(const double *tau, long long n, double mean_flux_desir
         return FSAMD_OK;
     }
     hipStream_t s = (hipStream_t)stream;
-    const int nblocks = (int)std::min<long long>(kMomentBlocks, (n + kFluxThreads - 1) / kFluxThreads);
+    constexpr long long kBlockPixels = (long long)kFluxThreads * kMomentPixels;
+    const int nblocks = (int)std::min<long long>(kMomentBlocks, (n + kBlockPixels - 1) / kBlockPixels);
+    const bool few = nblocks <= kMomentFew;
+    double host[kSums * kMomentFew];
     double *partial = nullptr;
     FSAMD_HIP(hipMalloc(&partial, sizeof(double) * kSums * (nblocks + 1)));
     double *total = partial + (size_t)kSums * nblocks;
@@ -786,14 +797,18 @@ int fsamd_mean_flux_scale(const double *tau, long long n, double mean_flux_desir
         double F, G;
         if (it == 0 || !taylor_step(sum, centre, scale, mean_flux_desired * sum[kMoments + 1], F, G)) {
             flux_moments_kernel<<<nblocks, kFluxThreads, 0, s>>>(tau, n, scale, thresh, partial);
-            row_sum_kernel<<<kSums, kFluxThreads, 0, s>>>(partial, nblocks, total);
+            if (!few) row_sum_kernel<<<kSums, kFluxThreads, 0, s>>>(partial, nblocks, total);
             hipError_t e = hipGetLastError();
-            if (e == hipSuccess) e = hipMemcpyAsync(sum, total, sizeof(sum), hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess)
+                e = hipMemcpyAsync(few ? host : sum, few ? partial : total, sizeof(double) * kSums * (few ? nblocks : 1),
+                                   hipMemcpyDeviceToHost, s);
             if (e == hipSuccess) e = hipStreamSynchronize(s);
             if (e != hipSuccess) {
                 rc = fail(FSAMD_ERR_HIP, std::string("flux moments: ") + hipGetErrorString(e));
                 break;
             }
+            for (int j = 0; few && j < kSums; ++j)
+                sum[j] = std::accumulate(host + j * nblocks, host + (j + 1) * nblocks, 0.0);
             centre = scale;
             F = sum[0];
             G = sum[1];

@@ -331,3 +331,14 @@ def test_longest_adjoint_rows(group, most):
     for x, y in zip(*grads):
         assert float((x - y).abs().max()) <= 1e-5 * float(y.abs().max())
     plan.close()
+
+
+# blocks of 4096 pixels, whose sums the host adds up where they are at most 32
+@pytest.mark.parametrize("n", [4096, 4097, 32 * 4096, 32 * 4096 + 1, 1536 * 4096 + 1])
+def test_mean_flux_of_few_and_many_blocks(n):
+    import fluxstats as FS
+    from fake_spectra_amd import fluxstatistics as GF
+    t = np.exp(2.0 * np.random.default_rng(n).standard_normal(n))
+    for target in (0.5, 0.95):
+        got, ref = GF.mean_flux(dev(t), target, 1e-10), FS.mean_flux_scale(t, target, 1e-10)
+        assert abs(got - ref) <= 1e-10 * ref      # the tolerance of the iteration
