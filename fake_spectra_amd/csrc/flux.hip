@@ -204,14 +204,19 @@ struct ResTile {
     int stride;                 // of a staged row, a multiple of kResOut
 };
 
-static ResTile res_tile(int ncol, int nw)
+// Parts a call has at least before short rows share a block: fewer than fill the
+// chip, they would only wait for each other (1000 rows of 50, 1 and 9 taps: 21.7 and
+// 22.3 us a call with 19 rows a block, 20.8 and 21.2 so).
+constexpr int kResParts = 512;
+
+static ResTile res_tile(int nrow, int ncol, int nw)
 {
     ResTile t;
     t.cols = std::min(ncol, kResCols);
     t.nchunk = (ncol + t.cols - 1) / t.cols;
     t.stride = (t.cols + kResOut - 1) / kResOut * kResOut + (std::min(nw, kResTaps) + kResOut) / kResOut * kResOut;
     const int groups = (t.cols + kResOut - 1) / kResOut;
-    t.rows = std::max(1, std::min(kFluxThreads / groups, kResLds / t.stride));
+    t.rows = std::max(1, std::min(std::min(kFluxThreads / groups, kResLds / t.stride), nrow / kResParts));
     return t;
 }
 
@@ -842,7 +847,7 @@ int fsamd_res_corr(const double *in, double *out, int nrow, int ncol, double sig
     FSAMD_HIP(hipMalloc(&dw, sizeof(double) * w.size()));
     hipError_t e = hipMemcpyAsync(dw, w.data(), sizeof(double) * w.size(), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
-        const ResTile t = res_tile(ncol, 2 * r + 1);
+        const ResTile t = res_tile(nrow, ncol, 2 * r + 1);
         const long long nparts = ((long long)nrow + t.rows - 1) / t.rows * t.nchunk;
         const size_t shm = sizeof(double) * ((size_t)t.rows * t.stride + (std::min(2 * r + 1, kResTaps) + 1) / 2 * 2);
         res_corr_kernel<<<(int)std::min<long long>(nparts, 4096), kFluxThreads, shm, s>>>(in, out, nrow, ncol, dw,

@@ -342,3 +342,18 @@ def test_mean_flux_of_few_and_many_blocks(n):
     for target in (0.5, 0.95):
         got, ref = GF.mean_flux(dev(t), target, 1e-10), FS.mean_flux_scale(t, target, 1e-10)
         assert abs(got - ref) <= 1e-10 * ref      # the tolerance of the iteration
+
+
+# rows of their own block, and short rows that share one from 1024 rows on, with a
+# remainder and none
+@pytest.mark.parametrize("nrow,ncol", [(1023, 5), (1024, 5), (1025, 50), (20001, 7), (40000, 3), (1600, 300)])
+@pytest.mark.parametrize("sigma", [0.1, 1.04, 31.9])
+def test_smoothing_of_rows_that_share_a_block(nrow, ncol, sigma):
+    """A weighted mean of nw pixels: eps sqrt(nw) of the largest, with 4 ulp for
+    the weights."""
+    import fluxstats as FS
+    from fake_spectra_amd import fluxstatistics as GF
+    x = np.random.default_rng(ncol).random((nrow, ncol))
+    dvbin = 8 / (2 * np.sqrt(2 * np.log(2))) / sigma
+    got = GF.res_corr(dev(x), dvbin, 8).cpu().numpy()
+    assert np.max(np.abs(got - FS.res_corr(x, dvbin, 8))) <= 2.3e-16 * (4 + np.sqrt(8 * sigma + 1)) * 2
