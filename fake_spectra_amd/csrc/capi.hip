@@ -789,7 +789,7 @@ int fsamd_tau_adjoint(fsamd_plan *P, int nbins, int kernel, double velfac, const
         A.grad_temp = grad_temp;
         A.grad_vel = grad_vel;
         fsamd_plan::ItemSet *set = nullptr;
-        const int slots = dev.ncu;
+        const int slots = dev.ncu;   // one block of the adjoint kernel fills a CU
         if ((rc = item_set(P, K, 1ll << 62, slots, kAdjointPart, &set))) return rc;
         if (set->host.empty()) continue;
         A.nitems = (int)set->host.size();

@@ -21,9 +21,8 @@ constexpr int kColThreads = 512;   // threads of a column-density block
 size_t deposit_lds_bytes(int nbins);
 // LDS a deposit kernel declares itself (queues, per-group state, tables):
 // the tau kernel at group width gsize and `waves` wavefronts per block, or
-// the column-density kernel; the adjoint kernel at group width gsize.
+// the column-density kernel.
 size_t deposit_static_lds(bool tau, int gsize, int waves);
-size_t adjoint_static_lds(int gsize);
 int launch_deposit(bool tau, bool lds, int gsize, int waves, const DepositArgs &A, const WorkItem *items, int item_base,
                    int nblocks, int use_queue, hipStream_t s);
 // fields: rows a column-density block holds (1 for tau)
@@ -33,8 +32,6 @@ int colden_fields(int nlines, int nbins);
 int effective_waves(bool lds, bool stats, int waves);
 // wide: the pass over the pairs that the other one left out (fix_count[1] & 2)
 int launch_tau_adjoint(int gsize, bool wide, const DepositArgs &A, const WorkItem *items, int nblocks, hipStream_t s);
-// one block of the adjoint kernel fills a CU
-bool adjoint_row_in_lds(int nbins);
 // the FP64 pairs tau_adjoint_kernel listed in A.fix (after it, on the same stream)
 int launch_tau_adjoint64(const DepositArgs &A, const WorkItem *items, int nblocks, hipStream_t s);
 int launch_tau_fixup(const DepositArgs &A, const WorkItem *items, int nblocks, hipStream_t s);

@@ -15,9 +15,11 @@
 //    pulls items heaviest-first from a queue; the row of the sightline lives
 //    in LDS as float64 and is flushed with coalesced stores (or FP64 atomics
 //    when a sightline's pairs are split across several items);
-//  * a wavefront handles one pair at a time with lanes on consecutive pixels;
-//    the sequential tail cut becomes a ballot: the first lane whose taulast
-//    falls below tautail ends the walk, lanes up to it deposit;
+//  * a wavefront sets up to 32 pairs up, one per lane, and its groups of 16 (32,
+//    64) lanes each walk one of them, lanes on consecutive pixels; the
+//    sequential tail cut becomes a ballot: the first lane whose taulast falls
+//    below tautail ends the walk, lanes up to it deposit.  A walk that reaches
+//    the far wing goes on by the whole wavefront, 64 pixels at a time;
 //  * the mapping position -> velocity -> pixel, the pixel and sub-sample
 //    offsets and the accumulation are FP64, as in the reference; the kernel
 //    weights and the Voigt profile are FP32 (voigt.h);
@@ -222,8 +224,6 @@ struct PairTau : PairRec {
     int fp64, wide;
     int np;          // sub-samples per pixel (1 = midpoint)
     int wing_ready;  // Cw computed
-    double inv_nm1;  // 1 / (np - 1)
-    double dv;       // sub-sample spacing bintov / (np - 1)
 };
 
 // u times its scale, u = (vv_i - vouter)/b of the kernel sample i - 3 = j from the
@@ -672,8 +672,6 @@ __device__ inline bool setup_pair(const DepositArgs &A, int line, const LineDesc
         P.ibs = voigt_uscale(P.vp, C.fp64 ? 0.0 : C.aa) * C.inv_b;
         P.qs = 0.25 * C.vhigh * P.ibs;
         P.wing_ready = 0;
-        P.inv_nm1 = C.np > 1 ? 1.0 / (C.np - 1) : 1.0;
-        P.dv = C.np > 1 ? bintov * P.inv_nm1 : 0.0;
     }
     wave_sync();
     return true;
@@ -1817,8 +1815,23 @@ int launch_tau_adjoint64(const DepositArgs &A, const WorkItem *items, int nblock
     return FSAMD_OK;
 }
 
-// Whether the adjoint keeps its row in LDS beside its records and table.
-bool adjoint_row_in_lds(int nbins) { return deposit_lds_bytes(nbins) + adjoint_static_lds(16) <= 160 * 1024; }
+// A kernel's static LDS, or a conservative 64 KiB if the runtime cannot say.
+static size_t static_lds(const void *fn)
+{
+    hipFuncAttributes a;
+    if (hipFuncGetAttributes(&a, fn) != hipSuccess) {
+        (void)hipGetLastError();
+        return 65536;
+    }
+    return a.sharedSizeBytes;
+}
+
+// Whether the adjoint keeps its row in LDS beside its records and table, whose
+// size is the same at every group width.
+static bool adjoint_row_in_lds(int nbins)
+{
+    return deposit_lds_bytes(nbins) + static_lds((const void *)tau_adjoint_kernel<16, true, false>) <= 160 * 1024;
+}
 
 template <int kG, bool kRow, bool kWide>
 static int launch_adjoint(const DepositArgs &A, const WorkItem *items, int nblocks, hipStream_t s)
@@ -2127,17 +2140,6 @@ static size_t colden_shm(bool lds, int nbins, int fields)
     return (size_t)fields * (lds ? colden_lds_bytes(nbins) : colden_lds_bytes(0));
 }
 
-// A kernel's static LDS, or a conservative 64 KiB if the runtime cannot say.
-static size_t static_lds(const void *fn)
-{
-    hipFuncAttributes a;
-    if (hipFuncGetAttributes(&a, fn) != hipSuccess) {
-        (void)hipGetLastError();
-        return 65536;
-    }
-    return a.sharedSizeBytes;
-}
-
 template <int kG>
 static size_t tau_static_lds(int waves)
 {
@@ -2153,12 +2155,6 @@ size_t deposit_static_lds(bool tau, int gsize, int waves)
     // (column density: with the densities of one field)
     if (!tau) return static_lds((const void *)colden_kernel<true>) + colden_lds_bytes(0);
     return gsize == 16 ? tau_static_lds<16>(waves) : gsize == 32 ? tau_static_lds<32>(waves) : tau_static_lds<64>(waves);
-}
-
-size_t adjoint_static_lds(int gsize)
-{
-    return static_lds(gsize == 16 ? (const void *)tau_adjoint_kernel<16, true, false>
-                      : gsize == 32 ? (const void *)tau_adjoint_kernel<32, true, false> : (const void *)tau_adjoint_kernel<64, true, false>);
 }
 
 int raise_lds_limit(const void *fn, size_t shm)

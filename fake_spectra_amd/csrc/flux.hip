@@ -197,7 +197,7 @@ static bool taylor_step(const double *sum, double c, double z, double target, do
 constexpr int kResOut = 4;
 constexpr int kResCols = kResOut * kFluxThreads;
 constexpr int kResTaps = 256;   // even: only the last stretch of taps has an odd one
-constexpr int kResLds = 2560;   // doubles of short rows in a block: 20 KB, eight blocks a CU
+constexpr int kResLds = 2560;   // doubles of short rows in a block: 20 KB, with the taps seven blocks a CU
 
 struct ResTile {
     int cols, rows, nchunk;     // a block's part: cols columns of rows rows; nchunk parts a row
@@ -729,7 +729,7 @@ __device__ inline int flux_bin(double f, int nb)
 // the two divides a pixel and the 256 copies read by one thread a bin gone; 50
 // bins, one copy before, a call on 20M pixels: 140 -> 105 us; 40000 bins, one
 // copy, on 1e5 pixels 60 -> 48 us.
-constexpr int kHistCounts = 10240;   // 40 KB: four blocks a CU
+constexpr int kHistCounts = 10240;   // 40 KB: with the table of exponentials three blocks a CU at the most copies
 constexpr int kHistBatch = 4;
 
 // kTable: exp by flux_exp's table, where the LDS holds it beside the bins

@@ -1,5 +1,8 @@
 """Generate dawson_table.h: piecewise polynomials for G(u) = 1 - 2u D(u).
 
+No kernel reads this table since profile_table.h took its place; the tests
+of the generated tables still check it against Dawson's integral.
+
 D is Dawson's integral; G(u) is D'(u), the real-axis factor of the first
 term of the Voigt function's expansion in the damping parameter a:
     Re w(u + ia) = exp(a^2 - u^2) cos(2au) - (2/sqrt(pi)) (a G(u) - a^3/6 D'''(u) + ...)

@@ -38,12 +38,10 @@
 namespace fsamd {
 
 constexpr float kA32Max = 0.04f;
-constexpr float kTwoOverSqrtPiF = 1.12837916709551257390f;
 constexpr float kInvSqrtPiF = 0.56418958354775628695f;
 constexpr double kSqrtPi = 1.77245385090551602729;
 constexpr double kTwoOverSqrtPi = 1.12837916709551257390;
 constexpr double kLog2E = 1.44269504088896340736;
-constexpr float kLog2EF = 1.44269504088896340736f;
 
 // Damping parameters up to which the deposit uses the light form of the
 // profile: without the a^3 term and with the Gaussian exponent cut to
