@@ -987,7 +987,11 @@ struct CutBand {
     double lo, hi;
 };
 
-__device__ inline CutBand cut_band(double tautail) { return CutBand{tautail - kGuard * tautail, tautail + kGuard * tautail}; }
+__device__ inline CutBand cut_band(double tautail)
+{
+    const double guard = kGuard * fabs(tautail);
+    return CutBand{tautail - guard, tautail + guard};
+}
 
 // A walk that has reached the far wing, by the whole wavefront, 64 pixels at a
 // time: |U| only grows from there, so this ends the walk.  zf: its next pixel,

@@ -357,3 +357,22 @@ def test_smoothing_of_rows_that_share_a_block(nrow, ncol, sigma):
     dvbin = 8 / (2 * np.sqrt(2 * np.log(2))) / sigma
     got = GF.res_corr(dev(x), dvbin, 8).cpu().numpy()
     assert np.max(np.abs(got - FS.res_corr(x, dvbin, 8))) <= 2.3e-16 * (4 + np.sqrt(8 * sigma + 1)) * 2
+
+
+# a negative cut that the first pixel lies within the guard band of, on either side
+@pytest.mark.parametrize("off", [-1e-5, 1e-5, -1e-3, 1e-3])
+def test_negative_cuts_of_negative_densities(oracle, off):
+    """The walk ends at the first pixel below tautail: with a negative density
+    (the difference of two fields) at once, or where it starts above, never."""
+    args = list(small_gas(1, 900.0, 1, 200, 1, 0.02))
+    args[12][:] = 0.0
+    args[13] *= -1
+    args[17] = args[11].astype(np.float64) + 1.0
+    args[10] = -1e300
+    whole = oracle.interpolate(*args)
+    assert np.all(whole < 0)
+    args[10] = float(whole.min()) * (1.0 + off)
+    ref, got = oracle.interpolate(*args), SP._Particle_Interpolate(*args)
+    assert np.count_nonzero(ref) < 200 if off < 0 else np.array_equal(ref, whole)
+    assert np.array_equal(got == 0, ref == 0)
+    assert np.max(np.abs(got - ref)) <= 1e-5 * np.max(np.abs(ref))
