@@ -503,7 +503,7 @@ __device__ inline bool cell_window(double x, double hr, double inv, int nc, int 
 
 // Supports that reach no sightline: no number, or infinite (los_accept, like the
 // reference's windows, is empty or undefined for them).
-__device__ inline bool finite_support(float hh) { return fabs((double)hh) < 1e300; }
+__device__ inline bool finite_support(float hh) { return __builtin_fabsf(hh) < __builtin_inff(); }
 
 // Visit every sightline accepted for particle p; f(sightline, dr2) returns
 // false to stop the visit early.
@@ -582,9 +582,10 @@ __global__ void bin_emit_kernel(BinArgs A, const long long *poff, int *keys, int
 
 // Whether one of the sightlines of the cell that holds the particle's own
 // point of the plane accepts it, on any axis.
+// (An infinite support is accepted here: finite_support, asked after this in the
+// kernel, costs nothing, and 2.5% of the call where a cell's reads wait for it.)
 __device__ inline bool own_cell_accepts(const BinArgs &A, const float *p, float hh)
 {
-    if (!finite_support(hh)) return false;
     for (int ai = 0; ai < 3; ++ai) {
         if (A.grid.nlos_axis[ai] == 0) continue;
         float first, second;
@@ -632,7 +633,8 @@ __global__ __launch_bounds__(256) void bin_any_kernel(BinArgs A, unsigned long l
             bool any = false;
             if (have) {
                 const float p[3] = {A.pos[3 * i], A.pos[3 * i + 1], A.pos[3 * i + 2]};
-                any = own_cell_accepts(A, p, A.h[i]);
+                const float hh = A.h[i];
+                any = own_cell_accepts(A, p, hh) && finite_support(hh);
             }
             const unsigned long long m = __ballot(any), open = __ballot(have && !any);
             int at = 0;
